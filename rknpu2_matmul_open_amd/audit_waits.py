@@ -173,7 +173,7 @@ def audit_function(name, lines):
     return violations
 
 
-def audit_text(asm_text, only=("gemm_wk_kernel", "gemm_stream_kernel")):
+def audit_text(asm_text, only=("gemm_wk_kernel", "gemm_wk_big_kernel", "gemm_stream_kernel")):
     """Violations in every kernel of an assembly file whose (mangled) name contains one of `only`."""
     violations, checked = [], 0
     lines = asm_text.splitlines()

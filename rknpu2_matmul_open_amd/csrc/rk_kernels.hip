@@ -1390,7 +1390,7 @@ static DensePlan effective_plan(int M, int N, int K, int w_int4) {
     static const char* forced = getenv("RK_NPU_HIP_GEMM_PLAN");
     if (forced) {
         int rows = 0, split = 0;
-        if (sscanf(forced, "%d:%d", &rows, &split) == 2 && (rows == 32 || rows == 64 || rows == 128) && split >= 1) {
+        if (sscanf(forced, "%d:%d", &rows, &split) == 2 && (rows == 32 || rows == 64 || rows == 128 || rows == 256) && split >= 1) {
             plan.bm = rows;
             plan.ksplit = split > min_ksplit(K, w_int4) ? split : min_ksplit(K, w_int4);
         }
@@ -1498,6 +1498,13 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
     return 0;
 }
 
+// Tiles of 256 x 256 (gemm_wk_big_kernel) where there are enough of them and they end sooner than tiles of
+// 128 x 256 would.
+static bool dense_big(const rkh_gemm_args& g) {
+    static const char* plan = getenv("RK_NPU_HIP_GEMM_PLAN"); // (a forced plan is the plan)
+    return !(plan && plan[0]) && min_ksplit(g.K, g.w_int4) == 1 && rkk::wk_big_applies(g.M, g.N, g.K, g.w_int4);
+}
+
 size_t rkh_gemm_scratch_bytes(int M, int N, int K, int w_int4) {
     if (M <= 8) return 0;
     const DensePlan plan = effective_plan(M, N, K, w_int4);
@@ -1514,6 +1521,7 @@ int rkh_gemm(void* stream, const rkh_gemm_args* args) {
     if (grouped) return launch_gemm_grouped(st, g);
     if (dense_streams(g)) return launch_gemm_grouped(st, g);
     if (const int tile_rows = dense_narrow(g)) return launch_gemm_wk_narrow(st, g, tile_rows);
+    if (dense_big(g)) return rkk::launch_gemm_wk(st, g, 256, 1);
     const DensePlan plan = effective_plan(g.M, g.N, g.K, g.w_int4);
     int ksplit = plan.ksplit;
     if (ksplit > 1 && !g.splitk_acc) {

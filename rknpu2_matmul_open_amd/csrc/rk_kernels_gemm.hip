@@ -55,8 +55,9 @@ namespace {
 // workgroup; on this multi-die part each one walks the die's L2, and 32
 // workgroups per die queueing for that cost more than the second launch.)
 constexpr int WK_NBUF = 16, WK_G = 4, WK_D = 12, WK_BUF = 8 * 1024;
-constexpr int WK_SCALES_OFF = WK_NBUF * WK_BUF;                   // fp32 scales of the tile: 128 rows, then 256 columns
-constexpr int WK_LDS_BYTES = WK_SCALES_OFF + (128 + 256) * 4;
+constexpr int WK_SCALES_OFF = WK_NBUF * WK_BUF;                   // fp32 scales of the tile: 256 rows, then 256 columns
+constexpr int WK_ROW_SCALES = 256;
+constexpr int WK_LDS_BYTES = WK_SCALES_OFF + (WK_ROW_SCALES + 256) * 4;
 
 typedef __attribute__((address_space(3))) uint8_t* lds_ptr_t;
 
@@ -80,16 +81,12 @@ __device__ __forceinline__ void wk_tile_coords(unsigned tile, unsigned mblocks, 
 #pragma clang diagnostic ignored "-Winline-asm" // m0 is set and clobbered on purpose below
 // TN: 32-column blocks per wave.  Two -- tiles of 256 columns; one -- tiles of 128 columns, for a few
 // hundred rows whose 256-column tiles would leave compute units without one (launch_gemm_wk_narrow).
-template <int TM, bool W4, int EPI, int TN = 2>
-__global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const uint8_t* h_W, int h_M, int h_K,
-                                                      int mblocks, int nblocks, int ksplit, int ksteps_per_part,
-                                                      rkh_gemm_args g) {
-    // (leading scalar arguments, see RK_GEMM_HEAD_PARAMS: everything the tile coordinates and the
-    // prologue's loads depend on, ten dwords, arrives in registers)
-    g.A = h_A; g.W = h_W; g.M = h_M; g.K = h_K;
-    RK_TS(0);
-    constexpr int KTS = 8 / TM, KTW = KTS / 2; // k-tiles per sub-step: all / this wave's
+template <int TM, bool W4, int EPI, int TN, bool RS>
+__device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw, int tile, int mblk, int nblk, int kpart,
+                                        int ksplit, int kstep0, int ksteps) {
+    constexpr int KTS = RS ? 1 : 8 / TM, KTW = RS ? 1 : KTS / 2; // k-tiles per sub-step: all / this wave's
     constexpr int NMF = TM * KTW * TN;         // MFMAs of a wave per sub-step
+    static_assert(!RS || (TM == 4 && TN == 2), "row-split waves: tiles of 256 x 256");
     static_assert(TN == 2 || (TN == 1 && EPI != RKH_EPI_SWIGLU), "gate / up pairs need two column blocks per wave");
     // Look-ahead: weights NSW - 1 sub-steps, activation copies D sub-steps.  The 128-row tile runs
     // one tile per compute unit, all of them at once, so what the prologue requests before the first
@@ -100,7 +97,10 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
     // 30.8 -> 30.25 us, int4 32.55 -> 32.15 us.  (The 64-row int4 tile measured the same with
     // either depth and keeps the deeper one.)
     constexpr int NSW = TM == 4 ? 4 : (TM == 2 && W4) ? 8 : 4;
-    constexpr int NBUF = WK_NBUF, G = WK_G, D = TM == 4 ? 8 : WK_D, BM = 32 * TM, BUF = WK_BUF;
+    constexpr int NBUF = WK_NBUF, G = WK_G, D = TM == 4 && !(RS && W4) ? 8 : WK_D, BM = RS ? 256 : 32 * TM, BUF = WK_BUF;
+    // (RS, int4: a super-tile is two sub-steps, loaded whole -- 16 bytes per lane -- at every even one;
+    // the ring's slots are super-tiles)
+    constexpr bool WPAIR = RS && W4;
     constexpr int UNR = 16;            // sub-steps per unrolled trip: multiple of NSW, NBUF, G and 2
     // int4 weights come in 1 KiB super-tiles of two k-tiles (16 bytes per lane).  When a
     // wave has two or more k-tiles per sub-step it takes WHOLE super-tiles (k-tiles
@@ -114,26 +114,17 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
     constexpr int NWREG = PAIRED ? (KTW / 2) * TN : KTW * TN;   // weight loads (registers of the ring) per sub-step
     constexpr int LPS = 1 + NWREG;                              // loads per sub-step and wave
     static_assert(UNR % NSW == 0 && UNR % NBUF == 0 && UNR % G == 0, "slot arithmetic must be compile-time");
-    static_assert(D >= NSW + G - 1 && NBUF >= D + G, "see the ordering rules above");
-    static_assert((NSW - 2) * LPS <= 63, "vmcnt field");
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[]; // WK_LDS_BYTES
+    static_assert(WPAIR ? D >= 2 * NSW - 2 + G && NBUF >= D + G : D >= NSW + G - 1 && NBUF >= D + G, "see the ordering rules above");
+    // loads of a wave that may be outstanding while it waits for the next weights: (NSW - 2) sub-steps' worth, or,
+    // with super-tiles of two sub-steps, the copies of the sub-steps since and the super-tiles behind the wanted one
+    constexpr int IN_FLIGHT = WPAIR ? 2 * (NSW - 1) - 1 + (NSW - 2) * NWREG : (NSW - 2) * LPS;
+    static_assert(IN_FLIGHT <= 63, "vmcnt field");
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
-    const int wn = wave & 3, wk = wave >> 2;
+    const int wn = wave & 3, wk = wave >> 2; // column group; k-half (RS: row half)
     const int Kp = (int)rkh_align_up(g.K, RKH_K_ALIGN);
     const int KB = Kp / 32;
-    const int ksteps_total = KB / KTS;
-
-    // ---- tile assignment: XCD-contiguous ranges, 4 row blocks per column sweep
-    const int tiles = mblocks * nblocks;
-    const int logical = xcd_remap(blockIdx.x, tiles * ksplit);
-    const int kpart = ksplit > 1 ? (int)((unsigned)logical / (unsigned)tiles) : 0;
-    const int tile = logical - kpart * tiles;
-    int mblk, nblk;
-    wk_tile_coords(tile, mblocks, nblocks, mblk, nblk);
-    const int kstep0 = kpart * ksteps_per_part;
-    const int ksteps = min(ksteps_per_part, ksteps_total - kstep0); // >= 1 by construction of the launch
 
     const uint8_t* Wb = g.W;
     const float* w_scale = g.w_scale;
@@ -141,7 +132,7 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 
     // ---- sources: wave-uniform base pointers (scalar registers) + a constant lane offset.
     // activation chunk of this wave: row block wave / KTS, k-tile wave % KTS of the sub-step
-    const uint8_t* asrc = g.A + ((size_t)(mblk * TM + wave / KTS) * KB + (size_t)kstep0 * KTS + wave % KTS) * 1024;
+    const uint8_t* asrc = g.A + ((size_t)(mblk * (BM / 32) + wave / KTS) * KB + (size_t)kstep0 * KTS + wave % KTS) * 1024;
     // int8 weights of a wave with four k-tiles per sub-step span 6 KiB; the base
     // sits in the middle so that the 13-bit signed instruction offset reaches all
     constexpr int W_BIAS = (!W4 && KTW > 2) ? 4096 : 0;
@@ -149,18 +140,19 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int pb = nblk * (4 * TN) + wn * TN + j;
-        wsrc[j] = W4 ? Wb + ((size_t)pb * (KB / 2) + (size_t)kstep0 * KTW) * 1024 + (PAIRED ? wk * 1024 : wk * 8)
-                     : Wb + ((size_t)pb * KB + (size_t)kstep0 * KTS + wk) * 1024 + W_BIAS;
+        wsrc[j] = RS   ? Wb + (size_t)pb * (W4 ? KB / 2 : KB) * 1024 // (K is not split over workgroups)
+                  : W4 ? Wb + ((size_t)pb * (KB / 2) + (size_t)kstep0 * KTW) * 1024 + (PAIRED ? wk * 1024 : wk * 8)
+                       : Wb + ((size_t)pb * KB + (size_t)kstep0 * KTS + wk) * 1024 + W_BIAS;
     }
     const unsigned lane_off = lane * 16;
-    constexpr int A_STEP = KTS * 1024, W_STEP = W4 ? KTW * 1024 : KTS * 1024;
-    using wraw_t = typename std::conditional<W4 && !PAIRED, v2i, v4i>::type;
+    constexpr int A_STEP = KTS * 1024, W_STEP = W4 && !RS ? KTW * 1024 : KTS * 1024; // (WPAIR: per super-tile)
+    using wraw_t = typename std::conditional<W4 && !PAIRED && !RS, v2i, v4i>::type;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds_raw;
     const uint32_t copy_dst = lds_base + wave * 1024; // this wave's chunk inside buffer 0
     // LDS byte addresses of this lane's fragment (row block 0, this wave's first k-tile) in buffers 0 and 8
-    uint32_t frag_lo = lds_base + wk * (PAIRED ? 2048 : 1024) + lane * 16;
+    uint32_t frag_lo = lds_base + wk * (RS ? 4096 : PAIRED ? 2048 : 1024) + lane * 16;
     uint32_t frag_hi = frag_lo + 8 * BUF;
-    int a_left = ksteps - 1, w_left = ksteps - 1; // how often the sources may still advance
+    int a_left = ksteps - 1, w_left = (WPAIR ? ksteps / 2 : ksteps) - 1; // how often the sources may still advance
 
     v16i acc[TM][TN];
 #pragma unroll
@@ -189,6 +181,8 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
             wraw_t r;
             if constexpr (PAIRED) // U counts this wave's super-tiles: every second one of the sub-step
                 asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(r) : "v"(off), "s"(base), "n"(U * 2048));
+            else if constexpr (WPAIR)
+                asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(r) : "v"(off), "s"(base));
             else if constexpr (W4)
                 asm volatile("global_load_dwordx2 %0, %1, %2 offset:%3" : "=v"(r) : "v"(off), "s"(base), "n"(U * 1024));
             else
@@ -199,9 +193,9 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
         for (int j = 0; j < TN; ++j) wsrc[j] += w_left > 0 ? W_STEP : 0;
         --w_left;
     };
-    // wait until at most (NSW-2)*LPS of this wave's loads are outstanding; regs become valid
+    // wait until at most IN_FLIGHT of this wave's loads are outstanding; regs become valid
     auto w_wait = [&](wraw_t* regs) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSW - 2) * LPS) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IN_FLIGHT) : "memory");
 #pragma unroll
         for (int e = 0; e < NWREG; ++e) asm volatile("" : "+v"(regs[e]));
     };
@@ -219,9 +213,13 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3])::"memory");
     };
     // ring register e of a sub-step -> its operand(s) in dst[NWOP]
-    auto unpack_item = [&](v4i* dst, const wraw_t* ring_regs, auto e_tag) {
+    auto unpack_item = [&](v4i* dst, const wraw_t* ring_regs, auto e_tag, auto half_tag) {
         constexpr int E = decltype(e_tag)::value;
-        if constexpr (PAIRED) {
+        if constexpr (WPAIR) { // the half of the super-tile that the sub-step is
+            const wraw_t raw = ring_regs[E];
+            const int x = decltype(half_tag)::value ? raw.z : raw.x, y = decltype(half_tag)::value ? raw.w : raw.y;
+            dst[E] = v4i{(x << 4) & (int)0xF0F0F0F0, x & (int)0xF0F0F0F0, (y << 4) & (int)0xF0F0F0F0, y & (int)0xF0F0F0F0};
+        } else if constexpr (PAIRED) {
             constexpr int V = E / TN, J = E % TN; // super-tile V of this wave = its k-tiles 2V, 2V + 1
             const wraw_t raw = ring_regs[E];
             dst[(2 * V) * TN + J] = v4i{(raw.x << 4) & (int)0xF0F0F0F0, raw.x & (int)0xF0F0F0F0,
@@ -246,7 +244,10 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
         // busy alone; the wave that is further into the barrier interval yields.
         __builtin_amdgcn_s_setprio(G - 1 - SLOT % G);
         copy_a((SLOT + D) % NBUF);
-        load_w(wring[(SLOT + NSW - 1) % NSW]);
+        if constexpr (!WPAIR) load_w(wring[(SLOT + NSW - 1) % NSW]);
+        else if constexpr (SLOT % 2 == 0) load_w(wring[(SLOT / 2 + NSW - 1) % NSW]);
+        constexpr int NEXT_W = WPAIR ? (SLOT + 1) / 2 % NSW : (SLOT + 1) % NSW; // ring slot of the next sub-step's weights
+        using NextHalf = std::integral_constant<int, (SLOT + 1) % 2>;
         __builtin_amdgcn_sched_barrier(0);
         static_assert(NMF >= 4 && NWREG <= ((NWREG + 3) / 4) * (NMF - 2), "the slots below: four fragment reads, the wait, the unpack items");
         static_for<NMF>([&](auto q_tag) {
@@ -259,12 +260,12 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
                                                                   acc[I][J], 0, 0, 0);
             // in the MFMA's shadow: one fragment read of the next sub-step, part of its unpack
             if constexpr (Q < 4) read_frag(afr[F ^ 1][Q], NextBuf{}, std::integral_constant<int, Q>{});
-            if constexpr (Q == 1) w_wait(wring[(SLOT + 1) % NSW]);
+            if constexpr (Q == 1 && !(WPAIR && SLOT % 2 == 0)) w_wait(wring[NEXT_W]); // (an odd half came with its even one)
             if constexpr (W4 && Q >= 2 && Q < 6) {
                 static_for<UPS>([&](auto t_tag) {
                     constexpr int E = (Q - 2) * UPS + decltype(t_tag)::value;
                     if constexpr (E < NWREG)
-                        unpack_item(wop[F ^ 1], wring[(SLOT + 1) % NSW], std::integral_constant<int, E>{});
+                        unpack_item(wop[F ^ 1], wring[NEXT_W], std::integral_constant<int, E>{}, NextHalf{});
                 });
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 #pragma unroll
     for (int t = -D; t < 0; ++t) {
         copy_a(t + D);
-        if (t + NSW - 1 >= 0) load_w(wring[t + NSW - 1]);
+        if (WPAIR ? t % 2 == 0 && t / 2 + NSW - 1 >= 0 : t + NSW - 1 >= 0) load_w(wring[(WPAIR ? t / 2 : t) + NSW - 1]);
     }
     RK_TS(1);
     // The tile's scales are fetched now, behind the prologue's loads, and handed
@@ -314,10 +315,10 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
         asm volatile("global_load_dword %0, %1, off" : "=v"(my_as) : "v"(pa));
         asm volatile("global_load_dword %0, %1, off" : "=v"(my_ws) : "v"(pw));
     }
-    w_wait(wring[0]); // weights of sub-step 0 and the copies of sub-steps 0..D-NSW+1 have landed
+    w_wait(wring[0]); // weights of sub-step 0 and the copies of sub-steps 0..D-NSW+1 (WPAIR: 0..D-2*NSW+2) have landed
     asm volatile("s_barrier" ::: "memory");
     static_for<4>([&](auto f_tag) { read_frag(afr[0][decltype(f_tag)::value], std::integral_constant<int, 0>{}, f_tag); });
-    static_for<NWREG>([&](auto e_tag) { unpack_item(wop[0], wring[0], e_tag); });
+    static_for<NWREG>([&](auto e_tag) { unpack_item(wop[0], wring[0], e_tag, std::integral_constant<int, 0>{}); });
     frags_wait(afr[0]);
     RK_TS(2);
 
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
         float* sc = reinterpret_cast<float*>(lds_raw + WK_SCALES_OFF);
         const int t = threadIdx.x;
         if (t < BM) sc[t] = as_valid ? my_as : 0.0f;
-        if (t < 128 * TN) sc[128 + t] = ws_valid ? my_ws : 0.0f;
+        if (t < 128 * TN) sc[WK_ROW_SCALES + t] = ws_valid ? my_ws : 0.0f;
     }
     lds_barrier();
 
@@ -359,11 +360,13 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
     // wk = 0 wave owns the block and its partner only hands over.
     auto finish = [&](auto wk_tag) {
         constexpr int WK = decltype(wk_tag)::value;
-        constexpr int KEEP = TM == 1 ? (WK == 0 ? 1 : 0) : TM / 2;  // row blocks kept
-        constexpr int GIVE = TM == 1 ? (WK == 1 ? 1 : 0) : TM / 2;  // row blocks handed over
-        constexpr int KEEP0 = TM == 1 ? 0 : WK * (TM / 2);          // first kept row block
+        constexpr int KEEP = RS ? TM : TM == 1 ? (WK == 0 ? 1 : 0) : TM / 2;  // row blocks kept
+        constexpr int GIVE = RS ? 0 : TM == 1 ? (WK == 1 ? 1 : 0) : TM / 2;   // row blocks handed over
+        constexpr int KEEP0 = RS || TM == 1 ? 0 : WK * (TM / 2);              // first kept row block
+        constexpr int ROW0 = RS ? WK * TM : KEEP0;                            // its place in the tile
         constexpr int GIVE0 = TM == 1 ? 0 : (WK ^ 1) * (TM / 2);    // first handed-over row block
         constexpr int XT = (TM == 1 ? 1 : TM / 2) * TN;             // tiles per exchange slot of a wave
+        if constexpr (!RS) {
         int* xch = reinterpret_cast<int*>(lds_raw);
         const int partner = wave ^ 4;
         static_assert(8 * XT * 16 * 64 * 4 <= WK_SCALES_OFF, "exchange area");
@@ -389,9 +392,10 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
             }
         }
         lds_barrier();
+        } // (RS: every wave holds finished sums)
         RK_TS(4);
 
-        if (ksplit > 1) {
+        if (!RS && ksplit > 1) {
             // partial tile in accumulator order: [tile][part][owning wave][kept tile][q][lane] x 4 ints
             constexpr int OWNERS = TM == 1 ? 4 : 8;
             constexpr int PER_WAVE = (TM == 1 ? 1 : TM / 2) * TN * 1024;
@@ -413,11 +417,11 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
             if constexpr (EPI != RKH_EPI_I32) {
                 const float* sc = reinterpret_cast<const float*>(lds_raw + WK_SCALES_OFF);
 #pragma unroll
-                for (int ii = 0; ii < KEEP; ++ii) as[ii] = sc[(KEEP0 + ii) * 32 + (lane & 31)];
+                for (int ii = 0; ii < KEEP; ++ii) as[ii] = sc[(ROW0 + ii) * 32 + (lane & 31)];
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) ws[j][r] = sc[128 + (wn * TN + j) * 32 + tile_col(r, lane)];
+                    for (int r = 0; r < 16; ++r) ws[j][r] = sc[WK_ROW_SCALES + (wn * TN + j) * 32 + tile_col(r, lane)];
             } else {
 #pragma unroll
                 for (int ii = 0; ii < KEEP; ++ii) as[ii] = 0.0f;
@@ -426,7 +430,7 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 #pragma unroll
             for (int ii = 0; ii < KEEP; ++ii) {
                 constexpr int i0 = KEEP0;
-                const int m0 = mblk * BM + (i0 + ii) * 32;
+                const int m0 = mblk * BM + (ROW0 + ii) * 32;
                 if constexpr (W4) {
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
@@ -449,6 +453,65 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
     if (wk == 0) finish(std::integral_constant<int, 0>{});
     else finish(std::integral_constant<int, 1>{});
     RK_TS(5);
+}
+
+// The tile of a workgroup: XCD-contiguous ranges, 4 row blocks per column sweep.
+template <int TM, bool W4, int EPI, int TN = 2>
+__global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const uint8_t* h_W, int h_M, int h_K,
+                                                      int mblocks, int nblocks, int ksplit, int ksteps_per_part,
+                                                      rkh_gemm_args g) {
+    // (leading scalar arguments, see RK_GEMM_HEAD_PARAMS: everything the tile coordinates and the
+    // prologue's loads depend on, ten dwords, arrives in registers)
+    g.A = h_A; g.W = h_W; g.M = h_M; g.K = h_K;
+    RK_TS(0);
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[]; // WK_LDS_BYTES
+    const int ksteps_total = (int)rkh_align_up(g.K, RKH_K_ALIGN) / 32 / (8 / TM);
+    const int tiles = mblocks * nblocks;
+    const int logical = xcd_remap(blockIdx.x, tiles * ksplit);
+    const int kpart = ksplit > 1 ? (int)((unsigned)logical / (unsigned)tiles) : 0;
+    const int tile = logical - kpart * tiles;
+    int mblk, nblk;
+    wk_tile_coords(tile, mblocks, nblocks, mblk, nblk);
+    const int kstep0 = kpart * ksteps_per_part;
+    const int ksteps = min(ksteps_per_part, ksteps_total - kstep0); // >= 1 by construction of the launch
+    wk_tile<TM, W4, EPI, TN, false>(g, lds_raw, tile, mblk, nblk, kpart, ksplit, kstep0, ksteps);
+}
+
+// Tiles of 256 x 256 (RS) -- `big` of them, the first in tile order -- and tiles of 128 x 256 for what is
+// left of the output: the tiles that would start a last, mostly empty round, each in two halves, and a
+// last strip of at most 128 rows.  Workgroup = 8 waves in 4 column groups x 2 row halves: a wave multiplies
+// 128 x 64 over the whole K, so there is no exchange of k-halves and all eight waves convert and store.
+// What bounds it: the power limit.  The loop keeps the matrix pipes 94 % busy (70 000 cycles for the 65 536
+// of its MFMAs at K = 4096) at the 1.41 GHz that int8 operands leave (int4 weights 1.62; a loop of nothing
+// but MFMAs 1.71); 9 of a tile's 58 us are outside it.  Against 128 x 256 tiles: the second operand of a
+// column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
+// cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, one box: int8 4096 x 4096 x
+// 14336 224 -> 204, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
+// (Measured and not kept: half of the compute units starting with a small tile so that the epilogues'
+// bursts of stores fall apart -- 204 -> 217, 195 -> 210: tiles in step share their operands in L2.)
+template <bool W4, int EPI>
+__global__ __launch_bounds__(512) void gemm_wk_big_kernel(const uint8_t* h_A, const uint8_t* h_W, int h_M, int h_K,
+                                                          int mblocks, int nblocks, int big, rkh_gemm_args g) {
+    g.A = h_A; g.W = h_W; g.M = h_M; g.K = h_K;
+    RK_TS(0);
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[]; // WK_LDS_BYTES
+    const int KB = (int)rkh_align_up(g.K, RKH_K_ALIGN) / 32;
+    int mblk, nblk;
+    if ((int)blockIdx.x < big) {
+        wk_tile_coords(xcd_remap(blockIdx.x, big), mblocks, nblocks, mblk, nblk);
+        wk_tile<4, W4, EPI, 2, true>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB);
+    } else {
+        const int halves = 2 * (mblocks * nblocks - big); // small tiles inside the last 256 x 256 ones, then the strip
+        const int t = xcd_remap(blockIdx.x - big, gridDim.x - big);
+        if (t < halves) {
+            wk_tile_coords(big + (t >> 1), mblocks, nblocks, mblk, nblk);
+            mblk = mblk * 2 + (t & 1);
+        } else {
+            mblk = mblocks * 2;
+            nblk = t - halves;
+        }
+        wk_tile<4, W4, EPI, 2, false>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB / 2);
+    }
 }
 #pragma clang diagnostic pop
 
@@ -569,6 +632,70 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
     return RKH_OK;
 }
 
+// How a dense launch is cut into 256 x 256 tiles (the first `big`, in tile order) and 128 x 256 ones, and
+// the microseconds to expect.  A 256 x 256 tile costs 9 us beside its loop, a 128 x 256 one 8 (time stamps:
+// prologue 2.5, epilogue and stores 5 - 6, the next workgroup's start 0.6), so one big tile is cheaper
+// than two small ones (K = 4096: 58 against 2 x 33 us, int8 weights) but leaves more compute units idle in
+// the last round: the tiles of that round go as halves where that ends sooner.
+struct BigPlan { int big, small; double us, us_128; };
+static BigPlan big_plan(int M, int N, int K, int w_int4) {
+    constexpr int cus = 256;
+    const int nblocks = (N + 255) / 256, strip = M % 256 > 0 && M % 256 <= 128;
+    const int tiles = (M / 256 + (M % 256 > 128)) * nblocks;
+    // microseconds per 64 k of a 128 x 256 tile with every compute unit at work: 554 - 580 cycles at the clock that
+    // the power limit leaves, 1.4 GHz with int8 operands, 1.6 with int4 weights (which ride as 16 * code)
+    const double loop = (w_int4 ? 0.35 : 0.39) * (rkh_align_up(K, RKH_K_ALIGN) / 64);
+    const double t_big = 2 * loop + 9.0, t_small = loop + 8.0;
+    BigPlan best{0, 0, 1e30, (((M + 127) / 128) * (long)nblocks + cus - 1) / cus * t_small};
+    for (int k = 0; k <= 16; ++k) {
+        const int big = tiles - k * 32;
+        if (big < 0) break;
+        const int small = 2 * (tiles - big) + strip * nblocks;
+        const int q = big / cus, rem = big % cus; // rounds of big tiles; compute units with one more
+        double us = (q + (rem > 0)) * t_big;
+        for (int r = 0; small;) { // rounds of small tiles on the compute units without the extra big one
+            const double t = q * t_big + ++r * t_small, after = t - (q + 1) * t_big;
+            const long late = after >= 0 ? (long)(after / t_small) : 0; // ... and on the others
+            if ((long)(cus - rem) * r + rem * late < small) continue;
+            if (t > us) us = t;
+            break;
+        }
+        if (us < best.us) best = {big, small, us, best.us_128};
+    }
+    return best;
+}
+
+int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g) {
+    const BigPlan plan = big_plan(g.M, g.N, g.K, g.w_int4);
+    const int nblocks = (g.N + 255) / 256, mblocks = g.M / 256 + (g.M % 256 > 128);
+    const dim3 grid(plan.big + plan.small), block(512);
+    mark(st, "gemm_wk_big_kernel");
+#define RK_WKB(W4, EPI)                                                                             \
+    do {                                                                                            \
+        static std::atomic<bool> opted_in[64] = {};                                                 \
+        int dev = 0;                                                                                \
+        RKH_CHECK(hipGetDevice(&dev));                                                              \
+        if (dev < 0 || dev >= 64) return RKH_ERR_RUNTIME;                                           \
+        if (!opted_in[dev].load(std::memory_order_acquire)) {                                       \
+            RKH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wk_big_kernel<W4, EPI>), \
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, WK_LDS_BYTES)); \
+            opted_in[dev].store(true, std::memory_order_release);                                   \
+        }                                                                                           \
+        hipLaunchKernelGGL((gemm_wk_big_kernel<W4, EPI>), grid, block, WK_LDS_BYTES, st,           \
+                           g.A, g.W, g.M, g.K, mblocks, nblocks, plan.big, g);                      \
+    } while (0)
+    switch (g.epilogue) {
+    case RKH_EPI_I32: if (g.w_int4) RK_WKB(true, RKH_EPI_I32); else RK_WKB(false, RKH_EPI_I32); break;
+    case RKH_EPI_F16: if (g.w_int4) RK_WKB(true, RKH_EPI_F16); else RK_WKB(false, RKH_EPI_F16); break;
+    case RKH_EPI_F32: if (g.w_int4) RK_WKB(true, RKH_EPI_F32); else RK_WKB(false, RKH_EPI_F32); break;
+    case RKH_EPI_SWIGLU: if (g.w_int4) RK_WKB(true, RKH_EPI_SWIGLU); else return RKH_ERR_RUNTIME; break;
+    default: return RKH_ERR_RUNTIME;
+    }
+#undef RK_WKB
+    RKH_CHECK(hipGetLastError());
+    return RKH_OK;
+}
+
 // Tiles of 64 or 128 rows x 128 columns (one column block per wave), K not split over workgroups: a few
 // hundred rows whose 256-column tiles would leave compute units without one.  The activation rows of a tile
 // go through LDS once for the eight waves, so a tile pulls K x (rows + 128) bytes through its compute unit.
@@ -618,8 +745,15 @@ namespace rkk {
 int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g, int tile_rows) {
     return tile_rows == 128 ? ::launch_gemm_wk_narrow<4>(st, g) : ::launch_gemm_wk_narrow<2>(st, g);
 }
+bool wk_big_applies(int M, int N, int K, int w_int4) {
+    // (up to 256 tiles of 128 x 256 run in one round: nothing to gain, and other plans may be better still)
+    if ((M + 127) / 128 * (long)((N + 255) / 256) <= 256) return false;
+    const BigPlan plan = big_plan(M, N, K, w_int4);
+    return plan.big > 0 && plan.us < plan.us_128;
+}
 size_t wk_scratch_bytes(long tiles, int bm, int ksplit) { return ::wk_scratch_bytes(tiles, bm, ksplit); }
 int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int tile_rows, int ksplit) {
+    if (tile_rows == 256) return ::launch_gemm_wk_big(st, g);
     if (tile_rows == 128) return ::launch_gemm_wk<4>(st, g, ksplit);
     if (tile_rows == 64) return ::launch_gemm_wk<2>(st, g, ksplit);
     return ::launch_gemm_wk<1>(st, g, ksplit);

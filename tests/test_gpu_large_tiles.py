@@ -1,0 +1,76 @@
+"""GPU parity of the 256 x 256 tiles of the large-tile GEMM (gemm_wk_big_kernel) against the CPU oracle.
+
+The kernel serves dense calls with more than 256 tiles of 128 x 256; the cases put the places where it can
+go wrong into small problems: rows that end in a strip of 128-row tiles, in a partly filled 256-row tile or
+exactly, a last round cut into halves, one and several trips of the unrolled K loop with and without a
+remainder, columns that are no multiple of anything, and every epilogue.  Integer sums and a fixed order of
+the floating-point steps: exact.
+"""
+import numpy as np
+import pytest
+
+from rknpu2_matmul_open_amd import capi, ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1100, 7500, 200),    # strip of 76 rows; one partial trip of the K loop
+          (1224, 7457, 300),    # last 256-row tile with 200 rows; odd columns
+          (2816, 6656, 513),    # 286 tiles of 256 x 256: the last round in halves; K remainder of one
+          (1025, 8200, 1000)]   # a strip of one row
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("kind", ["f16", "f32", "i32"])
+def test_int8_weights(sess, oracle, M, N, K, kind):
+    c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
+    if kind == "i32":
+        A = np.random.default_rng(M).integers(-128, 128, (M, K)).astype(np.int8)
+        op, dtype = ops.W8A8Linear(sess, capi.I8I8I32, M, c["B"]), np.int32
+        want = oracle.gemm_i8(A, c["B"])
+    elif kind == "f16":
+        A = c["A"]
+        op, dtype = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, M, c["B"], c["w_scale"]), np.uint16
+        want = oracle.w8a8(A, c["B"], c["w_scale"])["C"]
+    else:
+        A = workloads.normal_f32(K, (M, K))
+        op, dtype = ops.W8A8Linear(sess, capi.F32I8F32_DYNAMIC, M, c["B"], c["w_scale"]), np.float32
+        want = oracle.w8a8(A, c["B"], c["w_scale"])["C"]
+    dA, dC = sess.to_device(A), sess.empty_device(M * N * np.dtype(dtype).itemsize)
+    try:
+        assert op.run_device(dA, dC) == 0
+        assert sess.sync() == 0
+        got = sess.from_device(dC, (M, N), dtype)
+        assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, dtype).view(np.uint8))
+    finally:
+        sess.free_device(dA)
+        sess.free_device(dC)
+        op.close()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("kind", ["f16", "f32", "i32", "swiglu"])
+def test_int4_weights(sess, oracle, M, N, K, kind):
+    if kind == "swiglu":
+        N = (N + 63) // 64 * 64
+    c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
+    w = ops.W4A8Weights(sess, c["B"], c["w_scale"])
+    ws = ops.W4A8Workspace(sess, M, N, K)
+    try:
+        A32 = oracle.half_to_float(c["A"]).astype(np.float32).reshape(M, K)
+        if kind == "f16":
+            rc, got = ws.run_f16(w, c["A"])
+            want = oracle.w4a8(c["A"], c["B"], c["w_scale"])["C"]
+        elif kind == "f32":
+            rc, got = ws.run_f32(w, A32)
+            want = oracle.w4a8(A32, c["B"], c["w_scale"])["C"]
+        elif kind == "i32":
+            rc, got = ws.run_i32(w, A32)
+            want = oracle.w4a8(A32, c["B"], c["w_scale"])["acc"]
+        else:
+            rc, got = ws.run_swiglu_f32(w, A32)
+            want = oracle.w4a8_swiglu(A32, c["B"], c["w_scale"])["middle"]
+        assert rc == 0
+        assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, got.dtype).view(np.uint8))
+    finally:
+        ws.close()
+        w.close()
