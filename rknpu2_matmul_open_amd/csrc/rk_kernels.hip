@@ -1515,6 +1515,7 @@ int rkh_gemm(void* stream, const rkh_gemm_args* args) {
     const rkh_gemm_args& g = *args;
     hipStream_t st = (hipStream_t)stream;
     const bool grouped = g.blk_expert != nullptr;
+    if (const int cols = rkk::few_cols(g)) return rkk::launch_gemm_few(st, g, cols);
     const bool gemv_ok = !g.w_int4 || g.w_colsum; // (the int4 GEMV kernels need the column sums)
     if (!grouped && g.M <= gemv_max_rows(g) && g.epilogue != RKH_EPI_SWIGLU && gemv_ok) return dispatch_gemv(st, g, nullptr);
     if (gemv_swiglu_applies(g) && gemv_ok) return dispatch_gemv_swiglu(st, g, nullptr);
@@ -1532,7 +1533,9 @@ int rkh_gemm(void* stream, const rkh_gemm_args* args) {
 }
 
 int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_args* gargs) {
-    if (gemv_can_fuse(*qargs, *gargs)) return dispatch_gemv((hipStream_t)stream, *gargs, qargs);
+    // (int8 rows as given are staged by the decode kernel without a launch in front, whatever their length)
+    const bool few = rkk::few_cols(*gargs) != 0 && qargs->in_dtype != RKH_I8;
+    if (!few && gemv_can_fuse(*qargs, *gargs)) return dispatch_gemv((hipStream_t)stream, *gargs, qargs);
     if (gemv_swiglu_applies(*gargs) && gemv_can_fuse(*qargs, *gargs, true))
         return dispatch_gemv_swiglu((hipStream_t)stream, *gargs, qargs);
     if (qargs->mode == RKH_Q_REUSE_BITS) {
@@ -1545,7 +1548,7 @@ int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_arg
         scan.mode = RKH_Q_W4A8;
         scan.row_max_bits = nullptr;
         scan.row_max_parts = 0;
-        if (gemv_can_fuse(scan, *gargs)) return dispatch_gemv((hipStream_t)stream, *gargs, &scan);
+        if (!few && gemv_can_fuse(scan, *gargs)) return dispatch_gemv((hipStream_t)stream, *gargs, &scan);
     }
     // (int8 rows of 9..128-row calls: letting the streaming kernel read them from their row-major source
     // instead of a tiled copy saves the re-tiling launch but was slower -- a lane's 16 bytes then come from
