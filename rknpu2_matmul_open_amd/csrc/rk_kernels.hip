@@ -1465,8 +1465,8 @@ static bool dense_streams(const rkh_gemm_args& g) {
 // row blocks per wave before, which pulled 1 MB per tile where this one pulls 768 KB and which lost to the
 // other plans with int4 weights; those instantiations are gone.)  It loses where the tiles outnumber
 // the compute units (int8 4096 x 4096 at 768 rows 30.8 -> 31.9, 4096 x 14336 at 512 rows 41 -> 68; int4
-// 4096 x 11008 at 160 rows, 258 tiles: 20.6 -> 23.2) and for a long K (11008 x 4096 at 192 rows 33.2 -> 42:
-// there the K split pays), which is where the rule stops.  RK_NPU_HIP_NARROW_TILES = 0 switches it off,
+// 4096 x 11008 at 160 rows, 258 tiles: 20.6 -> 23.2) and for a long K on few tiles (below), which is where the
+// rule stops.  RK_NPU_HIP_NARROW_TILES = 0 switches it off,
 // 1 forces it (2: the 128-row tiles below) for every dense GEMM beyond the streaming kernel's rows that
 // needs no K split (tuning aid).
 static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: another plan
@@ -1477,7 +1477,21 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
     if (plan && plan[0]) return 0;
     const int cus = compute_units() > 0 ? compute_units() : 256;
     const long nblocks = (g.N + 127) / 128;
-    if (g.K <= 6144 && (long)((g.M + 63) / 64) * nblocks <= (g.w_int4 ? cus : cus + cus / 50)) return 64;
+    const long tiles64 = (long)((g.M + 63) / 64) * nblocks;
+    if (tiles64 <= (g.w_int4 ? cus : cus + cus / 50)) {
+        if (g.K <= 6144) return 64;
+        // A longer K: the other plan splits it over workgroups, whose int32 partial tiles (2 x 4 MN bytes per
+        // part) and reduce launch cost what the extra bytes of a narrow tile do when there are enough tiles; with
+        // fewer, each of them walks its K alone on a mostly idle device.  us as above, split -> 64 x 128 tiles:
+        //   96 tiles (160 rows x 4096, ...): int8 K 8192 23.9 -> 22.9 (11008 27.2 -> 29.3), int4 8192 23.1 -> 20.0,
+        //     11008 25.9 -> 23.9 (14336 a tie)
+        //   128: int8 8192 29.6 -> 26.5, 11008 a tie, 14336 39.0 -> 36.9; int4 8192 28.3 -> 23.4, 11008 29.3 -> 25.4,
+        //     14336 32.5 -> 30.3 (28672 49.0 -> 52.2)
+        //   192: int8 8192 35.2 -> 28.5, 14336 44.0 -> 42.8; int4 14336 44.1 -> 36.3, 28672 67.9 -> 63.6
+        //   256: int8 8192 39.3 -> 30.8, 14336 51.2 -> 47.4 (28672 90.9 -> 111.7); int4 14336 47.1 -> 42.1, 28672 81.9 -> 76.8
+        const long least = g.K <= (g.w_int4 ? 11264 : 8192) ? 96 : g.K <= 16384 ? 128 : g.w_int4 && g.K <= 32768 ? 192 : cus + 1L;
+        if (tiles64 >= cus * least / 256) return 64;
+    }
     // Beyond that, int8 weights: tiles of 128 rows x 128 columns of the same kernel while THEY give every
     // compute unit at most one and at least five in eight of them have one.  A tile pulls K x (128 + 128)
     // bytes for twice the products, and no K split means no reduce launch; a long K is no obstacle here.

@@ -1,0 +1,39 @@
+"""GPU parity of the 64 x 128 tiles of the LDS-ring GEMM on a long K (dense_narrow), against the CPU oracle.
+
+The rule takes them by K and by the number of tiles; the cases stand at its edges (the fewest tiles of each
+K range, and K just below and beyond a limit) with rows, columns and K that are no multiples of a tile.
+Integer sums and a fixed order of the floating-point steps: exact.
+"""
+import numpy as np
+import pytest
+
+from rknpu2_matmul_open_amd import capi, ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+# 97 tiles to K = 8192 (int8) / 11264 (int4), 129 to 16384, 192 beyond (int4), and one K past a limit (K split)
+@pytest.mark.parametrize("M,N,K", [(129, 4100, 6200), (129, 4100, 8500), (129, 5500, 8200)])
+def test_int8_weights(sess, oracle, M, N, K):
+    c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
+    op = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, M, c["B"], c["w_scale"])
+    try:
+        rc, got = op.run(c["A"])
+        want = oracle.w8a8(c["A"], c["B"], c["w_scale"])["C"]
+        assert rc == 0 and np.array_equal(got.view(np.uint16), np.asarray(want).view(np.uint16))
+    finally:
+        op.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 4100, 11200), (129, 4100, 11300), (129, 5500, 11300), (129, 8100, 16400)])
+def test_int4_weights(sess, oracle, M, N, K):
+    c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
+    w = ops.W4A8Weights(sess, c["B"], c["w_scale"])
+    ws = ops.W4A8Workspace(sess, M, N, K)
+    try:
+        rc, got = ws.run_f16(w, c["A"])
+        want = oracle.w4a8(c["A"], c["B"], c["w_scale"])["C"]
+        assert rc == 0 and np.array_equal(got.view(np.uint16), np.asarray(want).view(np.uint16))
+    finally:
+        ws.close()
+        w.close()
