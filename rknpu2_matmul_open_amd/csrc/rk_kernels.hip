@@ -158,16 +158,27 @@ __global__ __launch_bounds__(256) void pack_w4_kernel(const int8_t* __restrict__
 
 constexpr int QR_CACHE = 4; // 16-element chunks kept in registers per thread
 
-// `split` workgroups share a row (blockIdx.x = row * split + part), each taking a
+// `split` workgroups share a row (row * split + part, in contiguous ranges per die), each taking a
 // contiguous range of its 16-element chunks.  Only the modes that do not scan the
 // row for its maximum are launched with split > 1: re-quantization finds the
 // maximum in the partial maxima the GEMM left behind, which every part reads.
+// Bound by HBM, for few rows by latency.  What it was bound by: the codes went out as 16-byte
+// write-through stores from rows dealt round-robin over the dies.  Whole calls onto 1024 columns (us),
+// round-robin and written through -> contiguous rows, plain stores (either alone gives at most a third of it,
+// see store_codes_merged): int8 rows re-tiled 4096 x 4096 38.7 -> 29.7, 1024 x 4096 17.1 -> 15.3; fp32
+// 1024 x 11008 41.0 -> 36.7, fp16 512 x 14336 31.6 -> 28.7, 16 x 14336 12.6 -> 12.2; the FFN of 512 rows
+// x 4096 x 14336, whose middle it re-quantizes, 105.2 -> 102.4.
 template <typename T>
 __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, int split, rkh_quant_args a) {
     RK_QUANT_HEAD_APPLY(a);
     __shared__ float wave_max[4];
     __shared__ int wave_bad[4];
-    const int m = blockIdx.x / split, part = blockIdx.x - m * split, t = threadIdx.x;
+    // (Fewer than 256 int8 rows as given stay round-robin and written through: a few hundred KB without a maximum
+    // to wait for, where the write-back at the kernel's end counts: 128 x 4096 -> 11008 columns 14.1 us against 14.2.)
+    const bool merged = sizeof(T) > 1 || a.M >= 256;
+    const int bid = merged ? xcd_remap(blockIdx.x, a.M * split) // (gridDim would be a round trip to memory ahead of the row: 0.2 us)
+                           : (int)blockIdx.x;
+    const int m = bid / split, part = bid - m * split, t = threadIdx.x;
     if (a.active_blocks && m >= a.active_blocks[0] * 32) return;
     const int K = a.K, KB = (int)(rkh_align_up(K, RKH_K_ALIGN) / 32);
     const int row_chunks = (K + 15) >> 4;
@@ -182,8 +193,8 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
         // int8 input is re-tiled byte for byte (the full range -128..127 is legal
         // for the raw integer operator)
         const int8_t* brow = reinterpret_cast<const int8_t*>(row);
-        // (four chunks are fetched before the first is stored: the store is an asm statement the
-        // compiler keeps every load behind, and a thread that alternates load and store pays one
+        // (four chunks are fetched before the first is stored: the compiler cannot tell that the codes
+        // are not the rows and keeps every load behind a store, and a thread that alternates load and store pays one
         // memory latency per chunk)
         for (int c0 = chunk0 + t; c0 < nchunks; c0 += 4 * 256) {
             uint4 v[4];
@@ -205,7 +216,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int c = c0 + i * 256;
-                if (c < nchunks) store_codes(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
+                if (c < nchunks) {
+                    if (merged) store_codes_merged(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
+                    else store_codes(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
+                }
             }
         }
         return;
@@ -283,7 +297,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
 
     auto emit = [&](int c, const float* vals) {
         const uint4 packed = even ? quantize16<true>(vals, inv) : quantize16<false>(vals, inv);
-        store_codes(a.dst + tiled_chunk_offset(m, c, KB), packed);
+        store_codes_merged(a.dst + tiled_chunk_offset(m, c, KB), packed);
     };
     if (cached) {
 #pragma unroll
@@ -304,10 +318,12 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
 // 1024): one wave per row, four rows per workgroup.  The row maximum comes from
 // the partial maxima the SwiGLU epilogue left behind, so a row needs no
 // workgroup-wide reduction; with a workgroup per row three of its four waves
-// had nothing to do.  Rows of up to 64 * QR_CACHE chunks.
+// had nothing to do.  Rows of up to 64 * QR_CACHE chunks.  Contiguous rows per die and plain stores as
+// in quant_rows_kernel: the FFN of 2048 rows x 512 x 1024 24.6 -> 20.8 us, of 1024 x 1024 x 960
+// 21.9 -> 20.4, the MoE layer of 256 tokens 60.9 -> 60.3.
 __global__ __launch_bounds__(256) void requant_rows_wave_kernel(RK_QUANT_HEAD_PARAMS, rkh_quant_args a) {
     RK_QUANT_HEAD_APPLY(a);
-    const int lane = lane_id(), m = blockIdx.x * 4 + wave_id();
+    const int lane = lane_id(), m = xcd_remap(blockIdx.x, (a.M + 3) / 4) * 4 + wave_id();
     if (m >= a.M) return;
     // (The count of live row blocks is requested with the row, not ahead of it: rows beyond the
     // live blocks exist -- the buffers are sized for the most blocks a call can have -- so reading
@@ -345,7 +361,7 @@ __global__ __launch_bounds__(256) void requant_rows_wave_kernel(RK_QUANT_HEAD_PA
 #pragma unroll
     for (int i = 0; i < QR_CACHE; ++i)
         if (lane + 64 * i < nchunks)
-            store_codes(a.dst + tiled_chunk_offset(m, lane + 64 * i, KB),
+            store_codes_merged(a.dst + tiled_chunk_offset(m, lane + 64 * i, KB),
                         even ? quantize16<true>(v[i], inv) : quantize16<false>(v[i], inv));
 }
 
@@ -1291,8 +1307,13 @@ int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
     // 4096 elements, 4 rows: 8192): longer rows are read twice in a loop, and 256 rows of 11008 then
     // took 15 us where a workgroup per row takes 6.5.
     const int row_chunks = (args->K + 15) / 16;
+    // And only where that leaves workgroups for the device or the rows are too short for a workgroup: fp16 rows,
+    // whole calls onto 1024 columns, us, four rows -> one row per workgroup: 256 x 2048 8.4 -> 8.2, 256 x 4096
+    // 11.0 -> 10.4, 512 x 4096 (fp32) 14.2 -> 13.0, 700 x 4096 16.6 -> 16.5; but 300 x 500 7.9 -> 8.3, 999 x 1500
+    // 10.8 -> 11.1, 2048 x 2048 12.8 -> 13.4, 4096 x 4096 29.7 -> 32.3.
     const bool fits8 = row_chunks <= (256 / 8) * Q8_CACHE, fits4 = row_chunks <= (256 / 4) * Q8_CACHE;
-    if (args->M >= 256 && !args->active_blocks && args->in_dtype != RKH_I8 && fits4 &&
+    const int least_rows = row_chunks >= 128 ? 768 : 256;
+    if (args->M >= least_rows && !args->active_blocks && args->in_dtype != RKH_I8 && fits4 &&
         (mode == RKH_Q_W8_DYNAMIC || mode == RKH_Q_W4A8 || mode == RKH_Q_W8_STATIC)) {
         const bool rows4 = !fits8 || args->M < 8 * 2 * 256; // 8 rows would give fewer than two workgroups per compute unit
         const dim3 grid(rows4 ? (args->M + 3) / 4 : (args->M + 7) / 8);

@@ -234,6 +234,14 @@ __device__ __forceinline__ size_t tiled_chunk_offset(int row, int c, int KB) {
     return ((size_t)(row >> 5) * KB + kb) * 1024 + (size_t)((row & 31) + 32 * half) * 16;
 }
 
+__device__ __forceinline__ int xcd_remap(int bid, int total) {
+    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD one
+    // contiguous range of logical tiles so neighbours share its L2.
+    const int q = total >> 3, r = total & 7;
+    const int xcd = bid & 7, idx = bid >> 3;
+    return xcd * q + min(xcd, r) + idx;
+}
+
 // 16 quantized codes into the tiled matrix, as a write-through store (system scope, but not
 // streaming).  The next kernel reads these tiles.  A plain store leaves the line dirty in this
 // die's L2 until the write-back at the end of the kernel, which the launch then waits for
@@ -248,6 +256,12 @@ __device__ __forceinline__ void store_codes(uint8_t* dst, uint4 codes) {
     const v4i v = {(int)codes.x, (int)codes.y, (int)codes.z, (int)codes.w};
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
 }
+
+// The same as a plain store, for kernels whose workgroups hold single rows (or four) of a tile and are dealt
+// to the dies in contiguous ranges (xcd_remap): a row's chunks are 16-byte pieces of 128-byte lines that eight
+// consecutive rows share, and the die's L2 puts the lines together before they leave it.  Written through, every
+// piece is a memory write of its own; dealt round-robin, every die holds an eighth of every line.
+__device__ __forceinline__ void store_codes_merged(uint8_t* dst, uint4 codes) { *reinterpret_cast<uint4*>(dst) = codes; }
 
 // int8 code of v * inv as the low byte of the result.
 //   EVEN:  rint(clamp(q, -127, 127))            (ties to even)

@@ -8,14 +8,6 @@
 namespace {
 
 // ------------------------------------------------------------------ GEMM
-__device__ __forceinline__ int xcd_remap(int bid, int total) {
-    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD one
-    // contiguous range of logical tiles so neighbours share its L2.
-    const int q = total >> 3, r = total & 7;
-    const int xcd = bid & 7, idx = bid >> 3;
-    return xcd * q + min(xcd, r) + idx;
-}
-
 // LDS-only workgroup barrier: waits for this wave's LDS traffic and joins the
 // barrier, but leaves global loads in flight (the K loop keeps prefetches
 // outstanding across it).  The "memory" clobber stops the compiler from moving

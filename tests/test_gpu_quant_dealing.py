@@ -1,0 +1,63 @@
+"""GPU parity of the row quantization where its workgroups are dealt to the dies, against the CPU oracle.
+
+Workgroups take rows (or four rows, or parts of a row) in one contiguous range per die: row counts below, at
+and around multiples of eight and of 8 x 4, rows of less than a chunk and with a ragged last chunk, the line
+between one row and four rows per workgroup, and, for the re-quantized middle of an FFN, the wave-per-row kernel
+(up to 4096 columns) and rows shared by two to eight workgroups.  Exact.
+"""
+import numpy as np
+import pytest
+
+from rknpu2_matmul_open_amd import capi, ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(9, 40), (15, 2050), (33, 16400), (67, 300), (255, 2049), (256, 2030), (257, 2048), (767, 2033), (768, 2048)]
+
+
+@pytest.mark.parametrize("M,K", SHAPES)
+@pytest.mark.parametrize("kind", ["f16", "f32", "i32"])
+def test_rows(sess, oracle, M, K, kind):
+    N = 64
+    c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
+    if kind == "i32":
+        A = np.random.default_rng(M).integers(-128, 128, (M, K)).astype(np.int8)
+        op, dtype = ops.W8A8Linear(sess, capi.I8I8I32, M, c["B"]), np.int32
+        want = oracle.gemm_i8(A, c["B"])
+    elif kind == "f16":
+        A = c["A"]
+        op, dtype = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, M, c["B"], c["w_scale"]), np.uint16
+        want = oracle.w8a8(A, c["B"], c["w_scale"])["C"]
+    else:
+        A = workloads.normal_f32(K, (M, K))
+        op, dtype = ops.W8A8Linear(sess, capi.F32I8F32_DYNAMIC, M, c["B"], c["w_scale"]), np.float32
+        want = oracle.w8a8(A, c["B"], c["w_scale"])["C"]
+    dA, dC = sess.to_device(A), sess.empty_device(M * N * np.dtype(dtype).itemsize)
+    try:
+        assert op.run_device(dA, dC) == 0
+        assert sess.sync() == 0
+        got = sess.from_device(dC, (M, N), dtype)
+        assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, dtype).view(np.uint8))
+    finally:
+        sess.free_device(dA)
+        sess.free_device(dC)
+        op.close()
+
+
+@pytest.mark.parametrize("M,I", [(9, 992), (64, 992), (65, 1024), (131, 4096), (33, 4128), (70, 8224), (513, 4160)])
+def test_middle_of_an_ffn(sess, oracle, M, I):
+    H = 96
+    gu = workloads.w4a8_case(M, H, 2 * I, seed_w=I, seed_a=M)
+    dn = workloads.w4a8_case(M, I, H, seed_w=I + 1, seed_a=M)
+    A = workloads.normal_f32(M, (M, H))
+    gu_w, dn_w = ops.W4A8Weights(sess, gu["B"], gu["w_scale"]), ops.W4A8Weights(sess, dn["B"], dn["w_scale"])
+    gu_ws, dn_ws = ops.W4A8Workspace(sess, M, 2 * I, H), ops.W4A8Workspace(sess, M, H, I)
+    try:
+        rc, middle, out = ops.w4a8_ffn(sess, gu_ws, gu_w, dn_ws, dn_w, A)
+        want = oracle.w4a8_ffn(A, gu["B"], gu["w_scale"], dn["B"], dn["w_scale"])
+        assert rc == 0
+        assert np.array_equal(middle.view(np.uint32), np.asarray(want["middle"], np.float32).view(np.uint32))
+        assert np.array_equal(out.view(np.uint32), np.asarray(want["C"], np.float32).view(np.uint32))
+    finally:
+        for h in (gu_ws, dn_ws, gu_w, dn_w):
+            h.close()
