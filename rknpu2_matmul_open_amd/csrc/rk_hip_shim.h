@@ -177,6 +177,18 @@ int rkh_gemm(void* stream, const rkh_gemm_args* args);
  * into the GEMV kernel (one launch); otherwise the two kernels run back to back.
  * Either way qargs->dst / qargs->scale end up holding the quantized rows. */
 int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_args* gargs);
+/* The kernel family rkh_gemm takes for a dense problem of this shape (no GPU call: the rules are arithmetic on
+ * the shape), its tile -- columns of a workgroup for RKH_GEMM_FEW, rows of a tile for the RKH_GEMM_TILES* -- and
+ * how many workgroups share the K of a tile. */
+enum rkh_gemm_kernel {
+    RKH_GEMM_FEW = 0,          /* gemm_few_kernel                                      */
+    RKH_GEMM_GEMV = 1,         /* gemv_kernel                                          */
+    RKH_GEMM_GEMV_SWIGLU = 2,  /* gemv_swiglu_kernel                                   */
+    RKH_GEMM_STREAM = 3,       /* gemm_stream_kernel                                   */
+    RKH_GEMM_TILES_NARROW = 4, /* gemm_wk_kernel, tiles of 128 columns                 */
+    RKH_GEMM_TILES = 5         /* gemm_wk_kernel, tiles of 256 columns (256 rows: gemm_wk_big_kernel) */
+};
+int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, int* tile, int* ksplit);
 /* Bytes of split-K scratch rkh_gemm may use for a dense problem of this shape
  * (0 when it never splits K); the caller passes a zero-filled buffer of at
  * least this size in splitk_acc. */

@@ -1546,25 +1546,59 @@ size_t rkh_gemm_scratch_bytes(int M, int N, int K, int w_int4) {
     return wk_scratch_bytes(dense_tiles(M, N, plan.bm), plan.bm, plan.ksplit);
 }
 
+// What rkh_gemm does with a request: the first kernel family that takes it, in the order of the rules.
+struct GemmRoute {
+    int kernel;   // rkh_gemm_kernel
+    int tile;     // RKH_GEMM_FEW: columns of a workgroup; RKH_GEMM_TILES*: rows of a tile
+    int ksplit;   // RKH_GEMM_TILES: workgroups that share a tile's K (as planned, whether or not there is scratch)
+};
+static GemmRoute gemm_route(const rkh_gemm_args& g) {
+    if (const int cols = rkk::few_cols(g)) return {RKH_GEMM_FEW, cols, 1};
+    const bool gemv_ok = !g.w_int4 || g.w_colsum; // (the int4 GEMV kernels need the column sums)
+    if (!g.blk_expert && g.M <= gemv_max_rows(g) && g.epilogue != RKH_EPI_SWIGLU && gemv_ok) return {RKH_GEMM_GEMV, 0, 1};
+    if (gemv_swiglu_applies(g) && gemv_ok) return {RKH_GEMM_GEMV_SWIGLU, 0, 1};
+    if (g.blk_expert || dense_streams(g)) return {RKH_GEMM_STREAM, 0, 1};
+    if (const int tile_rows = dense_narrow(g)) return {RKH_GEMM_TILES_NARROW, tile_rows, 1};
+    if (dense_big(g)) return {RKH_GEMM_TILES, 256, 1};
+    const DensePlan plan = effective_plan(g.M, g.N, g.K, g.w_int4);
+    return {RKH_GEMM_TILES, plan.bm, plan.ksplit};
+}
+
+int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, int* tile, int* ksplit) {
+    static const int32_t some_sums = 0; // (never read: a dense int4 matrix has its column sums)
+    rkh_gemm_args g{};
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.w_int4 = w_int4;
+    g.epilogue = epilogue;
+    g.interleave_F = epilogue == RKH_EPI_SWIGLU ? N / 2 : 0;
+    g.w_colsum = w_int4 ? &some_sums : nullptr;
+    if (M < 1 || N < 1 || K < 1) return RKH_ERR_RUNTIME;
+    const GemmRoute r = gemm_route(g);
+    *kernel = r.kernel;
+    *tile = r.tile;
+    *ksplit = r.ksplit;
+    return RKH_OK;
+}
+
 int rkh_gemm(void* stream, const rkh_gemm_args* args) {
     const rkh_gemm_args& g = *args;
     hipStream_t st = (hipStream_t)stream;
-    const bool grouped = g.blk_expert != nullptr;
-    if (const int cols = rkk::few_cols(g)) return rkk::launch_gemm_few(st, g, cols);
-    const bool gemv_ok = !g.w_int4 || g.w_colsum; // (the int4 GEMV kernels need the column sums)
-    if (!grouped && g.M <= gemv_max_rows(g) && g.epilogue != RKH_EPI_SWIGLU && gemv_ok) return dispatch_gemv(st, g, nullptr);
-    if (gemv_swiglu_applies(g) && gemv_ok) return dispatch_gemv_swiglu(st, g, nullptr);
-    if (grouped) return launch_gemm_grouped(st, g);
-    if (dense_streams(g)) return launch_gemm_grouped(st, g);
-    if (const int tile_rows = dense_narrow(g)) return launch_gemm_wk_narrow(st, g, tile_rows);
-    if (dense_big(g)) return rkk::launch_gemm_wk(st, g, 256, 1);
-    const DensePlan plan = effective_plan(g.M, g.N, g.K, g.w_int4);
-    int ksplit = plan.ksplit;
-    if (ksplit > 1 && !g.splitk_acc) {
-        if (min_ksplit(g.K, g.w_int4) > 1) return RKH_ERR_RUNTIME;
-        ksplit = 1;
+    GemmRoute r = gemm_route(g);
+    switch (r.kernel) {
+    case RKH_GEMM_FEW: return rkk::launch_gemm_few(st, g, r.tile);
+    case RKH_GEMM_GEMV: return dispatch_gemv(st, g, nullptr);
+    case RKH_GEMM_GEMV_SWIGLU: return dispatch_gemv_swiglu(st, g, nullptr);
+    case RKH_GEMM_STREAM: return launch_gemm_grouped(st, g);
+    case RKH_GEMM_TILES_NARROW: return launch_gemm_wk_narrow(st, g, r.tile);
+    default: break;
     }
-    return rkk::launch_gemm_wk(st, g, plan.bm, ksplit);
+    if (r.ksplit > 1 && !g.splitk_acc) {
+        if (min_ksplit(g.K, g.w_int4) > 1) return RKH_ERR_RUNTIME;
+        r.ksplit = 1;
+    }
+    return rkk::launch_gemm_wk(st, g, r.tile, r.ksplit);
 }
 
 int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_args* gargs) {

@@ -155,7 +155,11 @@ namespace rkk {
 // Columns of a workgroup, or 0 where another kernel is better.  Both sides measured with fp16 rows,
 // quantization included, weights from HBM, us.
 int few_cols(const rkh_gemm_args& g) {
-    if (g.blk_expert || g.epilogue == RKH_EPI_SWIGLU || g.M < 2 || g.M > 64 || (g.w_int4 && g.K > 131072)) return 0;
+    if (g.blk_expert || g.epilogue == RKH_EPI_SWIGLU || g.M < 2 || g.M > 64) return 0;
+    // int4 weights ride as 16 * code: the int32 sum of more than 2^17 k may wrap.  int8: the kernel's descriptors
+    // hold the bytes of a column block over all of K, 32 K, in 32 bits, and K = 2^27 would read as none; the
+    // line lies well before that, and beyond anything measured here.
+    if (g.K > (g.w_int4 ? 1 << 17 : 1 << 24)) return 0;
     const long kp = (long)rkh_align_up(g.K, RKH_K_ALIGN);
     const bool narrow = g.N <= 4096; // at most one workgroup of 16 columns per compute unit
     if (g.M <= 8) {

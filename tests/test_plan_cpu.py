@@ -74,3 +74,36 @@ def test_which_moe_calls_take_the_two_launch_path():
     assert not f(13, 2048, 1024) and not f(256, 2048, 1024) and not f(0, 2048, 1024)
     assert not f(4, 32768 + 32, 1024) and not f(4, 2048, 3584 + 32) and not f(4, 2048, 8192)
     assert not f(4, 2040, 1024) and not f(4, 2048, 1000)   # (the layer's geometry is in multiples of 32)
+
+
+# ---- which kernel a dense call takes (the same rules rkh_gemm applies) ----
+FEW, GEMV, GEMV_SWIGLU, STREAM, TILES_NARROW, TILES = range(6)
+EPI_I32, EPI_F16, EPI_F32, EPI_SWIGLU = range(4)
+
+
+@pytest.fixture(scope="module")
+def route():
+    lib = capi.load_library()
+    f = lib.rkh_gemm_route
+    f.restype = C.c_int
+    f.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int)] * 3
+
+    def call(M, N, K, int4=0, epilogue=EPI_F16):
+        out = [C.c_int(-1) for _ in range(3)]
+        assert f(M, N, K, int4, epilogue, *[C.byref(v) for v in out]) == 0
+        return tuple(v.value for v in out)
+    return call
+
+
+@pytest.mark.parametrize("epilogue", [EPI_I32, EPI_F16, EPI_F32])
+def test_few_rows_of_a_k_beyond_a_descriptor(route, epilogue):
+    """gemm_few_kernel addresses a column block over all of K, 32 K bytes, through a 32-bit descriptor: from
+    K = 2^27 on its loads would return zeros.  The streaming kernel, whose strides are 64-bit, keeps such rows."""
+    for M in (9, 16, 17, 32, 40, 64):
+        for K in ((1 << 26) - 200, 1 << 26, 1 << 27, (1 << 27) + 256, (1 << 31) - 257):
+            for N in (1, 256, 5000):
+                assert route(M, N, K, 0, epilogue)[0] == STREAM, (M, N, K)
+    assert route(16, 4096, 14336, 0, epilogue) == (FEW, 16, 1)
+    # int4 weights ride as 16 x code in an int32 sum
+    for M in (9, 16, 32):
+        assert route(M, 256, 131072 + 256, 1, epilogue)[0] not in (FEW, STREAM)
