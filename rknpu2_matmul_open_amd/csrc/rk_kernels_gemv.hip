@@ -1041,6 +1041,9 @@ int gemv_max_rows(const rkh_gemm_args& g) {
         const int v = e ? atoi(e) : 8;
         return v >= 1 && v <= 8 ? v : 8;
     }();
+    // (int8 weights: a column block over all of K, 32 K bytes, has to fit a 32-bit descriptor and leave room for the
+    // offset that reads as zeros; the streaming kernel's strides are 64-bit)
+    if (!g.w_int4 && rkh_align_up(g.K, RKH_K_ALIGN) >= (1 << 27)) return 0;
     const bool wide = (g.N + 31) / 32 > 256;
     if (w4_wide_eight(g)) return min(rows, GEMV_W4_WIDE_ROWS);
     if (g.w_int4 && g.epilogue != RKH_EPI_SWIGLU && dense_stream_fits(g)) {

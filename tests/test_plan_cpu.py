@@ -107,3 +107,13 @@ def test_few_rows_of_a_k_beyond_a_descriptor(route, epilogue):
     # int4 weights ride as 16 x code in an int32 sum
     for M in (9, 16, 32):
         assert route(M, 256, 131072 + 256, 1, epilogue)[0] not in (FEW, STREAM)
+
+
+@pytest.mark.parametrize("epilogue", [EPI_I32, EPI_F16, EPI_F32])
+def test_decode_rows_of_a_k_beyond_a_descriptor(route, epilogue):
+    """The same 32-bit descriptor in the decode kernel: 32 K bytes of int8 weights have to be less than 2^32."""
+    for M in range(1, 9):
+        for K in (1 << 27, (1 << 27) - 255, (1 << 27) + 256, (1 << 31) - 257):
+            for N in (1, 256, 5000):
+                assert route(M, N, K, 0, epilogue)[0] == STREAM, (M, N, K)
+        assert route(M, 256, (1 << 27) - 256, 0, epilogue)[0] == GEMV
