@@ -1405,13 +1405,16 @@ static DensePlan dense_plan(int M, int N, int K, int w_int4) {
     return best;
 }
 // RK_NPU_HIP_GEMM_PLAN="rows:ksplit" forces the workgroup tile rows (32 / 64 /
-// 128) and the K split of dense launches (tuning aid).
+// 128) and the K split of dense launches (tuning aid).  "256:1" forces the 256 x 256 tiles, which walk all of
+// K in one accumulator: any other split of them is not a plan, and neither are they for int4 weights whose
+// sums of 16 * code need a split.
 static DensePlan effective_plan(int M, int N, int K, int w_int4) {
     DensePlan plan = dense_plan(M, N, K, w_int4);
     static const char* forced = getenv("RK_NPU_HIP_GEMM_PLAN");
     if (forced) {
         int rows = 0, split = 0;
-        if (sscanf(forced, "%d:%d", &rows, &split) == 2 && (rows == 32 || rows == 64 || rows == 128 || rows == 256) && split >= 1) {
+        if (sscanf(forced, "%d:%d", &rows, &split) == 2 &&
+            (((rows == 32 || rows == 64 || rows == 128) && split >= 1) || (rows == 256 && split == 1 && min_ksplit(K, w_int4) == 1))) {
             plan.bm = rows;
             plan.ksplit = split > min_ksplit(K, w_int4) ? split : min_ksplit(K, w_int4);
         }

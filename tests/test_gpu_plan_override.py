@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("plan", ["128:2", "64:3", "32:4", "128:1"])
+@pytest.mark.parametrize("plan", ["128:2", "64:3", "32:4", "128:1", "256:1"])
 def test_forced_dense_plan_matches_the_oracle(plan):
     env = dict(os.environ, RK_NPU_HIP_GEMM_PLAN=plan)
     child = subprocess.run([sys.executable, os.path.join(ROOT, "tests", "plan_override_child.py")], env=env,

@@ -2,6 +2,10 @@
 a workspace: the bytes of split-K scratch, = tiles x K split x tile rows x 256 columns x 4.  No GPU call
 is made (the plan is arithmetic on the shape)."""
 import ctypes as C
+import json
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -117,3 +121,38 @@ def test_decode_rows_of_a_k_beyond_a_descriptor(route, epilogue):
             for N in (1, 256, 5000):
                 assert route(M, N, K, 0, epilogue)[0] == STREAM, (M, N, K)
         assert route(M, 256, (1 << 27) - 256, 0, epilogue)[0] == GEMV
+
+
+_ROUTES = """
+import ctypes as C, json, sys
+from rknpu2_matmul_open_amd import capi
+f = capi.load_library().rkh_gemm_route
+got = []
+for shape in json.loads(sys.argv[1]):
+    out = [C.c_int(-1) for _ in range(3)]
+    assert f(*[C.c_int(v) for v in shape], *[C.byref(v) for v in out]) == 0
+    got.append([v.value for v in out])
+print(json.dumps(got))
+"""
+
+
+def _routes_under(env, shapes):
+    """Routes with environment switches set (the library reads them once per process)."""
+    child = subprocess.run([sys.executable, "-c", _ROUTES, json.dumps(shapes)], env=dict(os.environ, **env), text=True,
+                           capture_output=True, timeout=120, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert child.returncode == 0, child.stderr[-2000:]
+    return [tuple(r) for r in json.loads(child.stdout.strip().splitlines()[-1])]
+
+
+def test_forced_256_row_tiles_never_drop_a_k_split():
+    """256 x 256 tiles walk all of K in one accumulator: forced for int4 weights of more than 2^17 k, whose sums
+    of 16 x code may wrap, or with a split, they are no plan and the computed one stays."""
+    shapes = [[2000, 4096, 4096, 0, EPI_F16], [300, 512, 131072, 1, EPI_F32], [300, 512, 131072 + 256, 1, EPI_F32],
+              [2000, 4096, 3 * 131072, 1, EPI_F16]]
+    got = _routes_under({"RK_NPU_HIP_GEMM_PLAN": "256:1"}, shapes)
+    assert got[:2] == [(TILES, 256, 1)] * 2
+    for kernel, rows, ksplit in got[2:]:
+        assert kernel == TILES and rows <= 128 and ksplit >= 2
+    free = _routes_under({"RK_NPU_HIP_GEMM_PLAN": "none"}, shapes)  # (no plan, but read as a forced one: no other rule)
+    assert got[2:] == free[2:]
+    assert _routes_under({"RK_NPU_HIP_GEMM_PLAN": "256:2"}, shapes) == free
