@@ -1502,8 +1502,9 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
     const int cus = compute_units() > 0 ? compute_units() : 256;
     const long nblocks = (g.N + 127) / 128;
     const long tiles64 = (long)((g.M + 63) / 64) * nblocks;
-    if (tiles64 <= (g.w_int4 ? cus : cus + cus / 50)) {
-        if (g.K <= 6144) return 64;
+    if (g.K <= 6144) {
+        if (tiles64 <= (g.w_int4 ? cus : cus + cus / 50)) return 64;
+    } else if (tiles64 <= cus) {
         // A longer K: the other plan splits it over workgroups, whose int32 partial tiles (2 x 4 MN bytes per
         // part) and reduce launch cost what the extra bytes of a narrow tile do when there are enough tiles; with
         // fewer, each of them walks its K alone on a mostly idle device.  us as above, split -> 64 x 128 tiles:
@@ -1513,8 +1514,12 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
         //     14336 32.5 -> 30.3 (28672 49.0 -> 52.2)
         //   192: int8 8192 35.2 -> 28.5, 14336 44.0 -> 42.8; int4 14336 44.1 -> 36.3, 28672 67.9 -> 63.6
         //   256: int8 8192 39.3 -> 30.8, 14336 51.2 -> 47.4 (28672 90.9 -> 111.7); int4 14336 47.1 -> 42.1, 28672 81.9 -> 76.8
-        const long least = g.K <= (g.w_int4 ? 11264 : 8192) ? 96 : g.K <= 16384 ? 128 : g.w_int4 && g.K <= 32768 ? 192 : cus + 1L;
-        if (tiles64 >= cus * least / 256) return 64;
+        // One tile more than the compute units runs in a second round, which a longer K never pays for: 258 tiles
+        // (129 - 192 rows x 11008), us, 64 x 128 / 128 x 128 tiles: int8 K 6400 41.7 / 36.8, 8192 49.5 / 43.7,
+        // 11008 65.2 / 58.0, 28672 168.7 / 139.5.  (In one round the 64-row tiles are ahead of them: 240 - 252 tiles,
+        // K 8192 35.4 - 36.7 / 43.6 - 44.4, 14336 58.5 - 60.5 / 71.7 - 72.8.)
+        const long least = g.K <= (g.w_int4 ? 11264 : 8192) ? 96 : g.K <= 16384 ? 128 : g.w_int4 && g.K <= 32768 ? 192 : 0;
+        if (least && tiles64 >= cus * least / 256) return 64;
     }
     // Beyond that, int8 weights: tiles of 128 rows x 128 columns of the same kernel while THEY give every
     // compute unit at most one and at least five in eight of them have one.  A tile pulls K x (128 + 128)

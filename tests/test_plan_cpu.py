@@ -156,3 +156,16 @@ def test_forced_256_row_tiles_never_drop_a_k_split():
     free = _routes_under({"RK_NPU_HIP_GEMM_PLAN": "none"}, shapes)  # (no plan, but read as a forced one: no other rule)
     assert got[2:] == free[2:]
     assert _routes_under({"RK_NPU_HIP_GEMM_PLAN": "256:2"}, shapes) == free
+
+
+def test_64_row_tiles_of_a_long_k_run_in_one_round(route):
+    """Three row blocks of an 11008-wide matrix are 258 tiles of 64 x 128: on 256 compute units a second round of
+    two, which K <= 6144 tolerates and a longer K does not (the 128 x 128 tiles take it, whatever K)."""
+    for M in (129, 160, 192):
+        for K in (6145, 6400, 8192, 11008, 16384, 16385, 20480, 28672):
+            assert route(M, 11008, K) == (TILES_NARROW, 128, 1), (M, K)
+        for K in (2000, 6144):
+            assert route(M, 11008, K) == (TILES_NARROW, 64, 1), (M, K)
+        assert route(M, 10752, 8192) == (TILES_NARROW, 64, 1) and route(M, 10880, 14336) == (TILES_NARROW, 64, 1)
+        assert route(M, 10752, 28672) == (TILES_NARROW, 128, 1)   # (no number of tiles pays beyond K = 16384)
+        assert route(M, 11008, 8192, 1)[0] == TILES               # (int4 weights: no tiles of 128 x 128)
