@@ -158,7 +158,23 @@ __global__ __launch_bounds__(256) void pack_w4_kernel(const int8_t* __restrict__
 
 constexpr int QR_CACHE = 4; // 16-element chunks kept in registers per thread
 
-// `split` workgroups share a row (row * split + part, in contiguous ranges per die), each taking a
+// How the workgroups of a quantization launch are dealt to the dies (workgroup b runs on die b % 8):
+//   ROUND_ROBIN  row after row;
+//   RANGES       one contiguous range of rows per die;
+//   EIGHTS       groups of eight rows -- the rows whose chunks share the lines of the tiled matrix -- round-robin,
+//                for launches of which only the first rows are live (a range per die would leave all of those to
+//                a few dies).  The grid is a whole number of such rounds, rows past the last one exist in it.
+enum { DEAL_ROUND_ROBIN, DEAL_RANGES, DEAL_EIGHTS };
+constexpr int DEAL_THROUGH = 4; // + written through (store_codes) instead of merged in L2 (store_codes_merged)
+// Workgroup -> its place in row order.  `units`: workgroups of all rows; `log2_per_eight`: of eight rows.
+__host__ __device__ __forceinline__ int dealt_place(int b, int units, int log2_per_eight, int deal) {
+    if (deal == DEAL_RANGES) return xcd_remap(b, units);
+    if (deal == DEAL_ROUND_ROBIN) return b;
+    const int on_die = b >> 3, group = (on_die >> log2_per_eight) * 8 + (b & 7);
+    return (group << log2_per_eight) + (on_die & ((1 << log2_per_eight) - 1));
+}
+
+// 1 << log2_split workgroups share a row (row * split + part, dealt to the dies as `how` says), each taking a
 // contiguous range of its 16-element chunks.  Only the modes that do not scan the
 // row for its maximum are launched with split > 1: re-quantization finds the
 // maximum in the partial maxima the GEMM left behind, which every part reads.
@@ -169,20 +185,19 @@ constexpr int QR_CACHE = 4; // 16-element chunks kept in registers per thread
 // 1024 x 11008 41.0 -> 36.7, fp16 512 x 14336 31.6 -> 28.7, 16 x 14336 12.6 -> 12.2; the FFN of 512 rows
 // x 4096 x 14336, whose middle it re-quantizes, 105.2 -> 102.4.
 template <typename T>
-__global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, int split, rkh_quant_args a) {
+__global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, int log2_split, int how, rkh_quant_args a) {
     RK_QUANT_HEAD_APPLY(a);
     __shared__ float wave_max[4];
     __shared__ int wave_bad[4];
-    // (Fewer than 256 int8 rows as given stay round-robin and written through: a few hundred KB without a maximum
-    // to wait for, where the write-back at the kernel's end counts: 128 x 4096 -> 11008 columns 14.1 us against 14.2.)
-    const bool merged = sizeof(T) > 1 || a.M >= 256;
-    const int bid = merged ? xcd_remap(blockIdx.x, a.M * split) // (gridDim would be a round trip to memory ahead of the row: 0.2 us)
-                           : (int)blockIdx.x;
-    const int m = bid / split, part = bid - m * split, t = threadIdx.x;
+    const int split = 1 << log2_split;
+    // (a.M * split and not the grid's size, which would be a round trip to memory ahead of the row: 0.2 us)
+    const int place = dealt_place(blockIdx.x, a.M << log2_split, 3 + log2_split, how & 3);
+    const int m = place >> log2_split, part = place & (split - 1), t = threadIdx.x;
+    if (m >= a.M) return; // (DEAL_EIGHTS)
     if (a.active_blocks && m >= a.active_blocks[0] * 32) return;
     const int K = a.K, KB = (int)(rkh_align_up(K, RKH_K_ALIGN) / 32);
     const int row_chunks = (K + 15) >> 4;
-    const int per_part = (row_chunks + split - 1) / split;
+    const int per_part = (row_chunks + split - 1) >> log2_split;
     const int chunk0 = part * per_part;                         // this workgroup's chunks: chunk0 .. nchunks - 1
     const int nchunks = min(row_chunks, chunk0 + per_part);
     const T* row = static_cast<const T*>(a.src) + (size_t)m * K;
@@ -217,8 +232,8 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
             for (int i = 0; i < 4; ++i) {
                 const int c = c0 + i * 256;
                 if (c < nchunks) {
-                    if (merged) store_codes_merged(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
-                    else store_codes(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
+                    if (how & DEAL_THROUGH) store_codes(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
+                    else store_codes_merged(a.dst + tiled_chunk_offset(m, c, KB), v[i]);
                 }
             }
         }
@@ -320,10 +335,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
 // workgroup-wide reduction; with a workgroup per row three of its four waves
 // had nothing to do.  Rows of up to 64 * QR_CACHE chunks.  Contiguous rows per die and plain stores as
 // in quant_rows_kernel: the FFN of 2048 rows x 512 x 1024 24.6 -> 20.8 us, of 1024 x 1024 x 960
-// 21.9 -> 20.4, the MoE layer of 256 tokens 60.9 -> 60.3.
-__global__ __launch_bounds__(256) void requant_rows_wave_kernel(RK_QUANT_HEAD_PARAMS, rkh_quant_args a) {
+// 21.9 -> 20.4.  (The MoE layer, whose live rows are the first of more: quant_plan.)
+__global__ __launch_bounds__(256) void requant_rows_wave_kernel(RK_QUANT_HEAD_PARAMS, int how, rkh_quant_args a) {
     RK_QUANT_HEAD_APPLY(a);
-    const int lane = lane_id(), m = xcd_remap(blockIdx.x, (a.M + 3) / 4) * 4 + wave_id();
+    const int lane = lane_id(), m = dealt_place(blockIdx.x, (a.M + 3) / 4, 1, how) * 4 + wave_id();
     if (m >= a.M) return;
     // (The count of live row blocks is requested with the row, not ahead of it: rows beyond the
     // live blocks exist -- the buffers are sized for the most blocks a call can have -- so reading
@@ -1299,57 +1314,103 @@ int rkh_pack_w4(void* stream, const int8_t* src, int K, int N, int interleave_F,
     return RKH_OK;
 }
 
-int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
-    if (args->M <= 0) return RKH_OK;
-    const dim3 block(256);
-    const int mode = args->mode;
+// The launch of a quantization: which kernel, its grid, and how its workgroups are dealt.
+struct QuantPlan {
+    enum { ROWS8, ROWS4, WAVES, ROWS } kernel;
+    int grid;
+    int log2_split; // ROWS: workgroups that share a row
+    int how;        // WAVES, ROWS: DEAL_*
+};
+static QuantPlan quant_plan(const rkh_quant_args& a) {
+    const int mode = a.mode;
     // Several rows per workgroup only while a row fits the registers its threads hold it in (8 rows:
     // 4096 elements, 4 rows: 8192): longer rows are read twice in a loop, and 256 rows of 11008 then
     // took 15 us where a workgroup per row takes 6.5.
-    const int row_chunks = (args->K + 15) / 16;
+    const int row_chunks = (a.K + 15) / 16;
     // And only where that leaves workgroups for the device or the rows are too short for a workgroup: fp16 rows,
     // whole calls onto 1024 columns, us, four rows -> one row per workgroup: 256 x 2048 8.4 -> 8.2, 256 x 4096
     // 11.0 -> 10.4, 512 x 4096 (fp32) 14.2 -> 13.0, 700 x 4096 16.6 -> 16.5; but 300 x 500 7.9 -> 8.3, 999 x 1500
     // 10.8 -> 11.1, 2048 x 2048 12.8 -> 13.4, 4096 x 4096 29.7 -> 32.3.
     const bool fits8 = row_chunks <= (256 / 8) * Q8_CACHE, fits4 = row_chunks <= (256 / 4) * Q8_CACHE;
     const int least_rows = row_chunks >= 128 ? 768 : 256;
-    if (args->M >= least_rows && !args->active_blocks && args->in_dtype != RKH_I8 && fits4 &&
+    if (a.M >= least_rows && !a.active_blocks && a.in_dtype != RKH_I8 && fits4 &&
         (mode == RKH_Q_W8_DYNAMIC || mode == RKH_Q_W4A8 || mode == RKH_Q_W8_STATIC)) {
-        const bool rows4 = !fits8 || args->M < 8 * 2 * 256; // 8 rows would give fewer than two workgroups per compute unit
-        const dim3 grid(rows4 ? (args->M + 3) / 4 : (args->M + 7) / 8);
-        const hipStream_t st = (hipStream_t)stream;
-        mark(st, "quant_rows8_kernel");
-        if (args->in_dtype == RKH_F16) {
-            if (rows4) hipLaunchKernelGGL((quant_rows8_kernel<uint16_t, 4>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
-            else hipLaunchKernelGGL((quant_rows8_kernel<uint16_t, 8>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
-        } else {
-            if (rows4) hipLaunchKernelGGL((quant_rows8_kernel<float, 4>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
-            else hipLaunchKernelGGL((quant_rows8_kernel<float, 8>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
-        }
-        RKH_CHECK(hipGetLastError());
-        return RKH_OK;
+        // (8 rows would give fewer than two workgroups per compute unit below that)
+        if (!fits8 || a.M < 8 * 2 * 256) return {QuantPlan::ROWS4, (a.M + 3) / 4, 0, 0};
+        return {QuantPlan::ROWS8, (a.M + 7) / 8, 0, 0};
     }
+    // Rows of which only the first are live: see DEAL_EIGHTS.  One contiguous range per die left the live rows of
+    // a MoE call smaller than its workspace to the first dies.  us, ranges over the workspace's rows -> eights over
+    // the rows the call can have, workspaces for 256 tokens, 32 experts, top-4, 2048 x 1024: 16 tokens 47.4 -> 46.6, 32
+    // 49.1 -> 48.3, 200 53.5 -> 52.6, 256 56.7 -> 56.5; 8 experts, top-8, 512 x 2048: 32 tokens 28.1 -> 25.4.
+    // All rows live: ranges, which find the rows that the GEMM before wrote on the same die (the FFN of 2048 rows
+    // x 512 x 1024 20.8 us, with eights 25.7).
     const bool reuse = mode == RKH_Q_REUSE_BITS || mode == RKH_Q_REUSE_BITS_MOE;
-    if (reuse && args->in_dtype == RKH_F32 && args->M >= 64 && (args->K + 15) / 16 <= 64 * QR_CACHE) {
-        mark((hipStream_t)stream, "requant_rows_wave_kernel");
-        hipLaunchKernelGGL(requant_rows_wave_kernel, dim3((args->M + 3) / 4), block, 0, (hipStream_t)stream,
-                           RK_QUANT_HEAD(*args), *args);
-        RKH_CHECK(hipGetLastError());
-        return RKH_OK;
+    const int eights = ((a.M + 7) / 8 + 7) / 8 * 8;
+    if (reuse && a.in_dtype == RKH_F32 && a.M >= 64 && row_chunks <= 64 * QR_CACHE) {
+        if (a.active_blocks) return {QuantPlan::WAVES, eights * 2, 0, DEAL_EIGHTS};
+        return {QuantPlan::WAVES, (a.M + 3) / 4, 0, DEAL_RANGES};
     }
     // Re-quantization of a few long rows: several workgroups per row, about 256 chunks
     // each, until the grid has a few hundred workgroups.
-    int split = 1;
-    if (reuse) {
-        while (split < 8 && args->M * split < 512 && row_chunks / (split * 2) >= 128) split *= 2;
+    int log2_split = 0;
+    if (reuse)
+        while (log2_split < 3 && (a.M << log2_split) < 512 && (row_chunks >> (log2_split + 1)) >= 128) ++log2_split;
+    if (a.active_blocks) return {QuantPlan::ROWS, (eights * 8) << log2_split, log2_split, DEAL_EIGHTS};
+    // (Fewer than 256 int8 rows as given stay round-robin and written through: a few hundred KB without a maximum
+    // to wait for, where the write-back at the kernel's end counts: 128 x 4096 -> 11008 columns 14.1 us against 14.2.)
+    if (a.in_dtype == RKH_I8 && a.M < 256) return {QuantPlan::ROWS, a.M, 0, DEAL_ROUND_ROBIN + DEAL_THROUGH};
+    return {QuantPlan::ROWS, a.M << log2_split, log2_split, DEAL_RANGES};
+}
+
+int rkh_quant_row_of(const rkh_quant_args* args, int workgroup, int* workgroups, int* rows, int* part) {
+    const QuantPlan p = quant_plan(*args);
+    *workgroups = p.grid;
+    *part = 0;
+    if (p.kernel == QuantPlan::ROWS8 || p.kernel == QuantPlan::ROWS4) {
+        *rows = p.kernel == QuantPlan::ROWS8 ? 8 : 4;
+        return workgroup * *rows;
     }
-    const dim3 grid(args->M * split);
-    mark((hipStream_t)stream, "quant_rows_kernel");
-    switch (args->in_dtype) {
-    case RKH_F16: hipLaunchKernelGGL(quant_rows_kernel<uint16_t>, grid, block, 0, (hipStream_t)stream, RK_QUANT_HEAD(*args), split, *args); break;
-    case RKH_F32: hipLaunchKernelGGL(quant_rows_kernel<float>, grid, block, 0, (hipStream_t)stream, RK_QUANT_HEAD(*args), split, *args); break;
-    case RKH_I8: hipLaunchKernelGGL(quant_rows_kernel<int8_t>, grid, block, 0, (hipStream_t)stream, RK_QUANT_HEAD(*args), split, *args); break;
-    default: return RKH_ERR_RUNTIME;
+    if (p.kernel == QuantPlan::WAVES) {
+        *rows = 4;
+        return dealt_place(workgroup, (args->M + 3) / 4, 1, p.how) * 4;
+    }
+    *rows = 1;
+    const int place = dealt_place(workgroup, args->M << p.log2_split, 3 + p.log2_split, p.how & 3);
+    *part = place & ((1 << p.log2_split) - 1);
+    return place >> p.log2_split;
+}
+
+int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
+    if (args->M <= 0) return RKH_OK;
+    const QuantPlan p = quant_plan(*args);
+    const dim3 grid(p.grid), block(256);
+    const hipStream_t st = (hipStream_t)stream;
+    const bool fp16 = args->in_dtype == RKH_F16;
+    switch (p.kernel) {
+    case QuantPlan::ROWS8:
+        mark(st, "quant_rows8_kernel");
+        if (fp16) hipLaunchKernelGGL((quant_rows8_kernel<uint16_t, 8>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
+        else hipLaunchKernelGGL((quant_rows8_kernel<float, 8>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
+        break;
+    case QuantPlan::ROWS4:
+        mark(st, "quant_rows8_kernel");
+        if (fp16) hipLaunchKernelGGL((quant_rows8_kernel<uint16_t, 4>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
+        else hipLaunchKernelGGL((quant_rows8_kernel<float, 4>), grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
+        break;
+    case QuantPlan::WAVES:
+        mark(st, "requant_rows_wave_kernel");
+        hipLaunchKernelGGL(requant_rows_wave_kernel, grid, block, 0, st, RK_QUANT_HEAD(*args), p.how, *args);
+        break;
+    case QuantPlan::ROWS:
+        mark(st, "quant_rows_kernel");
+        switch (args->in_dtype) {
+        case RKH_F16: hipLaunchKernelGGL(quant_rows_kernel<uint16_t>, grid, block, 0, st, RK_QUANT_HEAD(*args), p.log2_split, p.how, *args); break;
+        case RKH_F32: hipLaunchKernelGGL(quant_rows_kernel<float>, grid, block, 0, st, RK_QUANT_HEAD(*args), p.log2_split, p.how, *args); break;
+        case RKH_I8: hipLaunchKernelGGL(quant_rows_kernel<int8_t>, grid, block, 0, st, RK_QUANT_HEAD(*args), p.log2_split, p.how, *args); break;
+        default: return RKH_ERR_RUNTIME;
+        }
+        break;
     }
     RKH_CHECK(hipGetLastError());
     return RKH_OK;

@@ -234,12 +234,12 @@ __device__ __forceinline__ size_t tiled_chunk_offset(int row, int c, int KB) {
     return ((size_t)(row >> 5) * KB + kb) * 1024 + (size_t)((row & 31) + 32 * half) * 16;
 }
 
-__device__ __forceinline__ int xcd_remap(int bid, int total) {
+__host__ __device__ __forceinline__ int xcd_remap(int bid, int total) {
     // Workgroups are dealt round-robin to the 8 XCDs; give each XCD one
     // contiguous range of logical tiles so neighbours share its L2.
     const int q = total >> 3, r = total & 7;
     const int xcd = bid & 7, idx = bid >> 3;
-    return xcd * q + min(xcd, r) + idx;
+    return xcd * q + (xcd < r ? xcd : r) + idx;
 }
 
 // 16 quantized codes into the tiled matrix, as a write-through store (system scope, but not

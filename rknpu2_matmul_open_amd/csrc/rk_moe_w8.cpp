@@ -230,7 +230,7 @@ int enqueue(rk_npu_moe_w8_workspace* ws, const rk_npu_moe_w8_weights* w, int row
     q2.src = ws->hidden.as<>();
     q2.in_dtype = RKH_F32;
     q2.mode = RKH_Q_REUSE_BITS_MOE;
-    q2.M = ws->sorted_rows;
+    q2.M = call_blocks * 32; // (the live row blocks are the first ones, of these at most)
     q2.K = I;
     q2.scale = ws->h_scale.as<float>();
     q2.dst = ws->h_tiled.as<>();

@@ -169,3 +169,61 @@ def test_64_row_tiles_of_a_long_k_run_in_one_round(route):
         assert route(M, 10752, 8192) == (TILES_NARROW, 64, 1) and route(M, 10880, 14336) == (TILES_NARROW, 64, 1)
         assert route(M, 10752, 28672) == (TILES_NARROW, 128, 1)   # (no number of tiles pays beyond K = 16384)
         assert route(M, 11008, 8192, 1)[0] == TILES               # (int4 weights: no tiles of 128 x 128)
+
+
+# ---- which rows the workgroups of a quantization launch take ----
+Q_W8_DYNAMIC, Q_W4A8, Q_COPY_I8, Q_REUSE, Q_REUSE_MOE = 0, 2, 4, 5, 6
+F16, F32, I8 = 0, 1, 2
+DIES = 8  # workgroup b of a launch runs on die b % 8
+
+
+class _QuantArgs(C.Structure):
+    _fields_ = [("src", C.c_void_p), ("in_dtype", C.c_int), ("mode", C.c_int), ("M", C.c_int), ("K", C.c_int),
+                ("scale", C.c_void_p), ("dst", C.c_void_p), ("bad_flag", C.c_void_p), ("row_max_bits", C.c_void_p),
+                ("row_max_parts", C.c_int), ("active_blocks", C.c_void_p), ("src_is_host", C.c_int)]
+
+
+@pytest.fixture(scope="module")
+def dealing():
+    f = capi.load_library().rkh_quant_row_of
+    f.restype = C.c_int
+    f.argtypes = [C.POINTER(_QuantArgs), C.c_int] + [C.POINTER(C.c_int)] * 3
+
+    def call(M, K, dtype, mode, grouped=False):
+        """[(die, first row, rows, part)] of every workgroup (grouped: only the first rows are live)"""
+        a = _QuantArgs(in_dtype=dtype, mode=mode, M=M, K=K, row_max_parts=K // 32, active_blocks=1 if grouped else None)
+        n, rows, part = C.c_int(1), C.c_int(0), C.c_int(0)
+        got, b = [], 0
+        while b < n.value:
+            first = f(C.byref(a), b, C.byref(n), C.byref(rows), C.byref(part))
+            got.append((b % DIES, first, rows.value, part.value))
+            b += 1
+        return got
+    return call
+
+
+@pytest.mark.parametrize("M", [1, 2, 7, 8, 9, 31, 32, 33, 61, 63, 64, 65, 100, 128, 255, 256, 257, 700, 767, 768, 1025, 4099])
+def test_every_row_is_quantized_once(dealing, M):
+    for K in (40, 1024, 2048, 4096, 4128, 8224, 14336, 20000):
+        for dtype, mode, grouped in ((F16, Q_W8_DYNAMIC, False), (F32, Q_W4A8, False), (I8, Q_COPY_I8, False),
+                                     (F32, Q_REUSE, False), (F32, Q_REUSE_MOE, True)):
+            seen = {}
+            for _, first, rows, part in dealing(M, K, dtype, mode, grouped):
+                assert first >= 0
+                for row in range(first, min(first + rows, M)):
+                    assert (row, part) not in seen
+                    seen[row, part] = True
+            parts = 1 + max(part for _, part in seen)
+            assert len(seen) == M * parts and (parts == 1 or mode in (Q_REUSE, Q_REUSE_MOE)), (K, dtype, mode)
+
+
+@pytest.mark.parametrize("I", [512, 1024, 4096, 4128, 8224])
+def test_live_rows_of_a_moe_call_are_spread_over_the_dies(dealing, I):
+    """A workspace holds more row blocks than a call fills, and the live ones are the first: whatever their
+    number, the dies' shares differ by a group of eight rows at most."""
+    capacity = 64 * 32
+    for live in (1, 2, 8, 9, 33, 64):
+        share = [0] * DIES
+        for die, first, rows, part in dealing(capacity, I, F32, Q_REUSE_MOE, True):
+            share[die] += sum(1 for row in range(first, first + rows) if row < live * 32 and part == 0)
+        assert sum(share) == live * 32 and max(share) - min(share) <= 8, (live, share)
