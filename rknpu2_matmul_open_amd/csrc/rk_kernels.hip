@@ -1331,8 +1331,12 @@ static QuantPlan quant_plan(const rkh_quant_args& a) {
     // whole calls onto 1024 columns, us, four rows -> one row per workgroup: 256 x 2048 8.4 -> 8.2, 256 x 4096
     // 11.0 -> 10.4, 512 x 4096 (fp32) 14.2 -> 13.0, 700 x 4096 16.6 -> 16.5; but 300 x 500 7.9 -> 8.3, 999 x 1500
     // 10.8 -> 11.1, 2048 x 2048 12.8 -> 13.4, 4096 x 4096 29.7 -> 32.3.
+    // fp32 rows that are fetched element by element (not 16-byte aligned) want the four rows from 513 on, more than
+    // two rows per compute unit: 560 x 4099 22.0 -> 19.7, 560 x 8191 33.8 -> 30.5, 700 x 2050 14.05 -> 13.1; 500 x 4099
+    // 16.35 -> 16.6.  (fp16 ones: 560 x 4099 23.7 with four rows against 21.9.)
     const bool fits8 = row_chunks <= (256 / 8) * Q8_CACHE, fits4 = row_chunks <= (256 / 4) * Q8_CACHE;
-    const int least_rows = row_chunks >= 128 ? 768 : 256;
+    const bool unaligned = a.in_dtype == RKH_F32 && ((a.K & 3) || (reinterpret_cast<uintptr_t>(a.src) & 15));
+    const int least_rows = row_chunks < 128 ? 256 : unaligned ? 513 : 768;
     if (a.M >= least_rows && !a.active_blocks && a.in_dtype != RKH_I8 && fits4 &&
         (mode == RKH_Q_W8_DYNAMIC || mode == RKH_Q_W4A8 || mode == RKH_Q_W8_STATIC)) {
         // (8 rows would give fewer than two workgroups per compute unit below that)
@@ -1358,8 +1362,15 @@ static QuantPlan quant_plan(const rkh_quant_args& a) {
         while (log2_split < 3 && (a.M << log2_split) < 512 && (row_chunks >> (log2_split + 1)) >= 128) ++log2_split;
     if (a.active_blocks) return {QuantPlan::ROWS, (eights * 8) << log2_split, log2_split, DEAL_EIGHTS};
     // (Fewer than 256 int8 rows as given stay round-robin and written through: a few hundred KB without a maximum
-    // to wait for, where the write-back at the kernel's end counts: 128 x 4096 -> 11008 columns 14.1 us against 14.2.)
+    // to wait for, where the write-back at the kernel's end counts: 128 x 4096 -> 11008 columns 14.15 us, 14.35 - 14.55
+    // merged, however dealt.)
     if (a.in_dtype == RKH_I8 && a.M < 256) return {QuantPlan::ROWS, a.M, 0, DEAL_ROUND_ROBIN + DEAL_THROUGH};
+    // Unaligned fp32 rows of up to 8192 elements (fewer than 513 here) go round-robin, merged.  us, written through
+    // round-robin / ranges -> this: 61 x 2050 8.55 / 8.55 -> 8.25, 16 x 2050 8.4 / 6.75 -> 6.45, 250 x 8191 16.55 / 17.6 -> 16.7,
+    // 300 x 4099 15.35 / 15.85 -> 15.2, 500 x 8191 25.0 / 25.1 -> 24.85.  Longer ones lose (512 x 9001 32.3 / 31.3 -> 35.2), and so
+    // do aligned rows (250 x 14336 25.2 / 23.7 -> 26.6, 64 x 4096 9.45 / 8.75 -> 8.85) and many fp16 ones
+    // (700 x 8191 44.3 / 34.0 -> 38.5).
+    if (unaligned && fits4 && !reuse) return {QuantPlan::ROWS, a.M, 0, DEAL_ROUND_ROBIN};
     return {QuantPlan::ROWS, a.M << log2_split, log2_split, DEAL_RANGES};
 }
 

@@ -2,8 +2,9 @@
 
 Workgroups take rows (or four rows, or parts of a row) in one contiguous range per die: row counts below, at
 and around multiples of eight and of 8 x 4, rows of less than a chunk and with a ragged last chunk, the line
-between one row and four rows per workgroup, and, for the re-quantized middle of an FFN, the wave-per-row kernel
-(up to 4096 columns) and rows shared by two to eight workgroups.  Exact.
+between one row and four rows per workgroup (at 513 for fp32 rows that are not 16-byte aligned), and, for the
+re-quantized middle of an FFN, the wave-per-row kernel (up to 4096 columns) and rows shared by two to eight
+workgroups.  Exact.
 """
 import numpy as np
 import pytest
@@ -12,7 +13,8 @@ from rknpu2_matmul_open_amd import capi, ops, workloads
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(9, 40), (15, 2050), (33, 16400), (67, 300), (255, 2049), (256, 2030), (257, 2048), (767, 2033), (768, 2048)]
+SHAPES = [(9, 40), (15, 2050), (33, 16400), (67, 300), (255, 2049), (256, 2030), (257, 2048), (767, 2033), (768, 2048),
+          (512, 2051), (513, 2051)]
 
 
 @pytest.mark.parametrize("M,K", SHAPES)

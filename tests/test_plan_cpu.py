@@ -227,3 +227,18 @@ def test_live_rows_of_a_moe_call_are_spread_over_the_dies(dealing, I):
         for die, first, rows, part in dealing(capacity, I, F32, Q_REUSE_MOE, True):
             share[die] += sum(1 for row in range(first, first + rows) if row < live * 32 and part == 0)
         assert sum(share) == live * 32 and max(share) - min(share) <= 8, (live, share)
+
+
+def test_unaligned_fp32_rows_go_round_robin(dealing):
+    """fp32 rows that are fetched element by element: one row per workgroup, round-robin over the dies, while a
+    compute unit gets at most two of up to 8192 elements; four rows per workgroup beyond.  Aligned rows, fp16 rows
+    and longer rows keep their ranges."""
+    for M, K in ((16, 2050), (61, 2050), (250, 8191), (512, 4099), (300, 8190)):
+        assert dealing(M, K, F32, Q_W8_DYNAMIC) == [(m % DIES, m, 1, 0) for m in range(M)], (M, K)
+    for M, K in ((513, 2050), (560, 4099), (700, 8191)):
+        assert all(rows == 4 for _, _, rows, _ in dealing(M, K, F32, Q_W4A8)), (M, K)
+    for M, K, dtype in ((61, 2048, F32), (61, 2050, F16), (250, 9001, F32), (560, 4099, F16)):
+        got = dealing(M, K, dtype, Q_W8_DYNAMIC)
+        for die in range(DIES):
+            mine = [first for d, first, rows, _ in got if d == die]
+            assert mine == list(range(mine[0], mine[0] + len(mine))), (M, K, dtype)
