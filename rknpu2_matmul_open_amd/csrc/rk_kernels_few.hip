@@ -156,6 +156,10 @@ namespace rkk {
 // quantization included, weights from HBM, us.
 int few_cols(const rkh_gemm_args& g) {
     if (g.blk_expert || g.epilogue == RKH_EPI_SWIGLU || g.M < 2 || g.M > 64) return 0;
+    // (tuning aids that say how one of the kernels below is used, or up to which row: the calls they mean are theirs)
+    static const bool decode_forced = getenv("RK_NPU_HIP_GEMV_COLS") || getenv("RK_NPU_HIP_GEMV_MAX_ROWS");
+    static const bool stream_forced = getenv("RK_NPU_HIP_STREAM_MAX_ROWS") != nullptr;
+    if (stream_forced || (decode_forced && g.M <= 8)) return 0;
     // int4 weights ride as 16 * code: the int32 sum of more than 2^17 k may wrap.  int8: the kernel's descriptors
     // hold the bytes of a column block over all of K, 32 K, in 32 bits, and K = 2^27 would read as none; the
     // line lies well before that, and beyond anything measured here.

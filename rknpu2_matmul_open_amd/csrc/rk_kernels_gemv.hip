@@ -1034,6 +1034,8 @@ bool dense_stream_fits(const rkh_gemm_args& g) { return !g.w_int4 || g.K <= 1310
 // blocks) whose rows fit the staging area eight at a time (the eight-row kernel, see gemv_mr); eight on
 // a narrower one with such rows; otherwise four or two, see below.  (The four-row dot products on a wide
 // matrix took 15.5 - 19.3 us for five to eight rows of 4096 x 11008 / 14336 against 12.3 - 12.9 streamed.)
+// (gemm_few_kernel comes first: rows that do not fit the staging area, int8 ones and int4 ones on up to 4096 columns,
+// get here only beyond its K or with one of the decode kernels' switches set.)
 // RK_NPU_HIP_GEMV_MAX_ROWS = 1..8 lowers the limit (tuning aid).
 int gemv_max_rows(const rkh_gemm_args& g) {
     static const int rows = [] {

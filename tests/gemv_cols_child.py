@@ -102,7 +102,8 @@ def main():
             sess.free_device(dA)
             sess.free_device(dC)
             op.close()
-    for M, K in ((4, 70000), (6, 33000)):
+    # (K > 2^17: up to there rows that do not fit the staging area leave the decode kernel from three on)
+    for M, K in ((4, 70000), (6, 33000), (2, 70000), (4, 140000), (6, 131400), (8, 133000)):
         B4 = np.full((K, N), -8, np.int8)
         B4[::3] = 7
         s4 = (rng.random(N).astype(np.float32) + 0.5) * np.float32(0.01)

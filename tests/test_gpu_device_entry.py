@@ -88,15 +88,14 @@ W4_SHAPES = [(1, 64, 64), (1, 65, 33), (1, 4096, 4096), (1, 2100, 8200), (1, 900
              # kernel from three rows on, two rows on the dot products
              (3, 8200, 1000), (5, 9000, 4096), (7, 8224, 300), (6, 14336, 4096), (4, 8200, 4100), (3, 8300, 4100),
              (2, 8300, 4100),
-             # a narrower matrix: eight rows that fit the staging area stay on the decode kernel, five to eight
-             # longer ones go to the streaming kernel; three and four rows stay up to K = 16384 (in chunks
-             # beyond 8192)
+             # a narrower matrix: rows that fit the staging area (eight of K = 4096, four of 8192) stay on the decode
+             # kernel, longer ones go to gemm_few_kernel (up to 4096 columns) or the streaming kernel
              (4, 2000, 8192), (3, 4100, 8300), (4, 2000, 4100), (5, 2000, 4100), (8, 2000, 4096), (3, 2000, 16500),
              # 129 .. 256 column blocks: whole blocks per workgroup, the eight-row kernel from three rows on
              (2, 5120, 4096), (3, 8192, 1000), (4, 6000, 300), (8, 5130, 4096), (2, 5100, 4100),
              # up to 128 blocks: 16 columns per workgroup for any number of rows
              (6, 4000, 1000), (8, 3000, 300), (2, 4000, 300),
-             # two rows that do not fit it (K > 16384): the streaming kernel beyond 4096 columns
+             # two rows that do not fit it (K > 16384): the streaming kernel beyond 4096 columns, gemm_few_kernel up to there
              (2, 4200, 16500), (2, 2000, 16500)]
 
 

@@ -158,6 +158,19 @@ def test_forced_256_row_tiles_never_drop_a_k_split():
     assert _routes_under({"RK_NPU_HIP_GEMM_PLAN": "256:2"}, shapes) == free
 
 
+def test_forced_kernels_take_their_rows():
+    """The switches that force a width or a row limit of the decode or the streaming kernel: gemm_few_kernel, which
+    takes rows of both by default, leaves these calls to them."""
+    decode = [[5, 72, 20000, 0, EPI_F16], [8, 300, 8192, 0, EPI_I32], [4, 72, 140000, 1, EPI_F16]]
+    more = [[16, 4096, 4096, 0, EPI_F16], [64, 8192, 4096, 0, EPI_F32], [16, 4096, 4096, 1, EPI_F16]]
+    assert [r[0] for r in _routes_under({}, decode + more)] == [FEW, FEW, GEMV, FEW, FEW, FEW]
+    for switch in ({"RK_NPU_HIP_GEMV_COLS": "16"}, {"RK_NPU_HIP_GEMV_MAX_ROWS": "8"}):
+        assert [r[0] for r in _routes_under(switch, decode + more)] == [GEMV] * 3 + [FEW] * 3
+    got = _routes_under({"RK_NPU_HIP_GEMV_MAX_ROWS": "2"}, decode[:2] + [[2, 72, 20000, 0, EPI_F16]])
+    assert [r[0] for r in got] == [STREAM, STREAM, GEMV]
+    assert [r[0] for r in _routes_under({"RK_NPU_HIP_STREAM_MAX_ROWS": "128"}, decode + more)] == [GEMV] * 3 + [STREAM] * 3
+
+
 def test_64_row_tiles_of_a_long_k_run_in_one_round(route):
     """Three row blocks of an 11008-wide matrix are 258 tiles of 64 x 128: on 256 compute units a second round of
     two, which K <= 6144 tolerates and a longer K does not (the 128 x 128 tiles take it, whatever K)."""
