@@ -182,7 +182,8 @@ int rkh_gemm(void* stream, const rkh_gemm_args* args);
 int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_args* gargs);
 /* The kernel family rkh_gemm takes for a dense problem of this shape (no GPU call: the rules are arithmetic on
  * the shape), its tile -- columns of a workgroup for RKH_GEMM_FEW, rows of a tile for the RKH_GEMM_TILES* -- and
- * how many workgroups share the K of a tile. */
+ * how many workgroups share the K of a tile; for tiles of 256 rows (else 0) how many of them there are and how many of
+ * 128 rows take the rest. */
 enum rkh_gemm_kernel {
     RKH_GEMM_FEW = 0,          /* gemm_few_kernel                                      */
     RKH_GEMM_GEMV = 1,         /* gemv_kernel                                          */
@@ -191,7 +192,7 @@ enum rkh_gemm_kernel {
     RKH_GEMM_TILES_NARROW = 4, /* gemm_wk_kernel, tiles of 128 columns                 */
     RKH_GEMM_TILES = 5         /* gemm_wk_kernel, tiles of 256 columns (256 rows: gemm_wk_big_kernel) */
 };
-int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, int* tile, int* ksplit);
+int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, int* tile, int* ksplit, int* big, int* small);
 /* Bytes of split-K scratch rkh_gemm may use for a dense problem of this shape
  * (0 when it never splits K); the caller passes a zero-filled buffer of at
  * least this size in splitk_acc. */

@@ -1615,9 +1615,9 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
 
 // Tiles of 256 x 256 (gemm_wk_big_kernel) where there are enough of them and they end sooner than tiles of
 // 128 x 256 would.
-static bool dense_big(const rkh_gemm_args& g) {
+static bool dense_big(const rkh_gemm_args& g, rkk::BigTiles* tiles) {
     static const char* plan = getenv("RK_NPU_HIP_GEMM_PLAN"); // (a forced plan is the plan)
-    return !(plan && plan[0]) && min_ksplit(g.K, g.w_int4) == 1 && rkk::wk_big_applies(g.M, g.N, g.K, g.w_int4);
+    return !(plan && plan[0]) && min_ksplit(g.K, g.w_int4) == 1 && rkk::wk_big_applies(g.M, g.N, g.K, g.w_int4, tiles);
 }
 
 size_t rkh_gemm_scratch_bytes(int M, int N, int K, int w_int4) {
@@ -1631,20 +1631,23 @@ struct GemmRoute {
     int kernel;   // rkh_gemm_kernel
     int tile;     // RKH_GEMM_FEW: columns of a workgroup; RKH_GEMM_TILES*: rows of a tile
     int ksplit;   // RKH_GEMM_TILES: workgroups that share a tile's K (as planned, whether or not there is scratch)
+    rkk::BigTiles cut; // RKH_GEMM_TILES of 256 rows
 };
 static GemmRoute gemm_route(const rkh_gemm_args& g) {
-    if (const int cols = rkk::few_cols(g)) return {RKH_GEMM_FEW, cols, 1};
+    if (const int cols = rkk::few_cols(g)) return {RKH_GEMM_FEW, cols, 1, {}};
     const bool gemv_ok = !g.w_int4 || g.w_colsum; // (the int4 GEMV kernels need the column sums)
-    if (!g.blk_expert && g.M <= gemv_max_rows(g) && g.epilogue != RKH_EPI_SWIGLU && gemv_ok) return {RKH_GEMM_GEMV, 0, 1};
-    if (gemv_swiglu_applies(g) && gemv_ok) return {RKH_GEMM_GEMV_SWIGLU, 0, 1};
-    if (g.blk_expert || dense_streams(g)) return {RKH_GEMM_STREAM, 0, 1};
-    if (const int tile_rows = dense_narrow(g)) return {RKH_GEMM_TILES_NARROW, tile_rows, 1};
-    if (dense_big(g)) return {RKH_GEMM_TILES, 256, 1};
+    if (!g.blk_expert && g.M <= gemv_max_rows(g) && g.epilogue != RKH_EPI_SWIGLU && gemv_ok) return {RKH_GEMM_GEMV, 0, 1, {}};
+    if (gemv_swiglu_applies(g) && gemv_ok) return {RKH_GEMM_GEMV_SWIGLU, 0, 1, {}};
+    if (g.blk_expert || dense_streams(g)) return {RKH_GEMM_STREAM, 0, 1, {}};
+    if (const int tile_rows = dense_narrow(g)) return {RKH_GEMM_TILES_NARROW, tile_rows, 1, {}};
+    rkk::BigTiles cut{};
+    if (dense_big(g, &cut)) return {RKH_GEMM_TILES, 256, 1, cut};
     const DensePlan plan = effective_plan(g.M, g.N, g.K, g.w_int4);
-    return {RKH_GEMM_TILES, plan.bm, plan.ksplit};
+    if (plan.bm == 256) cut = rkk::wk_big_tiles(g.M, g.N, g.K, g.w_int4); // (a forced plan)
+    return {RKH_GEMM_TILES, plan.bm, plan.ksplit, cut};
 }
 
-int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, int* tile, int* ksplit) {
+int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, int* tile, int* ksplit, int* big, int* small) {
     static const int32_t some_sums = 0; // (never read: a dense int4 matrix has its column sums)
     rkh_gemm_args g{};
     g.M = M;
@@ -1659,6 +1662,8 @@ int rkh_gemm_route(int M, int N, int K, int w_int4, int epilogue, int* kernel, i
     *kernel = r.kernel;
     *tile = r.tile;
     *ksplit = r.ksplit;
+    *big = r.cut.big;
+    *small = r.cut.small;
     return RKH_OK;
 }
 
@@ -1678,6 +1683,7 @@ int rkh_gemm(void* stream, const rkh_gemm_args* args) {
         if (min_ksplit(g.K, g.w_int4) > 1) return RKH_ERR_RUNTIME;
         r.ksplit = 1;
     }
+    if (r.tile == 256) return rkk::launch_gemm_wk_big(st, g, r.cut);
     return rkk::launch_gemm_wk(st, g, r.tile, r.ksplit);
 }
 

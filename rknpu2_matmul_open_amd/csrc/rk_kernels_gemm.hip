@@ -639,7 +639,7 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
 // the last round: the tiles of that round go as halves where that ends sooner.
 struct BigPlan { int big, small; double us, us_128; };
 static BigPlan big_plan(int M, int N, int K, int w_int4) {
-    constexpr int cus = 256;
+    const int cus = compute_units() > 0 ? compute_units() : 256;
     const int nblocks = (N + 255) / 256, strip = M % 256 > 0 && M % 256 <= 128;
     const int tiles = (M / 256 + (M % 256 > 128)) * nblocks;
     // microseconds per 64 k of a 128 x 256 tile with every compute unit at work: 554 - 580 cycles at the clock that
@@ -665,8 +665,7 @@ static BigPlan big_plan(int M, int N, int K, int w_int4) {
     return best;
 }
 
-int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g) {
-    const BigPlan plan = big_plan(g.M, g.N, g.K, g.w_int4);
+int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, rkk::BigTiles plan) {
     const int nblocks = (g.N + 255) / 256, mblocks = g.M / 256 + (g.M % 256 > 128);
     const dim3 grid(plan.big + plan.small), block(512);
     mark(st, "gemm_wk_big_kernel");
@@ -745,15 +744,20 @@ namespace rkk {
 int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g, int tile_rows) {
     return tile_rows == 128 ? ::launch_gemm_wk_narrow<4>(st, g) : ::launch_gemm_wk_narrow<2>(st, g);
 }
-bool wk_big_applies(int M, int N, int K, int w_int4) {
-    // (up to 256 tiles of 128 x 256 run in one round: nothing to gain, and other plans may be better still)
-    if ((M + 127) / 128 * (long)((N + 255) / 256) <= 256) return false;
+BigTiles wk_big_tiles(int M, int N, int K, int w_int4) {
     const BigPlan plan = big_plan(M, N, K, w_int4);
+    return {plan.big, plan.small};
+}
+bool wk_big_applies(int M, int N, int K, int w_int4, BigTiles* tiles) {
+    // (as many tiles of 128 x 256 as compute units run in one round: nothing to gain, and other plans may be better still)
+    if ((M + 127) / 128 * (long)((N + 255) / 256) <= (compute_units() > 0 ? compute_units() : 256)) return false;
+    const BigPlan plan = big_plan(M, N, K, w_int4);
+    *tiles = {plan.big, plan.small};
     return plan.big > 0 && plan.us < plan.us_128;
 }
+int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, BigTiles tiles) { return ::launch_gemm_wk_big(st, g, tiles); }
 size_t wk_scratch_bytes(long tiles, int bm, int ksplit) { return ::wk_scratch_bytes(tiles, bm, ksplit); }
 int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int tile_rows, int ksplit) {
-    if (tile_rows == 256) return ::launch_gemm_wk_big(st, g);
     if (tile_rows == 128) return ::launch_gemm_wk<4>(st, g, ksplit);
     if (tile_rows == 64) return ::launch_gemm_wk<2>(st, g, ksplit);
     return ::launch_gemm_wk<1>(st, g, ksplit);

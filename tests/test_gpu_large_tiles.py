@@ -2,7 +2,8 @@
 
 The kernel serves dense calls with more than 256 tiles of 128 x 256; the cases put the places where it can
 go wrong into small problems: rows that end in a strip of 128-row tiles, in a partly filled 256-row tile or
-exactly, a last round cut into halves, one and several trips of the unrolled K loop with and without a
+exactly, a last round cut into halves with and without a strip behind them (tests/test_plan_cpu.py holds the cut
+of each shape), one and several trips of the unrolled K loop with and without a
 remainder, columns that are no multiple of anything, and every epilogue.  Integer sums and a fixed order of
 the floating-point steps: exact.
 """
@@ -15,8 +16,10 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(1100, 7500, 200),    # strip of 76 rows; one partial trip of the K loop
           (1224, 7457, 300),    # last 256-row tile with 200 rows; odd columns
-          (2816, 6656, 513),    # 286 tiles of 256 x 256: the last round in halves; K remainder of one
-          (1025, 8200, 1000)]   # a strip of one row
+          (2816, 6656, 513),    # 286 tiles of 256 x 256, two rounds of them; K remainder of one
+          (1025, 8200, 1000),   # a strip of one row
+          (2304, 8192, 200),    # 288 tiles: 256 whole, the other 32 in halves
+          (2404, 8100, 300)]    # the same, and a strip of 100 rows behind the halves; ragged columns
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)

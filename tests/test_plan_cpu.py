@@ -90,12 +90,12 @@ def route():
     lib = capi.load_library()
     f = lib.rkh_gemm_route
     f.restype = C.c_int
-    f.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int)] * 3
+    f.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int)] * 5
 
-    def call(M, N, K, int4=0, epilogue=EPI_F16):
-        out = [C.c_int(-1) for _ in range(3)]
+    def call(M, N, K, int4=0, epilogue=EPI_F16, cut=False):
+        out = [C.c_int(-1) for _ in range(5)]
         assert f(M, N, K, int4, epilogue, *[C.byref(v) for v in out]) == 0
-        return tuple(v.value for v in out)
+        return tuple(v.value for v in out)[3 if cut else 0:5 if cut else 3]
     return call
 
 
@@ -129,9 +129,9 @@ from rknpu2_matmul_open_amd import capi
 f = capi.load_library().rkh_gemm_route
 got = []
 for shape in json.loads(sys.argv[1]):
-    out = [C.c_int(-1) for _ in range(3)]
+    out = [C.c_int(-1) for _ in range(5)]
     assert f(*[C.c_int(v) for v in shape], *[C.byref(v) for v in out]) == 0
-    got.append([v.value for v in out])
+    got.append([v.value for v in out[:3]])
 print(json.dumps(got))
 """
 
@@ -182,6 +182,18 @@ def test_64_row_tiles_of_a_long_k_run_in_one_round(route):
         assert route(M, 10752, 8192) == (TILES_NARROW, 64, 1) and route(M, 10880, 14336) == (TILES_NARROW, 64, 1)
         assert route(M, 10752, 28672) == (TILES_NARROW, 128, 1)   # (no number of tiles pays beyond K = 16384)
         assert route(M, 11008, 8192, 1)[0] == TILES               # (int4 weights: no tiles of 128 x 128)
+
+
+@pytest.mark.parametrize("int4", [0, 1])
+def test_cut_of_the_large_tiles(route, int4):
+    """How a launch is cut into 256 x 256 tiles and 128 x 256 ones -- halves of the last 256 x 256 tiles, then a last
+    strip of at most 128 rows; the shapes are those of test_gpu_large_tiles.py, which rely on it."""
+    for M, N, K, big, halves, strip in ((1100, 7500, 200, 120, 0, 30), (1224, 7457, 300, 150, 0, 0), (2816, 6656, 513, 286, 0, 0),
+                                        (1025, 8200, 1000, 132, 0, 33), (2304, 8192, 200, 256, 64, 0), (2404, 8100, 300, 256, 64, 32)):
+        assert route(M, N, K, int4) == (TILES, 256, 1), (M, N, K)
+        assert route(M, N, K, int4, cut=True) == (big, halves + strip), (M, N, K)
+    assert route(4096, 14336, 4096, int4, cut=True) == (768, 256)
+    assert route(2048, 4096, 4096, int4, cut=True) == (0, 0)
 
 
 # ---- which rows the workgroups of a quantization launch take ----
