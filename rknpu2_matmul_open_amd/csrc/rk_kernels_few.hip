@@ -177,6 +177,9 @@ int few_cols(const rkh_gemm_args& g) {
         const long rows = g.M == 2 ? 2 : g.M <= 4 ? 4 : 8;
         const bool staged = kp * rows <= (rows >= 4 && !g.w_int4 ? 65536 : 32768);
         if (g.w_int4) return !staged && narrow ? 16 : 0;
+        // (8192 x 13312 five / six / seven rows 22.1 / 23.1 / 24.0 -> 23.4 / 23.5 / 23.5, 14336 23.2 / 24.5 / 25.3 -> 23.9; 12288 and
+        // 16384 columns are ahead from five rows on.)
+        if (staged && g.M <= 6 && g.N > 12288 && g.N < 16384) return 0;
         return !staged || (g.M > 4 && kp >= 8192) ? 16 : 0;
     }
     if (g.w_int4) {
@@ -186,13 +189,44 @@ int few_cols(const rkh_gemm_args& g) {
     }
     // int8, 16 rows: 4096 x 4096 11.8 -> 8.7, 11008 x 4096 21.5 -> 14.4, 14336 x 4096 26.0 -> 17.1, 28672 x 4096 48.2 -> 32.4;
     // 32 columns 4096 x 8192 12.3 -> 11.0, 4096 x 11008 15.5 -> 14.7, 4096 x 28672 27.7 -> 24.8, 13824 x 5120 26.2 -> 21.0.
+    // What lies just past the 2048 k that the eight waves' first eight loads cover waits for memory once more:
+    // 2304 x 4128 16 / 32 rows 8.25 / 8.75 -> 8.95 / 9.7 (2048 9.0 -> 7.4 at 5120, 2304 x 8192 10.2 -> 9.5).
+    if (kp == 2304 && g.N > 4096 && g.N <= 6144) return 0;
+    if (g.M <= 16 && g.N > 8192) { // more than a workgroup per compute unit
+        // The same, 16 rows: 2304 x 9216 / 14336 / 28672 11.8 / 12.4 / 19.6 -> 12.6 / 12.9 / 20.1, 2560 x 9216 12.1 -> 12.7 (20480 18.7 -> 16.8,
+        // 2816 x 9216 12.85 -> 12.7); past two rounds 4608 x 9216 16.6 -> 17.0 (12288 a tie).  Short K: 512 x 20480 9.45 -> 10.4, 1024 x
+        // 28672 12.5 -> 13.5 (1024 x 20480 12.0 -> 11.4).  K = 8192 is slow here (8192 x 8320 24.4 where 7936 takes 21.6 and 8448 24.4;
+        // not for the channels that its power-of-two blocks share: starting each block at another k made it 26.3):
+        // 8320 / 10240 / 13312 / 28672 columns 23.8 / 24.8 / 26.25 / 47.4 -> 24.5 / 25.5 / 26.75 / 48.8 (8192 19.4 -> 18.6, 20480 42.8 ->
+        // 37.8, 30720 50.9 -> 49.7).
+        if (kp > 2048 && kp < 2816 && (g.N <= 16384 || g.N > 24576)) return 0;
+        if (kp > 4096 && kp < 4864 && g.N < 12288) return 0;
+        if (kp < 2048 && g.N > (kp < 1024 ? 16384 : 24576)) return 0;
+        if (kp == 8192 && (g.N < 14336 || (g.N > 24576 && g.N < 29696))) return 0;
+    }
     if (g.M <= 16) return narrow ? 16 : g.N <= 32768 ? 32 : 0;
     // 32 rows: 4096 x 4096 11.8 -> 10.3, 11008 x 4096 22.4 -> 18.1, 28672 x 4096 50.0 -> 42.0; 32 columns 4096 x 8192 12.9 -> 12.0,
     // 13824 x 5120 27.4 -> 25.4; 4096 x 12288 16.2 against 17.6: an activation tile for every weight tile is too much there.
     if (g.M <= 32) return narrow ? 16 : g.N <= 8192 ? 32 : 0;
-    // 40 / 64 rows, 32 columns: 4096 x 5120 14.6 / 14.7 -> 12.9 / 14.6, 4096 x 8192 15.7 / 16.4 -> 13.4 / 15.7, 13824 x 5120 33.6 / 34.0 ->
-    // 28.1 / 32.5; 4096 x 12288 40 / 56 / 64 rows 21.9 / 22.5 / 22.5 -> 19.6 / 21.7 / 23.4; 11008 x 4096 22.2 against 24.
-    return narrow ? 0 : g.N <= 8192 || (g.N <= 14336 && g.M <= 56) ? 32 : 0;
+    // 33 to 64 rows, 32 columns.  Up to 4096 columns the streaming kernel has tiles of 32 columns: 11008 x 4096 22.2 against 24.
+    if (narrow) return 0;
+    if (g.N <= 8192) {
+        // 40 / 64 rows: 4096 x 5120 14.6 / 14.7 -> 12.9 / 14.6, 4096 x 8192 15.7 / 16.4 -> 13.4 / 15.7, 13824 x 5120 33.6 / 34.0 ->
+        // 28.1 / 32.5, 2560 x 4128 10.65 / 10.7 -> 10.4 / 10.75, 1024 x 4128 8.6 / 8.55 -> 7.9 / 8.3.  In between, 40 / 48 / 64 rows:
+        // 2048 x 4128 8.7 / 8.7 / 8.8 -> 9.5 / 9.8 / 10.4, 2048 x 5120 9.8 / 9.9 / 9.9 -> 9.6 / 9.9 / 10.9, 1536 x 5120 8.35 / 8.35 /
+        // 8.4 -> 8.3 / 8.5 / 9.05, 2048 x 7168 10.5 / 10.6 / 10.7 -> 10.3 / 10.4 / 11.05, 2048 x 8192 10.8 / 10.8 / 10.95 -> 9.9 / 10.2 / 10.6.
+        const int most = kp <= 1024 || kp >= 2560 || g.N > 7680 ? 64 : g.N > 6144 ? 48 : g.N >= 5120 ? 40 : 0;
+        return g.M <= most ? 32 : 0;
+    }
+    // Wider, more than a workgroup per compute unit.  Up to 8448 columns, 264 tiles of the streaming kernel, that one is
+    // ahead (3072 x 8320 40 / 56 rows 15.0 / 15.15 -> 14.7 / 16.0, 5120 x 8448 21.65 / 22.0 -> 21.9 / 23.6, 8192 x 8320 29.2 / 30.1 ->
+    // 33.3 / 36.0); with 266 tiles it takes 15 % longer (3072 x 8512 17.2).  Beyond, 40 / 56 rows: 3072 x 8512 17.2 / 17.5 -> 14.9 / 16.3,
+    // 4096 x 12288 21.9 / 22.5 -> 19.6 / 21.7 (64: 22.5 -> 23.4), 14336 x 14336 61.3 / 62.3 -> 50.2 / 57.4; K = 8192 48 / 56 rows
+    // 8704 columns 35.1 / 35.7 -> 35.0 / 36.3, 12288 36.7 / 37.2 -> 36.2 / 37.9; 2048 x 9216 40 / 48 / 56 rows 14.1 / 14.2 / 14.2 ->
+    // 13.7 / 14.2 / 14.6; 1024 x 9216 9.9 -> 10.5 at 40.
+    if (g.N <= 8448 || g.N > 14336) return 0;
+    const int most = kp == 8192 ? 48 : kp >= 3072 ? 56 : kp >= 2048 ? 40 : 0;
+    return g.M <= most ? 32 : 0;
 }
 int launch_gemm_few(hipStream_t st, const rkh_gemm_args& g, int cols) {
     if (cols == 16) return g.M <= 16 ? launch_few<16, 1>(st, g) : launch_few<16, 2>(st, g);

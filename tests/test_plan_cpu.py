@@ -171,6 +171,24 @@ def test_forced_kernels_take_their_rows():
     assert [r[0] for r in _routes_under({"RK_NPU_HIP_STREAM_MAX_ROWS": "128"}, decode + more)] == [GEMV] * 3 + [STREAM] * 3
 
 
+def test_where_few_rows_keep_the_streaming_or_decode_kernel(route):
+    """int8 weights: shapes among those gemm_few_kernel is best for at which it measured slower than the kernel that
+    had them, and their neighbours on its side."""
+    def kernel(M, N, K):
+        return route(M, N, K)[0]
+    for M, N, K in ((16, 4128, 2304), (32, 5120, 2300), (16, 9216, 2304), (9, 12288, 2560), (16, 28672, 2304), (16, 9216, 4608),
+                    (9, 20480, 512), (16, 28672, 1024), (16, 8320, 8192), (12, 13312, 8192), (9, 28672, 8192),
+                    (40, 4128, 2048), (64, 5120, 2048), (56, 6144, 1536), (64, 7168, 2048),
+                    (33, 8320, 3072), (40, 8448, 5120), (56, 8320, 8192), (56, 9216, 8192), (56, 9216, 2048), (33, 9216, 1024), (57, 12288, 4096)):
+        assert kernel(M, N, K) == STREAM, (M, N, K)
+    for M, N, K in ((16, 4096, 2304), (16, 8192, 2304), (32, 4128, 2048), (16, 4128, 2560), (16, 20480, 2560), (16, 9216, 2816), (16, 12288, 4608),
+                    (9, 14336, 512), (16, 20480, 1024), (16, 8192, 8192), (16, 20480, 8192), (16, 32768, 8192),
+                    (64, 4128, 1024), (40, 5120, 2048), (48, 7168, 2048), (64, 8192, 2048), (64, 4128, 2560),
+                    (56, 8512, 3072), (48, 9216, 8192), (40, 9216, 2048), (56, 14336, 14336)):
+        assert kernel(M, N, K) == FEW, (M, N, K)
+    assert [kernel(M, 14336, 8192) for M in (5, 6, 7, 8)] == [GEMV, GEMV, FEW, FEW] and kernel(5, 12288, 8192) == FEW
+
+
 def test_64_row_tiles_of_a_long_k_run_in_one_round(route):
     """Three row blocks of an 11008-wide matrix are 258 tiles of 64 x 128: on 256 compute units a second round of
     two, which K <= 6144 tolerates and a longer K does not (the 128 x 128 tiles take it, whatever K)."""
