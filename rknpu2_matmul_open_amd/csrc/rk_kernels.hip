@@ -1579,18 +1579,22 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
     } else if (tiles64 <= cus) {
         // A longer K: the other plan splits it over workgroups, whose int32 partial tiles (2 x 4 MN bytes per
         // part) and reduce launch cost what the extra bytes of a narrow tile do when there are enough tiles; with
-        // fewer, each of them walks its K alone on a mostly idle device.  us as above, split -> 64 x 128 tiles:
-        //   96 tiles (160 rows x 4096, ...): int8 K 8192 23.9 -> 22.9 (11008 27.2 -> 29.3), int4 8192 23.1 -> 20.0,
-        //     11008 25.9 -> 23.9 (14336 a tie)
-        //   128: int8 8192 29.6 -> 26.5, 11008 a tie, 14336 39.0 -> 36.9; int4 8192 28.3 -> 23.4, 11008 29.3 -> 25.4,
-        //     14336 32.5 -> 30.3 (28672 49.0 -> 52.2)
-        //   192: int8 8192 35.2 -> 28.5, 14336 44.0 -> 42.8; int4 14336 44.1 -> 36.3, 28672 67.9 -> 63.6
-        //   256: int8 8192 39.3 -> 30.8, 14336 51.2 -> 47.4 (28672 90.9 -> 111.7); int4 14336 47.1 -> 42.1, 28672 81.9 -> 76.8
+        // fewer, each of them walks its K alone on a mostly idle device.  fp16 in / out, quantization included, us,
+        // split -> 64 x 128 tiles with the weights from HBM (from the last-level cache), 4096 columns except at 120 tiles:
+        //    96 tiles (192 rows): int8 K 6400 26.7 -> 27.4 (22.7 -> 20.1), 7168 27.5 -> 29.3 (22.7 -> 21.1), 8192 29.4 -> 32.6
+        //      (23.8 -> 22.7); int4 8192 28.6 -> 24.7 (27.6 -> 18.8), 9472 27.3 -> 28.6 (25.9 -> 21.3), 11008 28.4 -> 31.5
+        //   120: int8 7168 28.6 -> 29.5 (24.3 -> 21.1), 8192 30.6 -> 32.6 (26.1 -> 22.6); int4 11008 29.9 -> 31.4 (27.8 -> 23.1)
+        //   128: int8 8192 32.6 -> 32.6 (29.5 -> 23.3), 9472 33.9 -> 37.2 (28.9 -> 26.6), 14336 44.3 -> 52.4 (41.5 -> 35.5);
+        //      int4 11008 33.2 -> 31.8 (29.8 -> 24.1), 12800 34.7 -> 36.0 (31.5 -> 26.6), 14336 35.5 -> 38.7 (32.8 -> 28.3)
+        //   160: int8 9472 41.0 -> 38.0, 12800 48.0 -> 48.5 (40.3 -> 36.3), 14336 51.5 -> 53.7 (42.7 -> 39.7); int4 14336 43.4 -> 39.4
+        //   192: int4 20480 55.1 -> 53.9 (53.5 -> 44.6), 28672 69.7 -> 73.6 (67.2 -> 59.2); 224: 28672 77.9 -> 75.3
+        //   256: int8 8192 42.0 -> 34.5, 14336 57.7 -> 54.3 (28672 90.9 -> 111.7); int4 14336 49.2 -> 41.5, 28672 84.6 -> 76.8
         // One tile more than the compute units runs in a second round, which a longer K never pays for: 258 tiles
         // (129 - 192 rows x 11008), us, 64 x 128 / 128 x 128 tiles: int8 K 6400 41.7 / 36.8, 8192 49.5 / 43.7,
         // 11008 65.2 / 58.0, 28672 168.7 / 139.5.  (In one round the 64-row tiles are ahead of them: 240 - 252 tiles,
         // K 8192 35.4 - 36.7 / 43.6 - 44.4, 14336 58.5 - 60.5 / 71.7 - 72.8.)
-        const long least = g.K <= (g.w_int4 ? 11264 : 8192) ? 96 : g.K <= 16384 ? 128 : g.w_int4 && g.K <= 32768 ? 192 : 0;
+        const long least = g.K <= (g.w_int4 ? 8192 : 6656) ? 96 : g.K <= (g.w_int4 ? 11264 : 8192) ? 128
+                           : g.K <= 16384 ? 160 : !g.w_int4 ? 0 : g.K <= 24576 ? 192 : g.K <= 32768 ? 224 : 0;
         if (least && tiles64 >= cus * least / 256) return 64;
     }
     // Beyond that, int8 weights: tiles of 128 rows x 128 columns of the same kernel while THEY give every

@@ -12,8 +12,9 @@ from rknpu2_matmul_open_amd import capi, ops, workloads
 pytestmark = pytest.mark.gpu
 
 
-# 97 tiles to K = 8192 (int8) / 11264 (int4), 129 to 16384, 192 beyond (int4), and one K past a limit (K split)
-@pytest.mark.parametrize("M,N,K", [(129, 4100, 6200), (129, 4100, 8500), (129, 5500, 8200)])
+# 99 tiles to K = 6656 (int8) / 8192 (int4), 129 to 8192 / 11264, 162 to 16384, 192 and 224 beyond (int4), and one K past a
+# limit (K split)
+@pytest.mark.parametrize("M,N,K", [(129, 4100, 6200), (129, 4100, 8500), (129, 5500, 8200), (129, 5500, 8100), (129, 6900, 8200)])
 def test_int8_weights(sess, oracle, M, N, K):
     c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
     op = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, M, c["B"], c["w_scale"])
@@ -25,7 +26,8 @@ def test_int8_weights(sess, oracle, M, N, K):
         op.close()
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 4100, 11200), (129, 4100, 11300), (129, 5500, 11300), (129, 8100, 16400)])
+@pytest.mark.parametrize("M,N,K", [(129, 4100, 11200), (129, 4100, 11300), (129, 5500, 11300), (129, 8100, 16400), (129, 4100, 8100),
+                                   (129, 5500, 11200), (129, 6900, 11300)])
 def test_int4_weights(sess, oracle, M, N, K):
     c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
     w = ops.W4A8Weights(sess, c["B"], c["w_scale"])
