@@ -335,10 +335,12 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
 // workgroup-wide reduction; with a workgroup per row three of its four waves
 // had nothing to do.  Rows of up to 64 * QR_CACHE chunks.  Contiguous rows per die and plain stores as
 // in quant_rows_kernel: the FFN of 2048 rows x 512 x 1024 24.6 -> 20.8 us, of 1024 x 1024 x 960
-// 21.9 -> 20.4.  (The MoE layer, whose live rows are the first of more: quant_plan.)
-__global__ __launch_bounds__(256) void requant_rows_wave_kernel(RK_QUANT_HEAD_PARAMS, int how, rkh_quant_args a) {
+// 21.9 -> 20.4.  (The MoE layer, whose live rows are the first of more: quant_plan.  The dealing is a constant of the
+// instantiation: as an argument it cost the FFN of 800 rows x 1024 x 4096 0.5 of 39 us.)
+template <int DEAL>
+__global__ __launch_bounds__(256) void requant_rows_wave_kernel(RK_QUANT_HEAD_PARAMS, rkh_quant_args a) {
     RK_QUANT_HEAD_APPLY(a);
-    const int lane = lane_id(), m = dealt_place(blockIdx.x, (a.M + 3) / 4, 1, how) * 4 + wave_id();
+    const int lane = lane_id(), m = dealt_place(blockIdx.x, (a.M + 3) / 4, 1, DEAL) * 4 + wave_id();
     if (m >= a.M) return;
     // (The count of live row blocks is requested with the row, not ahead of it: rows beyond the
     // live blocks exist -- the buffers are sized for the most blocks a call can have -- so reading
@@ -1411,7 +1413,8 @@ int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
         break;
     case QuantPlan::WAVES:
         mark(st, "requant_rows_wave_kernel");
-        hipLaunchKernelGGL(requant_rows_wave_kernel, grid, block, 0, st, RK_QUANT_HEAD(*args), p.how, *args);
+        if (p.how == DEAL_EIGHTS) hipLaunchKernelGGL(requant_rows_wave_kernel<DEAL_EIGHTS>, grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
+        else hipLaunchKernelGGL(requant_rows_wave_kernel<DEAL_RANGES>, grid, block, 0, st, RK_QUANT_HEAD(*args), *args);
         break;
     case QuantPlan::ROWS:
         mark(st, "quant_rows_kernel");
