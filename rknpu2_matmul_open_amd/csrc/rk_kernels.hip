@@ -1,8 +1,9 @@
 // HIP kernels of the quantized-linear path for gfx950 (MI355X), and the C-ABI
 // launchers declared in rk_hip_shim.h.  Data layouts are described there.
-// This unit holds the C ABI and the small kernels; the three large kernel families are units
+// This unit holds the C ABI and the small kernels; the large kernel families are units
 // of their own: rk_kernels_gemv.hip (gemv_kernel, gemv_swiglu_kernel), rk_kernels_gemm.hip
-// (gemm_wk_kernel, gemm_wk_reduce_kernel), rk_kernels_stream.hip (gemm_stream_kernel).
+// (gemm_wk_kernel, gemm_wk_big_kernel, gemm_wk_reduce_kernel), rk_kernels_stream.hip
+// (gemm_stream_kernel), rk_kernels_few.hip (gemm_few_kernel).
 //
 // Kernel inventory (what bounds each one):
 //   pack_w8_kernel / pack_w4_kernel     weight re-tiling at upload                      (one-time)
@@ -14,6 +15,10 @@
 //   gemv_swiglu_kernel                  gate/up + SwiGLU of one or two rows              (HBM)
 //   gemm_wk_kernel                      int8 MFMA 32x32x32, (32..128) x 256 tiles, activations
 //                                       through an LDS ring, waves split K               (MFMA)
+//   gemm_wk_big_kernel                  256 x 256 tiles (128 x 256 for the rest), waves split
+//                                       the rows: more than one round of 128 x 256 tiles (MFMA)
+//   gemm_few_kernel                     2 .. 64 rows, 16 or 32 columns per workgroup, K
+//                                       interleaved over eight waves                    (HBM)
 //   gemm_wk_reduce_kernel               sum of K-split partial tiles + epilogue          (L2, small)
 //   gemm_stream_kernel                  32 x 256 tiles, operands straight to registers: MoE
 //                                       (grouped by expert) and dense GEMMs of 9..128 rows (HBM)

@@ -481,12 +481,12 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 // left of the output: the tiles that would start a last, mostly empty round, each in two halves, and a
 // last strip of at most 128 rows.  Workgroup = 8 waves in 4 column groups x 2 row halves: a wave multiplies
 // 128 x 64 over the whole K, so there is no exchange of k-halves and all eight waves convert and store.
-// What bounds it: the power limit.  The loop keeps the matrix pipes 94 % busy (70 000 cycles for the 65 536
-// of its MFMAs at K = 4096) at the 1.41 GHz that int8 operands leave (int4 weights 1.62; a loop of nothing
-// but MFMAs 1.71); 9 of a tile's 58 us are outside it.  Against 128 x 256 tiles: the second operand of a
-// column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
-// cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, one box: int8 4096 x 4096 x
-// 14336 224 -> 204, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
+// What bounds it: the matrix pipes at the clock that the power limit leaves -- 4096 x 4096 x 14336 int8 is 229 376 MFMA
+// cycles per SIMD in 199 us cold and 228 on average of 40 launches in a row, 2.4 - 2.1 POP/s where a loop of nothing but
+// MFMAs reaches 3.5 -- and about 9 of a tile's 58 us outside its loop (time stamps, RK_DEBUG_TS).  Against 128 x 256 tiles:
+// the second operand of a column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
+// cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, the calls among others: int8
+// 4096 x 4096 x 14336 241 -> 203, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
 // (Measured and not kept: half of the compute units starting with a small tile so that the epilogues'
 // bursts of stores fall apart -- 204 -> 217, 195 -> 210: tiles in step share their operands in L2.)
 template <bool W4, int EPI>
