@@ -1601,8 +1601,11 @@ static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: ano
         // (129 - 192 rows x 11008), us, 64 x 128 / 128 x 128 tiles: int8 K 6400 41.7 / 36.8, 8192 49.5 / 43.7,
         // 11008 65.2 / 58.0, 28672 168.7 / 139.5.  (In one round the 64-row tiles are ahead of them: 240 - 252 tiles,
         // K 8192 35.4 - 36.7 / 43.6 - 44.4, 14336 58.5 - 60.5 / 71.7 - 72.8.)
-        const long least = g.K <= (g.w_int4 ? 8192 : 6656) ? 96 : g.K <= (g.w_int4 ? 11264 : 8192) ? 128
-                           : g.K <= 16384 ? 160 : !g.w_int4 ? 0 : g.K <= 24576 ? 192 : g.K <= 32768 ? 224 : 0;
+        // The line is where what is lost from HBM is less than what is gained from the cache; 14336 x 4096 as the down
+        // projection of an int4 FFN of 256 rows, behind the gate / up weights, 75.5 with the tiles and 69.9 split.
+        const long least = g.w_int4 ? (g.K <= 9728 ? 96 : g.K <= 11264 ? 112 : g.K <= 13312 ? 128 : g.K <= 16384 ? 160
+                                       : g.K <= 24576 ? 192 : g.K <= 32768 ? 224 : 0)
+                                    : (g.K <= 6656 ? 96 : g.K <= 8192 ? 112 : g.K <= 16384 ? 160 : 0);
         if (least && tiles64 >= cus * least / 256) return 64;
     }
     // Beyond that, int8 weights: tiles of 128 rows x 128 columns of the same kernel while THEY give every

@@ -12,8 +12,8 @@ from rknpu2_matmul_open_amd import capi, ops, workloads
 pytestmark = pytest.mark.gpu
 
 
-# 99 tiles to K = 6656 (int8) / 8192 (int4), 129 to 8192 / 11264, 162 to 16384, 192 and 224 beyond (int4), and one K past a
-# limit (K split)
+# Row blocks x column blocks = 99 tiles (enough to K = 6656 int8 / 9728 int4), 129 (8192 / 13312), 162 (16384), 192 (24576, int4), and
+# one K past a limit (K split)
 @pytest.mark.parametrize("M,N,K", [(129, 4100, 6200), (129, 4100, 8500), (129, 5500, 8200), (129, 5500, 8100), (129, 6900, 8200)])
 def test_int8_weights(sess, oracle, M, N, K):
     c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
@@ -27,7 +27,7 @@ def test_int8_weights(sess, oracle, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(129, 4100, 11200), (129, 4100, 11300), (129, 5500, 11300), (129, 8100, 16400), (129, 4100, 8100),
-                                   (129, 5500, 11200), (129, 6900, 11300)])
+                                   (129, 5500, 11200), (129, 5500, 13400), (129, 6900, 13400)])
 def test_int4_weights(sess, oracle, M, N, K):
     c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
     w = ops.W4A8Weights(sess, c["B"], c["w_scale"])

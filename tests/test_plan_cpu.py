@@ -204,8 +204,9 @@ def test_64_row_tiles_of_a_long_k_run_in_one_round(route):
 
 def test_fewest_64_row_tiles_of_a_long_k(route):
     """Fewer tiles, each walking its K alone, are slower than the K split once the weights come from memory."""
-    for int4, K, least in ((0, 6656, 96), (0, 6657, 128), (0, 8192, 128), (0, 8193, 160), (0, 16384, 160),
-                           (1, 8192, 96), (1, 8193, 128), (1, 11264, 128), (1, 11265, 160), (1, 16384, 160), (1, 16385, 192), (1, 24576, 192), (1, 24577, 224), (1, 32768, 224)):
+    for int4, K, least in ((0, 6656, 96), (0, 6657, 112), (0, 8192, 112), (0, 8193, 160), (0, 16384, 160),
+                           (1, 9728, 96), (1, 9729, 112), (1, 11264, 112), (1, 11265, 128), (1, 13312, 128), (1, 13313, 160),
+                           (1, 16384, 160), (1, 16385, 192), (1, 24576, 192), (1, 24577, 224), (1, 32768, 224)):
         for tiles in (least - 4, least, 252):                # four row blocks x a quarter of the tiles
             kernel, rows, ksplit = route(256, tiles // 4 * 128, K, int4)
             if tiles >= least:
