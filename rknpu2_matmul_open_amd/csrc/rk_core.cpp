@@ -9,6 +9,7 @@
 #include <new>
 
 #include <cstring>
+#include <thread>
 
 #include "rk_host.h"
 #include "rk_npu_hip.h"
@@ -102,6 +103,47 @@ double StageTimer::span_us(int from, int to) {
     return us;
 }
 
+// Copies between a caller's buffer and a mirror are shared by several threads in pieces of this size.
+static constexpr size_t kPiece = size_t(512) << 10;
+
+// Runs `work` on this thread and beside it on one helper for every 2 MiB beyond the first, three at most; all have
+// ended when it returns.
+template <class Work>
+static void run_with_helpers(size_t bytes, const Work& work) {
+    std::thread helpers[3];
+    const size_t want = std::min<size_t>(3, bytes >> 21);
+    for (size_t i = 0; i < want; ++i) {
+        try {
+            helpers[i] = std::thread(work);
+        } catch (...) { // (no thread to be had: fewer copy)
+            break;
+        }
+    }
+    work();
+    for (std::thread& t : helpers)
+        if (t.joinable()) t.join();
+}
+
+// Copies `bytes` and tells whether the floating-point values among them are finite.
+template <class T>
+static bool copy_finite(T* __restrict__ to, const T* __restrict__ from, size_t n, T exponent) {
+    T bad = 0;
+    for (size_t i = 0; i < n; ++i) {
+        const T v = from[i];
+        to[i] = v;
+        bad |= (T)((v & exponent) == exponent);
+    }
+    return !bad;
+}
+static bool copy_checked(void* to, const void* from, size_t bytes, PanelPipe::Check check) {
+    if (check == PanelPipe::FINITE_F16)
+        return copy_finite(static_cast<uint16_t*>(to), static_cast<const uint16_t*>(from), bytes / 2, (uint16_t)0x7c00);
+    if (check == PanelPipe::FINITE_F32)
+        return copy_finite(static_cast<uint32_t*>(to), static_cast<const uint32_t*>(from), bytes / 4, 0x7f800000u);
+    std::memcpy(to, from, bytes);
+    return true;
+}
+
 HostStage::~HostStage() {
     for (void* e : events_) rkh_event_destroy(e);
     rkh_host_free(ptr_);
@@ -156,14 +198,146 @@ int HostStage::download(void* stream, void* user, const void* device, size_t byt
 }
 int HostStage::finish_download(void* stream, void* user, size_t bytes) {
     if (!staged_) return rkh_sync(stream);
-    size_t i = 0;
-    for (size_t off = 0; off < bytes; off += kChunk, ++i) {
-        const size_t n = bytes - off < kChunk ? bytes - off : kChunk;
-        const int rc = rkh_event_sync(events_[i]);
-        if (rc) return rc;
-        std::memcpy(static_cast<uint8_t*>(user) + off, static_cast<uint8_t*>(ptr_) + off, n);
+    const size_t count = (bytes + kChunk - 1) / kChunk;
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{RKH_OK};
+    run_with_helpers(bytes, [&] {
+        size_t passed = 0; // chunks known to have arrived
+        for (int rc = RKH_OK;;) {
+            const size_t at = next.fetch_add(1) * kPiece;
+            if (at >= bytes) return;
+            const size_t n = std::min(kPiece, bytes - at);
+            for (; passed * kChunk < at + n && !rc; ++passed) rc = rkh_event_sync(events_[passed]);
+            if (rc) return failed.store(rc);
+            std::memcpy(static_cast<uint8_t*>(user) + at, static_cast<const uint8_t*>(ptr_) + at, n);
+        }
+    });
+    // (a copy that was given up leaves downloads behind that still write the mirror)
+    int rc = failed.load();
+    for (size_t i = 0; rc && i < count; ++i) rkh_event_sync(events_[i]);
+    return rc;
+}
+
+PanelPipe::~PanelPipe() {
+    for (std::vector<void*>* v : {&up_, &down_})
+        for (void* e : *v) rkh_event_destroy(e);
+    if (before_) rkh_event_destroy(before_);
+}
+// Panels are whole groups of 128 rows (where a panel's tiles and scales can begin) of about 2 MiB: smaller ones pay
+// the 9 us that a DMA takes beside its bytes more often, larger ones leave more of the first and the last alone.
+int PanelPipe::panel_rows(int M, size_t a_row, size_t c_row) {
+    constexpr int kGroup = RKH_ROW_ALIGN;
+    const size_t group = std::max(a_row, c_row) * kGroup;
+    const size_t rows = std::max<size_t>(1, ((size_t(2) << 20) + group / 2) / group) * kGroup;
+    return rows < (size_t)M ? (int)rows : 0;
+}
+bool PanelPipe::plan(size_t a_row, size_t c_row) {
+    const size_t a_bytes = M_ * a_row, c_bytes = M_ * c_row;
+    if (!left_ || a_bytes <= HostStage::kLimit || c_bytes <= HostStage::kOutLimit) return false;
+    rows_ = panel_rows(M_, a_row, c_row);
+    if (!rows_) return false;
+    a_row_ = a_row;
+    c_row_ = c_row;
+    panels_ = ((size_t)M_ + rows_ - 1) / rows_;
+    return panels_ <= down_.size();
+}
+void PanelPipe::init(const Owner& owner, int M, size_t a_row, size_t c_row) {
+    if (M * a_row <= HostStage::kLimit || M * c_row <= HostStage::kOutLimit || M * a_row > HostStage::kPipeLimit ||
+        M * c_row > HostStage::kPipeLimit)
+        return;
+    const int rows = panel_rows(M, a_row, c_row);
+    if (!rows) return;
+    rk_npu_ctx* ctx = owner.ctx;
+    if (!ctx->up_stream && rkh_stream_create(ctx->device, &ctx->up_stream) != RKH_OK) return;
+    if (!ctx->second_stream && rkh_stream_create(ctx->device, &ctx->second_stream) != RKH_OK) return;
+    const size_t panels = ((size_t)M + rows - 1) / rows;
+    if (rkh_event_create(&before_) != RKH_OK) return;
+    for (std::vector<void*>* v : {&up_, &down_})
+        for (size_t i = 0; i < panels; ++i) {
+            void* e = nullptr;
+            if (rkh_event_create(&e) != RKH_OK) return;
+            v->push_back(e);
+        }
+    M_ = M;
+    left_.reset(new (std::nothrow) std::atomic<int>[panels]);
+}
+
+int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const HostStage& a, const HostStage& c, uint8_t* a_dev,
+                   uint8_t* c_dev, const void* A, void* C, Check check, bool* rejected,
+                   const std::function<int(const Panel&)>& multiply, const std::function<int()>& last) {
+    const uint8_t* from = static_cast<const uint8_t*>(A);
+    uint8_t* to = static_cast<uint8_t*>(C);
+    uint8_t *a_pin = static_cast<uint8_t*>(a.data()), *c_pin = static_cast<uint8_t*>(c.data());
+    const size_t a_bytes = M_ * a_row_, c_bytes = M_ * c_row_, a_panel = rows_ * a_row_, c_panel = rows_ * c_row_;
+    // pieces of a panel, which end with it
+    const size_t a_pieces = (a_panel + kPiece - 1) / kPiece, c_pieces = (c_panel + kPiece - 1) / kPiece;
+    for (size_t p = 0; p < panels_; ++p) left_[p].store((int)a_pieces);
+    std::atomic<size_t> a_next{0}, c_next{0}, a_left{a_pieces * panels_}, enqueued{0};
+    std::atomic<bool> bad{false};
+    std::atomic<int> failed{RKH_OK};
+    // one piece of A into the mirror; false: all are taken
+    auto fetch = [&] {
+        const size_t i = a_next.fetch_add(1), p = i / a_pieces;
+        if (p >= panels_) return false;
+        const size_t at = p * a_panel + i % a_pieces * kPiece, end = std::min(std::min(at + kPiece, (p + 1) * a_panel), a_bytes);
+        if (at < end && !copy_checked(a_pin + at, from + at, end - at, check)) bad.store(true);
+        left_[p].fetch_sub(1);
+        a_left.fetch_sub(1);
+        return true;
+    };
+    // the results on to C, piece by piece as they arrive
+    auto deliver = [&] {
+        while (a_left.load()) std::this_thread::yield(); // (every row has been looked at)
+        if (bad.load()) return;
+        for (size_t passed = 0;;) {
+            const size_t i = c_next.fetch_add(1), p = i / c_pieces;
+            if (p >= panels_) return;
+            const size_t at = p * c_panel + i % c_pieces * kPiece, end = std::min(std::min(at + kPiece, (p + 1) * c_panel), c_bytes);
+            while (enqueued.load() <= p && !failed.load()) std::this_thread::yield();
+            for (; passed <= p && !failed.load(); ++passed)
+                if (const int rc = map_error(rkh_event_sync(down_[passed]))) failed.store(rc);
+            if (failed.load()) return;
+            if (at < end) std::memcpy(to + at, c_pin + at, end - at);
+        }
+    };
+    const std::thread::id caller = std::this_thread::get_id();
+    run_with_helpers(c_bytes + a_bytes, [&] {
+        if (std::this_thread::get_id() == caller) {
+            // (device calls made before this one on the workspace may still be using its buffers)
+            int rc = map_error(rkh_event_record(before_, ctx->stream));
+            if (!rc) rc = map_error(rkh_stream_wait(ctx->second_stream, before_));
+            for (size_t p = 0; p < panels_ && !rc; ++p) {
+                const int row = (int)p * rows_;
+                const Panel panel{row, std::min(rows_, M_ - row), a_dev + p * a_panel, c_dev + p * c_panel,
+                                  p % 2 ? ctx->second_stream : ctx->stream};
+                while (left_[p].load())
+                    if (!fetch()) std::this_thread::yield();
+                rc = map_error(rkh_h2d(ctx->up_stream, a_dev + p * a_panel, a_pin + p * a_panel, panel.rows * a_row_));
+                if (!rc) rc = map_error(rkh_event_record(up_[p], ctx->up_stream));
+                if (!rc) rc = map_error(rkh_stream_wait(panel.stream, up_[p]));
+                if (!rc) rc = multiply(panel);
+                if (!rc) rc = map_error(rkh_d2h(panel.stream, c_pin + p * c_panel, panel.c, panel.rows * c_row_));
+                if (!rc) rc = map_error(rkh_event_record(down_[p], panel.stream));
+                if (!rc) enqueued.store(p + 1);
+            }
+            // (the last panels of both streams)
+            for (size_t p = panels_ > 1 ? panels_ - 2 : 0; p < panels_ && !rc; ++p) rc = map_error(rkh_stream_wait(ctx->stream, down_[p]));
+            if (!rc) rc = last();
+            if (rc) failed.store(rc);
+            submit.unlock();
+        }
+        while (fetch()) {
+        }
+        deliver();
+    });
+    *rejected = bad.load();
+    // (the downloads have been waited for, unless C is not to be written; `last` has not)
+    if (*rejected || failed.load()) {
+        for (void* stream : {ctx->up_stream, ctx->stream, ctx->second_stream})
+            if (const int rc = map_error(rkh_sync(stream))) failed.store(rc);
+        return failed.load();
     }
-    return RKH_OK;
+    return map_error(rkh_sync(ctx->stream));
 }
 
 BadFlag::~BadFlag() { rkh_host_free(host_); }
@@ -265,6 +439,8 @@ rk_npu_ctx* rk_npu_open(const char* dev) {
 void rk_npu_close(rk_npu_ctx* ctx) {
     if (!ctx) return;
     abandon_profile(ctx); // (a context closed between profile_begin and profile_end)
+    rkh_stream_destroy(ctx->up_stream);
+    rkh_stream_destroy(ctx->second_stream);
     rkh_close(ctx->device, ctx->stream);
     {
         // graphs that outlive their context only keep their executable; graph_free releases it

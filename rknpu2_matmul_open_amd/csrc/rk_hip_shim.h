@@ -87,6 +87,9 @@ int rkh_event_create(void** event);
 void rkh_event_destroy(void* event);
 int rkh_event_record(void* event, void* stream);
 int rkh_event_sync(void* event);                                /* blocks until the event has happened */
+int rkh_stream_create(int device, void** stream);
+void rkh_stream_destroy(void* stream);
+int rkh_stream_wait(void* stream, void* event);                 /* what is enqueued next waits for the event */
 int rkh_event_elapsed_us(void* start, void* stop, double* us); /* waits for stop */
 
 /* ---- weight re-tiling at upload ---- */

@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -42,6 +43,10 @@ struct rk_npu_ctx {
     // Device work of one context is issued on one stream; submissions from
     // different workspaces are serialised here so stream order == call order.
     std::mutex submit_mutex;
+    // For panelled host calls (PanelPipe): uploads, and every second panel.  Made with the first workspace that is
+    // large enough for them, under submit_mutex.
+    void* up_stream = nullptr;
+    void* second_stream = nullptr;
     // Per-kernel profile (rk_npu_hip_profile_begin / _end): one stream event in front of every
     // kernel launched on this context's stream while it is on.
     struct ProfileMark {
@@ -182,8 +187,10 @@ private:
 //    straight into the output's mirror, which adds ~1.5 us to a call.
 //  * Up to kPipeLimit bytes: the mirror is a staging buffer.  Uploads memcpy a
 //    chunk and enqueue its DMA while the next chunk is being copied; downloads
-//    enqueue one DMA per chunk with an event behind it and memcpy each chunk to
-//    the caller's buffer as soon as its event has passed.
+//    enqueue one DMA per chunk with an event behind it, and each chunk is copied to
+//    the caller's buffer as soon as its event has passed, large results by several
+//    threads: one thread reads what a DMA has just written at 27 GB/s, half the
+//    rate of the DMA (16.8 MB 608 us; two threads 327, four 196, eight 140).
 // Beyond that, or when the pinned allocation fails, the calls copy from / to
 // the caller's buffer as the runtime sees fit.
 class HostStage {
@@ -220,6 +227,53 @@ private:
     size_t bytes_ = 0;
     std::vector<void*> events_; // one per chunk of a staged download
     bool staged_ = false;       // the enqueued download went through the mirror
+};
+
+// Large blocking calls on host buffers, in panels of rows: while one panel is multiplied, the next one is on its way
+// up and the last one's result on its way down (both directions together run at 95 GB/s, one alone at 55).
+// Quantization is by row and sums are exact, so the panels give the bits of the whole.
+//
+// What it is bound by: the download of a panel, 38 us for 2 MiB, and the copies between the caller's buffers and the
+// mirrors, 27 GB/s on one thread once the four buffers exceed its caches (three helpers that live as long as the call
+// share them).  2048 x 4096 x 4096 on int4 weights, fp16 in and out: 1295 us as upload, kernels and download one after
+// the other with one copying thread -> 930.
+// Uploads go by the copy engine on a stream of their own.  Downloads are kernels of the runtime, and a kernel that
+// reads or writes host memory holds up the end of every kernel beside it until it is over (GEMMs of 10 us took
+// 35 - 80, whether the copy had 256 workgroups or 32).  So the panels take two streams in turn, each with
+// quantization, GEMM and download in order: a panel's kernels end with the download of the panel before, and its own
+// download follows at once.  Downloads behind an event on a third stream left 15 - 30 us between two of them.
+class PanelPipe {
+public:
+    enum Check { ANY, FINITE_F16, FINITE_F32 }; // what the elements of A have to be for C to be written
+    PanelPipe() = default;
+    PanelPipe(const PanelPipe&) = delete;
+    PanelPipe& operator=(const PanelPipe&) = delete;
+    ~PanelPipe();
+    // a_row / c_row: most bytes that a row has on the host.  Stays off where no call has a use for panels or
+    // something could not be made.  The caller holds the context's submission lock.
+    void init(const Owner& owner, int M, size_t a_row, size_t c_row);
+    // Cuts one call, whose rows have this many bytes; false: it is better off, or has to go, in one piece.
+    bool plan(size_t a_row, size_t c_row);
+    struct Panel {
+        int row, rows;    // the first, a multiple of RKH_ROW_ALIGN, and how many
+        const void* a;    // its rows on the device
+        void* c;
+        void* stream;     // for its kernels, which another panel's may run beside: no scratch is shared
+    };
+    // The planned call: A through a's mirror to a_dev, `multiply` -> RK_NPU_* for each panel, c_dev through c's mirror to C,
+    // and at the end `last` on ctx->stream.  Gives the submission lock back when everything is enqueued.  `check` fails: C
+    // is not written and *rejected set.  Returns with nothing of the call under way.
+    int run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const HostStage& a, const HostStage& c, uint8_t* a_dev,
+            uint8_t* c_dev, const void* A, void* C, Check check, bool* rejected, const std::function<int(const Panel&)>& multiply,
+            const std::function<int()>& last);
+
+private:
+    static int panel_rows(int M, size_t a_row, size_t c_row);
+    int M_ = 0, rows_ = 0;
+    size_t a_row_ = 0, c_row_ = 0, panels_ = 0; // of the planned call
+    std::vector<void*> up_, down_;              // per panel: uploaded, downloaded
+    void* before_ = nullptr;                    // what was on the context's stream before the call
+    std::unique_ptr<std::atomic<int>[]> left_;  // per panel: pieces that are not in the mirror yet
 };
 
 // Blocking check of one raw device flag (used by rk_npu_hip_sync).

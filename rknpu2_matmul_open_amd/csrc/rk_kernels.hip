@@ -1292,6 +1292,22 @@ int rkh_event_sync(void* event) {
     RKH_CHECK(hipEventSynchronize((hipEvent_t)event));
     return RKH_OK;
 }
+int rkh_stream_create(int device, void** stream) {
+    RKH_CHECK(hipSetDevice(device));
+    hipStream_t st;
+    RKH_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    *stream = st;
+    return RKH_OK;
+}
+void rkh_stream_destroy(void* stream) {
+    if (!stream) return;
+    (void)hipStreamSynchronize((hipStream_t)stream);
+    (void)hipStreamDestroy((hipStream_t)stream);
+}
+int rkh_stream_wait(void* stream, void* event) {
+    RKH_CHECK(hipStreamWaitEvent((hipStream_t)stream, (hipEvent_t)event, 0));
+    return RKH_OK;
+}
 int rkh_event_elapsed_us(void* start, void* stop, double* us) {
     RKH_CHECK(hipEventSynchronize((hipEvent_t)stop));
     float ms = 0.0f;

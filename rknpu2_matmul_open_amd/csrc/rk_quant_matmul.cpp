@@ -119,50 +119,57 @@ struct rk_npu_matmul_workspace {
     DeviceBuffer c_out;    // [M, N] result before the copy back
     DeviceBuffer splitk;   // int32 scratch when the shape may split K
     HostStage stage_a, stage_scale, stage_c; // pinned mirrors of small A / static scales / C
+    PanelPipe pipe;                          // large host calls
     BadFlag flag;
     std::atomic_flag busy = ATOMIC_FLAG_INIT;
 };
 
 namespace {
 
-rkh_gemm_args gemm_args(rk_npu_matmul_workspace* ws, const Weights& w, void* dC) {
+// `rows` rows of the workspace's from row r0 on (a multiple of RKH_ROW_ALIGN) that dC holds.
+rkh_gemm_args gemm_args(rk_npu_matmul_workspace* ws, const Weights& w, void* dC, int r0, int rows) {
     const auto& s = ws->strategy;
     rkh_gemm_args g{};
-    g.A = ws->a_tiled.as<>();
+    g.A = ws->a_tiled.as<>() + rkh_tiled_i8_bytes(r0, s.K, RKH_ROW_ALIGN);
     g.W = w.tiled.as<>();
-    g.M = s.M;
+    g.M = rows;
     g.N = s.N;
     g.K = s.K;
-    g.a_scale = ws->a_scale.as<float>();
+    g.a_scale = ws->a_scale.as<float>() + r0;
     g.w_scale = w.w_scale.as<float>();
     g.epilogue = ws->t.out_epi;
     g.C = dC;
     g.ldc = s.N;
-    g.splitk_acc = ws->splitk ? ws->splitk.as<int32_t>() : nullptr;
+    // (panels, which run beside each other, share no scratch: their K is not split)
+    g.splitk_acc = ws->splitk && rows == s.M ? ws->splitk.as<int32_t>() : nullptr;
     return g;
 }
 
 // Enqueue quantize + GEMM on the context's stream (one fused kernel for
 // decode-sized M, unless A is a pinned host mirror).  dA / dC are device-
 // visible pointers; static scales are expected in the workspace's a_scale buffer.
-int enqueue(rk_npu_matmul_workspace* ws, const Weights& w, const void* dA, void* dC, bool a_is_host = false) {
+int enqueue_rows(rk_npu_matmul_workspace* ws, const Weights& w, const void* dA, void* dC, bool a_is_host, int r0, int rows,
+                 void* stream) {
     const auto& s = ws->strategy;
     rkh_quant_args q{};
     q.src = dA;
     q.src_is_host = a_is_host ? 1 : 0;
     q.in_dtype = ws->t.in_dtype;
     q.mode = ws->t.quant == 0 ? RKH_Q_COPY_I8 : ws->t.quant == 1 ? RKH_Q_W8_DYNAMIC : RKH_Q_W8_STATIC;
-    q.M = s.M;
+    q.M = rows;
     q.K = s.K;
-    q.scale = ws->t.quant == 0 ? nullptr : ws->a_scale.as<float>();
-    q.dst = ws->a_tiled.as<>();
-    const rkh_gemm_args g = gemm_args(ws, w, dC);
-    return map_error(rkh_quant_gemm(ws->owner.ctx->stream, &q, &g));
+    q.scale = ws->t.quant == 0 ? nullptr : ws->a_scale.as<float>() + r0;
+    q.dst = ws->a_tiled.as<>() + rkh_tiled_i8_bytes(r0, s.K, RKH_ROW_ALIGN);
+    const rkh_gemm_args g = gemm_args(ws, w, dC, r0, rows);
+    return map_error(rkh_quant_gemm(stream, &q, &g));
+}
+int enqueue(rk_npu_matmul_workspace* ws, const Weights& w, const void* dA, void* dC, bool a_is_host = false) {
+    return enqueue_rows(ws, w, dA, dC, a_is_host, 0, ws->strategy.M, ws->owner.ctx->stream);
 }
 
 // GEMV / GEMM stage on the activations already quantized into the workspace.
 int enqueue_gemm(rk_npu_matmul_workspace* ws, const Weights& w, void* dC) {
-    const rkh_gemm_args g = gemm_args(ws, w, dC);
+    const rkh_gemm_args g = gemm_args(ws, w, dC, 0, ws->strategy.M);
     return map_error(rkh_gemm(ws->owner.ctx->stream, &g));
 }
 
@@ -195,6 +202,17 @@ int run_host(rk_npu_matmul_workspace* ws, const Weights* w, rk_npu_matmul_op_kin
     const void* src = direct_in ? ws->stage_a.fill(A, a_bytes) : ws->a_raw.as<>();
     const void* scale_src = a_scale;
     if (ws->t.quant == 2 && ws->stage_scale) scale_src = ws->stage_scale.fill(a_scale, scale_bytes);
+    if (ws->stage_a && ws->stage_c && ws->pipe.plan(a_bytes / s.M, c_bytes / s.M)) {
+        std::unique_lock<std::mutex> submit(ctx->submit_mutex);
+        if (!ctx->capturing) { // (a capture knows the context's stream only)
+            if (ws->t.quant == 2) rc = map_error(rkh_h2d(ctx->stream, ws->a_scale.as<>(), scale_src, scale_bytes));
+            if (rc) return rc;
+            bool rejected;
+            return ws->pipe.run(ctx, submit, ws->stage_a, ws->stage_c, ws->a_raw.as<>(), ws->c_out.as<>(), A, C, PanelPipe::ANY, &rejected,
+                                [&](const PanelPipe::Panel& p) { return enqueue_rows(ws, *w, p.a, p.c, false, p.row, p.rows, p.stream); },
+                                [] { return RK_NPU_OK; });
+        }
+    }
     {
         std::lock_guard<std::mutex> submit(ctx->submit_mutex);
         if (!direct_in) rc = map_error(ws->stage_a.upload(ctx->stream, ws->a_raw.as<>(), A, a_bytes));
@@ -322,6 +340,7 @@ rk_npu_matmul_workspace* rk_npu_matmul_workspace_create(rk_npu_iommu_domain* dom
     ws->stage_a.init((size_t)M * K * elem_bytes(ws->t.in_dtype));
     if (ws->t.quant == 2) ws->stage_scale.init((size_t)M * sizeof(float));
     ws->stage_c.init((size_t)M * N * elem_bytes(out_dtype(ws->t.out_epi)));
+    ws->pipe.init(ws->owner, M, (size_t)K * elem_bytes(ws->t.in_dtype), (size_t)N * elem_bytes(out_dtype(ws->t.out_epi)));
     if (rkh_sync(domain->ctx->stream)) return nullptr;
     return ws.release();
 }

@@ -235,6 +235,7 @@ struct rk_npu_w4a8_workspace {
     DeviceBuffer row_max;   // [align128(M)][N/64] partial row maxima of the SwiGLU middle
     DeviceBuffer splitk;
     HostStage stage_a, stage_c; // pinned mirrors of a small A / C that the kernels read / write in place
+    PanelPipe pipe;             // large host calls
     BadFlag flag;
     std::atomic_flag busy = ATOMIC_FLAG_INIT;
     ~rk_npu_w4a8_workspace() {
@@ -260,7 +261,22 @@ enum class Out { F32, F16, I32, SwiGLU };
 int enqueue_gemm(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, void* dC, Out out,
                  bool collect);
 rkh_gemm_args gemm_args(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, void* dC, Out out,
-                        bool collect);
+                        bool collect, int r0, int rows);
+
+// `rows` rows of the workspace's from row r0 on (a multiple of RKH_ROW_ALIGN), which A holds.
+rkh_quant_args quant_args(rk_npu_w4a8_workspace* ws, const void* A, bool half, bool a_is_host, int r0, int rows) {
+    rkh_quant_args q{};
+    q.src = A;
+    q.src_is_host = a_is_host ? 1 : 0;
+    q.in_dtype = half ? RKH_F16 : RKH_F32;
+    q.mode = RKH_Q_W4A8;
+    q.M = rows;
+    q.K = ws->config.K;
+    q.scale = ws->a_scale.as<float>() + r0;
+    q.dst = ws->a_tiled.as<>() + rkh_tiled_i8_bytes(r0, ws->config.K, RKH_ROW_ALIGN);
+    q.bad_flag = ws->flag.device();
+    return q;
+}
 
 // quantize (or re-quantize with reused row maxima) + GEMM.  `scale_source`
 // non-null: A is the fp32 middle of that workspace's SwiGLU run and its
@@ -268,25 +284,14 @@ rkh_gemm_args gemm_args(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w,
 int enqueue(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, const void* dA, bool half,
             void* dC, Out out, bool collect, rk_npu_w4a8_workspace* scale_source,
             StageTimer* timer, bool a_is_host = false) {
-    const auto& c = ws->config;
     void* stream = ws->owner.ctx->stream;
-    rkh_quant_args q{};
-    q.src = dA;
-    q.src_is_host = a_is_host ? 1 : 0;
-    q.in_dtype = half ? RKH_F16 : RKH_F32;
-    q.M = c.M;
-    q.K = c.K;
-    q.scale = ws->a_scale.as<float>();
-    q.dst = ws->a_tiled.as<>();
-    q.bad_flag = ws->flag.device();
+    rkh_quant_args q = quant_args(ws, dA, half, a_is_host, 0, ws->config.M);
     if (scale_source) {
         q.mode = RKH_Q_REUSE_BITS;
         q.row_max_bits = scale_source->row_max.as<uint32_t>();
         q.row_max_parts = scale_source->config.N / 64; // one partial per 32 middle columns
-    } else {
-        q.mode = RKH_Q_W4A8;
     }
-    const rkh_gemm_args g = gemm_args(ws, w, dC, out, collect);
+    const rkh_gemm_args g = gemm_args(ws, w, dC, out, collect, 0, ws->config.M);
     int rc;
     if (timer) {
         // separate launches so the stage timer can tell the two apart
@@ -301,21 +306,22 @@ int enqueue(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, const void*
 }
 
 rkh_gemm_args gemm_args(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, void* dC, Out out,
-                        bool collect) {
+                        bool collect, int r0, int rows) {
     const auto& c = ws->config;
     rkh_gemm_args g{};
-    g.A = ws->a_tiled.as<>();
+    g.A = ws->a_tiled.as<>() + rkh_tiled_i8_bytes(r0, c.K, RKH_ROW_ALIGN);
     g.W = w->tiled.as<>();
     g.w_int4 = 1;
-    g.M = c.M;
+    g.M = rows;
     g.N = c.N;
     g.K = c.K;
     g.interleave_F = w->interleave_F;
-    g.a_scale = ws->a_scale.as<float>();
+    g.a_scale = ws->a_scale.as<float>() + r0;
     g.w_scale = w->w_scale.as<float>();
     g.w_colsum = w->colsum.as<int32_t>();
     g.C = dC;
-    g.splitk_acc = ws->splitk ? ws->splitk.as<int32_t>() : nullptr;
+    // (panels, which run beside each other, share no scratch: their K is not split)
+    g.splitk_acc = ws->splitk && rows == c.M ? ws->splitk.as<int32_t>() : nullptr;
     switch (out) {
     case Out::F32: g.epilogue = RKH_EPI_F32; g.ldc = c.N; break;
     case Out::F16: g.epilogue = RKH_EPI_F16; g.ldc = c.N; break;
@@ -332,7 +338,7 @@ rkh_gemm_args gemm_args(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w,
 // GEMV / GEMM stage on the activations already quantized into the workspace.
 int enqueue_gemm(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, void* dC, Out out,
                  bool collect) {
-    const rkh_gemm_args g = gemm_args(ws, w, dC, out, collect);
+    const rkh_gemm_args g = gemm_args(ws, w, dC, out, collect, 0, ws->config.M);
     return map_error(rkh_gemm(ws->owner.ctx->stream, &g));
 }
 
@@ -365,6 +371,23 @@ int run_host(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, const void
     const size_t a_bytes = (size_t)c.M * c.K * (half ? 2 : 4);
     const size_t out_cols = swiglu ? (size_t)c.N / 2 : (size_t)c.N;
     const size_t c_bytes = (size_t)c.M * out_cols * (out == Out::F16 ? 2 : 4);
+    // (K beyond 2^17 has to be split, for which panels have no scratch; timings are of one launch each)
+    if (!timings && c.K <= 131072 && ws->stage_a && ws->stage_c && ws->pipe.plan(a_bytes / c.M, c_bytes / c.M)) {
+        std::unique_lock<std::mutex> submit(ctx->submit_mutex);
+        if (!ctx->capturing) { // (a capture knows the context's stream only)
+            bool rejected;
+            rc = ws->pipe.run(ctx, submit, ws->stage_a, ws->stage_c, ws->a_raw.as<>(), ws->c_out.as<>(), A, C,
+                              half ? PanelPipe::FINITE_F16 : PanelPipe::FINITE_F32, &rejected, [&](const PanelPipe::Panel& p) {
+                                  const rkh_quant_args q = quant_args(ws, p.a, half, false, p.row, p.rows);
+                                  const rkh_gemm_args g = gemm_args(ws, w, p.c, out, false, p.row, p.rows);
+                                  return map_error(rkh_quant_gemm(p.stream, &q, &g));
+                              },
+                              [&] { return ws->flag.enqueue_readback(ctx->stream); });
+            if (rc) return rc;
+            // (the kernels find what the copy found: NaN / Inf activation, C is not written)
+            return ws->flag.consume(ctx->stream) || rejected ? RK_NPU_ERR_PARAM : RK_NPU_OK;
+        }
+    }
     StageTimer timer(ctx->stream, timings != nullptr);
     // Small operands skip the copies: the kernels read A from / write the result
     // into the pinned mirrors (the caller's C is only written after the checks).
@@ -631,6 +654,7 @@ rk_npu_w4a8_workspace* rk_npu_w4a8_workspace_create_ex(rk_npu_iommu_domain* doma
     if (scratch && ws->splitk.alloc(ws->owner, scratch)) return nullptr;
     ws->stage_a.init((size_t)M * K * 4);
     ws->stage_c.init((size_t)M * N * 4);
+    ws->pipe.init(ws->owner, M, (size_t)K * 4, (size_t)N * 4);
     if (rkh_sync(domain->ctx->stream)) return nullptr;
     return ws.release();
 }
