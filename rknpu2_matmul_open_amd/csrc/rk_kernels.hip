@@ -180,9 +180,8 @@ __host__ __device__ __forceinline__ int dealt_place(int b, int units, int log2_p
 }
 
 // 1 << log2_split workgroups share a row (row * split + part, dealt to the dies as `how` says), each taking a
-// contiguous range of its 16-element chunks.  Only the modes that do not scan the
-// row for its maximum are launched with split > 1: re-quantization finds the
-// maximum in the partial maxima the GEMM left behind, which every part reads.
+// contiguous range of its 16-element chunks.  Re-quantization finds the maximum in the partial maxima the GEMM left
+// behind, which every part reads; where the row has to be scanned for it, every part reads the row (quant_plan).
 // Bound by HBM, for few rows by latency.  What it was bound by: the codes went out as 16-byte
 // write-through stores from rows dealt round-robin over the dies.  Whole calls onto 1024 columns (us),
 // round-robin and written through -> contiguous rows, plain stores (either alone gives at most a third of it,
@@ -202,8 +201,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
     if (a.active_blocks && m >= a.active_blocks[0] * 32) return;
     const int K = a.K, KB = (int)(rkh_align_up(K, RKH_K_ALIGN) / 32);
     const int row_chunks = (K + 15) >> 4;
-    const int per_part = (row_chunks + split - 1) >> log2_split;
-    const int chunk0 = part * per_part;                         // this workgroup's chunks: chunk0 .. nchunks - 1
+    const bool need_max = a.mode == RKH_Q_W8_DYNAMIC || a.mode == RKH_Q_W4A8;
+    // (every part of a row that is scanned reads all of it and keeps its 256 chunks)
+    const int per_part = need_max ? row_chunks : (row_chunks + split - 1) >> log2_split;
+    const int chunk0 = need_max ? 0 : part * per_part;          // this workgroup's chunks: chunk0 .. nchunks - 1
     const int nchunks = min(row_chunks, chunk0 + per_part);
     const T* row = static_cast<const T*>(a.src) + (size_t)m * K;
     const bool vec = ((reinterpret_cast<uintptr_t>(row) & 15) == 0);
@@ -244,7 +245,6 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
         }
         return;
     }
-    const bool need_max = mode == RKH_Q_W8_DYNAMIC || mode == RKH_Q_W4A8;
     const bool check = mode == RKH_Q_W4A8;
 
     float v[QR_CACHE][16];
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(RK_QUANT_HEAD_PARAMS, i
 #pragma unroll
         for (int i = 0; i < QR_CACHE; ++i) {
             const int c = chunk0 + t + i * 256;
-            if (c < nchunks) emit(c, v[i]);
+            if (c < nchunks && (!need_max || split == 1 || i == part)) emit(c, v[i]);
         }
     } else {
         for (int c = chunk0 + t; c < nchunks; c += 256) {
@@ -1344,7 +1344,8 @@ struct QuantPlan {
     int log2_split; // ROWS: workgroups that share a row
     int how;        // WAVES, ROWS: DEAL_*
 };
-static QuantPlan quant_plan(const rkh_quant_args& a) {
+// `ahead`: the launch stands in front of a GEMM of the same request (rkh_quant_gemm), which waits for it.
+static QuantPlan quant_plan(const rkh_quant_args& a, bool ahead = false) {
     const int mode = a.mode;
     // Several rows per workgroup only while a row fits the registers its threads hold it in (8 rows:
     // 4096 elements, 4 rows: 8192): longer rows are read twice in a loop, and 256 rows of 11008 then
@@ -1383,6 +1384,20 @@ static QuantPlan quant_plan(const rkh_quant_args& a) {
     int log2_split = 0;
     if (reuse)
         while (log2_split < 3 && (a.M << log2_split) < 512 && (row_chunks >> (log2_split + 1)) >= 128) ++log2_split;
+    // Few long rows that have to be scanned: two or four workgroups per row, each of which reads all of it -- its loads,
+    // which are in flight at once, and the maximum are the same latency for one workgroup and for four -- and quantizes
+    // the 256 chunks that are its own.  us, fp16 rows, whole calls, weights from HBM: int8 16 x 14336 x 4096 17.3 -> 16.5, 32 x 11008
+    // 17.25 -> 16.8, 6 x 11008 13.8 -> 13.2, 128 x 14336 32.3 -> 31.8; int4 16 x 14336 14.1 -> 13.3, 8 x 14336 13.05 -> 12.15,
+    // 16 x 8192 10.05 -> 9.8.  Up to a workgroup per compute unit: beyond, and with rows that are fetched element by element,
+    // the repeated reads cost more (100 x 9001 onto 2048 columns 23.3 -> 25.9, 200 x 4100 13.6 -> 14.9, fp32 120 x 12001 26.5 -> 30.5;
+    // aligned 250 x 8000 14.6 -> 15.2, but 128 rows of 16384 26.6 -> 26.1).
+    if (ahead && (mode == RKH_Q_W8_DYNAMIC || mode == RKH_Q_W4A8) && a.in_dtype != RKH_I8 && row_chunks > 256 &&
+        row_chunks <= 256 * QR_CACHE) {
+        const int parts = row_chunks > 512 ? 2 : 1;
+        const bool aligned = a.K % (a.in_dtype == RKH_F32 ? 4 : 8) == 0 && (reinterpret_cast<uintptr_t>(a.src) & 15) == 0;
+        // (host memory is read once)
+        if (!a.src_is_host && (a.M << parts <= 256 || (aligned && parts == 2 && a.M <= 128))) log2_split = parts;
+    }
     if (a.active_blocks) return {QuantPlan::ROWS, (eights * 8) << log2_split, log2_split, DEAL_EIGHTS};
     // (Fewer than 256 int8 rows as given stay round-robin and written through: a few hundred KB without a maximum
     // to wait for, where the write-back at the kernel's end counts: 128 x 4096 -> 11008 columns 14.15 us, 14.35 - 14.55
@@ -1393,7 +1408,7 @@ static QuantPlan quant_plan(const rkh_quant_args& a) {
     // 300 x 4099 15.35 / 15.85 -> 15.2, 500 x 8191 25.0 / 25.1 -> 24.85.  Longer ones lose (512 x 9001 32.3 / 31.3 -> 35.2), and so
     // do aligned rows (250 x 14336 25.2 / 23.7 -> 26.6, 64 x 4096 9.45 / 8.75 -> 8.85) and many fp16 ones
     // (700 x 8191 44.3 / 34.0 -> 38.5).
-    if (unaligned && fits4 && !reuse) return {QuantPlan::ROWS, a.M, 0, DEAL_ROUND_ROBIN};
+    if (unaligned && fits4 && !reuse && !log2_split) return {QuantPlan::ROWS, a.M, 0, DEAL_ROUND_ROBIN};
     return {QuantPlan::ROWS, a.M << log2_split, log2_split, DEAL_RANGES};
 }
 
@@ -1415,9 +1430,7 @@ int rkh_quant_row_of(const rkh_quant_args* args, int workgroup, int* workgroups,
     return place >> p.log2_split;
 }
 
-int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
-    if (args->M <= 0) return RKH_OK;
-    const QuantPlan p = quant_plan(*args);
+static int launch_quant(void* stream, const rkh_quant_args* args, const QuantPlan& p) {
     const dim3 grid(p.grid), block(256);
     const hipStream_t st = (hipStream_t)stream;
     const bool fp16 = args->in_dtype == RKH_F16;
@@ -1449,6 +1462,9 @@ int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
     }
     RKH_CHECK(hipGetLastError());
     return RKH_OK;
+}
+int rkh_quant_rows(void* stream, const rkh_quant_args* args) {
+    return args->M > 0 ? launch_quant(stream, args, quant_plan(*args)) : RKH_OK;
 }
 
 // Dense launch plan: rows per workgroup follow M, shrinking while the output
@@ -1739,7 +1755,7 @@ int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_arg
     // (int8 rows of 9..128-row calls: letting the streaming kernel read them from their row-major source
     // instead of a tiled copy saves the re-tiling launch but was slower -- a lane's 16 bytes then come from
     // 32 different cache lines per load: 128 x 4096 x 11008 26.8 -> 35.7 us, 128 x 11008 x 4096 25.3 -> 29.7.)
-    const int rc = rkh_quant_rows(stream, qargs);
+    const int rc = qargs->M > 0 ? launch_quant(stream, qargs, quant_plan(*qargs, true)) : RKH_OK;
     return rc ? rc : rkh_gemm(stream, gargs);
 }
 

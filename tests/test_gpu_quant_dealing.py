@@ -63,3 +63,35 @@ def test_middle_of_an_ffn(sess, oracle, M, I):
     finally:
         for h in (gu_ws, dn_ws, gu_w, dn_w):
             h.close()
+
+
+@pytest.mark.parametrize("M,K", [(9, 16384), (9, 4097), (33, 4111), (64, 8193), (65, 8193), (64, 12289), (128, 4112), (129, 4112),
+                                 (128, 8208), (40, 16385)])
+def test_long_rows_shared_by_workgroups(sess, oracle, M, K):
+    """Scanned rows of more than 256 chunks: two or four workgroups each (the last part whole, one chunk, or without
+    any), the row counts where that ends, rows too long for it; a value that is not finite in the last part."""
+    N = 64
+    c = workloads.w4a8_case(M, K, N, seed_w=M, seed_a=K)
+    w, ws = ops.W4A8Weights(sess, c["B"], c["w_scale"]), ops.W4A8Workspace(sess, M, N, K)
+    A = c["A"].copy()
+    try:
+        for dtype in (np.uint16, np.float32):
+            X = A if dtype is np.uint16 else oracle.half_to_float(A).astype(np.float32).reshape(M, K)
+            # (the largest value of a row in one part, of the next row in another)
+            X[np.arange(M), (np.arange(M) * 4099 + K - 1) % K] = 0x5500 if dtype is np.uint16 else 80.0
+            dA, dC = sess.to_device(X), sess.empty_device(M * N * X.itemsize)
+            run = sess.lib.rk_npu_w4a8_run_f16_device if dtype is np.uint16 else sess.lib.rk_npu_w4a8_run_f32_device
+            assert run(ws.h, w.h, dA, dC) == 0 and sess.sync() == 0
+            got = sess.from_device(dC, (M, N), dtype)
+            want = oracle.w4a8(X, c["B"], c["w_scale"])["C"]
+            assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, dtype).view(np.uint8))
+            sess.free_device(dA)
+            X = X.copy()
+            X[M - 1, K - 1] = 0x7c00 if dtype is np.uint16 else np.inf
+            dA = sess.to_device(X)
+            assert run(ws.h, w.h, dA, dC) == 0 and sess.sync() == capi.RK_NPU_ERR_PARAM
+            sess.free_device(dA)
+            sess.free_device(dC)
+    finally:
+        ws.close()
+        w.close()
