@@ -801,9 +801,12 @@ __global__ __launch_bounds__(512) void moe_decode_gate_kernel(RK_MOE_DECODE_HEAD
     // ---- gate block 2j and up block 2j + 1 of the expert.  Two groups of PF tiles per wave and
     // block are in flight: the first is requested now, the second when the token is quantized (one
     // token per call gained 0.3 us with the second group requested between the barriers of the
-    // quantization, four and eight tokens lost 1.5 and 3.5 us).  The loads are unconditional -- past
-    // the end of the block a wave reads its last tile again and does not use it -- so that the
-    // compiler counts them and the quantization waits for the row only, not for the tiles.
+    // quantization, four and eight tokens lost 1.5 and 3.5 us).  The loads are unconditional, so that the
+    // compiler counts them and the quantization waits for the row only, not for the tiles; those past
+    // the end of the block are outside its descriptor and touch no memory.  (Where a wave read its last tile
+    // again instead, an int4 layer of 2048 x 1024 -- four tiles per wave, a second group of nothing -- sent as much again
+    // through the compute unit's memory path: with the same in the down kernel, 4 / 8 / 12 tokens 17.4 / 25.8 / 39.3 ->
+    // 16.5 / 23.9 / 35.9 us, int8 12 tokens 51.1 -> 49.8.)
     // Against the first group requested ahead of the row, behind branches, and the rest in the
     // loop: 17.8 -> 15.7 / 24.1 -> 23.8 / 37.3 -> 35.9 us for one / four / eight tokens (both launches).
     const int e = slot.expert;
@@ -814,13 +817,17 @@ __global__ __launch_bounds__(512) void moe_decode_gate_kernel(RK_MOE_DECODE_HEAD
                               : a.gate_W + (size_t)(e - a.int4_experts) * a.gate_stride) + (size_t)(2 * j) * block_bytes;
     constexpr int PF = MOE_DECODE_PREFETCH;
     v4i cur[2][PF], nxt[2][PF];
+    __amdgpu_buffer_rsrc_t rsrc[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+        rsrc[b] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wb) + b * block_bytes, 0, (int)block_bytes, 0x00020000);
     auto load_group = [&](v4i (*regs)[PF], int grp) {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            const int idx = min(wave + 8 * (grp * PF + u), tiles - 1);
+            const int idx = wave + 8 * (grp * PF + u);
 #pragma unroll
             for (int b = 0; b < 2; ++b)
-                regs[b][u] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wb + b * block_bytes + (size_t)idx * 1024 + lane * 16));
+                regs[b][u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc[b], idx * 1024 + lane * 16, 0, 2 /* streaming */));
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -960,22 +967,24 @@ __global__ __launch_bounds__(512) void moe_decode_down_kernel(RK_MOE_DECODE_HEAD
     // a slot's tiles are walked in groups of 8 waves x PF tiles
     constexpr int PF = MOE_DECODE_PREFETCH;
     auto block_of = [&](int li, bool& int4, int& tiles) -> const uint8_t* {
-        const int e = live_expert[li];
+        const int e = __builtin_amdgcn_readfirstlane(live_expert[li]);
         int4 = e < a.int4_experts;
         tiles = int4 ? Ip / 64 : Ip / 32;
         return (int4 ? a.down_W4 + (size_t)e * a.down_stride4
                      : a.down_W + (size_t)(e - a.int4_experts) * a.down_stride) + (size_t)pb * tiles * 1024;
     };
-    // (unconditional loads -- past the end of a block a lane reads the block's last tile again and does
-    // not use it -- so that the compiler counts them: a wait for older data then leaves them in flight)
+    // (unconditional loads, so that the compiler counts them -- a wait for older data then leaves them in flight --
+    // through the block's descriptor: those past its end touch no memory.  A ring of eight tiles per wave across
+    // the slots, all of them with work, was slower: its bookkeeping per tile, 8 tokens 23.9 -> 29.6 us.)
     auto load_group = [&](int li, int grp, v4i* regs) {
         bool int4;
         int tiles;
         const uint8_t* wb = block_of(li, int4, tiles);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wb), 0, tiles * 1024, 0x00020000);
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            const int tile = min(((grp * PF + u) * 8 + wave) * TPL + sub, tiles - 1);
-            regs[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wb + (size_t)tile * 1024 + lane_byte));
+            const int tile = ((grp * PF + u) * 8 + wave) * TPL + sub;
+            regs[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(tile * 1024 + lane_byte), 0, 2 /* streaming */));
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -1051,9 +1060,9 @@ __global__ __launch_bounds__(512) void moe_decode_down_kernel(RK_MOE_DECODE_HEAD
         const uint8_t* codes = a_lds + (size_t)li * Ip;
         int acc = 0;
         for (int grp = 0; grp < groups; ++grp) {
-            // the next group: of this slot, else the first of the next slot, else (nothing left) this one again
+            // the next group: of this slot, else the first of the next slot, else (nothing left) one past the end
             const bool last = grp + 1 == groups, more = li + 1 < nlive;
-            load_group(last && more ? li + 1 : li, last ? (more ? 0 : grp) : grp + 1, nxt);
+            load_group(last && more ? li + 1 : li, last ? (more ? 0 : groups) : grp + 1, nxt);
 #pragma unroll
             for (int u = 0; u < PF; ++u) {
                 const int tile = ((grp * PF + u) * 8 + wave) * TPL + sub;

@@ -222,3 +222,11 @@ def test_random_geometries(sess, oracle):
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), what
         finally:
             moe.close()
+
+
+@pytest.mark.parametrize("T,H,I,flavour", [(1, 1024, 1024, "w8"), (4, 1280, 1280, "w8"), (3, 2304, 3584, "w8"), (4, 2048, 2048, "quant"),
+                                           (2, 2304, 2304, "quant"), (5, 4352, 256, "quant")])
+def test_ends_of_tile_groups(sess, oracle, T, H, I, flavour):
+    """Column blocks of exactly a group of tiles of the eight waves, a few tiles more, several groups, the longest
+    middle: what a wave loads past a block's end must not count."""
+    test_decode_sized_calls_bit_exact(sess, oracle, T, H, I, 5, 3, 0, flavour)
