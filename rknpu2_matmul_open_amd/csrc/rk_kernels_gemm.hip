@@ -166,11 +166,25 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     v4i afr[2][4];            // activation fragments (index u * TM + i), this sub-step / next
     v4i wop[2][NWOP];         // int4 only: unpacked operands (index u * TN + j), this sub-step / next
 
+    // Copies beyond K are issued like the others, for the count.  Tiles of 64 x 128 with int8 weights, which are bound by
+    // the compute unit's memory path, issue them for one lane: twelve sub-steps of 8 KiB that nothing reads, beside the
+    // 32 of K = 4096.  us, quantization included: 256 rows x 4096 x 4096 19.5 -> 18.8, 128 x 6144 x 11008 29.0 -> 28.2,
+    // 128 x 4096 x 11008 exact 14.0 -> 13.8, 512 x 14336 x 4096 54.8 -> 54.1.  Int4 weights, whose bytes are fewer, lose
+    // what the scalar instructions cost (256 x 4096 x 4096 13.3 -> 13.5), 128-row tiles gain nothing (1000 x 2048 x 3000
+    // 15.5 -> 15.6), and neither do the weights, of which three sub-steps lie beyond K.
+    constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
+    [[maybe_unused]] unsigned long long a_lanes = ~0ull;
     auto copy_a = [&](int buf) { // global -> LDS, 16 bytes per lane, lane-contiguous
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(asrc),
-                     "s"(copy_dst + buf * BUF)
-                     : "memory", "m0");
+        if constexpr (MASKED)    // (every lane is active here, and is again behind the copy)
+            asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lane_off),
+                         "s"(asrc), "s"(copy_dst + buf * BUF), "s"(a_lanes)
+                         : "memory", "m0");
+        else
+            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(asrc),
+                         "s"(copy_dst + buf * BUF)
+                         : "memory", "m0");
         asrc += a_left > 0 ? A_STEP : 0;
+        if constexpr (MASKED) a_lanes = a_left > 0 ? ~0ull : 1ull;
         --a_left;
     };
     auto load_w = [&](wraw_t* regs) {

@@ -39,3 +39,16 @@ def test_int4_weights(sess, oracle, M, N, K):
     finally:
         ws.close()
         w.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 2100, 40), (130, 4100, 512), (300, 3000, 1537), (320, 2900, 1792)])
+def test_fewer_sub_steps_than_the_look_ahead(sess, oracle, M, N, K):
+    """K of 2, 4, 14 (both) sub-steps where copies run twelve ahead: what is issued beyond K must not count."""
+    c = workloads.w8a8_case(2, K, N, seed_w=M, seed_a=K)
+    A = np.random.default_rng(K).integers(-128, 128, (M, K)).astype(np.int8)
+    op = ops.W8A8Linear(sess, capi.I8I8I32, M, c["B"])
+    try:
+        rc, got = op.run(A)
+        assert rc == 0 and np.array_equal(got, oracle.gemm_i8(A, c["B"]))
+    finally:
+        op.close()
