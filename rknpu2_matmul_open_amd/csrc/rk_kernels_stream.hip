@@ -31,7 +31,8 @@ namespace {
 // bank may hold int4 and int8 experts (routed INT4, shared int8): each format
 // has its launch over the same grid, and a workgroup whose row block belongs to
 // an expert of the other format exits at once.
-template <int EPI, int KS, bool W4, bool BAL = false, int TN = 2, int TM = 1>
+// DEEP: a balanced launch with few units per compute unit (launch_gemm_grouped).
+template <int EPI, int KS, bool W4, bool BAL = false, int TN = 2, int TM = 1, bool DEEP = false>
 __global__ __launch_bounds__(BAL ? 512 : 256) void gemm_stream_kernel(RK_GEMM_HEAD_PARAMS, int mblocks, int nblocks,
                                                                       rkh_gemm_args g) {
     RK_GEMM_HEAD_APPLY(g);
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(BAL ? 512 : 256) void gemm_stream_kernel(RK_GEMM_HE
     // it waits out a full memory latency per step: int8 128 x 4096 x 11008 took 37.9 us with 2,
     // 25.5 with 4, 25.9 with 8 (x 14336: 39.1 / 27.2 / 28.3).
     // (two row blocks per wave: four as well -- six and eight steps measured the same or slower)
-    constexpr int RING = KSPLIT ? 4 : BAL ? 2 : 4;
+    constexpr int RING = KSPLIT ? 4 : BAL && !DEEP ? 2 : 4;
     constexpr int AT = W4 ? 2 : 1;   // activation tiles per step
     constexpr int LPS = AT * TM + TN; // loads per step: TM activation tiles (int4: pairs), TN weight tiles
     static_assert((RING - 1) * LPS <= 63, "vmcnt field");
@@ -371,8 +372,21 @@ int launch_gemm_grouped(hipStream_t st, const rkh_gemm_args& g) {
 #define RK_LAUNCH_BAL(EPI)                                                                                          \
     do {                                                                                                            \
         if (any_int4) hipLaunchKernelGGL((gemm_stream_kernel<EPI, 1, true, true>), grid, block, 0, st, RK_GEMM_HEAD(g), mblocks, nblocks, g);  \
-        if (any_int8) hipLaunchKernelGGL((gemm_stream_kernel<EPI, 1, false, true>), grid, block, 0, st, RK_GEMM_HEAD(g), mblocks, nblocks, g); \
+        if (any_int8 && deep) {                                                                                     \
+            if constexpr (EPI == RKH_EPI_SWIGLU)                                                                    \
+                hipLaunchKernelGGL((gemm_stream_kernel<EPI, 1, false, true, 2, 1, true>), grid, block, 0, st, RK_GEMM_HEAD(g), mblocks, nblocks, g); \
+        } else if (any_int8)                                                                                        \
+            hipLaunchKernelGGL((gemm_stream_kernel<EPI, 1, false, true>), grid, block, 0, st, RK_GEMM_HEAD(g), mblocks, nblocks, g); \
     } while (0)
+        // Steps of a wave in flight: with at most six and a half units per compute unit (as many as the call can have) two
+        // steps of so few waves are too little for HBM, with more they are enough and a deeper ring only queues.  int8
+        // gate/up, whole layers, us, two -> four steps; units per compute unit: 4.5 (32 tokens, 32 experts, top-4, 2048 x 1024)
+        // 58.6 -> 56.9, 5 (256 tokens, 16 experts, top-8, 4096 x 512) 93.5 -> 84.1, 5.1 (100, 16, 8, 4096 x 1024) 87.2 -> 78.5, 6 (256, 64, 4,
+        // 2048 x 512) 67.3 -> 65.7, 6.5 (160, 32, 4, 2048 x 1024) 63.2 -> 61.8; 7 (192) 64.1 -> 64.1, 8 (256) 68.0 -> 69.9, 8.6 (200, 32, 6)
+        // 74.0 -> 76.5, 12 (256, 32, 8) 97.3 -> 98.7.  K up to 1024 gives no such line (6.5 (20, 50, 4, 1024 x 1024) 43.1 -> 43.6, 8 (256, 64,
+        // 8, 1024 x 512) 47.0 -> 48.1, 13.8 (200, 60, 8, 1024 x 1024) 73.7 -> 67.8).  Int4 weights (37.0 -> 38.0 at 128 tokens) keep two, and
+        // so does the down projection, which gains half as much and loses sooner.
+        const bool deep = g.epilogue == RKH_EPI_SWIGLU && g.K > 1024 && (long)mblocks * ((g.N + 63) / 64) * 2 <= 13L * cus;
         switch (g.epilogue) { // (grouped GEMMs are the MoE layer's: gate/up + SwiGLU and the fp32 down projection)
         case RKH_EPI_F32: RK_LAUNCH_BAL(RKH_EPI_F32); break;
         case RKH_EPI_SWIGLU: RK_LAUNCH_BAL(RKH_EPI_SWIGLU); break;
