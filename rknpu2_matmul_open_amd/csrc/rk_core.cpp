@@ -340,6 +340,15 @@ int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const 
     return map_error(rkh_sync(ctx->stream));
 }
 
+bool keeps_to_stream(rk_npu_ctx* ctx) {
+    {
+        std::lock_guard<std::mutex> lock(ctx->profile_mutex);
+        if (ctx->profiling) return true;
+    }
+    std::lock_guard<std::mutex> lock(ctx->pending_mutex);
+    return ctx->capturing;
+}
+
 BadFlag::~BadFlag() { rkh_host_free(host_); }
 int BadFlag::init(const Owner& owner) {
     int rc = dev_.alloc(owner, sizeof(int), true);

@@ -276,6 +276,9 @@ private:
     std::unique_ptr<std::atomic<int>[]> left_;  // per panel: pieces that are not in the mirror yet
 };
 
+// A capture or a per-kernel profile is on, which know the context's stream only: calls keep to it.
+bool keeps_to_stream(rk_npu_ctx* ctx);
+
 // Blocking check of one raw device flag (used by rk_npu_hip_sync).
 bool consume_device_flag(rk_npu_ctx* ctx, int* flag);
 void note_pending_flag(rk_npu_ctx* ctx, int* flag);

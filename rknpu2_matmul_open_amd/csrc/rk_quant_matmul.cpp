@@ -204,7 +204,7 @@ int run_host(rk_npu_matmul_workspace* ws, const Weights* w, rk_npu_matmul_op_kin
     if (ws->t.quant == 2 && ws->stage_scale) scale_src = ws->stage_scale.fill(a_scale, scale_bytes);
     if (ws->stage_a && ws->stage_c && ws->pipe.plan(a_bytes / s.M, c_bytes / s.M)) {
         std::unique_lock<std::mutex> submit(ctx->submit_mutex);
-        if (!ctx->capturing) { // (a capture knows the context's stream only)
+        if (!keeps_to_stream(ctx)) {
             if (ws->t.quant == 2) rc = map_error(rkh_h2d(ctx->stream, ws->a_scale.as<>(), scale_src, scale_bytes));
             if (rc) return rc;
             bool rejected;

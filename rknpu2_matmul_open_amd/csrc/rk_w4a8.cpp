@@ -374,7 +374,7 @@ int run_host(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, const void
     // (K beyond 2^17 has to be split, for which panels have no scratch; timings are of one launch each)
     if (!timings && c.K <= 131072 && ws->stage_a && ws->stage_c && ws->pipe.plan(a_bytes / c.M, c_bytes / c.M)) {
         std::unique_lock<std::mutex> submit(ctx->submit_mutex);
-        if (!ctx->capturing) { // (a capture knows the context's stream only)
+        if (!keeps_to_stream(ctx)) {
             bool rejected;
             rc = ws->pipe.run(ctx, submit, ws->stage_a, ws->stage_c, ws->a_raw.as<>(), ws->c_out.as<>(), A, C,
                               half ? PanelPipe::FINITE_F16 : PanelPipe::FINITE_F32, &rejected, [&](const PanelPipe::Panel& p) {

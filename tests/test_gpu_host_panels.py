@@ -88,3 +88,21 @@ def test_two_threads(sess, oracle):
     finally:
         for op in lin:
             op.close()
+
+
+def test_a_profile_sees_every_kernel(sess, oracle):
+    """While a per-kernel profile is on, which marks the context's stream, the call runs on it in one piece."""
+    import ctypes as C
+    M = 389
+    c = workloads.w8a8_case(2, K, N, seed_w=3, seed_a=1)
+    A = workloads.normal_f32(5, (M, K))
+    op = ops.W8A8Linear(sess, capi.F32I8F32_DYNAMIC, M, c["B"], c["w_scale"])
+    buf, us = C.create_string_buffer(4096), (C.c_double * 16)()
+    try:
+        assert sess.lib.rk_npu_hip_profile_begin(sess.ctx) == 0
+        rc, got = op.run(A)
+        n = sess.lib.rk_npu_hip_profile_end(sess.ctx, buf, len(buf), us, 16)
+        assert rc == 0 and 2 <= n <= 3  # quantization, GEMM and, if its K is split, the sum of the parts
+        assert np.array_equal(got.view(np.uint32), oracle.w8a8(A, c["B"], c["w_scale"])["C"].view(np.uint32))
+    finally:
+        op.close()
