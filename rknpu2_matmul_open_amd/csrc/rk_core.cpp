@@ -263,8 +263,8 @@ void PanelPipe::init(const Owner& owner, int M, size_t a_row, size_t c_row) {
 }
 
 int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const HostStage& a, const HostStage& c, uint8_t* a_dev,
-                   uint8_t* c_dev, const void* A, void* C, Check check, bool* rejected,
-                   const std::function<int(const Panel&)>& multiply, const std::function<int()>& last) {
+                   uint8_t* c_dev, const void* A, void* C, Check check, BadFlag* flag, bool* rejected,
+                   const std::function<int(const Panel&)>& multiply) {
     const uint8_t* from = static_cast<const uint8_t*>(A);
     uint8_t* to = static_cast<uint8_t*>(C);
     uint8_t *a_pin = static_cast<uint8_t*>(a.data()), *c_pin = static_cast<uint8_t*>(c.data());
@@ -296,15 +296,17 @@ int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const 
             while (enqueued.load() <= p && !failed.load()) std::this_thread::yield();
             for (; passed <= p && !failed.load(); ++passed)
                 if (const int rc = map_error(rkh_event_sync(down_[passed]))) failed.store(rc);
-            if (failed.load()) return;
+            // (the flag's read-back stands ahead of the first panel on the same stream)
+            if (failed.load() || (flag && flag->raised())) return;
             if (at < end) std::memcpy(to + at, c_pin + at, end - at);
         }
     };
     const std::thread::id caller = std::this_thread::get_id();
     run_with_helpers(c_bytes + a_bytes, [&] {
         if (std::this_thread::get_id() == caller) {
+            int rc = flag ? flag->enqueue_readback(ctx->stream) : RK_NPU_OK;
             // (device calls made before this one on the workspace may still be using its buffers)
-            int rc = map_error(rkh_event_record(before_, ctx->stream));
+            if (!rc) rc = map_error(rkh_event_record(before_, ctx->stream));
             if (!rc) rc = map_error(rkh_stream_wait(ctx->second_stream, before_));
             for (size_t p = 0; p < panels_ && !rc; ++p) {
                 const int row = (int)p * rows_;
@@ -322,7 +324,6 @@ int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const 
             }
             // (the last panels of both streams)
             for (size_t p = panels_ > 1 ? panels_ - 2 : 0; p < panels_ && !rc; ++p) rc = map_error(rkh_stream_wait(ctx->stream, down_[p]));
-            if (!rc) rc = last();
             if (rc) failed.store(rc);
             submit.unlock();
         }
@@ -330,13 +331,13 @@ int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const 
         }
         deliver();
     });
-    *rejected = bad.load();
-    // (the downloads have been waited for, unless C is not to be written; `last` has not)
-    if (*rejected || failed.load()) {
+    // (the downloads have been waited for, unless C is not to be written)
+    if (failed.load() || bad.load() || (flag && flag->raised()))
         for (void* stream : {ctx->up_stream, ctx->stream, ctx->second_stream})
             if (const int rc = map_error(rkh_sync(stream))) failed.store(rc);
-        return failed.load();
-    }
+    *rejected = bad.load() || (flag && flag->raised());
+    if (failed.load()) return failed.load();
+    if (*rejected) flag->rearm(ctx->stream); // (the kernels have raised it too where the copy found something)
     return map_error(rkh_sync(ctx->stream));
 }
 
@@ -363,10 +364,14 @@ int BadFlag::init(const Owner& owner) {
 int BadFlag::enqueue_readback(void* stream) {
     return map_error(rkh_d2h(stream, host_, dev_.as<>(), sizeof(int)));
 }
-bool BadFlag::consume(void* stream) {
-    if (!*host_) return false;
+bool BadFlag::raised() const { return *static_cast<const volatile int*>(host_) != 0; }
+void BadFlag::rearm(void* stream) {
     *host_ = 0;
     rkh_fill32(stream, dev_.as<>(), 0u, 1);
+}
+bool BadFlag::consume(void* stream) {
+    if (!raised()) return false;
+    rearm(stream);
     return true;
 }
 bool consume_device_flag(rk_npu_ctx* ctx, int* flag) {

@@ -169,6 +169,8 @@ public:
     int init(const Owner& owner);
     int* device() const { return dev_.as<int>(); }
     int enqueue_readback(void* stream);
+    bool raised() const; // as of the last read-back that has arrived
+    void rearm(void* stream);
     // After the stream wait: true when input was rejected; re-arms the flag.
     bool consume(void* stream);
 
@@ -260,12 +262,13 @@ public:
         void* c;
         void* stream;     // for its kernels, which another panel's may run beside: no scratch is shared
     };
-    // The planned call: A through a's mirror to a_dev, `multiply` -> RK_NPU_* for each panel, c_dev through c's mirror to C,
-    // and at the end `last` on ctx->stream.  Gives the submission lock back when everything is enqueued.  `check` fails: C
-    // is not written and *rejected set.  Returns with nothing of the call under way.
+    // The planned call: A through a's mirror to a_dev, `multiply` -> RK_NPU_* for each panel, c_dev through c's mirror to C.
+    // Gives the submission lock back when everything is enqueued.  `check` fails, or an earlier device call on the
+    // workspace has raised `flag` (null where there is nothing to check): C is not written, *rejected set and the flag
+    // re-armed.  Returns with nothing of the call under way.
     int run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const HostStage& a, const HostStage& c, uint8_t* a_dev,
-            uint8_t* c_dev, const void* A, void* C, Check check, bool* rejected, const std::function<int(const Panel&)>& multiply,
-            const std::function<int()>& last);
+            uint8_t* c_dev, const void* A, void* C, Check check, BadFlag* flag, bool* rejected,
+            const std::function<int(const Panel&)>& multiply);
 
 private:
     static int panel_rows(int M, size_t a_row, size_t c_row);

@@ -377,15 +377,13 @@ int run_host(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, const void
         if (!keeps_to_stream(ctx)) {
             bool rejected;
             rc = ws->pipe.run(ctx, submit, ws->stage_a, ws->stage_c, ws->a_raw.as<>(), ws->c_out.as<>(), A, C,
-                              half ? PanelPipe::FINITE_F16 : PanelPipe::FINITE_F32, &rejected, [&](const PanelPipe::Panel& p) {
+                              half ? PanelPipe::FINITE_F16 : PanelPipe::FINITE_F32, &ws->flag, &rejected,
+                              [&](const PanelPipe::Panel& p) {
                                   const rkh_quant_args q = quant_args(ws, p.a, half, false, p.row, p.rows);
                                   const rkh_gemm_args g = gemm_args(ws, w, p.c, out, false, p.row, p.rows);
                                   return map_error(rkh_quant_gemm(p.stream, &q, &g));
-                              },
-                              [&] { return ws->flag.enqueue_readback(ctx->stream); });
-            if (rc) return rc;
-            // (the kernels find what the copy found: NaN / Inf activation, C is not written)
-            return ws->flag.consume(ctx->stream) || rejected ? RK_NPU_ERR_PARAM : RK_NPU_OK;
+                              });
+            return rc ? rc : rejected ? RK_NPU_ERR_PARAM : RK_NPU_OK; // NaN / Inf activation: C is not written
         }
     }
     StageTimer timer(ctx->stream, timings != nullptr);

@@ -1,0 +1,180 @@
+// The host layer's large blocking calls over a device made of host memory: the shim below does at once, on the calling
+// thread, what the HIP side enqueues.  One check per run, named by the argument; ends with 0 or says what is wrong.
+#include <dlfcn.h>
+#include <pthread.h>
+#include <sched.h>
+#include <unistd.h>
+
+#include <atomic>
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <limits>
+#include <new>
+#include <vector>
+
+#include "rk_hip_shim.h"
+#include "rk_npu_hip.h"
+
+static std::atomic<int> g_threads{0};
+static std::atomic<int> g_syncs{0};          // waits for the context's stream
+static std::atomic<long> g_allocations{-1};  // allocations that still succeed; -1: all of them
+static char g_streams[3];                    // [0]: the context's
+static int g_made = 1;
+
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* x) {
+    static auto real = (int (*)(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*))dlsym(RTLD_NEXT, "pthread_create");
+    ++g_threads;
+    return real(t, a, f, x);
+}
+static bool may_allocate() { return g_allocations < 0 || g_allocations-- > 0; }
+void* operator new(size_t n) {
+    if (void* p = may_allocate() ? std::malloc(n ? n : 1) : nullptr) return p;
+    throw std::bad_alloc();
+}
+void* operator new(size_t n, const std::nothrow_t&) noexcept { return may_allocate() ? std::malloc(n ? n : 1) : nullptr; }
+void* operator new[](size_t n) { return operator new(n); }
+void* operator new[](size_t n, const std::nothrow_t& t) noexcept { return operator new(n, t); }
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+void operator delete[](void* p) noexcept { std::free(p); }
+void operator delete[](void* p, size_t) noexcept { std::free(p); }
+
+extern "C" {
+int rkh_device_count(void) { return 1; }
+int rkh_open(int, void** s, char* name, int, int* cus, int* khz) {
+    *s = g_streams;
+    name[0] = 0;
+    *cus = *khz = 1;
+    return RKH_OK;
+}
+void rkh_close(int, void*) {}
+int rkh_malloc(int, void** p, size_t n) { return (*p = std::malloc(n)) ? RKH_OK : RKH_ERR_NOMEM; }
+void rkh_free(int, void* p) { std::free(p); }
+int rkh_host_alloc(void** p, size_t n) { return rkh_malloc(0, p, n); }
+void rkh_host_free(void* p) { std::free(p); }
+int rkh_h2d(void*, void* d, const void* s, size_t n) { return std::memcpy(d, s, n), RKH_OK; }
+int rkh_d2h(void*, void* d, const void* s, size_t n) { return std::memcpy(d, s, n), RKH_OK; }
+int rkh_fill32(void*, void* d, uint32_t v, size_t n) {
+    for (size_t i = 0; i < n; ++i) static_cast<uint32_t*>(d)[i] = v;
+    return RKH_OK;
+}
+int rkh_sync(void* s) {
+    if (s == g_streams) ++g_syncs;
+    return RKH_OK;
+}
+int rkh_event_create(void** e) { return rkh_malloc(0, e, 1); }
+void rkh_event_destroy(void* e) { std::free(e); }
+int rkh_event_record(void*, void*) { return RKH_OK; }
+int rkh_event_sync(void*) { return RKH_OK; }
+int rkh_stream_create(int, void** s) { return *s = g_streams + g_made++, RKH_OK; }
+void rkh_stream_destroy(void*) {}
+int rkh_stream_wait(void*, void*) { return RKH_OK; }
+int rkh_static_scratch(int, void**, size_t*) { return RKH_ERR_RUNTIME; }
+void rkh_set_marker(rkh_marker_fn, void*) {}
+size_t rkh_gemm_scratch_bytes(int, int, int, int) { return 0; }
+int rkh_pack_w4(void*, const int8_t*, int, int, int, uint8_t*, int*, int32_t*) { return RKH_OK; }
+int rkh_pack_w8(void*, const int8_t*, int, int, int, uint8_t*) { return RKH_OK; }
+// C[m][n] = A[m][n % K], both fp32
+int rkh_quant_gemm(void*, const rkh_quant_args* q, const rkh_gemm_args* g) {
+    for (int m = 0; m < q->M; ++m) {
+        const float* a = static_cast<const float*>(q->src) + (size_t)m * q->K;
+        for (int k = 0; k < q->K; ++k)
+            if (q->mode == RKH_Q_W4A8 && !std::isfinite(a[k])) *q->bad_flag = 1;
+        for (int n = 0; n < g->N; ++n) static_cast<float*>(g->C)[(size_t)m * g->N + n] = a[n % q->K];
+    }
+    return RKH_OK;
+}
+int rkh_quant_rows(void*, const rkh_quant_args*) { return RKH_ERR_RUNTIME; }
+int rkh_gemm(void*, const rkh_gemm_args*) { return RKH_ERR_RUNTIME; }
+}
+
+#define CHECK(x)                                                         \
+    do {                                                                 \
+        if (!(x)) {                                                      \
+            std::fprintf(stderr, "line %d: %s\n", __LINE__, #x);         \
+            return 1;                                                    \
+        }                                                                \
+    } while (0)
+
+static constexpr int M = 1000, K = 1100, N = 4224; // A 4.4 MB, C 16.9 MB
+
+struct Calls {
+    rk_npu_ctx* ctx = rk_npu_open(nullptr);
+    rk_npu_iommu_domain* domain = rk_npu_iommu_domain_create(ctx, 0);
+    std::vector<float> A, C;
+    rk_npu_w4a8_weights* w4 = nullptr;
+    rk_npu_w4a8_workspace* ws4 = nullptr;
+    rk_npu_f32i8f32_weights* w8 = nullptr;
+    rk_npu_matmul_workspace* ws8 = nullptr;
+    rk_npu_w4a8_config config{};
+    rk_npu_matmul_strategy strategy{};
+    Calls() : A((size_t)M * K), C((size_t)M * N, 7.0f) {
+        for (size_t i = 0; i < A.size(); ++i) A[i] = (float)(i % 9973);
+        std::vector<int8_t> B((size_t)K * N, 1);
+        std::vector<float> scale(N, 1.0f);
+        rk_npu_w4a8_config_init(&config, M, N, K);
+        const rk_npu_i4_weight_config i4{K, N, config.k_tile};
+        w4 = rk_npu_w4a8_weights_create(domain, &i4, B.data(), scale.data());
+        ws4 = rk_npu_w4a8_workspace_create(domain, &config);
+        cpu_set_t set;
+        sched_getaffinity(0, sizeof(set), &set);
+        int cpu = 0;
+        while (!CPU_ISSET(cpu, &set)) ++cpu;
+        strategy.op_kind = RK_NPU_MATMUL_F32I8F32_DYNAMIC;
+        strategy.M = M, strategy.N = N, strategy.K = K, strategy.k_tile = K, strategy.n_tile = 1024;
+        strategy.npu_core_mask = 1, strategy.cpu_core_mask = 1ull << cpu, strategy.cpu_threads = 1;
+        rk_npu_matmul_weight_config i8{};
+        i8.K = K, i8.N = N, i8.k_tile = K;
+        w8 = rk_npu_f32i8f32_weights_create(domain, &i8, B.data(), scale.data());
+        ws8 = rk_npu_matmul_workspace_create(domain, &strategy);
+    }
+    bool made() const { return w4 && ws4 && w8 && ws8; }
+    int run4() { return rk_npu_w4a8_run_f32(ws4, w4, A.data(), C.data(), nullptr); }
+    int run8() { return rk_npu_f32i8f32_run_dynamic(ws8, w8, A.data(), C.data()); }
+    bool right() {
+        bool ok = true;
+        for (int m = 0; m < M; ++m)
+            for (int n = 0; n < N; ++n) ok = ok && C[(size_t)m * N + n] == A[(size_t)m * K + n % K];
+        C.assign(C.size(), 7.0f);
+        return ok;
+    }
+    bool untouched() const {
+        for (float v : C)
+            if (v != 7.0f) return false;
+        return true;
+    }
+};
+
+// An earlier device call rejected its input, which nothing has looked at since: the next blocking call says so and
+// leaves C alone, the one after it is a good one.
+static int rejected_before() {
+    Calls c;
+    CHECK(c.made());
+    std::vector<float> dC((size_t)M * N);
+    const float good = c.A[5];
+    c.A[5] = std::numeric_limits<float>::infinity();
+    CHECK(rk_npu_w4a8_run_f32_device(c.ws4, c.w4, c.A.data(), dC.data()) == RK_NPU_OK);
+    c.A[5] = good;
+    CHECK(c.run4() == RK_NPU_ERR_PARAM);
+    CHECK(c.untouched());
+    CHECK(c.run4() == RK_NPU_OK && c.right());
+    CHECK(rk_npu_hip_sync(c.ctx) == RK_NPU_OK);
+    // (and the call's own input, first and last row)
+    for (size_t at : {size_t(3), c.A.size() - 1}) {
+        const float keep = c.A[at];
+        c.A[at] = std::nanf("");
+        CHECK(c.run4() == RK_NPU_ERR_PARAM && c.untouched());
+        c.A[at] = keep;
+        CHECK(c.run4() == RK_NPU_OK && c.right());
+    }
+    return 0;
+}
+
+int main(int argc, char** argv) {
+    const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}};
+    for (const auto& c : checks)
+        if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.check();
+    return 2;
+}

@@ -2,7 +2,8 @@
 
 A and C are just large enough to be staged; the panels are 128 rows and the last one is whole, one row (the decode
 kernel), a few rows or nearly whole.  Also: the quantized rows that the call leaves in its workspace, given scales,
-rejected input in the first and the last panel (C stays as it was) and two threads at once.  Exact.
+rejected input in the first and the last panel or in an earlier device call (C stays as it was) and two threads at once.
+Exact.
 """
 import threading
 
@@ -60,6 +61,29 @@ def test_int4_weights(sess, oracle, M):
         rc, got = ws.run_f32(w, A)
         assert rc == 0 and np.array_equal(got.view(np.uint32), want.view(np.uint32))
     finally:
+        ws.close()
+        w.close()
+
+
+def test_an_earlier_device_call_rejected_its_input(sess, oracle):
+    """... and nothing has synchronized since: the blocking call says so and leaves C alone, the next one is good."""
+    M = 389
+    c = workloads.w4a8_case(M, K, N, seed_w=5, seed_a=M)
+    A = oracle.half_to_float(c["A"]).astype(np.float32).reshape(M, K)
+    bad = A.copy()
+    bad[M - 1, 0] = np.nan
+    w, ws = ops.W4A8Weights(sess, c["B"], c["w_scale"]), ops.W4A8Workspace(sess, M, N, K)
+    dA, dC, C = sess.to_device(bad), sess.empty_device(M * N * 4), np.full((M, N), 7.0, np.float32)
+    try:
+        assert sess.lib.rk_npu_w4a8_run_f32_device(ws.h, w.h, dA, dC) == 0
+        assert sess.lib.rk_npu_w4a8_run_f32(ws.h, w.h, capi.ptr(A), capi.ptr(C), None) == capi.RK_NPU_ERR_PARAM
+        assert np.all(C == 7.0)
+        rc, got = ws.run_f32(w, A)
+        assert rc == 0 and np.array_equal(got.view(np.uint32), oracle.w4a8(A, c["B"], c["w_scale"])["C"].view(np.uint32))
+        assert sess.sync() == 0
+    finally:
+        sess.free_device(dA)
+        sess.free_device(dC)
         ws.close()
         w.close()
 
