@@ -331,14 +331,17 @@ int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const 
         }
         deliver();
     });
-    // (the downloads have been waited for, unless C is not to be written)
-    if (failed.load() || bad.load() || (flag && flag->raised()))
-        for (void* stream : {ctx->up_stream, ctx->stream, ctx->second_stream})
-            if (const int rc = map_error(rkh_sync(stream))) failed.store(rc);
+    // The downloads have been waited for, unless C is not to be written.  (And nothing else is: other threads have been
+    // enqueueing on the context's stream since the lock was given back.)
     *rejected = bad.load() || (flag && flag->raised());
-    if (failed.load()) return failed.load();
+    for (size_t p = 0; *rejected && p < panels_ && !failed.load(); ++p)
+        if (const int rc = map_error(rkh_event_sync(down_[p]))) failed.store(rc);
+    if (failed.load()) {
+        for (void* stream : {ctx->up_stream, ctx->stream, ctx->second_stream}) rkh_sync(stream);
+        return failed.load();
+    }
     if (*rejected) flag->rearm(ctx->stream); // (the kernels have raised it too where the copy found something)
-    return map_error(rkh_sync(ctx->stream));
+    return RK_NPU_OK;
 }
 
 bool keeps_to_stream(rk_npu_ctx* ctx) {

@@ -172,8 +172,20 @@ static int rejected_before() {
     return 0;
 }
 
+// A call waits for its own copies and not for the context's stream, on which other threads go on enqueueing once the
+// call has given the submission lock back.
+static int own_work_only() {
+    Calls c;
+    CHECK(c.made());
+    g_syncs = 0;
+    CHECK(c.run4() == RK_NPU_OK && c.right());
+    CHECK(c.run8() == RK_NPU_OK && c.right());
+    CHECK(g_syncs == 0);
+    return 0;
+}
+
 int main(int argc, char** argv) {
-    const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}};
+    const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}, {"own_work_only", own_work_only}};
     for (const auto& c : checks)
         if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.check();
     return 2;
