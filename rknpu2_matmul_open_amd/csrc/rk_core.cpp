@@ -144,6 +144,16 @@ static bool copy_checked(void* to, const void* from, size_t bytes, PanelPipe::Ch
     return true;
 }
 
+// Room for `count` events; false: there is none (nothing is thrown through the C entry points).
+static bool reserve(std::vector<void*>& events, size_t count) {
+    try {
+        events.reserve(count);
+    } catch (...) {
+        return false;
+    }
+    return true;
+}
+
 HostStage::~HostStage() {
     for (void* e : events_) rkh_event_destroy(e);
     rkh_host_free(ptr_);
@@ -156,6 +166,7 @@ void HostStage::init(size_t bytes) {
     bytes_ = bytes;
     if (bytes > kLimit) { // (a mirror that may serve staged downloads)
         const size_t chunks = (bytes + kChunk - 1) / kChunk;
+        if (!reserve(events_, chunks)) return;
         for (size_t i = 0; i < chunks; ++i) {
             void* e = nullptr;
             if (rkh_event_create(&e) != RKH_OK) { // without its events the mirror only serves uploads
@@ -251,6 +262,7 @@ void PanelPipe::init(const Owner& owner, int M, size_t a_row, size_t c_row) {
     if (!ctx->up_stream && rkh_stream_create(ctx->device, &ctx->up_stream) != RKH_OK) return;
     if (!ctx->second_stream && rkh_stream_create(ctx->device, &ctx->second_stream) != RKH_OK) return;
     const size_t panels = ((size_t)M + rows - 1) / rows;
+    if (!reserve(up_, panels) || !reserve(down_, panels)) return;
     if (rkh_event_create(&before_) != RKH_OK) return;
     for (std::vector<void*>* v : {&up_, &down_})
         for (size_t i = 0; i < panels; ++i) {
@@ -264,7 +276,7 @@ void PanelPipe::init(const Owner& owner, int M, size_t a_row, size_t c_row) {
 
 int PanelPipe::run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const HostStage& a, const HostStage& c, uint8_t* a_dev,
                    uint8_t* c_dev, const void* A, void* C, Check check, BadFlag* flag, bool* rejected,
-                   const std::function<int(const Panel&)>& multiply) {
+                   const Multiply& multiply) {
     const uint8_t* from = static_cast<const uint8_t*>(A);
     uint8_t* to = static_cast<uint8_t*>(C);
     uint8_t *a_pin = static_cast<uint8_t*>(a.data()), *c_pin = static_cast<uint8_t*>(c.data());

@@ -10,7 +10,6 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
-#include <functional>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -262,13 +261,24 @@ public:
         void* c;
         void* stream;     // for its kernels, which another panel's may run beside: no scratch is shared
     };
+    // What multiplies a panel, by reference: a std::function would allocate for it in the call, and throw where it cannot.
+    class Multiply {
+    public:
+        template <class F>
+        explicit Multiply(const F& f) : f_(&f), call_([](const void* g, const Panel& p) { return (*static_cast<const F*>(g))(p); }) {}
+        int operator()(const Panel& p) const { return call_(f_, p); }
+
+    private:
+        const void* f_;
+        int (*call_)(const void*, const Panel&);
+    };
     // The planned call: A through a's mirror to a_dev, `multiply` -> RK_NPU_* for each panel, c_dev through c's mirror to C.
     // Gives the submission lock back when everything is enqueued.  `check` fails, or an earlier device call on the
     // workspace has raised `flag` (null where there is nothing to check): C is not written, *rejected set and the flag
     // re-armed.  Returns with nothing of the call under way.
     int run(rk_npu_ctx* ctx, std::unique_lock<std::mutex>& submit, const HostStage& a, const HostStage& c, uint8_t* a_dev,
             uint8_t* c_dev, const void* A, void* C, Check check, BadFlag* flag, bool* rejected,
-            const std::function<int(const Panel&)>& multiply);
+            const Multiply& multiply);
 
 private:
     static int panel_rows(int M, size_t a_row, size_t c_row);

@@ -208,9 +208,9 @@ int run_host(rk_npu_matmul_workspace* ws, const Weights* w, rk_npu_matmul_op_kin
             if (ws->t.quant == 2) rc = map_error(rkh_h2d(ctx->stream, ws->a_scale.as<>(), scale_src, scale_bytes));
             if (rc) return rc;
             bool rejected;
+            const auto multiply = [&](const PanelPipe::Panel& p) { return enqueue_rows(ws, *w, p.a, p.c, false, p.row, p.rows, p.stream); };
             return ws->pipe.run(ctx, submit, ws->stage_a, ws->stage_c, ws->a_raw.as<>(), ws->c_out.as<>(), A, C, PanelPipe::ANY,
-                                nullptr, &rejected,
-                                [&](const PanelPipe::Panel& p) { return enqueue_rows(ws, *w, p.a, p.c, false, p.row, p.rows, p.stream); });
+                                nullptr, &rejected, PanelPipe::Multiply(multiply));
         }
     }
     {

@@ -376,13 +376,14 @@ int run_host(rk_npu_w4a8_workspace* ws, const rk_npu_w4a8_weights* w, const void
         std::unique_lock<std::mutex> submit(ctx->submit_mutex);
         if (!keeps_to_stream(ctx)) {
             bool rejected;
+            const auto multiply = [&](const PanelPipe::Panel& p) {
+                const rkh_quant_args q = quant_args(ws, p.a, half, false, p.row, p.rows);
+                const rkh_gemm_args g = gemm_args(ws, w, p.c, out, false, p.row, p.rows);
+                return map_error(rkh_quant_gemm(p.stream, &q, &g));
+            };
             rc = ws->pipe.run(ctx, submit, ws->stage_a, ws->stage_c, ws->a_raw.as<>(), ws->c_out.as<>(), A, C,
                               half ? PanelPipe::FINITE_F16 : PanelPipe::FINITE_F32, &ws->flag, &rejected,
-                              [&](const PanelPipe::Panel& p) {
-                                  const rkh_quant_args q = quant_args(ws, p.a, half, false, p.row, p.rows);
-                                  const rkh_gemm_args g = gemm_args(ws, w, p.c, out, false, p.row, p.rows);
-                                  return map_error(rkh_quant_gemm(p.stream, &q, &g));
-                              });
+                              PanelPipe::Multiply(multiply));
             return rc ? rc : rejected ? RK_NPU_ERR_PARAM : RK_NPU_OK; // NaN / Inf activation: C is not written
         }
     }

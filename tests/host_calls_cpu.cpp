@@ -184,8 +184,38 @@ static int own_work_only() {
     return 0;
 }
 
+// Memory runs out at any allocation: a handle is not made, a run gives its code, and nothing is thrown at the caller.
+static int out_of_memory() {
+    Calls c;
+    CHECK(c.made());
+    int made = 0;
+    for (long n = 0; n < 64 && made < 2; ++n) {
+        g_allocations = n;
+        rk_npu_w4a8_workspace* ws4 = rk_npu_w4a8_workspace_create(c.domain, &c.config);
+        g_allocations = n;
+        rk_npu_matmul_workspace* ws8 = rk_npu_matmul_workspace_create(c.domain, &c.strategy);
+        g_allocations = -1;
+        made = (ws4 != nullptr) + (ws8 != nullptr);
+        for (int pass = 0; pass < 2; ++pass) { // (with what could be made, the calls work)
+            if (ws4) CHECK(rk_npu_w4a8_run_f32(ws4, c.w4, c.A.data(), c.C.data(), nullptr) == RK_NPU_OK && c.right());
+            if (ws8) CHECK(rk_npu_f32i8f32_run_dynamic(ws8, c.w8, c.A.data(), c.C.data()) == RK_NPU_OK && c.right());
+        }
+        rk_npu_w4a8_workspace_free(ws4);
+        rk_npu_matmul_workspace_free(ws8);
+    }
+    CHECK(made == 2);
+    for (int (Calls::*run)() : {&Calls::run4, &Calls::run8}) {
+        g_allocations = 0;
+        const int rc = (c.*run)();
+        g_allocations = -1;
+        CHECK(rc == RK_NPU_OK && c.right());
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
-    const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}, {"own_work_only", own_work_only}};
+    const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}, {"own_work_only", own_work_only},
+                                                                    {"out_of_memory", out_of_memory}};
     for (const auto& c : checks)
         if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.check();
     return 2;
