@@ -19,6 +19,7 @@
 
 static std::atomic<int> g_threads{0};
 static std::atomic<int> g_syncs{0};          // waits for the context's stream
+static std::atomic<int> g_waits{0};          // of one stream for another: panels
 static std::atomic<long> g_allocations{-1};  // allocations that still succeed; -1: all of them
 static char g_streams[3];                    // [0]: the context's
 static int g_made = 1;
@@ -70,7 +71,7 @@ int rkh_event_record(void*, void*) { return RKH_OK; }
 int rkh_event_sync(void*) { return RKH_OK; }
 int rkh_stream_create(int, void** s) { return *s = g_streams + g_made++, RKH_OK; }
 void rkh_stream_destroy(void*) {}
-int rkh_stream_wait(void*, void*) { return RKH_OK; }
+int rkh_stream_wait(void*, void*) { return ++g_waits, RKH_OK; }
 int rkh_static_scratch(int, void**, size_t*) { return RKH_ERR_RUNTIME; }
 void rkh_set_marker(rkh_marker_fn, void*) {}
 size_t rkh_gemm_scratch_bytes(int, int, int, int) { return 0; }
@@ -213,9 +214,32 @@ static int out_of_memory() {
     return 0;
 }
 
+// Helper threads: three at most, and one processor less than the process may run on; with none no panels.
+static int helpers() {
+    Calls c;
+    CHECK(c.made());
+    cpu_set_t all, few;
+    CHECK(sched_getaffinity(0, sizeof(all), &all) == 0);
+    CPU_ZERO(&few);
+    int cpus = 0;
+    for (int cpu = 0; cpu < CPU_SETSIZE; ++cpu) {
+        if (!CPU_ISSET(cpu, &all)) continue;
+        CPU_SET(cpu, &few);
+        ++cpus;
+        CHECK(sched_setaffinity(0, sizeof(few), &few) == 0);
+        for (int (Calls::*run)() : {&Calls::run4, &Calls::run8}) {
+            g_threads = g_waits = 0;
+            CHECK((c.*run)() == RK_NPU_OK && c.right());
+            CHECK(g_threads == (cpus > 3 ? 3 : cpus - 1));
+            CHECK((g_waits > 0) == (cpus > 1));
+        }
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}, {"own_work_only", own_work_only},
-                                                                    {"out_of_memory", out_of_memory}};
+                                                                    {"out_of_memory", out_of_memory}, {"helpers", helpers}};
     for (const auto& c : checks)
         if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.check();
     return 2;
