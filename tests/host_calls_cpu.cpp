@@ -87,8 +87,9 @@ int rkh_quant_gemm(void*, const rkh_quant_args* q, const rkh_gemm_args* g) {
     }
     return RKH_OK;
 }
-int rkh_quant_rows(void*, const rkh_quant_args*) { return RKH_ERR_RUNTIME; }
-int rkh_gemm(void*, const rkh_gemm_args*) { return RKH_ERR_RUNTIME; }
+static rkh_quant_args g_quantized; // (the two as launches of their own)
+int rkh_quant_rows(void*, const rkh_quant_args* q) { return g_quantized = *q, RKH_OK; }
+int rkh_gemm(void* s, const rkh_gemm_args* g) { return rkh_quant_gemm(s, &g_quantized, g); }
 }
 
 #define CHECK(x)                                                         \
