@@ -261,6 +261,16 @@ bool PanelPipe::plan(size_t a_row, size_t c_row) {
     a_row_ = a_row;
     c_row_ = c_row;
     panels_ = ((size_t)M_ + rows_ - 1) / rows_;
+    // Panels gain the time of the rows that are copied and uploaded beside another panel, and lose what a download takes
+    // longer beside uploads and kernels (50 us a panel and not 38) and what threads and streams cost whatever the size.
+    // The line is the best of its form over 70 shapes of 1 - 32 MB in and 4 - 33 MB out: the slower side loses 0.2 % on
+    // average and 4 % at most (always panels: 7 and 31; always one piece: 5 and 38).
+    // Whole calls, us, one piece -> panels, fp32: 512 x 560 x 2100 220 -> 289, 200 x 2048 x 8192 296 -> 353, 140 x 14336 x 8192
+    // 482 -> 599 (the second panel has 12 rows), 256 x 4200 x 4300 311 -> 305, 1024 x 1500 x 1500 407 -> 360, 600 x 4096 x 2048
+    // 561 -> 467; exact int8 2048 x 600 x 600 238 -> 309, 2048 x 1024 x 4096 1015 -> 1319, 1024 x 4200 x 3000 534 -> 612, 2048 x 3000 x
+    // 2048 735 -> 720.
+    const size_t beside = a_bytes - rows_ * a_row;
+    if (beside < (3 * panels_ + 7) * (size_t(128) << 10) + c_bytes / 16) return false;
     return panels_ <= down_.size();
 }
 void PanelPipe::init(const Owner& owner, int M, size_t a_row, size_t c_row) {

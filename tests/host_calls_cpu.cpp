@@ -100,7 +100,7 @@ int rkh_gemm(void* s, const rkh_gemm_args* g) { return rkh_quant_gemm(s, &g_quan
         }                                                                \
     } while (0)
 
-static constexpr int M = 1000, K = 1100, N = 4224; // A 4.4 MB, C 16.9 MB
+static constexpr int M = 1000, K = 1100, N = 2200; // A 4.4 MB, C 8.8 MB
 
 struct Calls {
     rk_npu_ctx* ctx = rk_npu_open(nullptr);
@@ -238,9 +238,42 @@ static int helpers() {
     return 0;
 }
 
+// Which calls go in panels (fp32 in and out): both sides of each line.
+static int panelled() {
+    Calls c;
+    CHECK(c.made());
+    const struct { int M, K, N; bool panels; } shapes[] = {
+        {1000, 1100, 1040, false},                            // less than 4 MiB out
+        {1000, 1013, 1100, false}, {1000, 1014, 1100, true},  // two panels
+        {200, 7338, 8192, false},  {200, 7339, 8192, true},   // of which the second is small
+        {500, 2228, 6600, false},  {500, 2229, 6600, true},   // four
+        {384, 2850, 4224, true},   {385, 2850, 4224, true},   // (the shapes of test_gpu_host_panels.py)
+        {387, 2850, 4224, true},   {389, 2850, 4224, true},   {510, 2850, 4224, true}};
+    for (const auto& s : shapes) {
+        const std::vector<int8_t> B((size_t)s.K * s.N, 1);
+        const std::vector<float> scale(s.N, 1.0f), A((size_t)s.M * s.K, 1.0f);
+        std::vector<float> C((size_t)s.M * s.N);
+        rk_npu_matmul_strategy strategy = c.strategy;
+        strategy.M = s.M, strategy.N = s.N, strategy.K = strategy.k_tile = s.K;
+        rk_npu_matmul_weight_config i8{};
+        i8.K = i8.k_tile = s.K, i8.N = s.N;
+        rk_npu_f32i8f32_weights* w = rk_npu_f32i8f32_weights_create(c.domain, &i8, B.data(), scale.data());
+        rk_npu_matmul_workspace* ws = rk_npu_matmul_workspace_create(c.domain, &strategy);
+        g_waits = 0;
+        CHECK(rk_npu_f32i8f32_run_dynamic(ws, w, A.data(), C.data()) == RK_NPU_OK);
+        for (float v : C) CHECK(v == 1.0f);
+        if ((g_waits > 0) != s.panels) std::fprintf(stderr, "%d x %d x %d\n", s.M, s.K, s.N);
+        CHECK((g_waits > 0) == s.panels);
+        rk_npu_matmul_workspace_free(ws);
+        rk_npu_f32i8f32_weights_free(w);
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const struct { const char* name; int (*check)(); } checks[] = {{"rejected_before", rejected_before}, {"own_work_only", own_work_only},
-                                                                    {"out_of_memory", out_of_memory}, {"helpers", helpers}};
+                                                                    {"out_of_memory", out_of_memory}, {"helpers", helpers},
+                                                                    {"panelled", panelled}};
     for (const auto& c : checks)
         if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.check();
     return 2;

@@ -1,6 +1,6 @@
 """GPU parity of large blocking calls on host buffers, which go in panels of rows, against the CPU oracle.
 
-A and C are just large enough to be staged; the panels are 128 rows and the last one is whole, one row (the decode
+A and C are just large enough for panels (tests/host_calls_cpu.cpp holds which calls are); the panels are 128 rows and the last one is whole, one row (the decode
 kernel), a few rows or nearly whole.  Also: the quantized rows that the call leaves in its workspace, given scales,
 rejected input in the first and the last panel or in an earlier device call (C stays as it was) and two threads at once.
 Exact.
@@ -14,7 +14,7 @@ from rknpu2_matmul_open_amd import capi, ops, workloads
 
 pytestmark = pytest.mark.gpu
 
-K, N = 1100, 4224  # 128 rows of fp32 results: 2.1 MiB, the size of a panel
+K, N = 2850, 4224  # 128 rows of fp32 results: 2.1 MiB, the size of a panel
 
 
 @pytest.mark.parametrize("M", [384, 385, 389, 510])
@@ -23,8 +23,8 @@ def test_int8_weights(sess, oracle, M, kind):
     c = workloads.w8a8_case(2, K, N, seed_w=M, seed_a=1)
     scale = None
     if kind == "i32":
-        A = np.random.default_rng(M).integers(-128, 128, (M, 2 * K)).astype(np.int8)  # (more than 1 MiB)
-        B = np.concatenate([c["B"], c["B"][::-1]])
+        A = np.random.default_rng(M).integers(-128, 128, (M, 4 * K)).astype(np.int8)  # (more than 4 MiB)
+        B = np.concatenate([c["B"], c["B"][::-1], c["B"][:, ::-1], c["B"]])
         op, want = ops.W8A8Linear(sess, capi.I8I8I32, M, B), oracle.gemm_i8(A, B)
     else:
         A = workloads.normal_f32(M, (M, K))

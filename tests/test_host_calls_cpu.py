@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("check", ["rejected_before", "own_work_only", "out_of_memory", "helpers"])
+@pytest.mark.parametrize("check", ["rejected_before", "own_work_only", "out_of_memory", "helpers", "panelled"])
 def test_blocking_calls(program, check):
     done = subprocess.run([program, check], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert done.returncode == 0, done.stdout
