@@ -18,7 +18,10 @@ with the same flags):
     can only make a wait stricter than this rule assumes);
   * LDS reads (ds_read from asm) are covered by the next s_waitcnt with lgkmcnt(0);
   * between an asm load and its covering wait no instruction may name one of its destination
-    registers.
+    registers;
+  * a load to LDS takes its address from M0, and needs one wait state behind a scalar write of M0: the
+    instruction in front of it may not be that write.  (The compiler inserts the wait state for
+    loads of its own; into an asm statement it does not look.)
 
 The check walks the control-flow graph of a kernel (basic blocks split at labels and branches):
 from every asm load it follows every path until the covering wait, carrying the number of loads
@@ -155,10 +158,33 @@ def _check_load(instrs, blocks, block_of, at, what, violations, seen):
     return uncovered_end
 
 
+_LDS_LOAD = re.compile(r"^\s*(global|buffer|scratch)_load_(lds_|\w+.*\blds\b)")
+_M0_WRITE = re.compile(r"^\s*s_\w+\s+m0\s*,")
+
+
+def _check_m0(name, instrs, violations):
+    """Loads to LDS directly behind a scalar write of M0 (in the same block or at the end of one before it)."""
+    blocks = _blocks(instrs)
+    for i, (text, _) in enumerate(instrs):
+        if not _LDS_LOAD.match(text):
+            continue
+        work, seen = [(lo, i) for lo, hi, _ in blocks.values() if lo <= i < hi], set()
+        while work:
+            lo, end = work.pop()
+            prev = [t for t, _ in instrs[lo:end] if not t.endswith(":")]
+            if prev:
+                if _M0_WRITE.match(prev[-1]):
+                    violations.append("%s: `%s` directly behind `%s` needs a wait state" % (name, text.strip(), prev[-1].strip()))
+            elif lo not in seen:
+                seen.add(lo)
+                work += [(first, hi) for first, hi, succ in blocks.values() if lo in succ]
+
+
 def audit_function(name, lines):
     """Violations (strings) of one kernel's assembly."""
     instrs = _instructions(lines)
     violations, seen = [], set()
+    _check_m0(name, instrs, violations)
     loads = [i for i, (t, a) in enumerate(instrs) if a and (_ASM_VLOAD.match(t) or _ASM_DSREAD.match(t))]
     if not loads:
         return violations

@@ -174,14 +174,18 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     // 15.5 -> 15.6), and neither do the weights, of which three sub-steps lie beyond K.
     constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
     [[maybe_unused]] unsigned long long a_lanes = ~0ull;
-    auto copy_a = [&](int buf) { // global -> LDS, 16 bytes per lane, lane-contiguous
+    // A load to LDS needs a wait state behind a scalar write of M0, which the compiler does not insert into an asm
+    // statement (the build checks for it): the change of priority that a sub-step begins with is put there.  (An s_nop
+    // beside it cost 0.3 - 0.8 % of a GEMM.)
+    auto copy_a = [&](int buf, auto prio_tag) { // global -> LDS, 16 bytes per lane, lane-contiguous
+        constexpr int PRIO = decltype(prio_tag)::value;
         if constexpr (MASKED)    // (every lane is active here, and is again behind the copy)
-            asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lane_off),
-                         "s"(asrc), "s"(copy_dst + buf * BUF), "s"(a_lanes)
+            asm volatile("s_mov_b32 m0, %2\n\ts_setprio %4\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lane_off),
+                         "s"(asrc), "s"(copy_dst + buf * BUF), "s"(a_lanes), "n"(PRIO)
                          : "memory", "m0");
         else
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(asrc),
-                         "s"(copy_dst + buf * BUF)
+            asm volatile("s_mov_b32 m0, %2\n\ts_setprio %3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(asrc),
+                         "s"(copy_dst + buf * BUF), "n"(PRIO)
                          : "memory", "m0");
         asrc += a_left > 0 ? A_STEP : 0;
         if constexpr (MASKED) a_lanes = a_left > 0 ? ~0ull : 1ull;
@@ -256,8 +260,7 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
         // The two waves of a SIMD drift apart between barriers (the older one wins
         // every issue conflict) and the one left behind cannot keep the matrix pipe
         // busy alone; the wave that is further into the barrier interval yields.
-        __builtin_amdgcn_s_setprio(G - 1 - SLOT % G);
-        copy_a((SLOT + D) % NBUF);
+        copy_a((SLOT + D) % NBUF, std::integral_constant<int, G - 1 - SLOT % G>{});
         if constexpr (!WPAIR) load_w(wring[(SLOT + NSW - 1) % NSW]);
         else if constexpr (SLOT % 2 == 0) load_w(wring[(SLOT / 2 + NSW - 1) % NSW]);
         constexpr int NEXT_W = WPAIR ? (SLOT + 1) / 2 % NSW : (SLOT + 1) % NSW; // ring slot of the next sub-step's weights
@@ -291,7 +294,7 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     // prologue: the same issue order as if the loop had run for sub-steps -D..-1
 #pragma unroll
     for (int t = -D; t < 0; ++t) {
-        copy_a(t + D);
+        copy_a(t + D, std::integral_constant<int, 0>{});
         if (WPAIR ? t % 2 == 0 && t / 2 + NSW - 1 >= 0 : t + NSW - 1 >= 0) load_w(wring[(WPAIR ? t / 2 : t) + NSW - 1]);
     }
     RK_TS(1);

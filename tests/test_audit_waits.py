@@ -109,6 +109,20 @@ def test_paths_through_branches_are_followed():
     assert len(found) == 1 and "v_add_u32" in found[0]
 
 
+def test_a_load_to_lds_needs_a_wait_state_behind_m0():
+    load = "\tglobal_load_lds_dwordx4 v1, s[2:3]\n"
+    for body, violations in (
+            (";;#ASMSTART\n\ts_mov_b32 m0, s4\n" + load + "\t;;#ASMEND", 1),
+            ("\ts_mov_b32 m0, s4\n\tbuffer_load_dwordx4 v1, s[8:11], 0 offen lds", 1),
+            ("\ts_mov_b32 m0, s4\n.LBB0_7:\n" + load + "\ts_cbranch_scc1 .LBB0_7", 1),  # (falls through into the loop)
+            ("\ts_mov_b32 m0, s4\n\ts_nop 0\n" + load, 0),
+            ("\ts_mov_b32 m0, s4\n\ts_mov_b64 exec, s[6:7]\n" + load + "\ts_mov_b64 exec, -1", 0),
+            (".LBB0_8:\n" + load + "\ts_add_u32 m0, m0, s5\n\ts_branch .LBB0_8", 0),   # (the branch is in between)
+            ("\ts_mov_b32 m0, s4\n\tglobal_load_dword v1, v2, off\n\ts_waitcnt vmcnt(0)", 0)):  # (to a register)
+        found, checked = audit_waits.audit_text(_kernel(body))
+        assert checked == 1 and len(found) == violations, body
+
+
 def test_other_kernels_and_compiler_loads_are_ignored():
     text = "_ZN1x11gemv_kernelILi1EEEvv:\n	global_load_dwordx4 v[10:13], v1, s[2:3]\n	v_mov_b32_e32 v1, v10\n	s_endpgm\n"
     assert audit_waits.audit_text(text) == ([], 0)
