@@ -26,3 +26,16 @@ def sess():
     s = ops.Session()
     yield s
     s.close()
+
+
+@pytest.fixture
+def one_piece(sess):
+    """one_piece(call) -> (what the call returns, the kernels it launched).  While a per-kernel profile is on, a large
+    call on host buffers does not go in panels of rows."""
+    from rknpu2_matmul_open_amd import ops
+
+    def run(call):
+        got = []
+        kernels = ops.profile_kernels(sess, lambda: got.append(call()), iters=1, warmup=0)
+        return got[0], [name for name, _ in kernels]
+    return run

@@ -52,7 +52,7 @@ def test_int8_weights(sess, oracle, M, N, K, kind):
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("kind", ["f16", "f32", "i32", "swiglu"])
-def test_int4_weights(sess, oracle, M, N, K, kind):
+def test_int4_weights(sess, oracle, one_piece, M, N, K, kind):
     if kind == "swiglu":
         N = (N + 63) // 64 * 64
     c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
@@ -61,18 +61,18 @@ def test_int4_weights(sess, oracle, M, N, K, kind):
     try:
         A32 = oracle.half_to_float(c["A"]).astype(np.float32).reshape(M, K)
         if kind == "f16":
-            rc, got = ws.run_f16(w, c["A"])
+            (rc, got), kernels = one_piece(lambda: ws.run_f16(w, c["A"]))
             want = oracle.w4a8(c["A"], c["B"], c["w_scale"])["C"]
         elif kind == "f32":
-            rc, got = ws.run_f32(w, A32)
+            (rc, got), kernels = one_piece(lambda: ws.run_f32(w, A32))
             want = oracle.w4a8(A32, c["B"], c["w_scale"])["C"]
         elif kind == "i32":
-            rc, got = ws.run_i32(w, A32)
+            (rc, got), kernels = one_piece(lambda: ws.run_i32(w, A32))
             want = oracle.w4a8(A32, c["B"], c["w_scale"])["acc"]
         else:
-            rc, got = ws.run_swiglu_f32(w, A32)
+            (rc, got), kernels = one_piece(lambda: ws.run_swiglu_f32(w, A32))
             want = oracle.w4a8_swiglu(A32, c["B"], c["w_scale"])["middle"]
-        assert rc == 0
+        assert rc == 0 and kernels[-1] == "gemm_wk_big_kernel"
         assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, got.dtype).view(np.uint8))
     finally:
         ws.close()

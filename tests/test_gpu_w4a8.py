@@ -377,7 +377,7 @@ def test_weight_info_and_k_tile_resolution(sess):
     sess.lib.rk_npu_w4a8_weights_free(h)
 
 
-def test_config2_full_output_and_properties(sess, oracle):
+def test_config2_full_output_and_properties(sess, oracle, one_piece):
     """BASELINE config 2 at full size (M=2048, K=4096, N=4096, seeds 4/5, 0.5% x20
     outliers): every int8 activation, every fp16 output and every int32
     accumulator exact against the oracle (all 2048 rows), plus a size-independent
@@ -396,10 +396,12 @@ def test_config2_full_output_and_properties(sess, oracle):
         assert want["rc"] == 0 and np.array_equal(_bits32(s), _bits32(want["a_scale"]))
         assert np.array_equal(q, want["q"])
         assert np.array_equal(got, want["C"])
-        # int32 accumulators of the whole problem through the probe entry point (same kernels,
-        # raw integer epilogue)
-        rc, acc = wsp.run_i32(w, oracle.half_to_float(c["A"]))
-        assert rc == 0 and np.array_equal(acc, want["acc"])
+        # the same in one piece, with the kernels of the device calls, and the int32 accumulators of the whole
+        # problem through the probe entry point (same kernels, raw integer epilogue)
+        (rc, got), kernels = one_piece(lambda: wsp.run_f16(w, c["A"]))
+        assert rc == 0 and np.array_equal(got, want["C"]) and kernels == ["quant_rows8_kernel", "gemm_wk_kernel"]
+        (rc, acc), kernels = one_piece(lambda: wsp.run_i32(w, oracle.half_to_float(c["A"])))
+        assert rc == 0 and np.array_equal(acc, want["acc"]) and kernels == ["quant_rows8_kernel", "gemm_wk_kernel"]
         half = (oracle.half_to_float(c["A"]) * np.float32(0.5)).astype(np.float16).view(np.uint16)
         rc, got_half = wsp.run_f16(w, half)
         assert rc == 0
@@ -461,7 +463,7 @@ def test_k_tile_resolution_against_reference_golden(sess):
                 sess.lib.rk_npu_w4a8_weights_free(h)
 
 
-def test_random_shapes_through_the_launch_plan(sess, oracle):
+def test_random_shapes_through_the_launch_plan(sess, oracle, one_piece):
     """Seeded random shapes of more than 128 rows: whatever tile height and K split the dense plan
     picks (long K with few columns is split over workgroups, wide matrices are not), the int32 sums
     and the fp32 output are the oracle's, for int4 weights here and int8 weights below."""
@@ -477,9 +479,9 @@ def test_random_shapes_through_the_launch_plan(sess, oracle):
         wsp = ops.W4A8Workspace(sess, M, N, K)
         try:
             want = oracle.w4a8(A, B, ws)
-            rc, acc = wsp.run_i32(w, A)
+            (rc, acc), _ = one_piece(lambda: wsp.run_i32(w, A))
             assert rc == 0 and np.array_equal(acc, want["acc"]), (case, M, N, K)
-            rc, got = wsp.run_f32(w, A)
+            (rc, got), _ = one_piece(lambda: wsp.run_f32(w, A))
             assert rc == 0 and np.array_equal(_bits32(got), _bits32(want["C"])), (case, M, N, K)
         finally:
             wsp.close()
@@ -493,7 +495,7 @@ def test_random_shapes_through_the_launch_plan(sess, oracle):
         A = rng.standard_normal((M, K)).astype(np.float32)
         op = ops.W8A8Linear(sess, capi.F32I8F32_DYNAMIC, M, B, ws)
         try:
-            rc, got = op.run(A)
+            (rc, got), _ = one_piece(lambda: op.run(A))
             want = oracle.w8a8(A, B, ws)["C"]
             assert rc == 0 and np.array_equal(_bits32(got), _bits32(want)), (case, M, N, K)
         finally:
