@@ -135,9 +135,10 @@ typedef struct rkh_quant_args {
     int src_is_host;
 } rkh_quant_args;
 int rkh_quant_rows(void* stream, const rkh_quant_args* args);
-/* The first of the *rows rows that workgroup `workgroup` of *workgroups takes in that launch (rows at or beyond
- * args->M do not exist), and which *part of its row where several workgroups share one.  No GPU call. */
-int rkh_quant_row_of(const rkh_quant_args* args, int workgroup, int* workgroups, int* rows, int* part);
+/* The first of the *rows rows that workgroup `workgroup` of *workgroups takes in that launch, or in the one that
+ * rkh_quant_gemm puts ahead of a GEMM (rows at or beyond args->M do not exist), and which *part of its row where
+ * several workgroups share one.  No GPU call. */
+int rkh_quant_row_of(const rkh_quant_args* args, int ahead, int workgroup, int* workgroups, int* rows, int* part);
 
 /* ---- GEMM / GEMV ---- */
 enum rkh_epilogue {

@@ -1397,8 +1397,8 @@ static QuantPlan quant_plan(const rkh_quant_args& a, bool ahead = false) {
     // which are in flight at once, and the maximum are the same latency for one workgroup and for four -- and quantizes
     // the 256 chunks that are its own.  us, fp16 rows, whole calls, weights from HBM: int8 16 x 14336 x 4096 17.3 -> 16.5, 32 x 11008
     // 17.25 -> 16.8, 6 x 11008 13.8 -> 13.2, 128 x 14336 32.3 -> 31.8; int4 16 x 14336 14.1 -> 13.3, 8 x 14336 13.05 -> 12.15,
-    // 16 x 8192 10.05 -> 9.8.  Up to a workgroup per compute unit: beyond, and with rows that are fetched element by element,
-    // the repeated reads cost more (100 x 9001 onto 2048 columns 23.3 -> 25.9, 200 x 4100 13.6 -> 14.9, fp32 120 x 12001 26.5 -> 30.5;
+    // 16 x 8192 10.05 -> 9.8.  Up to 256 workgroups, one per compute unit, or, of aligned rows that four share, two: beyond, and
+    // with more rows that are fetched element by element, the repeated reads cost more (100 x 9001 onto 2048 columns 23.3 -> 25.9, 200 x 4100 13.6 -> 14.9, fp32 120 x 12001 26.5 -> 30.5;
     // aligned 250 x 8000 14.6 -> 15.2, but 128 rows of 16384 26.6 -> 26.1).
     if (ahead && (mode == RKH_Q_W8_DYNAMIC || mode == RKH_Q_W4A8) && a.in_dtype != RKH_I8 && row_chunks > 256 &&
         row_chunks <= 256 * QR_CACHE) {
@@ -1421,8 +1421,8 @@ static QuantPlan quant_plan(const rkh_quant_args& a, bool ahead = false) {
     return {QuantPlan::ROWS, a.M << log2_split, log2_split, DEAL_RANGES};
 }
 
-int rkh_quant_row_of(const rkh_quant_args* args, int workgroup, int* workgroups, int* rows, int* part) {
-    const QuantPlan p = quant_plan(*args);
+int rkh_quant_row_of(const rkh_quant_args* args, int ahead, int workgroup, int* workgroups, int* rows, int* part) {
+    const QuantPlan p = quant_plan(*args, ahead != 0);
     *workgroups = p.grid;
     *part = 0;
     if (p.kernel == QuantPlan::ROWS8 || p.kernel == QuantPlan::ROWS4) {

@@ -243,15 +243,16 @@ class _QuantArgs(C.Structure):
 def dealing():
     f = capi.load_library().rkh_quant_row_of
     f.restype = C.c_int
-    f.argtypes = [C.POINTER(_QuantArgs), C.c_int] + [C.POINTER(C.c_int)] * 3
+    f.argtypes = [C.POINTER(_QuantArgs), C.c_int, C.c_int] + [C.POINTER(C.c_int)] * 3
 
-    def call(M, K, dtype, mode, grouped=False):
-        """[(die, first row, rows, part)] of every workgroup (grouped: only the first rows are live)"""
+    def call(M, K, dtype, mode, grouped=False, ahead=True):
+        """[(die, first row, rows, part)] of every workgroup (grouped: only the first rows are live; ahead: of a GEMM,
+        as nearly all of them are)"""
         a = _QuantArgs(in_dtype=dtype, mode=mode, M=M, K=K, row_max_parts=K // 32, active_blocks=1 if grouped else None)
         n, rows, part = C.c_int(1), C.c_int(0), C.c_int(0)
         got, b = [], 0
         while b < n.value:
-            first = f(C.byref(a), b, C.byref(n), C.byref(rows), C.byref(part))
+            first = f(C.byref(a), int(ahead), b, C.byref(n), C.byref(rows), C.byref(part))
             got.append((b % DIES, first, rows.value, part.value))
             b += 1
         return got
@@ -259,18 +260,38 @@ def dealing():
 
 
 @pytest.mark.parametrize("M", [1, 2, 7, 8, 9, 31, 32, 33, 61, 63, 64, 65, 100, 128, 255, 256, 257, 700, 767, 768, 1025, 4099])
-def test_every_row_is_quantized_once(dealing, M):
+@pytest.mark.parametrize("ahead", [False, True])
+def test_every_row_is_quantized_once(dealing, M, ahead):
     for K in (40, 1024, 2048, 4096, 4128, 8224, 14336, 20000):
         for dtype, mode, grouped in ((F16, Q_W8_DYNAMIC, False), (F32, Q_W4A8, False), (I8, Q_COPY_I8, False),
                                      (F32, Q_REUSE, False), (F32, Q_REUSE_MOE, True)):
             seen = {}
-            for _, first, rows, part in dealing(M, K, dtype, mode, grouped):
+            for _, first, rows, part in dealing(M, K, dtype, mode, grouped, ahead):
                 assert first >= 0
                 for row in range(first, min(first + rows, M)):
                     assert (row, part) not in seen
                     seen[row, part] = True
             parts = 1 + max(part for _, part in seen)
-            assert len(seen) == M * parts and (parts == 1 or mode in (Q_REUSE, Q_REUSE_MOE)), (K, dtype, mode)
+            # (scanned rows are shared only ahead of a GEMM, and only where the parts' registers hold a whole row)
+            scanned = ahead and mode in (Q_W8_DYNAMIC, Q_W4A8) and 4096 < K <= 16384
+            assert len(seen) == M * parts and (parts == 1 or mode in (Q_REUSE, Q_REUSE_MOE) or scanned), (K, dtype, mode)
+
+
+@pytest.mark.parametrize("M,K,dtype,parts", [
+    (1, 4096, F16, 1), (1, 4097, F16, 2), (128, 4104, F16, 2), (129, 4104, F16, 1), (128, 8192, F32, 2), (129, 8192, F32, 1),
+    (1, 8200, F16, 4), (64, 8200, F16, 4), (128, 8200, F16, 4), (129, 8200, F16, 1), (128, 16384, F32, 4), (128, 16400, F32, 1),
+    (64, 9001, F32, 4), (65, 9001, F32, 1), (64, 9001, F16, 4), (65, 9001, F16, 1), (128, 8196, F32, 4), (65, 8196, F16, 1)])
+def test_workgroups_that_share_a_scanned_row(dealing, M, K, dtype, parts):
+    """Two up to 8192 elements, four up to 16384, while that makes 256 workgroups at most, or 512 of rows whose chunks are
+    16-byte aligned and that four share; each part once, the parts of a row in consecutive places of one die's range."""
+    for mode in (Q_W8_DYNAMIC, Q_W4A8):
+        got = dealing(M, K, dtype, mode)
+        assert sorted((row, part) for _, row, _, part in got) == [(m, p) for m in range(M) for p in range(parts)]
+        assert len(dealing(M, K, dtype, mode, ahead=False)) == M
+        if parts > 1:
+            for die in range(DIES):
+                mine = [row * parts + part for d, row, _, part in got if d == die]
+                assert not mine or mine == list(range(mine[0], mine[0] + len(mine)))
 
 
 @pytest.mark.parametrize("I", [512, 1024, 4096, 4128, 8224])
