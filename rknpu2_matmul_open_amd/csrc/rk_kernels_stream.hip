@@ -367,7 +367,16 @@ int launch_gemm_grouped(hipStream_t st, const rkh_gemm_args& g) {
     if (forced && forced[0] == 't') balanced = false;
     if ((long)mblocks * ((g.N + 63) / 64) > 0x0fffffffL) balanced = false; // (the kernel deals the units in 32-bit arithmetic)
     if (balanced) {
-        mark(st, "gemm_stream_kernel<balanced>");
+        // Steps of a wave in flight: with at most six and a half units per compute unit (as many as the call can have) two
+        // steps of so few waves are too little for HBM, with more they are enough where K is longer than 1024.  int8
+        // gate/up, whole layers, us, two -> four steps; units per compute unit: 4.5 (32 tokens, 32 experts, top-4, 2048 x 1024)
+        // 58.6 -> 56.9, 5 (256 tokens, 16 experts, top-8, 4096 x 512) 93.5 -> 84.1, 5.1 (100, 16, 8, 4096 x 1024) 87.2 -> 78.5, 6 (256, 64, 4,
+        // 2048 x 512) 67.3 -> 65.7, 6.5 (160, 32, 4, 2048 x 1024) 63.2 -> 61.8; 7 (192) 64.1 -> 64.1, 8 (256) 68.0 -> 69.9, 8.6 (200, 32, 6)
+        // 74.0 -> 76.5, 12 (256, 32, 8) 97.3 -> 98.7.  K up to 1024 gives no such line, why is not known, and keeps two (6.5 (20, 50, 4, 1024 x 1024) 43.1 -> 43.6, 8 (256, 64,
+        // 8, 1024 x 512) 47.0 -> 48.1, 13.8 (200, 60, 8, 1024 x 1024) 73.7 -> 67.8).  Int4 weights (37.0 -> 38.0 at 128 tokens) keep two, and
+        // so does the down projection, which gains half as much and loses sooner.
+        const bool deep = g.epilogue == RKH_EPI_SWIGLU && g.K > 1024 && (long)mblocks * ((g.N + 63) / 64) * 2 <= 13L * cus;
+        mark(st, deep && any_int8 ? "gemm_stream_kernel<balanced, four steps>" : "gemm_stream_kernel<balanced>");
         const dim3 grid(cus), block(512);
 #define RK_LAUNCH_BAL(EPI)                                                                                          \
     do {                                                                                                            \
@@ -378,15 +387,6 @@ int launch_gemm_grouped(hipStream_t st, const rkh_gemm_args& g) {
         } else if (any_int8)                                                                                        \
             hipLaunchKernelGGL((gemm_stream_kernel<EPI, 1, false, true>), grid, block, 0, st, RK_GEMM_HEAD(g), mblocks, nblocks, g); \
     } while (0)
-        // Steps of a wave in flight: with at most six and a half units per compute unit (as many as the call can have) two
-        // steps of so few waves are too little for HBM, with more they are enough and a deeper ring only queues.  int8
-        // gate/up, whole layers, us, two -> four steps; units per compute unit: 4.5 (32 tokens, 32 experts, top-4, 2048 x 1024)
-        // 58.6 -> 56.9, 5 (256 tokens, 16 experts, top-8, 4096 x 512) 93.5 -> 84.1, 5.1 (100, 16, 8, 4096 x 1024) 87.2 -> 78.5, 6 (256, 64, 4,
-        // 2048 x 512) 67.3 -> 65.7, 6.5 (160, 32, 4, 2048 x 1024) 63.2 -> 61.8; 7 (192) 64.1 -> 64.1, 8 (256) 68.0 -> 69.9, 8.6 (200, 32, 6)
-        // 74.0 -> 76.5, 12 (256, 32, 8) 97.3 -> 98.7.  K up to 1024 gives no such line (6.5 (20, 50, 4, 1024 x 1024) 43.1 -> 43.6, 8 (256, 64,
-        // 8, 1024 x 512) 47.0 -> 48.1, 13.8 (200, 60, 8, 1024 x 1024) 73.7 -> 67.8).  Int4 weights (37.0 -> 38.0 at 128 tokens) keep two, and
-        // so does the down projection, which gains half as much and loses sooner.
-        const bool deep = g.epilogue == RKH_EPI_SWIGLU && g.K > 1024 && (long)mblocks * ((g.N + 63) / 64) * 2 <= 13L * cus;
         switch (g.epilogue) { // (grouped GEMMs are the MoE layer's: gate/up + SwiGLU and the fp32 down projection)
         case RKH_EPI_F32: RK_LAUNCH_BAL(RKH_EPI_F32); break;
         case RKH_EPI_SWIGLU: RK_LAUNCH_BAL(RKH_EPI_SWIGLU); break;

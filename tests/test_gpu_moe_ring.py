@@ -10,13 +10,13 @@ from rknpu2_matmul_open_amd import ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T,H,I,E,top_k,one_expert", [
-    (13, 1056, 1024, 48, 4, False),  # 49 row blocks x 32 pairs: 6.1 units per compute unit
-    (13, 1312, 1024, 52, 4, False),  # 53: 6.6
-    (32, 1088, 1024, 44, 4, True),   # 48, of which four are live
-    (13, 1024, 1024, 48, 4, False),  # the longest K that keeps the shallow ring
-    (64, 1056, 512, 60, 3, False)])
-def test_gate_up_ring(sess, oracle, T, H, I, E, top_k, one_expert):
+@pytest.mark.parametrize("T,H,I,E,top_k,one_expert,deep", [
+    (13, 1056, 1024, 48, 4, False, True),   # 49 row blocks x 32 pairs: 6.1 units per compute unit
+    (13, 1312, 1024, 52, 4, False, False),  # 53: 6.6
+    (32, 1088, 1024, 44, 4, True, True),    # 48, of which four are live
+    (13, 1024, 1024, 48, 4, False, False),  # the longest K that keeps the shallow ring
+    (64, 1056, 512, 60, 3, False, True)])
+def test_gate_up_ring(sess, oracle, T, H, I, E, top_k, one_expert, deep):
     rng = np.random.default_rng(T + H + E)
     experts = []
     for _ in range(E):
@@ -34,6 +34,8 @@ def test_gate_up_ring(sess, oracle, T, H, I, E, top_k, one_expert):
             assert sess.lib.rk_npu_moe_w8_run_f32_device(moe.ws, moe.w, T, dx, dids, drt, dout) == 0 and sess.sync() == 0 and rc2 == 0
             got = sess.from_device(dout, (T, H), np.float32)
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        kernels = ops.profile_kernels(sess, lambda: sess.lib.rk_npu_moe_w8_run_f32_device(moe.ws, moe.w, T, dx, dids, drt, dout), 1, 0)
+        assert kernels[1][0] == ("gemm_stream_kernel<balanced, four steps>" if deep else "gemm_stream_kernel<balanced>")
     finally:
         for d in (dx, dids, drt, dout):
             sess.free_device(d)
