@@ -750,10 +750,6 @@ __device__ __forceinline__ void moe_dot_tile(bool int4, const uint8_t* a_lds, in
         acc = __builtin_amdgcn_sdot4(a1.w, w.w & (int)0xF0F0F0F0, acc, false);
     }
 }
-__device__ __forceinline__ v4i moe_load_tile(const uint8_t* block, int idx, int tiles, int lane) {
-    return idx < tiles ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(block + (size_t)idx * 1024 + lane * 16))
-                       : v4i{0, 0, 0, 0};
-}
 
 constexpr int MOE_DECODE_PREFETCH = 4; // tiles per wave and column block requested ahead of the quantization
 
