@@ -10,9 +10,9 @@ the FFN, + route / combine for the MoE layer), enqueued through the
 device-pointer entry points of the C ABI and timed with HIP events on the
 context's stream (the stream the kernels are launched on).
 
-The headline workload is BASELINE config 1 (w8a8 decode GEMV, M=1, K=4096,
+The headline workload is configuration 1 (w8a8 decode GEMV, M=1, K=4096,
 N=14336), reported as weight GB/s.  The same line carries, under "also", every
-other BASELINE configuration (0, 2, 3, 4) and the int4 decode GEMV, each with
+other configuration (0, 2, 3, 4) and the int4 decode GEMV, each with
 its own roofline block (bound, dominant kernel, algorithmic bytes / operations,
 fraction of the datasheet peak), a per-kernel breakdown from stream events, and
 under "practical" what a read-only stream and a pure-MFMA loop reach on the box
@@ -608,7 +608,7 @@ def main():
     ap.add_argument("--steps", type=int, default=200)
     ap.add_argument("--warmup", type=int, default=20)
     ap.add_argument("--workload", default="all", choices=["c1", "all"],
-                    help="all: the headline line with every BASELINE configuration under \"also\" (default); "
+                    help="all: the headline line with every configuration under \"also\" (default); "
                          "c1: config 1, config 2 and the int4 GEMV only")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--only", default=None, choices=["c0", "c1", "c1w4", "c2", "c2w8", "c3", "c4", "llm_i8", "copy", "probes"],

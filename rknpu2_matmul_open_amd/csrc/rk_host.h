@@ -182,7 +182,7 @@ private:
 // memory and the device is staged and waited for inside the runtime (15-20 us
 // per direction when small; 36 GB/s up, 17 GB/s down when large); a DMA from /
 // to pinned memory costs 8-12 us when small and runs at 55 GB/s; a plain
-// memcpy runs at 80 GB/s.
+// memcpy runs at 75-80 GB/s while its buffers fit a core's caches and at 27 beyond.
 //  * Up to kLimit bytes ("direct"): no copy at all.  The quantization kernel
 //    reads A from the mirror (each row once) and the GEMM writes its result
 //    straight into the output's mirror, which adds ~1.5 us to a call.
@@ -230,8 +230,9 @@ private:
     bool staged_ = false;       // the enqueued download went through the mirror
 };
 
-// Large blocking calls on host buffers, in panels of rows: while one panel is multiplied, the next one is on its way
-// up and the last one's result on its way down (both directions together run at 95 GB/s, one alone at 55).
+// Large blocking calls on host buffers, in panels of rows: while one panel is multiplied or its result on its way down,
+// the next ones are copied and on their way up (both directions together run at 95 GB/s, one alone at 55).  Kernels
+// and downloads overlap only so far that a panel's kernels start beside the download before and end with it (below).
 // Quantization is by row and sums are exact, so the panels give the bits of the whole.
 //
 // What it is bound by: the download of a panel, 38 us for 2 MiB, and the copies between the caller's buffers and the

@@ -175,8 +175,8 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
     [[maybe_unused]] unsigned long long a_lanes = ~0ull;
     // A load to LDS needs a wait state behind a scalar write of M0, which the compiler does not insert into an asm
-    // statement (the build checks for it): the change of priority that a sub-step begins with is put there.  (An s_nop
-    // beside it cost 0.3 - 0.8 % of a GEMM.)
+    // statement (the build checks for it): the change of priority that a sub-step begins with is put there, so that
+    // the loop has no instruction more.  (With an s_nop 4096 x 4096 x 14336 int8 took 212.5 instead of 211.8 us.)
     auto copy_a = [&](int buf, auto prio_tag) { // global -> LDS, 16 bytes per lane, lane-contiguous
         constexpr int PRIO = decltype(prio_tag)::value;
         if constexpr (MASKED)    // (every lane is active here, and is again behind the copy)

@@ -221,7 +221,7 @@ def test_moe_extreme_codes_and_magnitudes(sess, oracle):
 
 
 def test_config4_full(sess, oracle):
-    """256 tokens, hidden 2048, 32 experts, top-4, intermediate 1024."""
+    """Configuration 4: 256 tokens, hidden 2048, 32 experts, top-4, intermediate 1024."""
     c = workloads.CONFIGS[4]()
     moe = ops.MoeW8(sess, c["H"], c["I"], c["E"], 0, c["top_k"], 256, c["experts"])
     try:

@@ -378,7 +378,7 @@ def test_weight_info_and_k_tile_resolution(sess):
 
 
 def test_config2_full_output_and_properties(sess, oracle, one_piece):
-    """BASELINE config 2 at full size (M=2048, K=4096, N=4096, seeds 4/5, 0.5% x20
+    """Configuration 2 at full size (M=2048, K=4096, N=4096, seeds 4/5, 0.5% x20
     outliers): every int8 activation, every fp16 output and every int32
     accumulator exact against the oracle (all 2048 rows), plus a size-independent
     property on the whole output: scaling a token by a power of two scales its
@@ -414,7 +414,7 @@ def test_config2_full_output_and_properties(sess, oracle, one_piece):
 
 
 def test_config3_ffn_full(sess, oracle):
-    """M=128, hidden 4096, intermediate 14336, seeds 6-9."""
+    """Configuration 3: M=128, hidden 4096, intermediate 14336, seeds 6-9."""
     c = workloads.CONFIGS[3]()
     M, H, I = c["M"], c["H"], c["I"]
     gw, dw = ops.W4A8Weights(sess, c["B_gu"], c["s_gu"]), ops.W4A8Weights(sess, c["B_down"], c["s_down"])

@@ -283,7 +283,7 @@ def test_rounding_ties_neighbours_saturation_and_nan(sess, oracle):
 
 
 def test_config0_full(sess, oracle):
-    """M=64, K=2048, N=2048, seeds 0/1."""
+    """Configuration 0: M=64, K=2048, N=2048, seeds 0/1."""
     c = workloads.CONFIGS[0]()
     op = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, c["M"], c["B"], c["w_scale"])
     try:
@@ -305,7 +305,7 @@ def test_config0_full(sess, oracle):
 
 
 def test_config1_full_decode(sess, oracle):
-    """M=1, K=4096, N=14336, seeds 2/3 (GEMV path)."""
+    """Configuration 1: M=1, K=4096, N=14336, seeds 2/3 (GEMV path)."""
     c = workloads.CONFIGS[1]()
     op = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, 1, c["B"], c["w_scale"])
     try:
