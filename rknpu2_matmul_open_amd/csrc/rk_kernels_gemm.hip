@@ -168,8 +168,8 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
 
     // Copies beyond K are issued like the others, for the count.  Tiles of 64 x 128 with int8 weights, which are bound by
     // the compute unit's memory path, issue them for one lane: twelve sub-steps of 8 KiB that nothing reads, beside the
-    // 32 of K = 4096.  us, quantization included: 256 rows x 4096 x 4096 19.5 -> 18.8, 128 x 6144 x 11008 29.0 -> 28.2,
-    // 128 x 4096 x 11008 exact 14.0 -> 13.8, 512 x 14336 x 4096 54.8 -> 54.1.  Int4 weights, whose bytes are fewer, lose
+    // 32 of K = 4096.  us, quantization included, two layers in turn: 256 rows x 4096 x 4096 28.8 -> 28.4, 128 x 6144 x 11008 58.9 ->
+    // 57.5, 128 x 4096 x 11008 exact 39.2 -> 37.4, 512 x 14336 x 4096 108.1 -> 105.9.  Int4 weights, whose bytes are fewer, lose
     // what the scalar instructions cost (256 x 4096 x 4096 13.3 -> 13.5), 128-row tiles gain nothing (1000 x 2048 x 3000
     // 15.5 -> 15.6), and neither do the weights, of which three sub-steps lie beyond K.
     constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
