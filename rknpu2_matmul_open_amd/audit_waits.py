@@ -16,7 +16,9 @@ with the same flags):
     younger load is, so the wait that covers a load is the first one behind it with N <= the
     number of loads issued since (stores are not counted: they may complete out of order, which
     can only make a wait stricter than this rule assumes);
-  * LDS reads (ds_read from asm) are covered by the next s_waitcnt with lgkmcnt(0);
+  * LDS operations of a wave complete in issue order as well, so an asm ds_read is covered by the first
+    s_waitcnt lgkmcnt(N) with N <= the number of LDS operations issued since (scalar loads, which share
+    the counter, can only make that wait stricter);
   * between an asm load and its covering wait no instruction may name one of its destination
     registers;
   * a load to LDS takes its address from M0, and needs one wait state behind a scalar write of M0: the
@@ -40,7 +42,8 @@ _VM_LOAD = re.compile(r"^\s*(global_load|buffer_load|flat_load|scratch_load)")
 _ASM_VLOAD = re.compile(r"^\s*global_load_dwordx?(\d*)\s+(v\[\d+:\d+\]|v\d+)\s*,")
 _ASM_DSREAD = re.compile(r"^\s*ds_read_b(\d+)\s+(v\[\d+:\d+\]|v\d+)\s*,")
 _VMCNT = re.compile(r"vmcnt\((\d+)\)")
-_LGKM0 = re.compile(r"lgkmcnt\(0\)")
+_LGKMCNT = re.compile(r"lgkmcnt\((\d+)\)")
+_DS_OP = re.compile(r"^\s*ds_")
 _REG = re.compile(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b")
 _LABEL = re.compile(r"^(\.LBB\d+_\d+):")
 _BRANCH = re.compile(r"^\s*s_cbranch_\w+\s+(\.LBB\d+_\d+)|^\s*s_branch\s+(\.LBB\d+_\d+)")
@@ -124,16 +127,12 @@ def _check_load(instrs, blocks, block_of, at, what, violations, seen):
             if t.endswith(":"):
                 continue
             if "s_waitcnt" in t:
-                if m:
-                    c = _VMCNT.search(t)
-                    if c and int(c.group(1)) <= issued:
-                        covered = True
-                        break
-                elif _LGKM0.search(t):
+                c = (_VMCNT if m else _LGKMCNT).search(t)
+                if c and int(c.group(1)) <= issued:
                     covered = True
                     break
                 continue
-            if m and _VM_LOAD.match(t):
+            if (_VM_LOAD if m else _DS_OP).match(t):
                 issued += 1
             parts = t.split(None, 1)
             hit = dst & _regs(parts[1] if len(parts) > 1 else "")

@@ -13,7 +13,7 @@
 //   gemv_kernel                         M <= 8 decode path: dot4, no MFMA, optional fused
 //                                       per-token quantization                           (HBM)
 //   gemv_swiglu_kernel                  gate/up + SwiGLU of one or two rows              (HBM)
-//   gemm_wk_kernel                      int8 MFMA 32x32x32, (32..128) x 256 tiles, activations
+//   gemm_wk_kernel                      int8 MFMA 16x16x64, (32..128) x 256 / 128 tiles, activations
 //                                       through an LDS ring, waves split K               (MFMA)
 //   gemm_wk_big_kernel                  256 x 256 tiles (128 x 256 for the rest), waves split
 //                                       the rows: more than one round of 128 x 256 tiles (MFMA)

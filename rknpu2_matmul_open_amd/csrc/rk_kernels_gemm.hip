@@ -5,48 +5,50 @@
 
 namespace {
 
-// ---- tiles of (32 * TM) rows x 256 columns, waves split K --------------------
-// Eight waves = 4 column groups (wn) x 2 k-halves (wk): wave (wn, wk)
-// accumulates the whole (32*TM) x 64 strip of column group wn, but only over
-// every second 32-deep k-tile (k-tile % 2 == wk); the two halves are summed
-// once, through LDS, before the epilogue.  Compared with splitting the rows
-// between the two waves that share a SIMD, no weight byte is loaded (or
-// unpacked) by two waves, which takes a third off the traffic through the
-// vector memory path and halves the int4 unpack work.
+// ---- tiles of (32 * TM) rows x (128 * TN) columns ------------------------------
+// v_mfma_i32_16x16x64_i8.  Large launches run at the clock that the power limit leaves, so energy per product
+// is what counts: a loop of nothing but MFMAs on quantized activations (codes of N(0, 2.5) with outliers) and
+// N(0, 30) weights reaches 3.53 POP/s with 32x32x32 and 4.19 with 16x16x64 (int4 weights as 16 * code: 3.77 and 4.67),
+// presumably because an instruction moves half the accumulator bytes per product.  Calls with quantization, us, from
+// 32x32x32 with each sub-step's loads issued together to this loop, one box: int4 2048 x 4096 x 4096 39.1 -> 34.8, 4096^3
+// 68.5 -> 59.5, int8 4096 x 4096 x 14336 202 -> 190, 1000 x 4096 x 4096 26.2 -> 24.2; int4 512 x 14336 x 4096 40.0 -> 36.3,
+// the FFN 4096 -> 14336 -> 4096 of 128 / 512 rows 42.6 -> 40.8 / 102 -> 94.
 //
-// A sub-step always covers 8 KiB of activations = (32*TM) rows x (8/TM)
-// k-tiles, i.e. 64 / 128 / 256 k for TM = 4 / 2 / 1, so that whatever the tile
-// height a wave issues per sub-step one 1 KiB activation copy, four 16-byte
-// fragment reads and eight MFMAs.
+// Eight waves = 4 column groups (wn) x 2.  In the tiles of up to 128 rows the two waves of a column group
+// split K (k-half wk): each accumulates all rows x 32 * TN columns over every second 128 k, and the halves are
+// summed once, through LDS, before the epilogue -- no weight byte is loaded (or unpacked) by two waves.  In
+// the tiles of 256 x 256 (RS) they split the rows (row half wk): 128 x 64 each over the whole K, no exchange.
 //
-// Activations: every wave copies its 1 KiB share of a sub-step global -> LDS
-// directly (no registers), D sub-steps ahead (WK_D; 8 for the 128-row tile), into
-// a ring of WK_NBUF buffers.  Weights: global -> registers, NSW-1 sub-steps ahead (8 bytes per
-// lane and k-tile pair for int4, 16 per k-tile for int8).  The fragments of
-// the NEXT sub-step are read and, for int4, its operands unpacked in the
-// shadow of this sub-step's MFMAs.
+// For a wave K goes in units of 64 k: RM activation operands of 16 rows and CN weight operands of 16 columns, RM x CN MFMAs.
+// A step -- what is copied to LDS at a time -- is one or two units of every wave (two where int4 super-tiles are
+// shared by a pair of units, and where one would be less than 8 KiB of activations).  A k-tile is 32 rows x 32 k with 16 bytes per lane; operand lane (r, q) = (l % 16, l / 16)
+// takes row 16 h + r, k-half q % 2 of k-tile q / 2 of the unit's two, i.e. both operands are read with per-lane addresses in
+// pieces of 256 contiguous bytes (which k a lane group holds is free as long as both operands agree).  Int4 super-tiles
+// hold 64 k in 16 bytes per lane: one load brings the words of both units, lane group q the k-half q % 2 of super-tile
+// q / 2 of the step's two, and unit u takes k-tile u of each.
 //
-// A workgroup barrier costs a good part of a sub-step's MFMA time (the matrix
-// pipes drain while the waves meet), so there is only one every WK_G
-// sub-steps.
+// Activations: every wave copies NC KiB of a step global -> LDS directly (no registers), D steps ahead, into a
+// ring of NBUF buffers.  Weights: global -> registers, NSW - 1 units ahead (int4: steps).  An operand of the next
+// unit is read from LDS into the registers of the one that the last CN MFMAs have used, and waited for one unit later:
+// LDS reads complete in order, so a counted wait leaves the younger RM - 1 in flight.
 //
-// All loads of the loop are inline assembly and every wait is explicit.  (The
-// compiler's own bookkeeping orders each LDS read and each register load after
-// ALL outstanding global -> LDS copies, which would undo the prefetch.)  The
-// waits rely on vector memory loads completing in issue order and on every
-// sub-step issuing exactly LPS loads -- copy first, then weights -- also
-// beyond the end of K, where the source pointers simply stop advancing (those
-// loads hit the L1 and their results are never used).  With that:
-//  * weights of sub-step s+1 were issued at s+1-(NSW-1); (NSW-2) * LPS loads
-//    have been issued since, hence vmcnt((NSW-2) * LPS);
-//  * publication: the fragments read during sub-steps B+1..B+G (B = last
-//    sub-step before a barrier) belong to sub-steps <= B+G+1; their copies
-//    were issued at sub-steps <= B+G+1-D, before the weights a wave waits for
-//    during sub-step B, so they have landed when it reaches the barrier
-//    (needs D >= NSW + G - 1);
-//  * reuse: the copy issued at sub-step s overwrites the buffer that held
-//    sub-step s+D-NBUF, last read at sub-step s+D-NBUF-1 <= s-G-1, which is
-//    before the latest barrier (needs NBUF >= D + G).
+// The loads of a unit are spread between its MFMAs.  Issued together behind a barrier, the eight waves' loads queue in front of
+// the compute unit's 64 B per clock and a wave stands still until its own have been taken (256 x 256 tiles, int8:
+// 1274 cycles per 64 k of which 1024 are MFMAs; spread 1124).
+//
+// All loads of the loop are inline assembly and every wait is explicit.  (The compiler's own bookkeeping orders each
+// LDS read after ALL outstanding global -> LDS copies, which would undo the prefetch.)  The waits rely on vector
+// memory loads completing in issue order and on every unit issuing the same loads -- copies first, then weights -- also
+// beyond the end of K, where the source pointers stop advancing (those loads hit the L1 and nothing uses them):
+//  * weights: unit t ends with the wait for those of unit t + 1, issued in unit t + 2 - NSW; the loads of the
+//    NSW - 2 units since may be outstanding.  (int4: the second unit of step s waits, ahead of its unpacking, for the
+//    weights of step s + 1, issued in the first unit of step s + 2 - NSW.)
+//  * publication: between the barrier at the end of step B and the next one, G steps later, waves read operands of steps up to
+//    B + G + 1.  Those were copied in steps up to B + G + 1 - D: the last wait ahead of the barrier leaves no older copy
+//    in flight (in_flight() is the smaller of the two bounds).
+//  * reuse: the copy issued in step s overwrites the buffer of step x = s + D - NBUF, whose last reads were
+//    issued in the first unit of step x and waited for in its second, ahead of the barrier that ends a step in x .. s - 1
+//    (needs NBUF >= D + G).
 //
 // Split K over workgroups (ksplit > 1, small M): every part stores its int32
 // tile in accumulator order to scratch and gemm_wk_reduce_kernel, launched
@@ -54,10 +56,12 @@ namespace {
 // kernel, in the part that arrives last, needs a device-scope release per
 // workgroup; on this multi-die part each one walks the die's L2, and 32
 // workgroups per die queueing for that cost more than the second launch.)
-constexpr int WK_NBUF = 16, WK_G = 4, WK_D = 12, WK_BUF = 8 * 1024;
-constexpr int WK_SCALES_OFF = WK_NBUF * WK_BUF;                   // fp32 scales of the tile: 256 rows, then 256 columns
+constexpr int WK_RING_BYTES = 128 * 1024;
+constexpr int WK_SCALES_OFF = WK_RING_BYTES;                      // fp32 scales of the tile: 256 rows, then 256 columns
 constexpr int WK_ROW_SCALES = 256;
 constexpr int WK_LDS_BYTES = WK_SCALES_OFF + (WK_ROW_SCALES + 256) * 4;
+constexpr int WK_STAGE = 2 * 16 * 144;                            // a wave's staging area: two units of 16 rows x 32 columns
+constexpr int WK_PART_K = 256;                                    // granularity of a K split over workgroups
 
 typedef __attribute__((address_space(3))) uint8_t* lds_ptr_t;
 
@@ -77,433 +81,471 @@ __device__ __forceinline__ void wk_tile_coords(unsigned tile, unsigned mblocks, 
     nblk = (int)col;
 }
 
+// ---- 16 x 16 accumulator tiles --------------------------------------------------
+// The weights are the FIRST MFMA operand: lane (r, q) owns output row r of the tile and its columns 4 q .. 4 q + 3.
+// Two neighbouring tiles make a unit of 16 rows x 32 columns, the width of a column block.
+
+// Stage a unit in one half of the wave's staging area and read it back as 16-byte pieces of rows.  LDS operations of a wave
+// complete in issue order, so nothing is waited for between the two; the fence keeps the compiler from swapping them.
+template <typename T>
+struct StagedUnit {
+    static constexpr int ES = sizeof(T), PITCH = 32 * ES + 16, PIECES = ES / 2; // 16-byte pieces of a lane
+    v4i piece[PIECES];
+    __device__ __forceinline__ void exchange(const T (&vals)[8], uint8_t* stage, int lane) {
+        const int r = lane & 15, q = lane >> 4;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            T* dst = reinterpret_cast<T*>(stage + r * PITCH + (16 * h + 4 * q) * ES);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst[e] = vals[4 * h + e];
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < PIECES; ++t) {
+            const int c = lane + 64 * t;
+            piece[t] = *reinterpret_cast<const v4i*>(stage + c / (2 * ES) * PITCH + c % (2 * ES) * 16);
+        }
+    }
+    template <bool ALL_ROWS>
+    __device__ __forceinline__ void store(T* C, int ldc, int m0, int n0, int m_limit, int lane) const {
+#pragma unroll
+        for (int t = 0; t < PIECES; ++t) {
+            const int c = lane + 64 * t, row = c / (2 * ES);
+            if (ALL_ROWS || m0 + row < m_limit) // the output is not read again by this kernel: streaming store
+                __builtin_nontemporal_store(piece[t], reinterpret_cast<v4i*>(reinterpret_cast<uint8_t*>(C) + ((size_t)(m0 + row) * ldc + n0) * ES +
+                                                                             c % (2 * ES) * 16));
+        }
+    }
+};
+
+// A unit whose columns end inside it, or whose rows are not 16-byte aligned in C.
+template <typename T>
+__device__ __forceinline__ void store_unit_plain(T* C, int ldc, int m0, int n0, int m_limit, int n_limit, const T (&vals)[8], int lane) {
+    const int m = m0 + (lane & 15);
+    if (m >= m_limit) return;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int n = n0 + 16 * (e >> 2) + 4 * (lane >> 4) + (e & 3);
+        if (n < n_limit) C[(size_t)m * ldc + n] = vals[e];
+    }
+}
+
+template <int EPI>
+using wk_out_t = typename std::conditional<EPI == RKH_EPI_I32, int, typename std::conditional<EPI == RKH_EPI_F16, __half, float>::type>::type;
+
+// Scale, convert and store ROWS x (16 * CN) sums of a wave: acc_of(i, j) is the tile of rows m0 + 16 i and physical columns
+// pb0 * 32 + 16 j, as(i) / ws(j, e) the lane's row scale and column scales.
+template <int ROWS, int CN, bool W4, int EPI, class Acc, class RowScale, class ColScale>
+__device__ __forceinline__ void wk_store(const rkh_gemm_args& g, Acc&& acc_of, RowScale&& as, ColScale&& ws, int m0, int pb0,
+                                         int m_limit, uint8_t* stage, int lane) {
+    using T = wk_out_t<EPI>;
+    constexpr bool SWIGLU = EPI == RKH_EPI_SWIGLU;
+    constexpr int NB = SWIGLU ? 1 : CN / 2; // column blocks stored per 16 rows
+    T* C = static_cast<T*>(g.C);
+    int n0[NB], n_end = SWIGLU ? g.interleave_F : g.N;
+    bool live[NB], whole[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        // padding blocks beyond the matrix hold zeros; with interleaved columns their logical index would alias a real
+        // column, so the block itself is tested
+        const int pb = pb0 + b;
+        n0[b] = SWIGLU ? (pb0 >> 1) * 32 : block_first_col(pb, g.interleave_F);
+        live[b] = SWIGLU ? n0[b] < n_end : g.interleave_F ? pb < g.N / 32 : pb * 32 < g.N;
+        whole[b] = n0[b] + 32 <= n_end &&
+                   ((reinterpret_cast<uintptr_t>(C) | ((size_t)g.ldc * sizeof(T)) | ((size_t)n0[b] * sizeof(T))) & 15) == 0;
+    }
+    uint32_t bits[ROWS];
+    const auto values = [&](T (&vals)[8], int i, int b) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int j = 2 * b + (e >> 2);
+            int sum = acc_of(i, j)[e & 3];
+            if (W4) sum >>= 4;
+            if constexpr (EPI == RKH_EPI_I32) {
+                vals[e] = sum;
+            } else if constexpr (SWIGLU) {
+                int up = acc_of(i, CN / 2 + j)[e & 3];
+                if (W4) up >>= 4;
+                const float gate = dequant(sum, as(i), ws(j, e & 3));
+                const float y = __fmul_rn(silu_poly(gate), dequant(up, as(i), ws(CN / 2 + j, e & 3)));
+                top = max(top, __float_as_uint(y) & 0x7fffffffu);
+                vals[e] = y;
+            } else if constexpr (EPI == RKH_EPI_F16) {
+                vals[e] = __float2half_rn(dequant(sum, as(i), ws(j, e & 3)));
+            } else {
+                vals[e] = dequant(sum, as(i), ws(j, e & 3));
+            }
+        }
+        bits[i] = top;
+    };
+    bool full = m0 + 16 * ROWS <= m_limit;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) full = full && live[b] && whole[b];
+    if (full) { // straight-line code: a unit is stored behind the exchange of the next one
+        StagedUnit<T> held[2];
+#pragma unroll
+        for (int u = 0; u < ROWS * NB; ++u) {
+            T vals[8];
+            values(vals, u / NB, u % NB);
+            held[u & 1].exchange(vals, stage + (u & 1) * (WK_STAGE / 2), lane);
+            if (u > 0) held[(u - 1) & 1].template store<true>(C, g.ldc, m0 + 16 * ((u - 1) / NB), n0[(u - 1) % NB], m_limit, lane);
+        }
+        held[(ROWS * NB - 1) & 1].template store<true>(C, g.ldc, m0 + 16 * (ROWS - 1), n0[NB - 1], m_limit, lane);
+    } else {
+#pragma unroll
+        for (int u = 0; u < ROWS * NB; ++u) {
+            const int i = u / NB, b = u % NB;
+            if (!live[b]) continue;
+            T vals[8];
+            values(vals, i, b);
+            StagedUnit<T> unit;
+            if (whole[b]) {
+                unit.exchange(vals, stage + (u & 1) * (WK_STAGE / 2), lane);
+                unit.template store<false>(C, g.ldc, m0 + 16 * i, n0[b], m_limit, lane);
+            } else {
+                store_unit_plain(C, g.ldc, m0 + 16 * i, n0[b], m_limit, n_end, vals, lane);
+            }
+        }
+    }
+    if constexpr (SWIGLU) {
+        if (g.row_max_bits && live[0]) { // largest |middle| per row and 32 columns
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i) {
+                uint32_t top = max(bits[i], (uint32_t)__shfl_xor((int)bits[i], 16));
+                top = max(top, (uint32_t)__shfl_xor((int)top, 32));
+                const int m = m0 + 16 * i + lane;
+                if (lane < 16 && m < m_limit) g.row_max_bits[(size_t)m * (n_end / 32) + (pb0 >> 1)] = top;
+            }
+        }
+    }
+}
+
+template <int N> __device__ __forceinline__ void wait_lds(v4i& x) { asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory"); }
+template <int OFF> __device__ __forceinline__ void read_lds(v4i& x, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x) : "v"(addr), "n"(OFF));
+}
+template <int OFF> __device__ __forceinline__ void load_regs(v4i& x, unsigned lane_off, const uint8_t* base) {
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(x) : "v"(lane_off), "s"(base), "n"(OFF));
+}
+__device__ __forceinline__ void keep(v4i& x) { asm volatile("" : "+v"(x)); }
+
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm" // m0 is set and clobbered on purpose below
-// TN: 32-column blocks per wave.  Two -- tiles of 256 columns; one -- tiles of 128 columns, for a few
-// hundred rows whose 256-column tiles would leave compute units without one (launch_gemm_wk_narrow).
+// 16 bytes per lane, lane-contiguous, global -> LDS; the offset counts on both sides.  A load to LDS needs a wait state
+// behind a scalar write of M0, which the compiler does not insert into an asm statement (the build checks for it): the
+// change of the wave's priority is put there.
+template <int OFF, int PRIO> __device__ __forceinline__ void copy_lds(unsigned lane_off, const uint8_t* src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_setprio %4\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(lane_off), "s"(src), "s"(dst), "n"(OFF), "n"(PRIO)
+                 : "memory", "m0");
+}
+// The same for the lanes of a mask (every lane is active here, and is again behind the copy).
+template <int OFF, int PRIO> __device__ __forceinline__ void copy_lds(unsigned lane_off, const uint8_t* src, uint32_t dst, unsigned long long lanes) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_setprio %4\n\ts_mov_b64 exec, %5\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3\n\ts_mov_b64 exec, -1" ::"v"(lane_off),
+                 "s"(src), "s"(dst), "n"(OFF), "n"(PRIO), "s"(lanes) : "memory", "m0");
+}
+__device__ __forceinline__ void copy_lds_dword(const float* src, uint32_t dst) { // 4 bytes per lane, likewise
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// The shape of a tile and of its pipeline.
+template <int TM, bool W4, int TN, bool RS>
+struct WkShape {
+    static_assert(!RS || (TM == 4 && TN == 2), "row-split waves: tiles of 256 x 256");
+    static constexpr bool ONE = TM == 4 && !W4;                 // a step is one unit
+    static constexpr int U = ONE ? 1 : 2;
+    static constexpr int RM = 2 * TM, CN = 2 * TN;              // operands of 16 rows / columns per wave
+    static constexpr int BM = RS ? 256 : 32 * TM;               // rows of a tile
+    static constexpr int KT = (RS ? 2 : 4) * U;                 // k-tiles of a step
+    static constexpr int BUF = BM / 32 * KT * 1024, NBUF = ONE ? 6 : TM == 4 ? 4 : 8;
+    static constexpr int NC = BUF / 8192;                       // 1 KiB copies of a wave per step
+    static constexpr int NW = CN;                               // weight loads per unit (int4: per step, in its first unit)
+    static constexpr int NSW = ONE ? 3 : TM == 4 ? 2 : 4;       // slots of the weight ring
+    static constexpr int G = ONE || (W4 && TM < 4) ? 2 : 1;             // steps between barriers
+    static constexpr int D = ONE ? 4 : W4 && TM < 4 ? 5 : 3;         // look-ahead of the copies
+    static constexpr int UNR = NBUF;                            // steps of an unrolled trip
+    static constexpr int copies(int unit) { return U == 1 ? NC : NC == 1 ? (unit & 1 ? 0 : 1) : NC / 2; }
+    static constexpr bool loads_w(int unit) { return !W4 || !(unit & 1); }
+    static constexpr int items(int unit) { return copies(unit) + (loads_w(unit) ? NW : 0); }
+    static constexpr int per_step() { return items(0) + (U == 2 ? items(1) : 0); }
+    // loads of a wave that may be outstanding at the wait of unit `u` of a step (int4: 1)
+    static constexpr int in_flight(int u) {
+        int weights = 0;                                        // issued since the next weights
+        if (W4) weights = items(1) + (NSW - 2) * per_step();
+        else for (int t = 0; t < NSW - 2; ++t) weights += items(U == 1 ? 0 : (u + t) & 1);
+        // issued since the last copy of step B + G + 1 - D
+        const int copied = (W4 ? (NC == 1 ? NW : 0) : U == 2 && NC == 1 ? 2 * NW : NW) + (D - G - 1) * per_step();
+        return u == U - 1 && copied < weights ? copied : weights;
+    }
+    // weights loaded in `unit`: of which unit (int4: step)
+    static constexpr int loaded(int unit) { return W4 ? (unit >> 1) + NSW - 1 : unit + NSW - 1; }
+    // what the prologue has issued since the copies that its wait is to see (its first steps load no weights)
+    static constexpr int prologue_since() {
+        int n = 0;
+        for (int unit = U * (G + 1 - D); unit < 0; ++unit) n += copies(unit) + (loads_w(unit) && loaded(unit) >= 0 ? NW : 0);
+        return n;
+    }
+    static_assert(D >= G + 1 && NBUF >= D + G && UNR % G == 0 && (W4 ? UNR : U * UNR) % NSW == 0, "see the ordering rules above");
+    static constexpr int first_wait() { return in_flight(U - 1) < prologue_since() ? in_flight(U - 1) : prologue_since(); }
+    static_assert(in_flight(0) <= 63 && in_flight(U - 1) <= 63, "the vmcnt field");
+    static_assert(NBUF * BUF <= WK_RING_BYTES && 4 * RM * CN * 1024 <= WK_RING_BYTES, "the ring; the exchange of k-halves");
+};
+
 template <int TM, bool W4, int EPI, int TN, bool RS>
 __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw, int tile, int mblk, int nblk, int kpart,
-                                        int ksplit, int kstep0, int ksteps) {
-    constexpr int KTS = RS ? 1 : 8 / TM, KTW = RS ? 1 : KTS / 2; // k-tiles per sub-step: all / this wave's
-    constexpr int NMF = TM * KTW * TN;         // MFMAs of a wave per sub-step
-    static_assert(!RS || (TM == 4 && TN == 2), "row-split waves: tiles of 256 x 256");
+                                        int ksplit, int kt0, int kts) { // the part's first k-tile and their number, a multiple of 8
+    using S = WkShape<TM, W4, TN, RS>;
     static_assert(TN == 2 || (TN == 1 && EPI != RKH_EPI_SWIGLU), "gate / up pairs need two column blocks per wave");
-    // Look-ahead: weights NSW - 1 sub-steps, activation copies D sub-steps.  The 128-row tile runs
-    // one tile per compute unit, all of them at once, so what the prologue requests before the first
-    // MFMA (D copies + NSW - 1 weight groups per wave, 152 KB per compute unit with 8 / 12) is
-    // issue-bound in the vector memory path: in-kernel time stamps showed 1.9 us until the requests
-    // were out and 3.1 us until the first MFMA.  4 / 8 is enough to cover the latency (a sub-step
-    // is ~570 cycles) and starts the loop sooner: 2048 x 4096 x 4096, same box, int8 weights
-    // 30.8 -> 30.25 us, int4 32.55 -> 32.15 us.  (The 64-row int4 tile measured the same with
-    // either depth and keeps the deeper one.)
-    constexpr int NSW = TM == 4 ? 4 : (TM == 2 && W4) ? 8 : 4;
-    constexpr int NBUF = WK_NBUF, G = WK_G, D = TM == 4 && !(RS && W4) ? 8 : WK_D, BM = RS ? 256 : 32 * TM, BUF = WK_BUF;
-    // (RS, int4: a super-tile is two sub-steps, loaded whole -- 16 bytes per lane -- at every even one;
-    // the ring's slots are super-tiles)
-    constexpr bool WPAIR = RS && W4;
-    constexpr int UNR = 16;            // sub-steps per unrolled trip: multiple of NSW, NBUF, G and 2
-    // int4 weights come in 1 KiB super-tiles of two k-tiles (16 bytes per lane).  When a
-    // wave has two or more k-tiles per sub-step it takes WHOLE super-tiles (k-tiles
-    // 4v + 2*wk, 4v + 2*wk + 1), one 16-byte load each; taking every second k-tile
-    // instead would make both k-halves fetch every cache line for half of its bytes,
-    // which doubles the weight traffic through the L1 and makes that the limit of the
-    // 64- and 32-row tiles.  (With one k-tile per wave and sub-step, TM = 4, the two
-    // halves of a super-tile necessarily go to the two waves, 8 bytes per lane each.)
-    constexpr bool PAIRED = W4 && KTW >= 2;
-    constexpr int NWOP = KTW * TN;                              // weight operands (k-tile x column block) per sub-step
-    constexpr int NWREG = PAIRED ? (KTW / 2) * TN : KTW * TN;   // weight loads (registers of the ring) per sub-step
-    constexpr int LPS = 1 + NWREG;                              // loads per sub-step and wave
-    static_assert(UNR % NSW == 0 && UNR % NBUF == 0 && UNR % G == 0, "slot arithmetic must be compile-time");
-    static_assert(WPAIR ? D >= 2 * NSW - 2 + G && NBUF >= D + G : D >= NSW + G - 1 && NBUF >= D + G, "see the ordering rules above");
-    // loads of a wave that may be outstanding while it waits for the next weights: (NSW - 2) sub-steps' worth, or,
-    // with super-tiles of two sub-steps, the copies of the sub-steps since and the super-tiles behind the wanted one
-    constexpr int IN_FLIGHT = WPAIR ? 2 * (NSW - 1) - 1 + (NSW - 2) * NWREG : (NSW - 2) * LPS;
-    static_assert(IN_FLIGHT <= 63, "vmcnt field");
+    constexpr int U = S::U, RM = S::RM, CN = S::CN, KT = S::KT, BUF = S::BUF, NBUF = S::NBUF, NSW = S::NSW;
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
     const int wn = wave & 3, wk = wave >> 2; // column group; k-half (RS: row half)
-    const int Kp = (int)rkh_align_up(g.K, RKH_K_ALIGN);
-    const int KB = Kp / 32;
-
-    const uint8_t* Wb = g.W;
-    const float* w_scale = g.w_scale;
-    const int m_limit = g.M;
+    const int KB = (int)rkh_align_up(g.K, RKH_K_ALIGN) / 32;
 
     // ---- sources: wave-uniform base pointers (scalar registers) + a constant lane offset.
-    // activation chunk of this wave: row block wave / KTS, k-tile wave % KTS of the sub-step
-    const uint8_t* asrc = g.A + ((size_t)(mblk * (BM / 32) + wave / KTS) * KB + (size_t)kstep0 * KTS + wave % KTS) * 1024;
-    // int8 weights of a wave with four k-tiles per sub-step span 6 KiB; the base
-    // sits in the middle so that the 13-bit signed instruction offset reaches all
-    constexpr int W_BIAS = (!W4 && KTW > 2) ? 4096 : 0;
-    const uint8_t* wsrc[TN];
+    // The step's copies of a wave are NC consecutive KiB: of row block wave * NC / KT, from k-tile wave * NC % KT on
+    const uint8_t* asrc = g.A + ((size_t)(mblk * (S::BM / 32) + wave * S::NC / KT) * KB + kt0 + wave * S::NC % KT) * 1024;
+    const uint8_t* wsrc[TN]; // (int4: two k-tiles per KiB)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int pb = nblk * (4 * TN) + wn * TN + j;
-        wsrc[j] = RS   ? Wb + (size_t)pb * (W4 ? KB / 2 : KB) * 1024 // (K is not split over workgroups)
-                  : W4 ? Wb + ((size_t)pb * (KB / 2) + (size_t)kstep0 * KTW) * 1024 + (PAIRED ? wk * 1024 : wk * 8)
-                       : Wb + ((size_t)pb * KB + (size_t)kstep0 * KTS + wk) * 1024 + W_BIAS;
-    }
+    for (int j = 0; j < TN; ++j)
+        wsrc[j] = g.W + ((size_t)(nblk * (4 * TN) + wn * TN + j) * KB + kt0 + (RS ? 0 : wk * 2 * U)) * (W4 ? 512 : 1024);
+    const int q = lane >> 4;
     const unsigned lane_off = lane * 16;
-    constexpr int A_STEP = KTS * 1024, W_STEP = W4 && !RS ? KTW * 1024 : KTS * 1024; // (WPAIR: per super-tile)
-    using wraw_t = typename std::conditional<W4 && !PAIRED && !RS, v2i, v4i>::type;
+    const unsigned piece_off = (q >> 1) * 1024 + (q & 1) * 512 + (lane & 15) * 16; // this lane's piece of an operand
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds_raw;
-    const uint32_t copy_dst = lds_base + wave * 1024; // this wave's chunk inside buffer 0
-    // LDS byte addresses of this lane's fragment (row block 0, this wave's first k-tile) in buffers 0 and 8
-    uint32_t frag_lo = lds_base + wk * (RS ? 4096 : PAIRED ? 2048 : 1024) + lane * 16;
-    uint32_t frag_hi = frag_lo + 8 * BUF;
-    int a_left = ksteps - 1, w_left = (WPAIR ? ksteps / 2 : ksteps) - 1; // how often the sources may still advance
+    const uint32_t copy_dst = lds_base + wave * S::NC * 1024; // this wave's chunk inside buffer 0
+    // LDS byte addresses of this lane's piece of the wave's first operand in buffer 0 and 64 KiB on
+    const uint32_t frag_lo = lds_base + (RS ? wk * (RM / 2) * KT : wk * 2 * U) * 1024 + (W4 ? piece_off + (q >> 1) * 1024 : piece_off);
+    const uint32_t frag_hi = frag_lo + 65536;
+    const int ksteps = kts / KT;
+    int a_left = ksteps - 1, w_left = ksteps - 1; // how often the sources may still advance
 
-    v16i acc[TM][TN];
+    v4i acc[RM][CN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < RM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+        for (int j = 0; j < CN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
 
-    wraw_t wring[NSW][NWREG]; // weight prefetch ring, index u * TN + j
-    v4i afr[2][4];            // activation fragments (index u * TM + i), this sub-step / next
-    v4i wop[2][NWOP];         // int4 only: unpacked operands (index u * TN + j), this sub-step / next
+    v4i a[RM];                  // activation operands
+    v4i wring[NSW][CN];         // weights as loaded: of a unit, or, int4, of a step
+    [[maybe_unused]] v4i wop[2][CN]; // int4 only: unpacked operands, this unit / next
 
     // Copies beyond K are issued like the others, for the count.  Tiles of 64 x 128 with int8 weights, which are bound by
-    // the compute unit's memory path, issue them for one lane: twelve sub-steps of 8 KiB that nothing reads, beside the
-    // 32 of K = 4096.  us, quantization included, two layers in turn: 256 rows x 4096 x 4096 28.8 -> 28.4, 128 x 6144 x 11008 58.9 ->
-    // 57.5, 128 x 4096 x 11008 exact 39.2 -> 37.4, 512 x 14336 x 4096 108.1 -> 105.9.  Int4 weights, whose bytes are fewer, lose
-    // what the scalar instructions cost (256 x 4096 x 4096 13.3 -> 13.5), 128-row tiles gain nothing (1000 x 2048 x 3000
-    // 15.5 -> 15.6), and neither do the weights, of which three sub-steps lie beyond K.
+    // the compute unit's memory path, issue them for one lane: three steps of 16 KiB that nothing reads, beside the 16 of
+    // K = 4096 (exact 128 x 4096 x 11008 13.9 -> 13.65 us, 512 x 4096 x 4096 16.5 -> 16.3; int4 weights and wider tiles gain nothing).
     constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
     [[maybe_unused]] unsigned long long a_lanes = ~0ull;
-    // A load to LDS needs a wait state behind a scalar write of M0, which the compiler does not insert into an asm
-    // statement (the build checks for it): the change of priority that a sub-step begins with is put there, so that
-    // the loop has no instruction more.  (With an s_nop 4096 x 4096 x 14336 int8 took 212.5 instead of 211.8 us.)
-    auto copy_a = [&](int buf, auto prio_tag) { // global -> LDS, 16 bytes per lane, lane-contiguous
-        constexpr int PRIO = decltype(prio_tag)::value;
-        if constexpr (MASKED)    // (every lane is active here, and is again behind the copy)
-            asm volatile("s_mov_b32 m0, %2\n\ts_setprio %4\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lane_off),
-                         "s"(asrc), "s"(copy_dst + buf * BUF), "s"(a_lanes), "n"(PRIO)
-                         : "memory", "m0");
-        else
-            asm volatile("s_mov_b32 m0, %2\n\ts_setprio %3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(asrc),
-                         "s"(copy_dst + buf * BUF), "n"(PRIO)
-                         : "memory", "m0");
-        asrc += a_left > 0 ? A_STEP : 0;
-        if constexpr (MASKED) a_lanes = a_left > 0 ? ~0ull : 1ull;
-        --a_left;
+    auto copy_a = [&](int buf, auto c_tag, auto prio_tag) { // one of the step's copies
+        constexpr int C = decltype(c_tag)::value, PRIO = decltype(prio_tag)::value;
+        if constexpr (MASKED) copy_lds<C * 1024, PRIO>(lane_off, asrc, copy_dst + buf * BUF, a_lanes);
+        else copy_lds<C * 1024, PRIO>(lane_off, asrc, copy_dst + buf * BUF);
+        if constexpr (C == S::NC - 1) {
+            asrc += a_left > 0 ? KT * 1024 : 0;
+            if constexpr (MASKED) a_lanes = a_left > 0 ? ~0ull : 1ull;
+            --a_left;
+        }
     };
-    auto load_w = [&](wraw_t* regs) {
-        static_for<NWREG>([&](auto e_tag) {
-            constexpr int E = decltype(e_tag)::value, U = E / TN, J = E % TN;
-            const unsigned off = lane_off; // (locals: asm operands cannot name captures of an enclosing lambda)
-            const uint8_t* base = wsrc[J];
-            wraw_t r;
-            if constexpr (PAIRED) // U counts this wave's super-tiles: every second one of the sub-step
-                asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(r) : "v"(off), "s"(base), "n"(U * 2048));
-            else if constexpr (WPAIR)
-                asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(r) : "v"(off), "s"(base));
-            else if constexpr (W4)
-                asm volatile("global_load_dwordx2 %0, %1, %2 offset:%3" : "=v"(r) : "v"(off), "s"(base), "n"(U * 1024));
-            else
-                asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(r) : "v"(off), "s"(base), "n"(U * 2048 - W_BIAS));
-            regs[E] = r;
-        });
+    auto load_w = [&](v4i* regs, auto half_tag, auto e_tag) { // operand e of unit HALF of a step (int4: of both)
+        constexpr int HALF = W4 || U == 1 ? 0 : decltype(half_tag)::value, E = decltype(e_tag)::value;
+        load_regs<HALF * 2048 + (E & 1) * 256>(regs[E], piece_off, wsrc[E / 2]);
+        if constexpr (E == CN - 1 && (W4 || HALF == U - 1)) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) wsrc[j] += w_left > 0 ? W_STEP : 0;
-        --w_left;
+            for (int j = 0; j < TN; ++j) wsrc[j] += w_left > 0 ? KT * (W4 ? 512 : 1024) : 0;
+            --w_left;
+        }
     };
-    // wait until at most IN_FLIGHT of this wave's loads are outstanding; regs become valid
-    auto w_wait = [&](wraw_t* regs) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IN_FLIGHT) : "memory");
+    auto w_wait = [&](v4i* regs, auto n_tag) { // regs become valid
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n_tag)::value) : "memory");
 #pragma unroll
-        for (int e = 0; e < NWREG; ++e) asm volatile("" : "+v"(regs[e]));
+        for (int e = 0; e < CN; ++e) keep(regs[e]);
     };
-    // fragment f = u * TM + i of buffer buf; completion is awaited by frags_wait()
-    auto read_frag = [&](v4i& dst, auto buf_tag, auto f_tag) {
-        constexpr int BUFI = decltype(buf_tag)::value, FI = decltype(f_tag)::value;
-        constexpr int U = FI / TM, I = FI % TM;
-        constexpr int KT = PAIRED ? (U / 2) * 4 + U % 2 : 2 * U; // this wave's u-th k-tile, relative to its first
-        constexpr int OFF = (BUFI % 8) * BUF + (I * KTS + KT) * 1024;
-        static_assert(OFF < 65536, "ds_read offset field");
-        const uint32_t addr = BUFI < 8 ? frag_lo : frag_hi;
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
+    auto read_a = [&](auto unit_tag, auto i_tag) { // operand i of a unit of the trip; awaited by wait_lds
+        constexpr int UNIT = decltype(unit_tag)::value, I = decltype(i_tag)::value, B = UNIT / U % NBUF, PER = 65536 / BUF;
+        read_lds<B % PER * BUF + (I / 2) * KT * 1024 + (UNIT % U) * (W4 ? 1024 : 2048) + (I & 1) * 256>(a[I], B < PER ? frag_lo : frag_hi);
     };
-    auto frags_wait = [&](v4i* f) {
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3])::"memory");
-    };
-    // ring register e of a sub-step -> its operand(s) in dst[NWOP]
-    auto unpack_item = [&](v4i* dst, const wraw_t* ring_regs, auto e_tag, auto half_tag) {
-        constexpr int E = decltype(e_tag)::value;
-        if constexpr (WPAIR) { // the half of the super-tile that the sub-step is
-            const wraw_t raw = ring_regs[E];
-            const int x = decltype(half_tag)::value ? raw.z : raw.x, y = decltype(half_tag)::value ? raw.w : raw.y;
+    auto unpack = [&](v4i* dst, const v4i* raw, auto half_tag, auto e_tag) { // k-tile HALF of each super-tile
+        if constexpr (W4) {
+            constexpr int HALF = decltype(half_tag)::value, E = decltype(e_tag)::value;
+            const int x = HALF ? raw[E].z : raw[E].x, y = HALF ? raw[E].w : raw[E].y;
             dst[E] = v4i{(x << 4) & (int)0xF0F0F0F0, x & (int)0xF0F0F0F0, (y << 4) & (int)0xF0F0F0F0, y & (int)0xF0F0F0F0};
-        } else if constexpr (PAIRED) {
-            constexpr int V = E / TN, J = E % TN; // super-tile V of this wave = its k-tiles 2V, 2V + 1
-            const wraw_t raw = ring_regs[E];
-            dst[(2 * V) * TN + J] = v4i{(raw.x << 4) & (int)0xF0F0F0F0, raw.x & (int)0xF0F0F0F0,
-                                        (raw.y << 4) & (int)0xF0F0F0F0, raw.y & (int)0xF0F0F0F0};
-            dst[(2 * V + 1) * TN + J] = v4i{(raw.z << 4) & (int)0xF0F0F0F0, raw.z & (int)0xF0F0F0F0,
-                                            (raw.w << 4) & (int)0xF0F0F0F0, raw.w & (int)0xF0F0F0F0};
-        } else if constexpr (W4) {
-            const wraw_t raw = ring_regs[E];
-            dst[E] = v4i{(raw.x << 4) & (int)0xF0F0F0F0, raw.x & (int)0xF0F0F0F0, (raw.y << 4) & (int)0xF0F0F0F0,
-                         raw.y & (int)0xF0F0F0F0};
         }
     };
 
-    // Sub-step s; SLOT = s % UNR.
-    auto k_step = [&](auto slot_tag) {
-        constexpr int SLOT = decltype(slot_tag)::value;
-        constexpr int F = SLOT & 1;
-        using NextBuf = std::integral_constant<int, (SLOT + 1) % NBUF>;
-        constexpr int UPS = (NWREG + 3) / 4; // unpack items per MFMA slot (slots 2..5)
-        // The two waves of a SIMD drift apart between barriers (the older one wins
-        // every issue conflict) and the one left behind cannot keep the matrix pipe
-        // busy alone; the wave that is further into the barrier interval yields.
-        copy_a((SLOT + D) % NBUF, std::integral_constant<int, G - 1 - SLOT % G>{});
-        if constexpr (!WPAIR) load_w(wring[(SLOT + NSW - 1) % NSW]);
-        else if constexpr (SLOT % 2 == 0) load_w(wring[(SLOT / 2 + NSW - 1) % NSW]);
-        constexpr int NEXT_W = WPAIR ? (SLOT + 1) / 2 % NSW : (SLOT + 1) % NSW; // ring slot of the next sub-step's weights
-        using NextHalf = std::integral_constant<int, (SLOT + 1) % 2>;
-        __builtin_amdgcn_sched_barrier(0);
-        static_assert(NMF >= 4 && NWREG <= ((NWREG + 3) / 4) * (NMF - 2), "the slots below: four fragment reads, the wait, the unpack items");
-        static_for<NMF>([&](auto q_tag) {
-            constexpr int Q = decltype(q_tag)::value;
-            constexpr int U = Q / (TN * TM), J = Q % (TN * TM) / TM, I = Q % TM;
-            if constexpr (W4)
-                acc[I][J] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wop[F][U * TN + J], afr[F][U * TM + I], acc[I][J], 0, 0, 0);
-            else
-                acc[I][J] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wring[SLOT % NSW][U * TN + J], afr[F][U * TM + I],
-                                                                  acc[I][J], 0, 0, 0);
-            // in the MFMA's shadow: one fragment read of the next sub-step, part of its unpack
-            if constexpr (Q < 4) read_frag(afr[F ^ 1][Q], NextBuf{}, std::integral_constant<int, Q>{});
-            if constexpr (Q == 1 && !(WPAIR && SLOT % 2 == 0)) w_wait(wring[NEXT_W]); // (an odd half came with its even one)
-            if constexpr (W4 && Q >= 2 && Q < 6) {
-                static_for<UPS>([&](auto t_tag) {
-                    constexpr int E = (Q - 2) * UPS + decltype(t_tag)::value;
-                    if constexpr (E < NWREG)
-                        unpack_item(wop[F ^ 1], wring[NEXT_W], std::integral_constant<int, E>{}, NextHalf{});
-                });
-            }
+    // Unit t of the trip.
+    auto k_unit = [&](auto unit_tag) {
+        constexpr int T = decltype(unit_tag)::value, STEP = T / U, UN = T % U, MF = RM * CN;
+        constexpr int ITEMS = S::items(UN), LAST = W4 ? MF / 2 : MF, SPACE = LAST / (ITEMS + 1) > 0 ? LAST / (ITEMS + 1) : 1; // loads: behind every SPACE-th MFMA
+        static_assert(ITEMS * SPACE <= (W4 && UN == 0 ? MF : LAST), "every load of a unit goes out before its wait");
+        constexpr int NEXT_W = W4 ? (STEP + 1) % NSW : (T + 1) % NSW;                 // slot of the next unit's (step's) weights
+        constexpr int LOAD_SLOT = W4 ? (STEP + NSW - 1) % NSW : (T + NSW - 1) % NSW;
+        using Half = std::integral_constant<int, (T + NSW - 1) & 1>;                  // place in its step of the unit whose weights are loaded
+        // The two waves of a SIMD drift apart between barriers (the older one wins every issue conflict) and the one left
+        // behind cannot keep the matrix pipe busy alone: the wave that is further into the barrier interval yields.
+        // (4096 x 4096 x 14336 int8 185.4 -> 182.7 us, 200 x 4096 x 14336 int4 18.1 -> 17.5)
+        using Priority = std::integral_constant<int, 3 - 4 * (T % (U * S::G)) / (U * S::G)>;
+        static_for<RM>([&](auto i_tag) {
+            constexpr int I = decltype(i_tag)::value;
+            wait_lds<RM - 1>(a[I]);
+            static_for<CN>([&](auto j_tag) {
+                constexpr int J0 = decltype(j_tag)::value, J = I & 1 ? CN - 1 - J0 : J0, AT = I * CN + J0; // (there and back: one operand stays)
+                if constexpr (W4) acc[I][J] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wop[UN][J], a[I], acc[I][J], 0, 0, 0);
+                else acc[I][J] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wring[T % NSW][J], a[I], acc[I][J], 0, 0, 0);
+                if constexpr (AT % SPACE == SPACE - 1 && AT / SPACE < ITEMS) {
+                    constexpr int Q = AT / SPACE, NCU = S::copies(UN);
+                    if constexpr (Q < NCU) copy_a((STEP + S::D) % NBUF, std::integral_constant<int, Q + (UN ? S::copies(0) : 0)>{}, Priority{});
+                    else load_w(wring[LOAD_SLOT], Half{}, std::integral_constant<int, Q - NCU>{});
+                }
+                if constexpr (W4) { // the next unit's operands, in the second half of this one
+                    if constexpr (UN == 1 && AT == MF / 2 - 1) w_wait(wring[NEXT_W], std::integral_constant<int, S::in_flight(1)>{});
+                    constexpr int EVERY = MF / 2 / CN, K = AT - MF / 2;
+                    if constexpr (K >= 0 && K % EVERY == 0)
+                        unpack(wop[UN ^ 1], wring[UN ? NEXT_W : STEP % NSW], std::integral_constant<int, UN ^ 1>{}, std::integral_constant<int, K / EVERY>{});
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            read_a(std::integral_constant<int, (T + 1) % (U * S::UNR)>{}, i_tag);
             __builtin_amdgcn_sched_barrier(0);
         });
-        frags_wait(afr[F ^ 1]);
-        if constexpr ((SLOT + 1) % G == 0) asm volatile("s_barrier" ::: "memory");
+        if constexpr (!W4) w_wait(wring[NEXT_W], std::integral_constant<int, S::in_flight(UN)>{});
+        if constexpr (UN == U - 1 && (STEP + 1) % S::G == 0) asm volatile("s_barrier" ::: "memory");
+    };
+    auto k_step = [&](auto step_tag) {
+        static_for<U>([&](auto u_tag) { k_unit(std::integral_constant<int, U * decltype(step_tag)::value + decltype(u_tag)::value>{}); });
     };
 
-    // prologue: the same issue order as if the loop had run for sub-steps -D..-1
-#pragma unroll
-    for (int t = -D; t < 0; ++t) {
-        copy_a(t + D, std::integral_constant<int, 0>{});
-        if (WPAIR ? t % 2 == 0 && t / 2 + NSW - 1 >= 0 : t + NSW - 1 >= 0) load_w(wring[(WPAIR ? t / 2 : t) + NSW - 1]);
-    }
+    // prologue: the same issue order as if the loop had run for steps -D..-1
+    static_for<U * S::D>([&](auto t_tag) {
+        constexpr int T = decltype(t_tag)::value - U * S::D, UN = (T + U * S::D) % U, OF = S::loaded(T);
+        static_for<S::copies(UN)>([&](auto c_tag) {
+            copy_a((T + U * S::D) / U, std::integral_constant<int, decltype(c_tag)::value + (UN ? S::copies(0) : 0)>{}, std::integral_constant<int, 0>{});
+        });
+        if constexpr (S::loads_w(T) && OF >= 0)
+            static_for<CN>([&](auto e_tag) { load_w(wring[OF % NSW], std::integral_constant<int, OF & 1>{}, e_tag); });
+    });
     RK_TS(1);
-    // The tile's scales are fetched now, behind the prologue's loads, and handed
-    // to the epilogue through LDS after the loop, so the epilogue does not start
-    // with a round trip to memory: thread t holds the row scale of row t
-    // (t < BM) and the column scale of physical column t (t < 256).  (Two more
-    // loads in the queue only make the first sub-steps' waits stricter.  Ahead of
-    // the prologue's loads they cost the 128-row tile 0.2 us: the first copies
-    // leave later.)  They are in flight until the wait of the loop's third
-    // sub-step, or the closing wait; like every register an asm load writes they
-    // must not be touched before -- which the build verifies in the compiled code
-    // (audit_waits.py) rather than trusting the allocator.
-    float my_as = 0.0f, my_ws = 0.0f;
-    bool as_valid = false, ws_valid = false;
+    // The tile's scales follow, straight to LDS, so that the epilogue does not start with a round trip to memory: thread t
+    // brings the scale of row t % BM and of physical column t % (128 TN).  (Two more loads in the queue only make the
+    // first units' waits stricter.  Ahead of the prologue's loads they cost the 128-row tile 0.2 us: the first copies
+    // leave later.  Rows and columns beyond the matrix take some valid scale: nothing is stored for them.)
     if constexpr (EPI != RKH_EPI_I32) {
-        const int t = threadIdx.x;
-        const int m = mblk * BM + (t & (BM - 1));
-        const int pb = nblk * (4 * TN) + ((t & (128 * TN - 1)) >> 5);
-        int n;
-        if constexpr (EPI == RKH_EPI_SWIGLU) {
-            // pb even = gate, odd = up block of middle columns (pb / 2) * 32
-            const int F = g.interleave_F;
-            const int nl = (pb >> 1) * 32 + (t & 31);
-            n = (pb & 1 ? F : 0) + nl;
-            ws_valid = nl < F;
-        } else {
-            const bool live = g.interleave_F ? pb < g.N / 32 : pb * 32 < g.N;
-            n = block_first_col(pb, g.interleave_F) + (t & 31);
-            ws_valid = live && n < g.N;
-        }
-        as_valid = m < m_limit;
-        const float* pa = g.a_scale + (as_valid ? m : 0);
-        const float* pw = w_scale + (ws_valid ? n : 0);
-        asm volatile("global_load_dword %0, %1, off" : "=v"(my_as) : "v"(pa));
-        asm volatile("global_load_dword %0, %1, off" : "=v"(my_ws) : "v"(pw));
+        const int row = threadIdx.x & (S::BM - 1), col = threadIdx.x & (128 * TN - 1);
+        const int pb = nblk * (4 * TN) + (col >> 5);
+        const int n = EPI == RKH_EPI_SWIGLU && (pb >> 1) * 32 >= g.interleave_F ? 0 : block_first_col(pb, g.interleave_F) + (col & 31);
+        copy_lds_dword(g.a_scale + min(mblk * S::BM + row, g.M - 1), lds_base + WK_SCALES_OFF + (wave * 64 & (S::BM - 1)) * 4);
+        copy_lds_dword(g.w_scale + min(n, g.N - 1), lds_base + WK_SCALES_OFF + (WK_ROW_SCALES + (wave * 64 & (128 * TN - 1))) * 4);
     }
-    w_wait(wring[0]); // weights of sub-step 0 and the copies of sub-steps 0..D-NSW+1 (WPAIR: 0..D-2*NSW+2) have landed
+    w_wait(wring[0], std::integral_constant<int, S::first_wait()>{}); // weights of unit 0 and the copies of steps 0..G have landed
     asm volatile("s_barrier" ::: "memory");
-    static_for<4>([&](auto f_tag) { read_frag(afr[0][decltype(f_tag)::value], std::integral_constant<int, 0>{}, f_tag); });
-    static_for<NWREG>([&](auto e_tag) { unpack_item(wop[0], wring[0], e_tag, std::integral_constant<int, 0>{}); });
-    frags_wait(afr[0]);
+    static_for<RM>([&](auto i_tag) { read_a(std::integral_constant<int, 0>{}, i_tag); });
+    static_for<CN>([&](auto e_tag) { unpack(wop[0], wring[0], std::integral_constant<int, 0>{}, e_tag); });
     RK_TS(2);
 
     int s = 0;
-    for (; s + UNR <= ksteps; s += UNR) static_for<UNR>([&](auto slot) { k_step(slot); });
-    // (the remaining sub-steps as a chain that ends at the first one beyond K: the control flow
-    // then only holds the sequences of sub-steps that can happen, which is what the static check
+    for (; s + S::UNR <= ksteps; s += S::UNR) static_for<S::UNR>([&](auto step) { k_step(step); });
+    // (the remaining steps as a chain that ends at the first one beyond K: the control flow
+    // then only holds the sequences of steps that can happen, which is what the static check
     // of the waits, audit_waits.py, walks)
-    static_while<UNR>([&](auto slot) {
-        if (s + decltype(slot)::value >= ksteps) return false;
-        k_step(slot);
+    static_while<S::UNR - 1>([&](auto step) {
+        if (s + decltype(step)::value >= ksteps) return false;
+        k_step(step);
         return true;
     });
     __builtin_amdgcn_s_setprio(0);
     RK_TS(3);
 
-    // ---- epilogue.  Drain the look-ahead copies (they write LDS) and the scale
-    // loads; then every wave is past its last fragment read and LDS is reused.
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(my_as), "+v"(my_ws)::"memory");
-    // The weight loads issued for sub-steps beyond K were in flight until this
-    // wait, while the compiler regards their destination registers as dead: the
-    // uses below keep it from giving one of them to an epilogue value ahead of
-    // the wait (the load would then land on top of that value).
+    // ---- epilogue.  Drain the look-ahead copies (they write LDS), the operands read ahead and the scale
+    // loads; then every wave is past its last operand and LDS is reused.
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    // What was loaded for units beyond K was in flight until this wait, while the compiler regards
+    // the destination registers as dead: the uses below keep it from giving one of them to an epilogue value
+    // ahead of the wait (the load would then land on top of that value).
+#pragma unroll
+    for (int i = 0; i < RM; ++i) keep(a[i]);
 #pragma unroll
     for (int t = 0; t < NSW; ++t)
 #pragma unroll
-        for (int e = 0; e < NWREG; ++e) asm volatile("" : "+v"(wring[t][e]));
-    if constexpr (EPI != RKH_EPI_I32) {
-        float* sc = reinterpret_cast<float*>(lds_raw + WK_SCALES_OFF);
-        const int t = threadIdx.x;
-        if (t < BM) sc[t] = as_valid ? my_as : 0.0f;
-        if (t < 128 * TN) sc[WK_ROW_SCALES + t] = ws_valid ? my_ws : 0.0f;
-    }
+        for (int e = 0; e < CN; ++e) keep(wring[t][e]);
     lds_barrier();
 
-    // The k-half index is a template tag so that accumulator registers are
-    // indexed with constants.  After the exchange a wave owns KEEP row blocks
-    // of its strip: TM = 4: blocks 2*wk, 2*wk+1; TM = 2: block wk; TM = 1: the
-    // wk = 0 wave owns the block and its partner only hands over.
-    auto finish = [&](auto wk_tag) {
-        constexpr int WK = decltype(wk_tag)::value;
-        constexpr int KEEP = RS ? TM : TM == 1 ? (WK == 0 ? 1 : 0) : TM / 2;  // row blocks kept
-        constexpr int GIVE = RS ? 0 : TM == 1 ? (WK == 1 ? 1 : 0) : TM / 2;   // row blocks handed over
-        constexpr int KEEP0 = RS || TM == 1 ? 0 : WK * (TM / 2);              // first kept row block
-        constexpr int ROW0 = RS ? WK * TM : KEEP0;                            // its place in the tile
-        constexpr int GIVE0 = TM == 1 ? 0 : (WK ^ 1) * (TM / 2);    // first handed-over row block
-        constexpr int XT = (TM == 1 ? 1 : TM / 2) * TN;             // tiles per exchange slot of a wave
-        if constexpr (!RS) {
-        int* xch = reinterpret_cast<int*>(lds_raw);
-        const int partner = wave ^ 4;
-        static_assert(8 * XT * 16 * 64 * 4 <= WK_SCALES_OFF, "exchange area");
+    // The k-halves meet: a wave hands half of the rows of its strip to its partner and keeps operands wk * RM / 2 .. (RS:
+    // every wave holds finished sums).  Accumulators are indexed with constants, hence the two branches.
+    constexpr int KEEP = RS ? RM : RM / 2;
+    const int row0 = wk * KEEP * 16; // of the kept rows in the tile
+    v4i sum[KEEP][CN];
+    if constexpr (RS) {
 #pragma unroll
-        for (int t = 0; t < GIVE * TN; ++t) {
-            const v16i& give = acc[GIVE0 + t / TN][t % TN];
+        for (int t = 0; t < RM * CN; ++t) sum[t / CN][t % CN] = acc[t / CN][t % CN];
+    } else {
+        constexpr int XT = KEEP * CN; // tiles per exchange slot
+        v4i* xch = reinterpret_cast<v4i*>(lds_raw);
+        const auto hand_over = [&](auto wk_tag) {
+            constexpr int GIVE0 = (decltype(wk_tag)::value ^ 1) * KEEP, KEEP0 = decltype(wk_tag)::value * KEEP;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<v4i*>(xch + (((wave * XT + t) * 4 + q) * 64 + lane) * 4) =
-                    v4i{give[q * 4], give[q * 4 + 1], give[q * 4 + 2], give[q * 4 + 3]};
-        }
+            for (int t = 0; t < XT; ++t) xch[(wave * XT + t) * 64 + lane] = acc[GIVE0 + t / CN][t % CN];
+#pragma unroll
+            for (int t = 0; t < XT; ++t) sum[t / CN][t % CN] = acc[KEEP0 + t / CN][t % CN];
+        };
+        if (wk == 0) hand_over(std::integral_constant<int, 0>{});
+        else hand_over(std::integral_constant<int, 1>{});
         lds_barrier();
 #pragma unroll
-        for (int t = 0; t < KEEP * TN; ++t) {
-            v16i& keep = acc[KEEP0 + t / TN][t % TN];
+        for (int t = 0; t < XT; ++t) sum[t / CN][t % CN] += xch[((wave ^ 4) * XT + t) * 64 + lane];
+        if (ksplit > 1) { // partial tile in accumulator order: [tile][part][wave][kept tile][lane] x 4 ints
+            v4i* dst = reinterpret_cast<v4i*>(g.splitk_acc) + (((size_t)tile * ksplit + kpart) * 8 + wave) * (XT * 64);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const v4i got = *reinterpret_cast<const v4i*>(xch + (((partner * XT + t) * 4 + q) * 64 + lane) * 4);
-                keep[q * 4] += got.x;
-                keep[q * 4 + 1] += got.y;
-                keep[q * 4 + 2] += got.z;
-                keep[q * 4 + 3] += got.w;
-            }
-        }
-        lds_barrier();
-        } // (RS: every wave holds finished sums)
-        RK_TS(4);
-
-        if (!RS && ksplit > 1) {
-            // partial tile in accumulator order: [tile][part][owning wave][kept tile][q][lane] x 4 ints
-            constexpr int OWNERS = TM == 1 ? 4 : 8;
-            constexpr int PER_WAVE = (TM == 1 ? 1 : TM / 2) * TN * 1024;
-            const int owner = TM == 1 ? wn : wave;
-            int* dst0 = g.splitk_acc + ((size_t)tile * ksplit + kpart) * (OWNERS * PER_WAVE) + owner * PER_WAVE;
-#pragma unroll
-            for (int t = 0; t < KEEP * TN; ++t) {
-                const v16i& mine = acc[KEEP0 + t / TN][t % TN];
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    *reinterpret_cast<v4i*>(dst0 + t * 1024 + (q * 64 + lane) * 4) =
-                        v4i{mine[q * 4], mine[q * 4 + 1], mine[q * 4 + 2], mine[q * 4 + 3]};
-            }
+            for (int t = 0; t < XT; ++t) dst[t * 64 + lane] = sum[t / CN][t % CN];
             return;
         }
-
-        if constexpr (KEEP > 0) {
-            float as[KEEP], ws[TN][16];
-            if constexpr (EPI != RKH_EPI_I32) {
-                const float* sc = reinterpret_cast<const float*>(lds_raw + WK_SCALES_OFF);
+        lds_barrier();
+    }
+    RK_TS(4);
+    float as[KEEP];
+    v4f ws[CN];
+    if constexpr (EPI != RKH_EPI_I32) {
+        const float* sc = reinterpret_cast<const float*>(lds_raw + WK_SCALES_OFF);
 #pragma unroll
-                for (int ii = 0; ii < KEEP; ++ii) as[ii] = sc[(ROW0 + ii) * 32 + (lane & 31)];
+        for (int i = 0; i < KEEP; ++i) as[i] = sc[row0 + i * 16 + (lane & 15)];
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) ws[j][r] = sc[WK_ROW_SCALES + (wn * TN + j) * 32 + tile_col(r, lane)];
-            } else {
-#pragma unroll
-                for (int ii = 0; ii < KEEP; ++ii) as[ii] = 0.0f;
-            }
-            uint8_t* stage_lds = lds_raw + wave * (32 * (32 * 4 + 8));
-#pragma unroll
-            for (int ii = 0; ii < KEEP; ++ii) {
-                constexpr int i0 = KEEP0;
-                const int m0 = mblk * BM + (ROW0 + ii) * 32;
-                if constexpr (W4) {
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[i0 + ii][j][r] >>= 4;
-                }
-                const int pb0 = nblk * (4 * TN) + wn * TN;
-                if constexpr (EPI == RKH_EPI_SWIGLU) {
-                    epilogue_swiglu_scaled(g, acc[i0 + ii][0], acc[i0 + ii][TN - 1], m0, pb0, lane, as[ii], ws[0], ws[TN - 1],
-                                           m_limit, stage_lds);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        epilogue_tile_scaled<EPI>(g, acc[i0 + ii][j], m0, pb0 + j, lane, as[ii], ws[j], m_limit,
-                                                  stage_lds);
-                }
-            }
-        }
-    };
-    if (wk == 0) finish(std::integral_constant<int, 0>{});
-    else finish(std::integral_constant<int, 1>{});
+        for (int j = 0; j < CN; ++j) ws[j] = *reinterpret_cast<const v4f*>(sc + WK_ROW_SCALES + (wn * CN + j) * 16 + 4 * q);
+    }
+    wk_store<KEEP, CN, W4, EPI>(g, [&](int i, int j) -> const v4i& { return sum[i][j]; }, [&](int i) { return as[i]; },
+                                [&](int j, int e) { return ws[j][e]; }, mblk * S::BM + row0, nblk * (4 * TN) + wn * TN, g.M,
+                                lds_raw + wave * WK_STAGE, lane);
     RK_TS(5);
 }
 
 // The tile of a workgroup: XCD-contiguous ranges, 4 row blocks per column sweep.
 template <int TM, bool W4, int EPI, int TN = 2>
 __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const uint8_t* h_W, int h_M, int h_K,
-                                                      int mblocks, int nblocks, int ksplit, int ksteps_per_part,
+                                                      int mblocks, int nblocks, int ksplit, int units_per_part,
                                                       rkh_gemm_args g) {
     // (leading scalar arguments, see RK_GEMM_HEAD_PARAMS: everything the tile coordinates and the
     // prologue's loads depend on, ten dwords, arrives in registers)
     g.A = h_A; g.W = h_W; g.M = h_M; g.K = h_K;
     RK_TS(0);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[]; // WK_LDS_BYTES
-    const int ksteps_total = (int)rkh_align_up(g.K, RKH_K_ALIGN) / 32 / (8 / TM);
+    const int units = (int)rkh_align_up(g.K, RKH_K_ALIGN) / WK_PART_K;
     const int tiles = mblocks * nblocks;
     const int logical = xcd_remap(blockIdx.x, tiles * ksplit);
     const int kpart = ksplit > 1 ? (int)((unsigned)logical / (unsigned)tiles) : 0;
     const int tile = logical - kpart * tiles;
     int mblk, nblk;
     wk_tile_coords(tile, mblocks, nblocks, mblk, nblk);
-    const int kstep0 = kpart * ksteps_per_part;
-    const int ksteps = min(ksteps_per_part, ksteps_total - kstep0); // >= 1 by construction of the launch
-    wk_tile<TM, W4, EPI, TN, false>(g, lds_raw, tile, mblk, nblk, kpart, ksplit, kstep0, ksteps);
+    const int first = kpart * units_per_part; // (at least one unit by construction of the launch)
+    wk_tile<TM, W4, EPI, TN, false>(g, lds_raw, tile, mblk, nblk, kpart, ksplit, first * (WK_PART_K / 32),
+                                    min(units_per_part, units - first) * (WK_PART_K / 32));
 }
 
 // Tiles of 256 x 256 (RS) -- `big` of them, the first in tile order -- and tiles of 128 x 256 for what is
 // left of the output: the tiles that would start a last, mostly empty round, each in two halves, and a
 // last strip of at most 128 rows.  Workgroup = 8 waves in 4 column groups x 2 row halves: a wave multiplies
 // 128 x 64 over the whole K, so there is no exchange of k-halves and all eight waves convert and store.
-// What bounds it: the matrix pipes at the clock that the power limit leaves -- 4096 x 4096 x 14336 int8 is 229 376 MFMA
-// cycles per SIMD in 199 us cold and 228 on average of 40 launches in a row, 2.4 - 2.1 POP/s where a loop of nothing but
-// MFMAs reaches 3.5 -- and about 9 of a tile's 58 us outside its loop (time stamps, RK_DEBUG_TS).  Against 128 x 256 tiles:
-// the second operand of a column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
-// cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, the calls among others: int8
-// 4096 x 4096 x 14336 241 -> 203, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
+// What bounds it: the matrix pipes at the clock that the power limit leaves, and 6 - 9 us of a tile outside its loop.
+// Against 128 x 256 tiles: the second operand of a column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
+// cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, when the tiles were
+// introduced: int8 4096 x 4096 x 14336 241 -> 203, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
 // (Measured and not kept: half of the compute units starting with a small tile so that the epilogues'
 // bursts of stores fall apart -- 204 -> 217, 195 -> 210: tiles in step share their operands in L2.)
 template <bool W4, int EPI>
@@ -527,65 +569,50 @@ __global__ __launch_bounds__(512) void gemm_wk_big_kernel(const uint8_t* h_A, co
             mblk = mblocks * 2;
             nblk = t - halves;
         }
-        wk_tile<4, W4, EPI, 2, false>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB / 2);
+        wk_tile<4, W4, EPI, 2, false>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB);
     }
 }
-#pragma clang diagnostic pop
-
-// Second half of a K-split launch.  Workgroup = one wave = one owner of kept
-// tiles of an output tile (the wave -> tile ownership gemm_wk_kernel has after
-// its k-half exchange): blockIdx.x = tile * OWNERS + owner.  Adds the ksplit
-// partial tiles and runs the epilogue.
+// Second half of a K-split launch.  Workgroup = one wave = what one wave of gemm_wk_kernel kept of an output tile:
+// blockIdx.x = tile * 8 + wave.  Adds the ksplit partial tiles and runs the epilogue.
 template <int TM, bool W4, int EPI>
 __global__ __launch_bounds__(64) void gemm_wk_reduce_kernel(rkh_gemm_args g, int mblocks, int nblocks, int ksplit) {
-    constexpr int TN = 2, BM = 32 * TM;
-    constexpr int OWNERS = TM == 1 ? 4 : 8;
-    constexpr int KEEP = TM == 1 ? 1 : TM / 2;             // row blocks per owner
-    constexpr int PER_WAVE = KEEP * TN * 1024;
-    __shared__ __attribute__((aligned(16))) uint8_t stage_lds[32 * (32 * 4 + 8)];
+    constexpr int TN = 2, CN = 4, BM = 32 * TM, KEEP = TM; // (rows of operands a wave keeps)
+    __shared__ __attribute__((aligned(16))) uint8_t stage_lds[WK_STAGE];
     const int lane = lane_id();
-    const int tile = blockIdx.x / OWNERS, owner = blockIdx.x % OWNERS;
-    const int wn = owner & 3, wk = owner >> 2;             // TM == 1: owners are the wk == 0 waves
+    const int tile = blockIdx.x / 8, wave = blockIdx.x % 8, wn = wave & 3, wk = wave >> 2;
     int mblk, nblk;
     wk_tile_coords(tile, mblocks, nblocks, mblk, nblk);
-    const int keep0 = TM == 1 ? 0 : wk * (TM / 2);
-    const int* src0 = g.splitk_acc + (size_t)tile * ksplit * (OWNERS * PER_WAVE) + owner * PER_WAVE;
-    const int pb0 = nblk * 8 + wn * TN;
+    const int m0 = mblk * BM + wk * KEEP * 16, pb0 = nblk * 8 + wn * TN;
+    const v4i* src = reinterpret_cast<const v4i*>(g.splitk_acc) + ((size_t)tile * ksplit * 8 + wave) * (KEEP * CN * 64) + lane;
+    v4i sum[KEEP][CN];
 #pragma unroll
-    for (int ii = 0; ii < KEEP; ++ii) {
-        v16i sum[TN];
+    for (int t = 0; t < KEEP * CN; ++t) sum[t / CN][t % CN] = v4i{0, 0, 0, 0};
+    for (int p = 0; p < ksplit; ++p, src += 8 * KEEP * CN * 64) {
+        // int4 weights ride as 16 * code: a part's sum is an exact multiple of 16 that fits
+        // int32 (a part spans at most 2^17 k), but the sum of the parts times 16 need not --
+        // so the factor comes off each part before it is added
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sum[j][r] = 0;
-        for (int p = 0; p < ksplit; ++p) {
-            const int* src = src0 + (size_t)p * (OWNERS * PER_WAVE) + ii * TN * 1024;
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    // int4 weights ride as 16 * code: a part's sum is an exact multiple of 16 that fits
-                    // int32 (a part spans at most 2^17 k), but the sum of the parts times 16 need not --
-                    // so the factor comes off each part before it is added
-                    constexpr int SH = W4 ? 4 : 0;
-                    const v4i got = *reinterpret_cast<const v4i*>(src + j * 1024 + (q * 64 + lane) * 4);
-                    sum[j][q * 4] += got.x >> SH;
-                    sum[j][q * 4 + 1] += got.y >> SH;
-                    sum[j][q * 4 + 2] += got.z >> SH;
-                    sum[j][q * 4 + 3] += got.w >> SH;
-                }
-        }
-        const int m0 = mblk * BM + (keep0 + ii) * 32;
-        if constexpr (EPI == RKH_EPI_SWIGLU) {
-            epilogue_swiglu(g, sum[0], sum[1], m0, pb0, lane, g.a_scale, g.w_scale, g.M, stage_lds);
-        } else {
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                epilogue_tile<EPI>(g, sum[j], m0, pb0 + j, lane, g.a_scale, g.w_scale, g.M, stage_lds);
-        }
+        for (int t = 0; t < KEEP * CN; ++t) sum[t / CN][t % CN] += src[t * 64] >> (W4 ? 4 : 0);
     }
+    float as[KEEP], ws[CN][4];
+    if constexpr (EPI != RKH_EPI_I32) {
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i) {
+            const int m = m0 + 16 * i + (lane & 15);
+            as[i] = m < g.M ? g.a_scale[m] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < CN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int pb = pb0 + j / 2, n = block_first_col(pb, g.interleave_F) + 16 * (j & 1) + 4 * (lane >> 4) + e;
+                const bool live = g.interleave_F ? pb < g.N / 32 : n < g.N;
+                ws[j][e] = live ? g.w_scale[n] : 0.0f;
+            }
+    }
+    wk_store<KEEP, CN, false, EPI>(g, [&](int i, int j) -> const v4i& { return sum[i][j]; }, [&](int i) { return as[i]; },
+                                   [&](int j, int e) { return ws[j][e]; }, m0, pb0, g.M, stage_lds, lane);
 }
-
 
 // Bytes of split-K scratch for `tiles` output tiles of bm rows split into
 // ksplit parts: the int32 partial tiles.
@@ -595,24 +622,23 @@ static size_t wk_scratch_bytes(long tiles, int bm, int ksplit) {
 
 // Workgroups of a launch with this tile height and K split (what launch_gemm_wk makes of `ksplit`).
 static int wk_grid(const rkh_gemm_args& g, int tile_rows, int& ksplit) {
-    const int kts = 8 / (tile_rows / 32);
     const int mblocks = (g.M + tile_rows - 1) / tile_rows, nblocks = (g.N + 255) / 256;
-    const int ksteps_total = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / 32 / kts);
-    if (ksplit > ksteps_total) ksplit = ksteps_total;
+    const int units = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / WK_PART_K);
+    if (ksplit > units) ksplit = units;
     if (ksplit < 1) ksplit = 1;
-    const int per = (ksteps_total + ksplit - 1) / ksplit;
-    ksplit = (ksteps_total + per - 1) / per; // no empty part
+    const int per = (units + ksplit - 1) / ksplit;
+    ksplit = (units + per - 1) / per; // no empty part
     return mblocks * nblocks * ksplit;
 }
 
 template <int TM>
 int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
-    constexpr int BM = 32 * TM, KTS = 8 / TM;
+    constexpr int BM = 32 * TM;
     const int mblocks = (g.M + BM - 1) / BM;
     const int nblocks = (g.N + 255) / 256;
-    const int ksteps_total = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / 32 / KTS);
+    const int units = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / WK_PART_K);
     const dim3 grid(wk_grid(g, BM, ksplit)), block(512);
-    const int per = (ksteps_total + ksplit - 1) / ksplit;
+    const int per = (units + ksplit - 1) / ksplit;
     mark(st, "gemm_wk_kernel");
 #define RK_WK(W4, EPI)                                                                              \
     do {                                                                                            \
@@ -633,7 +659,7 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
         if (ksplit > 1) mark(st, "gemm_wk_reduce_kernel");                                          \
         if (ksplit > 1)                                                                             \
             hipLaunchKernelGGL((gemm_wk_reduce_kernel<TM, W4, EPI>),                                \
-                               dim3(mblocks * nblocks * (TM == 1 ? 4 : 8)), dim3(64), 0, st, g,     \
+                               dim3(mblocks * nblocks * 8), dim3(64), 0, st, g,     \
                                mblocks, nblocks, ksplit);                                           \
     } while (0)
     // (a dense SwiGLU GEMM exists for int4 weights only: the w4a8 FFN; the MoE layer's is grouped)
@@ -717,9 +743,9 @@ int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, rkk::BigTiles pla
 // go through LDS once for the eight waves, so a tile pulls K x (rows + 128) bytes through its compute unit.
 template <int TM>
 int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g) {
-    constexpr int TN = 1, KTS = 8 / TM;
+    constexpr int TN = 1;
     const int mblocks = (g.M + 32 * TM - 1) / (32 * TM), nblocks = (g.N + 127) / 128;
-    const int ksteps_total = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / 32 / KTS);
+    const int units = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / WK_PART_K);
     const dim3 grid(mblocks * nblocks), block(512);
     mark(st, TM == 2 ? "gemm_wk_kernel<64 x 128>" : "gemm_wk_kernel<128 x 128>");
 #define RK_WKN(W4, EPI)                                                                             \
@@ -734,7 +760,7 @@ int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g) {
             opted_in[dev].store(true, std::memory_order_release);                                   \
         }                                                                                           \
         hipLaunchKernelGGL((gemm_wk_kernel<TM, W4, EPI, TN>), grid, block, WK_LDS_BYTES, st,       \
-                           g.A, g.W, g.M, g.K, mblocks, nblocks, 1, ksteps_total, g);               \
+                           g.A, g.W, g.M, g.K, mblocks, nblocks, 1, units, g);               \
     } while (0)
     // (int4 weights: the 64-row tiles only -- the 128-row ones measured slower than the other plans everywhere)
 #define RK_WKN_W(EPI)                                                                               \

@@ -1,0 +1,59 @@
+"""GPU parity of the LDS-ring GEMM's K loop against the CPU oracle: every tile shape of gemm_wk_kernel with K from less than
+one block of 256 to more than a trip of the unrolled loop, so that each remainder of the trip (0 .. 7 steps) and K that ends
+inside a step occurs; rows and columns end inside a tile.  (gemm_wk_big_kernel: tests/test_gpu_large_tiles.py.)  Integer
+sums and a fixed order of the floating-point steps: exact.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from rknpu2_matmul_open_amd import capi, ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+NARROW, TILES = 4, 5  # rkh_gemm_kernel
+KS = (130, 256, 500, 768, 1024, 1200, 1500, 1792, 2048, 2300)
+I32, F16, SWIGLU = 0, 1, 3
+
+
+def _route(M, N, K, w4, epi):
+    v = [C.c_int() for _ in range(5)]
+    assert capi.load_library().rkh_gemm_route(M, N, K, w4, epi, *[C.byref(x) for x in v]) == 0
+    return v[0].value, v[1].value
+
+
+@pytest.mark.parametrize("K", KS)
+@pytest.mark.parametrize("M,N,kernel,rows", [(129, 4100, NARROW, 64), (1000, 2500, NARROW, 128), (1800, 2900, TILES, 128)])
+def test_int8_weights(sess, oracle, M, N, K, kernel, rows):
+    assert _route(M, N, K, 0, I32) == (kernel, rows)
+    rng = np.random.default_rng(K)
+    A, B = rng.integers(-128, 128, (M, K)).astype(np.int8), rng.integers(-128, 128, (K, N)).astype(np.int8)
+    op = ops.W8A8Linear(sess, capi.I8I8I32, M, B)
+    try:
+        rc, got = op.run(A)
+        assert rc == 0 and np.array_equal(got, oracle.gemm_i8(A, B))
+    finally:
+        op.close()
+
+
+@pytest.mark.parametrize("K", KS)
+@pytest.mark.parametrize("M,N,epi,kernel,rows", [(129, 4100, F16, NARROW, 64), (700, 3000, F16, TILES, 64), (1800, 2304, F16, TILES, 128),
+                                                 (300, 6016, SWIGLU, TILES, 32), (900, 4032, SWIGLU, TILES, 64)])
+def test_int4_weights(sess, oracle, one_piece, M, N, K, epi, kernel, rows):
+    assert _route(M, N, K, 1, epi) == (kernel, rows)
+    c = workloads.w4a8_case(M, K, N, seed_w=K, seed_a=M)
+    w = ops.W4A8Weights(sess, c["B"], c["w_scale"])
+    ws = ops.W4A8Workspace(sess, M, N, K)
+    try:
+        if epi == F16:
+            (rc, got), _ = one_piece(lambda: ws.run_f16(w, c["A"]))
+            want = oracle.w4a8(c["A"], c["B"], c["w_scale"])["C"]
+        else:
+            A32 = oracle.half_to_float(c["A"]).astype(np.float32).reshape(M, K)
+            (rc, got), _ = one_piece(lambda: ws.run_swiglu_f32(w, A32))
+            want = oracle.w4a8_swiglu(A32, c["B"], c["w_scale"])["middle"]
+        assert rc == 0 and np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, got.dtype).view(np.uint8))
+    finally:
+        ws.close()
+        w.close()
