@@ -25,6 +25,10 @@ with the same flags):
     instruction in front of it may not be that write.  (The compiler inserts the wait state for
     loads of its own; into an asm statement it does not look.)
 
+  * a product (v_mfma) from asm takes no part in the compiler's bookkeeping of hazards: no vector instruction may write one
+    of its operands in the two wait states ahead of it, nor any other instruction read its result in the eleven behind it
+    (a product may: the hardware orders those).
+
 The check walks the control-flow graph of a kernel (basic blocks split at labels and branches):
 from every asm load it follows every path until the covering wait, carrying the number of loads
 issued since; a block is visited again only when reached with a smaller count (fewer loads
@@ -179,11 +183,80 @@ def _check_m0(name, instrs, violations):
                 work += [(first, hi) for first, hi, succ in blocks.values() if lo in succ]
 
 
+_MFMA = re.compile(r"^\s*v_mfma_")
+_NOP = re.compile(r"^\s*s_nop\s+(\d+)")
+_VALU = re.compile(r"^\s*v_(?!mfma_)")
+_READS_ALL = re.compile(r"^\s*(ds_write|global_store|buffer_store|scratch_store|global_load_lds|v_cmp)")
+
+
+def _operands(text):
+    """(registers written, registers read) of an instruction, as far as the rules below need it."""
+    parts = text.split(None, 1)
+    if len(parts) < 2:
+        return set(), set()
+    if _READS_ALL.match(text):
+        return set(), _regs(parts[1])
+    first, _, rest = parts[1].partition(",")
+    return _regs(first), _regs(rest)
+
+
+def _check_mfma(name, instrs, violations):
+    """Wait states around products from asm, along every path."""
+    blocks = _blocks(instrs)
+    block_of, cur = {}, 0
+    for i in range(len(instrs)):
+        cur = i if i in blocks else cur
+        block_of[i] = cur
+    preds = {}
+    for lo, _, succ in blocks.values():
+        for nxt in succ:
+            preds.setdefault(nxt, []).append(lo)
+    for i, (text, in_asm) in enumerate(instrs):
+        if not in_asm or not _MFMA.match(text):
+            continue
+        result, operands = _operands(text)
+        work, seen = [(i - 1, block_of[i], 0)], set()
+        while work:                                  # back: who writes the operands
+            j, lo, states = work.pop()
+            while j >= lo and states < 2:
+                t = instrs[j][0]
+                if not t.endswith(":"):
+                    if _VALU.match(t) and _operands(t)[0] & operands:
+                        violations.append("%s: `%s` writes an operand of `%s` %d wait states ahead of it" % (name, t.strip(), text.strip(), states))
+                    nop = _NOP.match(t)
+                    states += 1 + (int(nop.group(1)) if nop else 0)
+                j -= 1
+            if states < 2 and (lo, states) not in seen:
+                seen.add((lo, states))
+                work += [(blocks[p][1] - 1, p, states) for p in preds.get(lo, [])]
+        work, seen = [(i + 1, 0)], set()
+        while work:                                  # on: who reads the result
+            j, states = work.pop()
+            if j >= len(instrs):
+                continue
+            _, hi, succ = blocks[block_of[j]]
+            while j < hi and states < 11:
+                t = instrs[j][0]
+                if not t.endswith(":"):
+                    written, read = _operands(t)
+                    if not _MFMA.match(t) and (read | (written if _VALU.match(t) else set())) & result:
+                        violations.append("%s: `%s` touches the result of `%s` %d wait states behind it" % (name, t.strip(), text.strip(), states))
+                    nop = _NOP.match(t)
+                    states += 1 + (int(nop.group(1)) if nop else 0)
+                j += 1
+            if states < 11:
+                for nxt in succ:
+                    if (nxt, states) not in seen:
+                        seen.add((nxt, states))
+                        work.append((nxt, states))
+
+
 def audit_function(name, lines):
     """Violations (strings) of one kernel's assembly."""
     instrs = _instructions(lines)
     violations, seen = [], set()
     _check_m0(name, instrs, violations)
+    _check_mfma(name, instrs, violations)
     loads = [i for i, (t, a) in enumerate(instrs) if a and (_ASM_VLOAD.match(t) or _ASM_DSREAD.match(t))]
     if not loads:
         return violations

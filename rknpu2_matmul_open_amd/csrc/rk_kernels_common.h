@@ -38,7 +38,7 @@ bool dense_stream_fits(const rkh_gemm_args& g);
 int gemv_max_rows(const rkh_gemm_args& g);
 bool gemv_can_fuse(const rkh_quant_args& q, const rkh_gemm_args& g, bool swiglu = false);
 // rk_kernels_gemm.hip: tiles of 256 x 256 with 128-row ones for the rest, or tile_rows = 128 / 64 / 32
-struct BigTiles { int big, small; };
+struct BigTiles { int big, small, rounds; };
 BigTiles wk_big_tiles(int M, int N, int K, int w_int4);
 bool wk_big_applies(int M, int N, int K, int w_int4, BigTiles* tiles); // tiles: how the launch is cut if it does
 int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, BigTiles tiles);

@@ -57,10 +57,10 @@ namespace {
 // workgroup; on this multi-die part each one walks the die's L2, and 32
 // workgroups per die queueing for that cost more than the second launch.)
 constexpr int WK_RING_BYTES = 128 * 1024;
-constexpr int WK_SCALES_OFF = WK_RING_BYTES;                      // fp32 scales of the tile: 256 rows, then 256 columns
-constexpr int WK_ROW_SCALES = 256;
-constexpr int WK_LDS_BYTES = WK_SCALES_OFF + (WK_ROW_SCALES + 256) * 4;
-constexpr int WK_STAGE = 2 * 16 * 144;                            // a wave's staging area: two units of 16 rows x 32 columns
+constexpr int WK_SCALES_OFF = WK_RING_BYTES;                      // fp32 scales of the tile: 256 rows, then 256 columns; twice
+constexpr int WK_ROW_SCALES = 256, WK_SCALES = (WK_ROW_SCALES + 256) * 4;
+constexpr int WK_STAGE_OFF = WK_SCALES_OFF + 2 * WK_SCALES, WK_STAGE = 16 * 144; // per wave: 16 rows x 32 columns
+constexpr int WK_LDS_BYTES = WK_STAGE_OFF + 8 * WK_STAGE;
 constexpr int WK_PART_K = 256;                                    // granularity of a K split over workgroups
 
 typedef __attribute__((address_space(3))) uint8_t* lds_ptr_t;
@@ -85,8 +85,8 @@ __device__ __forceinline__ void wk_tile_coords(unsigned tile, unsigned mblocks, 
 // The weights are the FIRST MFMA operand: lane (r, q) owns output row r of the tile and its columns 4 q .. 4 q + 3.
 // Two neighbouring tiles make a unit of 16 rows x 32 columns, the width of a column block.
 
-// Stage a unit in one half of the wave's staging area and read it back as 16-byte pieces of rows.  LDS operations of a wave
-// complete in issue order, so nothing is waited for between the two; the fence keeps the compiler from swapping them.
+// Stage a unit in the wave's staging area and read it back as 16-byte pieces of rows.  LDS operations of a wave complete in
+// issue order, so nothing is waited for between the two, or ahead of the next unit; the fence keeps the compiler from swapping them.
 template <typename T>
 struct StagedUnit {
     static constexpr int ES = sizeof(T), PITCH = 32 * ES + 16, PIECES = ES / 2; // 16-byte pieces of a lane
@@ -188,7 +188,7 @@ __device__ __forceinline__ void wk_store(const rkh_gemm_args& g, Acc&& acc_of, R
         for (int u = 0; u < ROWS * NB; ++u) {
             T vals[8];
             values(vals, u / NB, u % NB);
-            held[u & 1].exchange(vals, stage + (u & 1) * (WK_STAGE / 2), lane);
+            held[u & 1].exchange(vals, stage, lane);
             if (u > 0) held[(u - 1) & 1].template store<true>(C, g.ldc, m0 + 16 * ((u - 1) / NB), n0[(u - 1) % NB], m_limit, lane);
         }
         held[(ROWS * NB - 1) & 1].template store<true>(C, g.ldc, m0 + 16 * (ROWS - 1), n0[NB - 1], m_limit, lane);
@@ -201,7 +201,7 @@ __device__ __forceinline__ void wk_store(const rkh_gemm_args& g, Acc&& acc_of, R
             values(vals, i, b);
             StagedUnit<T> unit;
             if (whole[b]) {
-                unit.exchange(vals, stage + (u & 1) * (WK_STAGE / 2), lane);
+                unit.exchange(vals, stage, lane);
                 unit.template store<false>(C, g.ldc, m0 + 16 * i, n0[b], m_limit, lane);
             } else {
                 store_unit_plain(C, g.ldc, m0 + 16 * i, n0[b], m_limit, n_end, vals, lane);
@@ -221,12 +221,28 @@ __device__ __forceinline__ void wk_store(const rkh_gemm_args& g, Acc&& acc_of, R
     }
 }
 
-template <int N> __device__ __forceinline__ void wait_lds(v4i& x) { asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory"); }
+// NAMED: x becomes valid -- what keeps the compiler's own products behind the wait; for products that are asm statements their
+// order is enough, and a statement that "writes" an operand would get a wait state behind it.
+template <int N, bool NAMED> __device__ __forceinline__ void wait_lds(v4i& x) {
+    if constexpr (NAMED) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory");
+    else asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
 template <int OFF> __device__ __forceinline__ void read_lds(v4i& x, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x) : "v"(addr), "n"(OFF));
 }
 template <int OFF> __device__ __forceinline__ void load_regs(v4i& x, unsigned lane_off, const uint8_t* base) {
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(x) : "v"(lane_off), "s"(base), "n"(OFF));
+}
+// The product as an asm statement, for the chained tiles: sums stay in one place (left to itself the compiler rotates 128
+// sums through the register file, and with the next tile's weights beside them spills some around the tile's first products).
+// What the compiler then does not order: a vector instruction that writes an operand has to be two wait states ahead
+// of the product -- the weights are unpacked well ahead --, and one that reads a sum waits for the last products, settle().
+// The build checks both in the compiled code (audit_waits.py).
+__device__ __forceinline__ void mfma(v4i& sum, const v4i& w, const v4i& a) {
+    asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(sum) : "v"(w), "v"(a));
+}
+__device__ __forceinline__ void mfma_first(v4i& sum, const v4i& w, const v4i& a) {
+    asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, 0" : "=&v"(sum) : "v"(w), "v"(a));
 }
 __device__ __forceinline__ void keep(v4i& x) { asm volatile("" : "+v"(x)); }
 
@@ -254,17 +270,21 @@ template <int TM, bool W4, int TN, bool RS>
 struct WkShape {
     static_assert(!RS || (TM == 4 && TN == 2), "row-split waves: tiles of 256 x 256");
     static constexpr bool ONE = TM == 4 && !W4;                 // a step is one unit
+    static constexpr bool ASM = RS;                             // products as asm statements, see mfma()
     static constexpr int U = ONE ? 1 : 2;
     static constexpr int RM = 2 * TM, CN = 2 * TN;              // operands of 16 rows / columns per wave
     static constexpr int BM = RS ? 256 : 32 * TM;               // rows of a tile
     static constexpr int KT = (RS ? 2 : 4) * U;                 // k-tiles of a step
-    static constexpr int BUF = BM / 32 * KT * 1024, NBUF = ONE ? 6 : TM == 4 ? 4 : 8;
+    static constexpr int BUF = BM / 32 * KT * 1024, NBUF = ONE ? (RS ? 8 : 6) : TM == 4 ? 4 : 8;
     static constexpr int NC = BUF / 8192;                       // 1 KiB copies of a wave per step
     static constexpr int NW = CN;                               // weight loads per unit (int4: per step, in its first unit)
-    static constexpr int NSW = ONE ? 3 : TM == 4 ? 2 : 4;       // slots of the weight ring
+    static constexpr int NSW = ONE ? (RS ? 4 : 3) : TM == 4 ? 2 : 4; // slots of the weight ring
     static constexpr int G = ONE || (W4 && TM < 4) ? 2 : 1;             // steps between barriers
     static constexpr int D = ONE ? 4 : W4 && TM < 4 ? 5 : 3;         // look-ahead of the copies
-    static constexpr int UNR = NBUF;                            // steps of an unrolled trip
+    static constexpr int UNR = RS ? NBUF / 2 : NBUF;            // steps of an unrolled trip (RS: 256 k, half the ring)
+    // RS: the step of a trip whose copies (weights) are a tile's last ones: in the tile's last trip but one (last trip)
+    static constexpr int A_TURN = ((-D - 1) % UNR + UNR) % UNR, W_TURN = (-(W4 ? NSW - 1 : (NSW - 1) / U) - 1 + 2 * UNR) % UNR;
+    static_assert(!RS || ((D + UNR - 1) / UNR == (A_TURN == UNR - 1 ? 1 : 2) && W_TURN == 0 && NSW - 1 < UNR * (W4 ? 1 : U)), "the trips of the turns");
     static constexpr int copies(int unit) { return U == 1 ? NC : NC == 1 ? (unit & 1 ? 0 : 1) : NC / 2; }
     static constexpr bool loads_w(int unit) { return !W4 || !(unit & 1); }
     static constexpr int items(int unit) { return copies(unit) + (loads_w(unit) ? NW : 0); }
@@ -280,24 +300,36 @@ struct WkShape {
     }
     // weights loaded in `unit`: of which unit (int4: step)
     static constexpr int loaded(int unit) { return W4 ? (unit >> 1) + NSW - 1 : unit + NSW - 1; }
-    // what the prologue has issued since the copies that its wait is to see (its first steps load no weights)
+    // what the prologue has issued since the last of what the first unit and the reads up to the first barrier need: the
+    // weights of unit 0 and the copies of steps 0 .. G
     static constexpr int prologue_since() {
-        int n = 0;
-        for (int unit = U * (G + 1 - D); unit < 0; ++unit) n += copies(unit) + (loads_w(unit) && loaded(unit) >= 0 ? NW : 0);
-        return n;
+        int n = 0, last = 0;
+        for (int t = 0; t < U * D; ++t) {
+            n += copies(t % U);
+            if (t / U <= G) last = n;
+            if (loads_w(t % U) && loaded(t - U * D) >= 0) n += NW;
+            if (loads_w(t % U) && loaded(t - U * D) == 0) last = n;
+        }
+        return n - last;
     }
     static_assert(D >= G + 1 && NBUF >= D + G && UNR % G == 0 && (W4 ? UNR : U * UNR) % NSW == 0, "see the ordering rules above");
-    static constexpr int first_wait() { return in_flight(U - 1) < prologue_since() ? in_flight(U - 1) : prologue_since(); }
     static_assert(in_flight(0) <= 63 && in_flight(U - 1) <= 63, "the vmcnt field");
     static_assert(NBUF * BUF <= WK_RING_BYTES && 4 * RM * CN * 1024 <= WK_RING_BYTES, "the ring; the exchange of k-halves");
 };
 
+// Where a load is issued: the wave's priority there and the step of the trip, -1 in the prologue.
+template <int P, int STEP> struct WkAt { static constexpr int PRIO = P, AT = STEP; };
+// The tiles that a workgroup of gemm_wk_big_kernel multiplies one after the other: v, v + stride, .. below `big`.
+struct WkChain { int v, stride, big, mblocks, nblocks; };
+
 template <int TM, bool W4, int EPI, int TN, bool RS>
 __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw, int tile, int mblk, int nblk, int kpart,
-                                        int ksplit, int kt0, int kts) { // the part's first k-tile and their number, a multiple of 8
+                                        int ksplit, int kt0, int kts, // the part's first k-tile and their number, a multiple of 8
+                                        [[maybe_unused]] WkChain chain = {}) {
     using S = WkShape<TM, W4, TN, RS>;
     static_assert(TN == 2 || (TN == 1 && EPI != RKH_EPI_SWIGLU), "gate / up pairs need two column blocks per wave");
     constexpr int U = S::U, RM = S::RM, CN = S::CN, KT = S::KT, BUF = S::BUF, NBUF = S::NBUF, NSW = S::NSW;
+    constexpr int A_STEP = KT * 1024, W_STEP = KT * (W4 ? 512 : 1024);
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
@@ -306,27 +338,45 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
 
     // ---- sources: wave-uniform base pointers (scalar registers) + a constant lane offset.
     // The step's copies of a wave are NC consecutive KiB: of row block wave * NC / KT, from k-tile wave * NC % KT on
-    const uint8_t* asrc = g.A + ((size_t)(mblk * (S::BM / 32) + wave * S::NC / KT) * KB + kt0 + wave * S::NC % KT) * 1024;
-    const uint8_t* wsrc[TN]; // (int4: two k-tiles per KiB)
+    const auto a_from = [&](int mb) { return g.A + ((size_t)(mb * (S::BM / 32) + wave * S::NC / KT) * KB + kt0 + wave * S::NC % KT) * 1024; };
+    const auto w_from = [&](int nb, int j) { // (int4: two k-tiles per KiB)
+        return g.W + ((size_t)(nb * (4 * TN) + wn * TN + j) * KB + kt0 + (RS ? 0 : wk * 2 * U)) * (W4 ? 512 : 1024);
+    };
+    const uint8_t* asrc = a_from(mblk);
+    const uint8_t* wsrc[TN];
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-        wsrc[j] = g.W + ((size_t)(nblk * (4 * TN) + wn * TN + j) * KB + kt0 + (RS ? 0 : wk * 2 * U)) * (W4 ? 512 : 1024);
+    for (int j = 0; j < TN; ++j) wsrc[j] = w_from(nblk, j);
     const int q = lane >> 4;
     const unsigned lane_off = lane * 16;
     const unsigned piece_off = (q >> 1) * 1024 + (q & 1) * 512 + (lane & 15) * 16; // this lane's piece of an operand
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds_raw;
-    const uint32_t copy_dst = lds_base + wave * S::NC * 1024; // this wave's chunk inside buffer 0
+    uint32_t copy_lo = lds_base + wave * S::NC * 1024, copy_hi = copy_lo + 65536; // this wave's chunk inside buffer 0, and 64 KiB on
     // LDS byte addresses of this lane's piece of the wave's first operand in buffer 0 and 64 KiB on
-    const uint32_t frag_lo = lds_base + (RS ? wk * (RM / 2) * KT : wk * 2 * U) * 1024 + (W4 ? piece_off + (q >> 1) * 1024 : piece_off);
-    const uint32_t frag_hi = frag_lo + 65536;
+    uint32_t frag_lo = lds_base + (RS ? wk * (RM / 2) * KT : wk * 2 * U) * 1024 + (W4 ? piece_off + (q >> 1) * 1024 : piece_off);
+    uint32_t frag_hi = frag_lo + 65536;
     const int ksteps = kts / KT;
     int a_left = ksteps - 1, w_left = ksteps - 1; // how often the sources may still advance
+    // RS: where they go from there, the chain's next tile or, behind the last, nowhere
+    [[maybe_unused]] const uint8_t *a_next = nullptr, *w_next[TN] = {};
+    [[maybe_unused]] int a_step = A_STEP, w_step = W_STEP, mblk_next = 0, nblk_next = 0;
+    [[maybe_unused]] bool more = false, a_turn = false, w_turn = false; // a_turn, w_turn: in this trip
+    [[maybe_unused]] const auto find_next = [&]() {
+        more = chain.v + chain.stride < chain.big;
+        if (more) wk_tile_coords(xcd_remap(chain.v + chain.stride, chain.big), chain.mblocks, chain.nblocks, mblk_next, nblk_next);
+        a_next = more ? a_from(mblk_next) : a_from(mblk) + (size_t)(ksteps - 1) * A_STEP;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) w_next[j] = more ? w_from(nblk_next, j) : w_from(nblk, j) + (size_t)(ksteps - 1) * W_STEP;
+    };
+    // (the prologue reaches the end of a tile only if there is no other, see launch_gemm_wk_big)
+    if constexpr (RS) a_next = asrc + (size_t)(ksteps - 1) * A_STEP;
 
     v4i acc[RM][CN];
+    if constexpr (!RS) {
 #pragma unroll
-    for (int i = 0; i < RM; ++i)
+        for (int i = 0; i < RM; ++i)
 #pragma unroll
-        for (int j = 0; j < CN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+            for (int j = 0; j < CN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    }
 
     v4i a[RM];                  // activation operands
     v4i wring[NSW][CN];         // weights as loaded: of a unit, or, int4, of a step
@@ -337,22 +387,38 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     // K = 4096 (exact 128 x 4096 x 11008 13.9 -> 13.65 us, 512 x 4096 x 4096 16.5 -> 16.3; int4 weights and wider tiles gain nothing).
     constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
     [[maybe_unused]] unsigned long long a_lanes = ~0ull;
-    auto copy_a = [&](int buf, auto c_tag, auto prio_tag) { // one of the step's copies
-        constexpr int C = decltype(c_tag)::value, PRIO = decltype(prio_tag)::value;
-        if constexpr (MASKED) copy_lds<C * 1024, PRIO>(lane_off, asrc, copy_dst + buf * BUF, a_lanes);
-        else copy_lds<C * 1024, PRIO>(lane_off, asrc, copy_dst + buf * BUF);
-        if constexpr (C == S::NC - 1) {
-            asrc += a_left > 0 ? KT * 1024 : 0;
+    auto copy_a = [&](auto buf_tag, auto c_tag, auto at_tag) { // one of the step's copies
+        constexpr int C = decltype(c_tag)::value, PRIO = decltype(at_tag)::PRIO;
+        constexpr int B = decltype(buf_tag)::value % NBUF, PER = 65536 / BUF;
+        const uint32_t dst = (B < PER ? copy_lo : copy_hi) + B % PER * BUF;
+        if constexpr (MASKED) copy_lds<C * 1024, PRIO>(lane_off, asrc, dst, a_lanes);
+        else copy_lds<C * 1024, PRIO>(lane_off, asrc, dst);
+        // RS: a trip turns to the next tile behind one of its steps (a choice behind every step cost the loop 2.5 %)
+        if constexpr (C == S::NC - 1 && RS && decltype(at_tag)::AT >= 0 && decltype(at_tag)::AT != S::A_TURN) {
+            asrc += a_step;
+        } else if constexpr (C == S::NC - 1 && RS) {
+            const bool turn = decltype(at_tag)::AT < 0 ? a_left-- == 0 : a_turn;
+            asrc = turn ? a_next : asrc + a_step;
+            a_step = turn && !more ? 0 : a_step;
+        } else if constexpr (C == S::NC - 1) {
+            asrc += a_left > 0 ? A_STEP : 0;
             if constexpr (MASKED) a_lanes = a_left > 0 ? ~0ull : 1ull;
             --a_left;
         }
     };
-    auto load_w = [&](v4i* regs, auto half_tag, auto e_tag) { // operand e of unit HALF of a step (int4: of both)
+    auto load_w = [&](v4i* regs, auto half_tag, auto e_tag, [[maybe_unused]] auto at_tag) { // operand e of unit HALF of a step (int4: of both)
         constexpr int HALF = W4 || U == 1 ? 0 : decltype(half_tag)::value, E = decltype(e_tag)::value;
         load_regs<HALF * 2048 + (E & 1) * 256>(regs[E], piece_off, wsrc[E / 2]);
-        if constexpr (E == CN - 1 && (W4 || HALF == U - 1)) {
+        if constexpr (E == CN - 1 && RS && decltype(at_tag)::AT != S::W_TURN) {
 #pragma unroll
-            for (int j = 0; j < TN; ++j) wsrc[j] += w_left > 0 ? KT * (W4 ? 512 : 1024) : 0;
+            for (int j = 0; j < TN; ++j) wsrc[j] += w_step;
+        } else if constexpr (E == CN - 1 && RS) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wsrc[j] = w_turn ? w_next[j] : wsrc[j] + w_step;
+            w_step = w_turn && !more ? 0 : w_step;
+        } else if constexpr (E == CN - 1 && (W4 || HALF == U - 1)) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wsrc[j] += w_left > 0 ? W_STEP : 0;
             --w_left;
         }
     };
@@ -370,11 +436,12 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
             constexpr int HALF = decltype(half_tag)::value, E = decltype(e_tag)::value;
             const int x = HALF ? raw[E].z : raw[E].x, y = HALF ? raw[E].w : raw[E].y;
             dst[E] = v4i{(x << 4) & (int)0xF0F0F0F0, x & (int)0xF0F0F0F0, (y << 4) & (int)0xF0F0F0F0, y & (int)0xF0F0F0F0};
+            if constexpr (S::ASM) keep(dst[E]); // (here, not in front of the product, see mfma())
         }
     };
 
-    // Unit t of the trip.
-    auto k_unit = [&](auto unit_tag) {
+    // Unit t of the trip.  FRESH: the accumulators start here.
+    auto k_unit = [&](auto unit_tag, auto fresh_tag) {
         constexpr int T = decltype(unit_tag)::value, STEP = T / U, UN = T % U, MF = RM * CN;
         constexpr int ITEMS = S::items(UN), LAST = W4 ? MF / 2 : MF, SPACE = LAST / (ITEMS + 1) > 0 ? LAST / (ITEMS + 1) : 1; // loads: behind every SPACE-th MFMA
         static_assert(ITEMS * SPACE <= (W4 && UN == 0 ? MF : LAST), "every load of a unit goes out before its wait");
@@ -384,18 +451,20 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
         // The two waves of a SIMD drift apart between barriers (the older one wins every issue conflict) and the one left
         // behind cannot keep the matrix pipe busy alone: the wave that is further into the barrier interval yields.
         // (4096 x 4096 x 14336 int8 185.4 -> 182.7 us, 200 x 4096 x 14336 int4 18.1 -> 17.5)
-        using Priority = std::integral_constant<int, 3 - 4 * (T % (U * S::G)) / (U * S::G)>;
+        using At = WkAt<3 - 4 * (T % (U * S::G)) / (U * S::G), STEP>;
         static_for<RM>([&](auto i_tag) {
             constexpr int I = decltype(i_tag)::value;
-            wait_lds<RM - 1>(a[I]);
+            wait_lds<RM - 1, !S::ASM>(a[I]);
             static_for<CN>([&](auto j_tag) {
                 constexpr int J0 = decltype(j_tag)::value, J = I & 1 ? CN - 1 - J0 : J0, AT = I * CN + J0; // (there and back: one operand stays)
-                if constexpr (W4) acc[I][J] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wop[UN][J], a[I], acc[I][J], 0, 0, 0);
-                else acc[I][J] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wring[T % NSW][J], a[I], acc[I][J], 0, 0, 0);
+                const v4i& w = W4 ? wop[UN][J] : wring[T % NSW][J];
+                if constexpr (!S::ASM) acc[I][J] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, a[I], acc[I][J], 0, 0, 0);
+                else if constexpr (decltype(fresh_tag)::value && T == 0) mfma_first(acc[I][J], w, a[I]);
+                else mfma(acc[I][J], w, a[I]);
                 if constexpr (AT % SPACE == SPACE - 1 && AT / SPACE < ITEMS) {
                     constexpr int Q = AT / SPACE, NCU = S::copies(UN);
-                    if constexpr (Q < NCU) copy_a((STEP + S::D) % NBUF, std::integral_constant<int, Q + (UN ? S::copies(0) : 0)>{}, Priority{});
-                    else load_w(wring[LOAD_SLOT], Half{}, std::integral_constant<int, Q - NCU>{});
+                    if constexpr (Q < NCU) copy_a(std::integral_constant<int, STEP + S::D>{}, std::integral_constant<int, Q + (UN ? S::copies(0) : 0)>{}, At{});
+                    else load_w(wring[LOAD_SLOT], Half{}, std::integral_constant<int, Q - NCU>{}, At{});
                 }
                 if constexpr (W4) { // the next unit's operands, in the second half of this one
                     if constexpr (UN == 1 && AT == MF / 2 - 1) w_wait(wring[NEXT_W], std::integral_constant<int, S::in_flight(1)>{});
@@ -405,80 +474,137 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
-            read_a(std::integral_constant<int, (T + 1) % (U * S::UNR)>{}, i_tag);
+            read_a(std::integral_constant<int, T + 1>{}, i_tag);
             __builtin_amdgcn_sched_barrier(0);
         });
         if constexpr (!W4) w_wait(wring[NEXT_W], std::integral_constant<int, S::in_flight(UN)>{});
         if constexpr (UN == U - 1 && (STEP + 1) % S::G == 0) asm volatile("s_barrier" ::: "memory");
     };
-    auto k_step = [&](auto step_tag) {
-        static_for<U>([&](auto u_tag) { k_unit(std::integral_constant<int, U * decltype(step_tag)::value + decltype(u_tag)::value>{}); });
+    auto k_step = [&](auto step_tag, auto fresh_tag) {
+        static_for<U>([&](auto u_tag) { k_unit(std::integral_constant<int, U * decltype(step_tag)::value + decltype(u_tag)::value>{}, fresh_tag); });
     };
 
     // prologue: the same issue order as if the loop had run for steps -D..-1
     static_for<U * S::D>([&](auto t_tag) {
         constexpr int T = decltype(t_tag)::value - U * S::D, UN = (T + U * S::D) % U, OF = S::loaded(T);
         static_for<S::copies(UN)>([&](auto c_tag) {
-            copy_a((T + U * S::D) / U, std::integral_constant<int, decltype(c_tag)::value + (UN ? S::copies(0) : 0)>{}, std::integral_constant<int, 0>{});
+            copy_a(std::integral_constant<int, (T + U * S::D) / U>{}, std::integral_constant<int, decltype(c_tag)::value + (UN ? S::copies(0) : 0)>{}, WkAt<0, -1>{});
         });
         if constexpr (S::loads_w(T) && OF >= 0)
-            static_for<CN>([&](auto e_tag) { load_w(wring[OF % NSW], std::integral_constant<int, OF & 1>{}, e_tag); });
+            static_for<CN>([&](auto e_tag) { load_w(wring[OF % NSW], std::integral_constant<int, OF & 1>{}, e_tag, WkAt<0, -1>{}); });
     });
     RK_TS(1);
     // The tile's scales follow, straight to LDS, so that the epilogue does not start with a round trip to memory: thread t
     // brings the scale of row t % BM and of physical column t % (128 TN).  (Two more loads in the queue only make the
     // first units' waits stricter.  Ahead of the prologue's loads they cost the 128-row tile 0.2 us: the first copies
     // leave later.  Rows and columns beyond the matrix take some valid scale: nothing is stored for them.)
-    if constexpr (EPI != RKH_EPI_I32) {
-        const int row = threadIdx.x & (S::BM - 1), col = threadIdx.x & (128 * TN - 1);
-        const int pb = nblk * (4 * TN) + (col >> 5);
-        const int n = EPI == RKH_EPI_SWIGLU && (pb >> 1) * 32 >= g.interleave_F ? 0 : block_first_col(pb, g.interleave_F) + (col & 31);
-        copy_lds_dword(g.a_scale + min(mblk * S::BM + row, g.M - 1), lds_base + WK_SCALES_OFF + (wave * 64 & (S::BM - 1)) * 4);
-        copy_lds_dword(g.w_scale + min(n, g.N - 1), lds_base + WK_SCALES_OFF + (WK_ROW_SCALES + (wave * 64 & (128 * TN - 1))) * 4);
-    }
-    w_wait(wring[0], std::integral_constant<int, S::first_wait()>{}); // weights of unit 0 and the copies of steps 0..G have landed
+    const auto fetch_scales = [&](uint32_t to) {
+        if constexpr (EPI != RKH_EPI_I32) {
+            int t = threadIdx.x;
+            asm volatile("" : "+v"(t)); // (opaque: addresses made from it are not worth registers in the loop)
+            const int row = t & (S::BM - 1), col = t & (128 * TN - 1);
+            const int pb = nblk * (4 * TN) + (col >> 5);
+            const int n = EPI == RKH_EPI_SWIGLU && (pb >> 1) * 32 >= g.interleave_F ? 0 : block_first_col(pb, g.interleave_F) + (col & 31);
+            copy_lds_dword(g.a_scale + min(mblk * S::BM + row, g.M - 1), lds_base + to + (wave * 64 & (S::BM - 1)) * 4);
+            copy_lds_dword(g.w_scale + min(n, g.N - 1), lds_base + to + (WK_ROW_SCALES + (wave * 64 & (128 * TN - 1))) * 4);
+        }
+    };
+    fetch_scales(WK_SCALES_OFF);
+    if constexpr (RS) find_next(); // (while the first loads are on their way)
+    w_wait(wring[0], std::integral_constant<int, S::prologue_since() + (EPI != RKH_EPI_I32 ? 2 : 0)>{}); // weights of unit 0 and the copies of steps 0..G have landed
     asm volatile("s_barrier" ::: "memory");
-    static_for<RM>([&](auto i_tag) { read_a(std::integral_constant<int, 0>{}, i_tag); });
-    static_for<CN>([&](auto e_tag) { unpack(wop[0], wring[0], std::integral_constant<int, 0>{}, e_tag); });
+    const auto first_operands = [&]() {
+        static_for<RM>([&](auto i_tag) { read_a(std::integral_constant<int, 0>{}, i_tag); });
+        static_for<CN>([&](auto e_tag) { unpack(wop[0], wring[0], std::integral_constant<int, 0>{}, e_tag); });
+    };
+    first_operands();
     RK_TS(2);
 
+    using Old = std::false_type;
+    // Scale, convert and store the rows from row0 of the tile on
+    const auto store = [&](auto rows_tag, auto&& sum_of, int row0, int scales) {
+        constexpr int ROWS = decltype(rows_tag)::value;
+        int l = lane; // (opaque, as in fetch_scales)
+        asm volatile("" : "+v"(l));
+        const float* sc = reinterpret_cast<const float*>(lds_raw + scales);
+        float as[ROWS];
+        v4f ws[CN];
+        if constexpr (EPI != RKH_EPI_I32) {
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i) as[i] = sc[row0 + i * 16 + (l & 15)];
+#pragma unroll
+            for (int j = 0; j < CN; ++j) ws[j] = *reinterpret_cast<const v4f*>(sc + WK_ROW_SCALES + (wn * CN + j) * 16 + 4 * (l >> 4));
+        }
+        wk_store<ROWS, CN, W4, EPI>(g, sum_of, [&](int i) { return as[i]; }, [&](int j, int e) { return ws[j][e]; },
+                                    mblk * S::BM + row0, nblk * (4 * TN) + wn * TN, g.M, lds_raw + WK_STAGE_OFF + wave * WK_STAGE, l);
+    };
+    const auto settle = [&]() { // the operands that were read beyond the tile's last unit; see below for why they are named
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < RM; ++i) keep(a[i]);
+#pragma unroll
+        for (int t = 0; t < RM * CN; ++t) keep(acc[t / CN][t % CN]);
+    };
+    if constexpr (RS) {
+        // The steps of the chain's tiles follow one another: the copies and weights that run ahead of a tile's end are the
+        // next tile's first ones, and stay in the ring and in registers while the tile is converted and stored.
+        for (int scales = WK_SCALES_OFF;; scales ^= WK_SCALES_OFF ^ (WK_SCALES_OFF + WK_SCALES)) {
+            const auto trip = [&](auto fresh_tag, int k) {
+                a_turn = k + 2 * S::UNR == ksteps, w_turn = k + S::UNR == ksteps;
+                static_for<S::UNR>([&](auto step) { k_step(step, fresh_tag); });
+                const uint32_t f = frag_lo, c = copy_lo;
+                frag_lo = frag_hi, frag_hi = f, copy_lo = copy_hi, copy_hi = c;
+            };
+            trip(std::true_type{}, 0);
+            for (int k = S::UNR; k < ksteps; k += S::UNR) trip(Old{}, k);
+            RK_TS(3);
+            settle();
+            // behind the last tile: a load to LDS must not outlive the workgroup (waited for here, not behind the stores)
+            if (!more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            RK_TS(4);
+            store(std::integral_constant<int, RM>{}, [&](int i, int j) -> const v4i& { return acc[i][j]; }, wk * RM * 16, scales);
+            RK_TS(5);
+            if (!more) break;
+            chain.v += chain.stride;
+            mblk = mblk_next, nblk = nblk_next;
+            find_next();
+            fetch_scales(scales ^ WK_SCALES_OFF ^ (WK_SCALES_OFF + WK_SCALES));
+            first_operands();
+        }
+        return;
+    }
+
     int s = 0;
-    for (; s + S::UNR <= ksteps; s += S::UNR) static_for<S::UNR>([&](auto step) { k_step(step); });
+    for (; s + S::UNR <= ksteps; s += S::UNR) static_for<S::UNR>([&](auto step) { k_step(step, Old{}); });
     // (the remaining steps as a chain that ends at the first one beyond K: the control flow
     // then only holds the sequences of steps that can happen, which is what the static check
     // of the waits, audit_waits.py, walks)
     static_while<S::UNR - 1>([&](auto step) {
         if (s + decltype(step)::value >= ksteps) return false;
-        k_step(step);
+        k_step(step, Old{});
         return true;
     });
-    __builtin_amdgcn_s_setprio(0);
     RK_TS(3);
 
     // ---- epilogue.  Drain the look-ahead copies (they write LDS), the operands read ahead and the scale
     // loads; then every wave is past its last operand and LDS is reused.
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    settle();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // What was loaded for units beyond K was in flight until this wait, while the compiler regards
     // the destination registers as dead: the uses below keep it from giving one of them to an epilogue value
     // ahead of the wait (the load would then land on top of that value).
-#pragma unroll
-    for (int i = 0; i < RM; ++i) keep(a[i]);
 #pragma unroll
     for (int t = 0; t < NSW; ++t)
 #pragma unroll
         for (int e = 0; e < CN; ++e) keep(wring[t][e]);
     lds_barrier();
 
-    // The k-halves meet: a wave hands half of the rows of its strip to its partner and keeps operands wk * RM / 2 .. (RS:
-    // every wave holds finished sums).  Accumulators are indexed with constants, hence the two branches.
-    constexpr int KEEP = RS ? RM : RM / 2;
-    const int row0 = wk * KEEP * 16; // of the kept rows in the tile
-    v4i sum[KEEP][CN];
-    if constexpr (RS) {
-#pragma unroll
-        for (int t = 0; t < RM * CN; ++t) sum[t / CN][t % CN] = acc[t / CN][t % CN];
-    } else {
-        constexpr int XT = KEEP * CN; // tiles per exchange slot
+    // The k-halves meet: a wave hands half of the rows of its strip to its partner and keeps operands wk * RM / 2 ..
+    // Accumulators are indexed with constants, hence the two branches.
+    if constexpr (!RS) {
+        constexpr int KEEP = RM / 2, XT = KEEP * CN; // operands kept; tiles per exchange slot
+        v4i sum[KEEP][CN];
         v4i* xch = reinterpret_cast<v4i*>(lds_raw);
         const auto hand_over = [&](auto wk_tag) {
             constexpr int GIVE0 = (decltype(wk_tag)::value ^ 1) * KEEP, KEEP0 = decltype(wk_tag)::value * KEEP;
@@ -498,22 +624,10 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
             for (int t = 0; t < XT; ++t) dst[t * 64 + lane] = sum[t / CN][t % CN];
             return;
         }
-        lds_barrier();
+        RK_TS(4);
+        store(std::integral_constant<int, KEEP>{}, [&](int i, int j) -> const v4i& { return sum[i][j]; }, wk * KEEP * 16, WK_SCALES_OFF);
+        RK_TS(5);
     }
-    RK_TS(4);
-    float as[KEEP];
-    v4f ws[CN];
-    if constexpr (EPI != RKH_EPI_I32) {
-        const float* sc = reinterpret_cast<const float*>(lds_raw + WK_SCALES_OFF);
-#pragma unroll
-        for (int i = 0; i < KEEP; ++i) as[i] = sc[row0 + i * 16 + (lane & 15)];
-#pragma unroll
-        for (int j = 0; j < CN; ++j) ws[j] = *reinterpret_cast<const v4f*>(sc + WK_ROW_SCALES + (wn * CN + j) * 16 + 4 * q);
-    }
-    wk_store<KEEP, CN, W4, EPI>(g, [&](int i, int j) -> const v4i& { return sum[i][j]; }, [&](int i) { return as[i]; },
-                                [&](int j, int e) { return ws[j][e]; }, mblk * S::BM + row0, nblk * (4 * TN) + wn * TN, g.M,
-                                lds_raw + wave * WK_STAGE, lane);
-    RK_TS(5);
 }
 
 // The tile of a workgroup: XCD-contiguous ranges, 4 row blocks per column sweep.
@@ -542,7 +656,10 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 // left of the output: the tiles that would start a last, mostly empty round, each in two halves, and a
 // last strip of at most 128 rows.  Workgroup = 8 waves in 4 column groups x 2 row halves: a wave multiplies
 // 128 x 64 over the whole K, so there is no exchange of k-halves and all eight waves convert and store.
-// What bounds it: the matrix pipes at the clock that the power limit leaves, and 6 - 9 us of a tile outside its loop.
+// What bounds it: the matrix pipes at the clock that the power limit leaves, and the conversion and stores of a tile.
+// A workgroup per compute unit multiplies its tiles one after the other as one stream of steps (wk_tile, RS), so that only its first
+// tile waits for memory: int8 4000 x 1024 x 14336 77.9 -> 73.2 us, 4000 x 512 x 14336 67.3 -> 62.4, 4096 x 4096 x 14336 187 -> 184;
+// a launch of one round measures the same.
 // Against 128 x 256 tiles: the second operand of a column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
 // cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, when the tiles were
 // introduced: int8 4096 x 4096 x 14336 241 -> 203, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
@@ -550,18 +667,27 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 // bursts of stores fall apart -- 204 -> 217, 195 -> 210: tiles in step share their operands in L2.)
 template <bool W4, int EPI>
 __global__ __launch_bounds__(512) void gemm_wk_big_kernel(const uint8_t* h_A, const uint8_t* h_W, int h_M, int h_K,
-                                                          int mblocks, int nblocks, int big, rkh_gemm_args g) {
+                                                          int mblocks, int nblocks, int big, int small, int rounds, rkh_gemm_args g) {
     g.A = h_A; g.W = h_W; g.M = h_M; g.K = h_K;
     RK_TS(0);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[]; // WK_LDS_BYTES
     const int KB = (int)rkh_align_up(g.K, RKH_K_ALIGN) / 32;
+    const int groups = gridDim.x, b = blockIdx.x;
     int mblk, nblk;
-    if ((int)blockIdx.x < big) {
-        wk_tile_coords(xcd_remap(blockIdx.x, big), mblocks, nblocks, mblk, nblk);
-        wk_tile<4, W4, EPI, 2, true>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB);
-    } else {
-        const int halves = 2 * (mblocks * nblocks - big); // small tiles inside the last 256 x 256 ones, then the strip
-        const int t = xcd_remap(blockIdx.x - big, gridDim.x - big);
+    if (b < big) {
+        wk_tile_coords(xcd_remap(b, big), mblocks, nblocks, mblk, nblk);
+        wk_tile<4, W4, EPI, 2, true>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB, WkChain{b, groups, big, mblocks, nblocks});
+    }
+    // The small tiles: `rounds` for every workgroup without a big one in the last round, the rest for the others.  (Without
+    // rounds -- a workgroup per tile -- they follow the big ones.)
+    const int extra = rounds ? big % groups : big, without = groups - extra;
+    const int first = b >= extra ? b - extra : without * rounds + b, stride = b >= extra ? without : extra;
+    const int end = !rounds ? b >= extra ? first + 1 : 0 : b >= extra ? min(small, without * rounds) : small;
+    const int halves = 2 * (mblocks * nblocks - big); // small tiles inside the last 256 x 256 ones, then the strip
+    if (first < end) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (no load is in flight, but only the chain's loop knows that)
+    for (int s = first; s < end; s += stride) {
+        lds_barrier(); // every wave is past the tile before: the ring and the staging areas are free
+        const int t = xcd_remap(s, small);
         if (t < halves) {
             wk_tile_coords(big + (t >> 1), mblocks, nblocks, mblk, nblk);
             mblk = mblk * 2 + (t & 1);
@@ -572,6 +698,7 @@ __global__ __launch_bounds__(512) void gemm_wk_big_kernel(const uint8_t* h_A, co
         wk_tile<4, W4, EPI, 2, false>(g, lds_raw, 0, mblk, nblk, 0, 1, 0, KB);
     }
 }
+
 // Second half of a K-split launch.  Workgroup = one wave = what one wave of gemm_wk_kernel kept of an output tile:
 // blockIdx.x = tile * 8 + wave.  Adds the ksplit partial tiles and runs the epilogue.
 template <int TM, bool W4, int EPI>
@@ -680,7 +807,8 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
 // prologue 2.5, epilogue and stores 5 - 6, the next workgroup's start 0.6), so one big tile is cheaper
 // than two small ones (K = 4096: 58 against 2 x 33 us, int8 weights) but leaves more compute units idle in
 // the last round: the tiles of that round go as halves where that ends sooner.
-struct BigPlan { int big, small; double us, us_128; };
+// `rounds`: small tiles that a compute unit without one of the last round's big tiles multiplies; the rest go to the others.
+struct BigPlan { int big, small, rounds; double us, us_128; };
 static BigPlan big_plan(int M, int N, int K, int w_int4) {
     const int cus = compute_units() > 0 ? compute_units() : 256;
     const int nblocks = (N + 255) / 256, strip = M % 256 > 0 && M % 256 <= 128;
@@ -689,28 +817,33 @@ static BigPlan big_plan(int M, int N, int K, int w_int4) {
     // the power limit leaves, 1.4 GHz with int8 operands, 1.6 with int4 weights (which ride as 16 * code)
     const double loop = (w_int4 ? 0.35 : 0.39) * (rkh_align_up(K, RKH_K_ALIGN) / 64);
     const double t_big = 2 * loop + 9.0, t_small = loop + 8.0;
-    BigPlan best{0, 0, 1e30, (((M + 127) / 128) * (long)nblocks + cus - 1) / cus * t_small};
+    BigPlan best{0, 0, 0, 1e30, (((M + 127) / 128) * (long)nblocks + cus - 1) / cus * t_small};
     for (int k = 0; k <= 16; ++k) {
         const int big = tiles - k * 32;
         if (big < 0) break;
         const int small = 2 * (tiles - big) + strip * nblocks;
         const int q = big / cus, rem = big % cus; // rounds of big tiles; compute units with one more
         double us = (q + (rem > 0)) * t_big;
-        for (int r = 0; small;) { // rounds of small tiles on the compute units without the extra big one
+        int r = 0;
+        while (small) { // rounds of small tiles on the compute units without the extra big one
             const double t = q * t_big + ++r * t_small, after = t - (q + 1) * t_big;
             const long late = after >= 0 ? (long)(after / t_small) : 0; // ... and on the others
             if ((long)(cus - rem) * r + rem * late < small) continue;
             if (t > us) us = t;
             break;
         }
-        if (us < best.us) best = {big, small, us, best.us_128};
+        if (us < best.us) best = {big, small, r, us, best.us_128};
     }
     return best;
 }
 
 int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, rkk::BigTiles plan) {
     const int nblocks = (g.N + 255) / 256, mblocks = g.M / 256 + (g.M % 256 > 128);
-    const dim3 grid(plan.big + plan.small), block(512);
+    // A workgroup per compute unit takes tile after tile; a K of fewer steps than the look-ahead, where the loads that run ahead
+    // would have to pass over a whole tile, gets a workgroup per tile.
+    const int cus = compute_units() > 0 ? compute_units() : 256, total = plan.big + plan.small;
+    const bool chained = rkh_align_up(g.K, RKH_K_ALIGN) >= 512 && total > cus;
+    const dim3 grid(chained ? cus : total), block(512);
     mark(st, "gemm_wk_big_kernel");
 #define RK_WKB(W4, EPI)                                                                             \
     do {                                                                                            \
@@ -724,7 +857,7 @@ int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, rkk::BigTiles pla
             opted_in[dev].store(true, std::memory_order_release);                                   \
         }                                                                                           \
         hipLaunchKernelGGL((gemm_wk_big_kernel<W4, EPI>), grid, block, WK_LDS_BYTES, st,           \
-                           g.A, g.W, g.M, g.K, mblocks, nblocks, plan.big, g);                      \
+                           g.A, g.W, g.M, g.K, mblocks, nblocks, plan.big, plan.small, chained ? plan.rounds : 0, g);                      \
     } while (0)
     switch (g.epilogue) {
     case RKH_EPI_I32: if (g.w_int4) RK_WKB(true, RKH_EPI_I32); else RK_WKB(false, RKH_EPI_I32); break;
@@ -789,13 +922,13 @@ int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g, int tile_rows)
 }
 BigTiles wk_big_tiles(int M, int N, int K, int w_int4) {
     const BigPlan plan = big_plan(M, N, K, w_int4);
-    return {plan.big, plan.small};
+    return {plan.big, plan.small, plan.rounds};
 }
 bool wk_big_applies(int M, int N, int K, int w_int4, BigTiles* tiles) {
     // (as many tiles of 128 x 256 as compute units run in one round: nothing to gain, and other plans may be better still)
     if ((M + 127) / 128 * (long)((N + 255) / 256) <= (compute_units() > 0 ? compute_units() : 256)) return false;
     const BigPlan plan = big_plan(M, N, K, w_int4);
-    *tiles = {plan.big, plan.small};
+    *tiles = {plan.big, plan.small, plan.rounds};
     return plan.big > 0 && plan.us < plan.us_128;
 }
 int launch_gemm_wk_big(hipStream_t st, const rkh_gemm_args& g, BigTiles tiles) { return ::launch_gemm_wk_big(st, g, tiles); }

@@ -129,3 +129,52 @@ def test_other_kernels_and_compiler_loads_are_ignored():
     # a load the compiler issued itself (outside an asm block) is the compiler's business
     body = "	global_load_dwordx4 v[10:13], v1, s[2:3]\n	s_waitcnt vmcnt(0)\n	v_mov_b32_e32 v1, v10"
     assert audit_waits.audit_text(_kernel(body)) == ([], 1)
+
+
+# products from inline assembly: the compiler puts no wait states around them
+MFMA_OK = """
+	v_and_b32_e32 v10, 0xf0f0f0f0, v5
+	s_nop 1
+	;;#ASMSTART
+	v_mfma_i32_16x16x64_i8 v[20:23], v[10:13], v[40:43], v[20:23]
+	;;#ASMEND
+	;;#ASMSTART
+	v_mfma_i32_16x16x64_i8 v[20:23], v[14:17], v[40:43], v[20:23]
+	;;#ASMEND
+	s_nop 7
+	s_nop 7
+	v_add_u32_e32 v50, v20, v51
+"""
+
+
+def test_products_with_their_wait_states_are_accepted():
+    assert audit_waits.audit_text(_kernel(MFMA_OK)) == ([], 1)
+
+
+def test_an_operand_written_just_ahead_of_a_product_is_flagged():
+    found, _ = audit_waits.audit_text(_kernel(MFMA_OK.replace("	s_nop 1\n", "")))
+    assert found and "writes an operand" in found[0]
+
+
+def test_a_sum_read_just_behind_a_product_is_flagged():
+    found, _ = audit_waits.audit_text(_kernel(MFMA_OK.replace("	s_nop 7\n	s_nop 7\n", "	s_nop 3\n")))
+    assert found and "touches the result" in found[0]
+
+
+# LDS reads complete in order: a counted wait covers the older one
+def test_counted_waits_for_lds_reads():
+    body = """
+	;;#ASMSTART
+	ds_read_b128 v[10:13], v1 offset:0
+	;;#ASMEND
+	;;#ASMSTART
+	ds_read_b128 v[14:17], v1 offset:256
+	;;#ASMEND
+	;;#ASMSTART
+	s_waitcnt lgkmcnt(1)
+	;;#ASMEND
+	v_mov_b32_e32 v50, v%d
+"""
+    assert audit_waits.audit_text(_kernel(body % 10))[0] == []
+    found, _ = audit_waits.audit_text(_kernel(body % 14))
+    assert found and "v[14:17]" in found[0]

@@ -77,3 +77,25 @@ def test_int4_weights(sess, oracle, one_piece, M, N, K, kind):
     finally:
         ws.close()
         w.close()
+
+
+# A workgroup multiplies several 256 x 256 tiles as one stream of steps, then its share of the small ones: two and five trips of the
+# loop per tile, three rounds with a last one of which some workgroups have no large tile
+@pytest.mark.parametrize("M,N,K", [(4700, 8200, 512), (3000, 14336, 1100)])
+@pytest.mark.parametrize("int4", [False, True])
+def test_several_tiles_of_a_workgroup(sess, oracle, one_piece, M, N, K, int4):
+    if int4:
+        c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
+        w, ws = ops.W4A8Weights(sess, c["B"], c["w_scale"]), ops.W4A8Workspace(sess, M, N, K)
+        (rc, got), kernels = one_piece(lambda: ws.run_f16(w, c["A"]))
+        want = oracle.w4a8(c["A"], c["B"], c["w_scale"])["C"]
+        ws.close()
+        w.close()
+    else:
+        c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
+        op = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, M, c["B"], c["w_scale"])
+        (rc, got), kernels = one_piece(lambda: op.run(c["A"]))
+        want = oracle.w8a8(c["A"], c["B"], c["w_scale"])["C"]
+        op.close()
+    assert rc == 0 and kernels[-1] == "gemm_wk_big_kernel"
+    assert np.array_equal(got.view(np.uint16), np.asarray(want).view(np.uint16))
