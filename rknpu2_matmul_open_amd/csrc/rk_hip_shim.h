@@ -178,6 +178,9 @@ typedef struct rkh_gemm_args {
     const uint8_t* W4;
     int int4_experts;
     size_t w4_expert_stride;
+    /* Set by rkh_quant_gemm alone: int8 rows [M, K] that the kernel multiplies in the place of A, into
+     * which it writes their tiles. */
+    const uint8_t* A_rows;
 } rkh_gemm_args;
 int rkh_gemm(void* stream, const rkh_gemm_args* args);
 /* quantize + GEMM as one request: for decode-sized M the quantization is fused

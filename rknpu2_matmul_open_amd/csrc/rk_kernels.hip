@@ -1760,6 +1760,15 @@ int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_arg
     // (int8 rows of 9..128-row calls: letting the streaming kernel read them from their row-major source
     // instead of a tiled copy saves the re-tiling launch but was slower -- a lane's 16 bytes then come from
     // 32 different cache lines per load: 128 x 4096 x 11008 26.8 -> 35.7 us, 128 x 11008 x 4096 25.3 -> 29.7.)
+    // Exact products on narrow tiles of the LDS-ring kernel take the caller's rows in whole lines (wk_tile, RAW).
+    if (qargs->mode == RKH_Q_COPY_I8 && qargs->in_dtype == RKH_I8 && !qargs->src_is_host && qargs->M > 0) {
+        const GemmRoute r = gemm_route(*gargs);
+        if (r.kernel == RKH_GEMM_TILES_NARROW && rkk::wk_takes_rows(*gargs, qargs->src, r.tile)) {
+            rkh_gemm_args g = *gargs;
+            g.A_rows = static_cast<const uint8_t*>(qargs->src);
+            return launch_gemm_wk_narrow((hipStream_t)stream, g, r.tile);
+        }
+    }
     const int rc = qargs->M > 0 ? launch_quant(stream, qargs, quant_plan(*qargs, true)) : RKH_OK;
     return rc ? rc : rkh_gemm(stream, gargs);
 }

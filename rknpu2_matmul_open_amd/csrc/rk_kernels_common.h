@@ -47,6 +47,7 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int tile_rows, int ks
 // rk_kernels_stream.hip
 int launch_gemm_grouped(hipStream_t st, const rkh_gemm_args& g);
 int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g, int tile_rows);
+bool wk_takes_rows(const rkh_gemm_args& g, const void* rows, int tile_rows); // ... with the caller's int8 rows in g.A_rows
 // rk_kernels_few.hip: columns of a workgroup (16 / 32), or 0 where another kernel is better
 int few_cols(const rkh_gemm_args& g);
 int launch_gemm_few(hipStream_t st, const rkh_gemm_args& g, int cols);

@@ -233,6 +233,7 @@ template <int OFF> __device__ __forceinline__ void read_lds(v4i& x, uint32_t add
 template <int OFF> __device__ __forceinline__ void load_regs(v4i& x, unsigned lane_off, const uint8_t* base) {
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(x) : "v"(lane_off), "s"(base), "n"(OFF));
 }
+__device__ __forceinline__ void load_far(v4i& x, const uint8_t* src) { asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(x) : "v"(src)); }
 // The product as an asm statement, for the chained tiles: sums stay in one place (left to itself the compiler rotates 128
 // sums through the register file, and with the next tile's weights beside them spills some around the tile's first products).
 // What the compiler then does not order: a vector instruction that writes an operand has to be two wait states ahead
@@ -322,14 +323,23 @@ template <int P, int STEP> struct WkAt { static constexpr int PRIO = P, AT = STE
 // The tiles that a workgroup of gemm_wk_big_kernel multiplies one after the other: v, v + stride, .. below `big`.
 struct WkChain { int v, stride, big, mblocks, nblocks; };
 
-template <int TM, bool W4, int EPI, int TN, bool RS>
+// RAW: the activations are the caller's int8 rows (g.A_rows, rows and K of 16-byte pieces), not tiles of them.  A copy then brings whole
+// 128-byte lines, 4 or 8 rows of one step; piece p of a row lies in slot p ^ swizzle(row) of the row's 16 or 8, so that the 16
+// rows of an operand, which are a multiple of 128 bytes apart, are read from 16 different places.  The tiles that the call owes its
+// caller (g.A) are written by the workgroups of a row block together, up to RAW_TILES per wave: fetched behind the
+// prologue, stored behind the loop.  Without the re-tiling launch in front, us: exact
+// 128 x 4096 x 11008 13.6 -> 12.1, 512 x 4096 x 4096 15.3 -> 13.2, 1000 x 2048 x 4096 15.4 -> 13.1, 300 x 14336 x 4096 38.2 -> 33.4.
+constexpr int RAW_TILES = 4;
+
+template <int TM, bool W4, int EPI, int TN, bool RS, bool RAW = false>
 __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw, int tile, int mblk, int nblk, int kpart,
                                         int ksplit, int kt0, int kts, // the part's first k-tile and their number, a multiple of 8
                                         [[maybe_unused]] WkChain chain = {}) {
     using S = WkShape<TM, W4, TN, RS>;
+    static_assert(!RAW || (!RS && !W4 && EPI == RKH_EPI_I32 && S::NC == 2), "int8 rows as given: the exact product on narrow tiles");
     static_assert(TN == 2 || (TN == 1 && EPI != RKH_EPI_SWIGLU), "gate / up pairs need two column blocks per wave");
     constexpr int U = S::U, RM = S::RM, CN = S::CN, KT = S::KT, BUF = S::BUF, NBUF = S::NBUF, NSW = S::NSW;
-    constexpr int A_STEP = KT * 1024, W_STEP = KT * (W4 ? 512 : 1024);
+    constexpr int A_STEP = RAW ? KT * 32 : KT * 1024, W_STEP = KT * (W4 ? 512 : 1024);
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
@@ -342,7 +352,7 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     const auto w_from = [&](int nb, int j) { // (int4: two k-tiles per KiB)
         return g.W + ((size_t)(nb * (4 * TN) + wn * TN + j) * KB + kt0 + (RS ? 0 : wk * 2 * U)) * (W4 ? 512 : 1024);
     };
-    const uint8_t* asrc = a_from(mblk);
+    const uint8_t* asrc = RAW ? g.A_rows + (size_t)(mblk * S::BM) * g.K : a_from(mblk);
     const uint8_t* wsrc[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) wsrc[j] = w_from(nblk, j);
@@ -355,7 +365,29 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     uint32_t frag_lo = lds_base + (RS ? wk * (RM / 2) * KT : wk * 2 * U) * 1024 + (W4 ? piece_off + (q >> 1) * 1024 : piece_off);
     uint32_t frag_hi = frag_lo + 65536;
     const int ksteps = kts / KT;
-    int a_left = ksteps - 1, w_left = ksteps - 1; // how often the sources may still advance
+    // RAW: this lane's places in the rows of the step's two copies, the same for the step that K ends in (pieces beyond K: the row's
+    // first, any would do -- the weights there are zero), and its first piece of the operands of each unit of a step
+    constexpr int PIECES = KT * 2, COPY_ROWS = 64 / PIECES, SWIZZLE = PIECES == 16 ? 0 : 1; // swizzle(row) = row >> SWIZZLE, modulo PIECES
+    [[maybe_unused]] unsigned row_off[2], row_off_end[2];
+    [[maybe_unused]] uint32_t raw_lo[U], raw_hi[U];
+    if constexpr (RAW) {
+        const unsigned in_step = (g.K - 1) % (KT * 32) + 1; // k of the last step with any
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int row = (wave * 2 + c) * COPY_ROWS + lane / PIECES;
+            const unsigned piece = ((lane % PIECES) ^ (row >> SWIZZLE)) % PIECES;
+            row_off[c] = (unsigned)min(row, g.M - 1 - mblk * S::BM) * (unsigned)g.K + piece * 16;
+            row_off_end[c] = piece * 16 < in_step ? row_off[c] : row_off[c] - piece * 16;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int r = lane & 15, piece = ((wk * 4 * U + u * 4 + q) ^ (r >> SWIZZLE)) % PIECES;
+            raw_lo[u] = lds_base + r * (PIECES * 16) + piece * 16;
+            raw_hi[u] = raw_lo[u] + 65536;
+        }
+    }
+    // how often the sources may still advance (RAW: rows end with K, which a step of 128 k may lie beyond)
+    int a_left = (RAW ? (g.K + KT * 32 - 1) / (KT * 32) : ksteps) - 1, w_left = ksteps - 1;
     // RS: where they go from there, the chain's next tile or, behind the last, nowhere
     [[maybe_unused]] const uint8_t *a_next = nullptr, *w_next[TN] = {};
     [[maybe_unused]] int a_step = A_STEP, w_step = W_STEP, mblk_next = 0, nblk_next = 0;
@@ -385,13 +417,14 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     // Copies beyond K are issued like the others, for the count.  Tiles of 64 x 128 with int8 weights, which are bound by
     // the compute unit's memory path, issue them for one lane: three steps of 16 KiB that nothing reads, beside the 16 of
     // K = 4096 (exact 128 x 4096 x 11008 13.9 -> 13.65 us, 512 x 4096 x 4096 16.5 -> 16.3; int4 weights and wider tiles gain nothing).
-    constexpr bool MASKED = TM == 2 && TN == 1 && !W4;
+    constexpr bool MASKED = (TM == 2 && TN == 1 && !W4) || RAW;
     [[maybe_unused]] unsigned long long a_lanes = ~0ull;
     auto copy_a = [&](auto buf_tag, auto c_tag, auto at_tag) { // one of the step's copies
         constexpr int C = decltype(c_tag)::value, PRIO = decltype(at_tag)::PRIO;
         constexpr int B = decltype(buf_tag)::value % NBUF, PER = 65536 / BUF;
         const uint32_t dst = (B < PER ? copy_lo : copy_hi) + B % PER * BUF;
-        if constexpr (MASKED) copy_lds<C * 1024, PRIO>(lane_off, asrc, dst, a_lanes);
+        if constexpr (RAW) copy_lds<0, PRIO>(a_left > 0 ? row_off[C & 1] : row_off_end[C & 1], asrc, dst + C * 1024, a_lanes);
+        else if constexpr (MASKED) copy_lds<C * 1024, PRIO>(lane_off, asrc, dst, a_lanes);
         else copy_lds<C * 1024, PRIO>(lane_off, asrc, dst);
         // RS: a trip turns to the next tile behind one of its steps (a choice behind every step cost the loop 2.5 %)
         if constexpr (C == S::NC - 1 && RS && decltype(at_tag)::AT >= 0 && decltype(at_tag)::AT != S::A_TURN) {
@@ -429,7 +462,8 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     };
     auto read_a = [&](auto unit_tag, auto i_tag) { // operand i of a unit of the trip; awaited by wait_lds
         constexpr int UNIT = decltype(unit_tag)::value, I = decltype(i_tag)::value, B = UNIT / U % NBUF, PER = 65536 / BUF;
-        read_lds<B % PER * BUF + (I / 2) * KT * 1024 + (UNIT % U) * (W4 ? 1024 : 2048) + (I & 1) * 256>(a[I], B < PER ? frag_lo : frag_hi);
+        if constexpr (RAW) read_lds<B % PER * BUF + I * (PIECES * 256)>(a[I], B < PER ? raw_lo[UNIT % U] : raw_hi[UNIT % U]);
+        else read_lds<B % PER * BUF + (I / 2) * KT * 1024 + (UNIT % U) * (W4 ? 1024 : 2048) + (I & 1) * 256>(a[I], B < PER ? frag_lo : frag_hi);
     };
     auto unpack = [&](v4i* dst, const v4i* raw, auto half_tag, auto e_tag) { // k-tile HALF of each super-tile
         if constexpr (W4) {
@@ -510,8 +544,25 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
         }
     };
     fetch_scales(WK_SCALES_OFF);
+    // RAW: this wave's tiles of the caller's copy, tile `kb` of the row block `rb` of this workgroup's rows
+    [[maybe_unused]] v4i copied[RAW_TILES];
+    [[maybe_unused]] const auto raw_tile = [&](int t, auto&& f) { // f(source, destination) for this lane's 16 bytes if there are any
+        const int tiles = S::BM / 32 * KB, nb = (g.N + 128 * TN - 1) / (128 * TN), per = (tiles + nb - 1) / nb;
+        const int mine = wave + 8 * t, tile_of = nblk * per + mine;
+        const int rb = tile_of / KB, kb = tile_of - rb * KB, m = mblk * S::BM + rb * 32 + (lane & 31), k = kb * 32 + (lane >> 5) * 16;
+        if (mine < per && tile_of < tiles && m < g.M && k < g.K)
+            f(g.A_rows + (size_t)m * g.K + k, const_cast<uint8_t*>(g.A) + ((size_t)(mblk * (S::BM / 32) + rb) * KB + kb) * 1024 + lane * 16);
+    };
+    if constexpr (RAW) {
+#pragma unroll
+        for (int t = 0; t < RAW_TILES; ++t) {
+            const uint8_t* from = g.A_rows; // (every wave issues every load, for the count)
+            raw_tile(t, [&](const uint8_t* src, uint8_t*) { from = src; });
+            load_far(copied[t], from);
+        }
+    }
     if constexpr (RS) find_next(); // (while the first loads are on their way)
-    w_wait(wring[0], std::integral_constant<int, S::prologue_since() + (EPI != RKH_EPI_I32 ? 2 : 0)>{}); // weights of unit 0 and the copies of steps 0..G have landed
+    w_wait(wring[0], std::integral_constant<int, S::prologue_since() + (EPI != RKH_EPI_I32 ? 2 : 0) + (RAW ? RAW_TILES : 0)>{}); // weights of unit 0 and the copies of steps 0..G have landed
     asm volatile("s_barrier" ::: "memory");
     const auto first_operands = [&]() {
         static_for<RM>([&](auto i_tag) { read_a(std::integral_constant<int, 0>{}, i_tag); });
@@ -598,6 +649,13 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     for (int t = 0; t < NSW; ++t)
 #pragma unroll
         for (int e = 0; e < CN; ++e) keep(wring[t][e]);
+    if constexpr (RAW) {
+#pragma unroll
+        for (int t = 0; t < RAW_TILES; ++t) {
+            keep(copied[t]);
+            raw_tile(t, [&](const uint8_t*, uint8_t* dst) { *reinterpret_cast<v4i*>(dst) = copied[t]; });
+        }
+    }
     lds_barrier();
 
     // The k-halves meet: a wave hands half of the rows of its strip to its partner and keeps operands wk * RM / 2 ..
@@ -631,7 +689,7 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
 }
 
 // The tile of a workgroup: XCD-contiguous ranges, 4 row blocks per column sweep.
-template <int TM, bool W4, int EPI, int TN = 2>
+template <int TM, bool W4, int EPI, int TN = 2, bool RAW = false>
 __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const uint8_t* h_W, int h_M, int h_K,
                                                       int mblocks, int nblocks, int ksplit, int units_per_part,
                                                       rkh_gemm_args g) {
@@ -648,7 +706,7 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
     int mblk, nblk;
     wk_tile_coords(tile, mblocks, nblocks, mblk, nblk);
     const int first = kpart * units_per_part; // (at least one unit by construction of the launch)
-    wk_tile<TM, W4, EPI, TN, false>(g, lds_raw, tile, mblk, nblk, kpart, ksplit, first * (WK_PART_K / 32),
+    wk_tile<TM, W4, EPI, TN, false, RAW>(g, lds_raw, tile, mblk, nblk, kpart, ksplit, first * (WK_PART_K / 32),
                                     min(units_per_part, units - first) * (WK_PART_K / 32));
 }
 
@@ -881,29 +939,32 @@ int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g) {
     const int units = (int)(rkh_align_up(g.K, RKH_K_ALIGN) / WK_PART_K);
     const dim3 grid(mblocks * nblocks), block(512);
     mark(st, TM == 2 ? "gemm_wk_kernel<64 x 128>" : "gemm_wk_kernel<128 x 128>");
-#define RK_WKN(W4, EPI)                                                                             \
+#define RK_WKN(W4, EPI, RAW)                                                                        \
     do {                                                                                            \
         static std::atomic<bool> opted_in[64] = {};                                                 \
         int dev = 0;                                                                                \
         RKH_CHECK(hipGetDevice(&dev));                                                              \
         if (dev < 0 || dev >= 64) return RKH_ERR_RUNTIME;                                           \
         if (!opted_in[dev].load(std::memory_order_acquire)) {                                       \
-            RKH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wk_kernel<TM, W4, EPI, TN>), \
+            RKH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wk_kernel<TM, W4, EPI, TN, RAW>), \
                                           hipFuncAttributeMaxDynamicSharedMemorySize, WK_LDS_BYTES)); \
             opted_in[dev].store(true, std::memory_order_release);                                   \
         }                                                                                           \
-        hipLaunchKernelGGL((gemm_wk_kernel<TM, W4, EPI, TN>), grid, block, WK_LDS_BYTES, st,       \
+        hipLaunchKernelGGL((gemm_wk_kernel<TM, W4, EPI, TN, RAW>), grid, block, WK_LDS_BYTES, st,       \
                            g.A, g.W, g.M, g.K, mblocks, nblocks, 1, units, g);               \
     } while (0)
     // (int4 weights: the 64-row tiles only -- the 128-row ones measured slower than the other plans everywhere)
 #define RK_WKN_W(EPI)                                                                               \
     do {                                                                                            \
-        if (!g.w_int4) RK_WKN(false, EPI);                                                          \
-        else if constexpr (TM == 2) RK_WKN(true, EPI);                                              \
+        if (!g.w_int4) RK_WKN(false, EPI, false);                                                   \
+        else if constexpr (TM == 2) RK_WKN(true, EPI, false);                                            \
         else return RKH_ERR_RUNTIME;                                                                \
     } while (0)
     switch (g.epilogue) {
-    case RKH_EPI_I32: RK_WKN_W(RKH_EPI_I32); break;
+    case RKH_EPI_I32:
+        if (g.A_rows && !g.w_int4) RK_WKN(false, RKH_EPI_I32, true);
+        else RK_WKN_W(RKH_EPI_I32);
+        break;
     case RKH_EPI_F16: RK_WKN_W(RKH_EPI_F16); break;
     case RKH_EPI_F32: RK_WKN_W(RKH_EPI_F32); break;
     default: return RKH_ERR_RUNTIME;
@@ -917,6 +978,13 @@ int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g) {
 } // namespace
 
 namespace rkk {
+// (the tiles owed to the caller are written a few per wave, at most RAW_TILES: K up to 4 N for 64 rows, 2 N for 128; a lane's
+// place in its rows is 32 bits)
+bool wk_takes_rows(const rkh_gemm_args& g, const void* rows, int tile_rows) {
+    const long nb = (g.N + 127) / 128, tiles = tile_rows / 32 * (long)(rkh_align_up(g.K, RKH_K_ALIGN) / 32);
+    return !g.w_int4 && g.epilogue == RKH_EPI_I32 && g.K % 16 == 0 && reinterpret_cast<uintptr_t>(rows) % 16 == 0 && g.K <= 1 << 24 &&
+           (tiles + nb - 1) / nb <= 8 * RAW_TILES;
+}
 int launch_gemm_wk_narrow(hipStream_t st, const rkh_gemm_args& g, int tile_rows) {
     return tile_rows == 128 ? ::launch_gemm_wk_narrow<4>(st, g) : ::launch_gemm_wk_narrow<2>(st, g);
 }

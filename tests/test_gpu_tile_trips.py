@@ -57,3 +57,30 @@ def test_int4_weights(sess, oracle, one_piece, M, N, K, epi, kernel, rows):
     finally:
         ws.close()
         w.close()
+
+
+# Exact products of 64- and 128-row tiles read the caller's int8 rows where these allow 16-byte pieces: K that ends in a step's
+# first piece, at its end and, with steps of 128 k, one whole step before the padded end; a last row block of one row
+@pytest.mark.parametrize("K", [16, 128, 144, 256, 272, 1040, 1536, 40])
+@pytest.mark.parametrize("M,N,rows,offset", [(129, 4100, 64, 0), (129, 4100, 64, 16), (129, 4100, 64, 4), (1000, 2500, 128, 0), (897, 2500, 128, 32)])
+def test_rows_as_given(sess, oracle, M, N, K, rows, offset):
+    assert _route(M, N, K, 0, I32) == (NARROW, rows)
+    rng = np.random.default_rng(K + M)
+    A, B = rng.integers(-128, 128, (M, K)).astype(np.int8), rng.integers(-128, 128, (K, N)).astype(np.int8)
+    op = ops.W8A8Linear(sess, capi.I8I8I32, M, B)
+    base = sess.to_device(np.concatenate([np.zeros(offset, np.int8), A.reshape(-1)]))
+    dC = sess.empty_device(M * N * 4)
+    try:
+        kernels = [name for name, _ in ops.profile_kernels(sess, lambda: op.run_device(base + offset, dC), 1, 1)]
+        assert ("quant_rows_kernel" in kernels) == (K % 16 != 0 or offset % 16 != 0), kernels
+        want = oracle.gemm_i8(A, B)
+        assert np.array_equal(sess.from_device(dC, (M, N), np.int32), want)
+        q, s = np.empty((M, K), np.int8), np.empty(M, np.float32)
+        assert sess.lib.rk_npu_matmul_workspace_read_quantized(op.ws, capi.ptr(q), capi.ptr(s)) == 0
+        assert np.array_equal(q, A)
+        assert sess.lib.rk_npu_matmul_workspace_rerun_gemm_device(op.ws, op.w, dC) == 0 and sess.sync() == 0
+        assert np.array_equal(sess.from_device(dC, (M, N), np.int32), want)
+    finally:
+        sess.free_device(base)
+        sess.free_device(dC)
+        op.close()
