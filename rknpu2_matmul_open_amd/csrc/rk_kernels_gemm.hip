@@ -328,7 +328,7 @@ struct WkChain { int v, stride, big, mblocks, nblocks; };
 // rows of an operand, which are a multiple of 128 bytes apart, are read from 16 different places.  The tiles that the call owes its
 // caller (g.A) are written by the workgroups of a row block together, up to RAW_TILES per wave: fetched behind the
 // prologue, stored behind the loop.  Without the re-tiling launch in front, us: exact
-// 128 x 4096 x 11008 13.6 -> 12.1, 512 x 4096 x 4096 15.3 -> 13.2, 1000 x 2048 x 4096 15.4 -> 13.1, 300 x 14336 x 4096 38.2 -> 33.4.
+// 128 x 4096 x 11008 13.6 -> 11.8, 512 x 4096 x 4096 15.3 -> 12.8, 1000 x 2048 x 4096 15.4 -> 13.1, 300 x 14336 x 4096 38.2 -> 33.6.
 constexpr int RAW_TILES = 4;
 
 template <int TM, bool W4, int EPI, int TN, bool RS, bool RAW = false>
@@ -546,23 +546,29 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     fetch_scales(WK_SCALES_OFF);
     // RAW: this wave's tiles of the caller's copy, tile `kb` of the row block `rb` of this workgroup's rows
     [[maybe_unused]] v4i copied[RAW_TILES];
+    [[maybe_unused]] const int raw_all = S::BM / 32 * KB, raw_nb = (g.N + 128 * TN - 1) / (128 * TN), raw_per = (raw_all + raw_nb - 1) / raw_nb;
+    [[maybe_unused]] const bool raw_many = RAW && raw_per > 8; // (more than one per wave; loads that bring nothing cost 0.3 us)
     [[maybe_unused]] const auto raw_tile = [&](int t, auto&& f) { // f(source, destination) for this lane's 16 bytes if there are any
-        const int tiles = S::BM / 32 * KB, nb = (g.N + 128 * TN - 1) / (128 * TN), per = (tiles + nb - 1) / nb;
-        const int mine = wave + 8 * t, tile_of = nblk * per + mine;
+        const int mine = wave + 8 * t, tile_of = nblk * raw_per + mine;
         const int rb = tile_of / KB, kb = tile_of - rb * KB, m = mblk * S::BM + rb * 32 + (lane & 31), k = kb * 32 + (lane >> 5) * 16;
-        if (mine < per && tile_of < tiles && m < g.M && k < g.K)
+        if (mine < raw_per && tile_of < raw_all && m < g.M && k < g.K)
             f(g.A_rows + (size_t)m * g.K + k, const_cast<uint8_t*>(g.A) + ((size_t)(mblk * (S::BM / 32) + rb) * KB + kb) * 1024 + lane * 16);
     };
+    [[maybe_unused]] const auto raw_fetch = [&](int t) {
+        const uint8_t* from = g.A_rows; // (every lane loads, for the count)
+        raw_tile(t, [&](const uint8_t* src, uint8_t*) { from = src; });
+        load_far(copied[t], from);
+    };
+    if constexpr (RS) find_next(); // (while the first loads are on their way)
     if constexpr (RAW) {
+        raw_fetch(0);
+        if (raw_many) {
 #pragma unroll
-        for (int t = 0; t < RAW_TILES; ++t) {
-            const uint8_t* from = g.A_rows; // (every wave issues every load, for the count)
-            raw_tile(t, [&](const uint8_t* src, uint8_t*) { from = src; });
-            load_far(copied[t], from);
+            for (int t = 1; t < RAW_TILES; ++t) raw_fetch(t);
         }
     }
-    if constexpr (RS) find_next(); // (while the first loads are on their way)
-    w_wait(wring[0], std::integral_constant<int, S::prologue_since() + (EPI != RKH_EPI_I32 ? 2 : 0) + (RAW ? RAW_TILES : 0)>{}); // weights of unit 0 and the copies of steps 0..G have landed
+    // weights of unit 0 and the copies of steps 0..G land (RAW: one load or RAW_TILES behind them, the count of one)
+    w_wait(wring[0], std::integral_constant<int, S::prologue_since() + (EPI != RKH_EPI_I32 ? 2 : 0) + (RAW ? 1 : 0)>{});
     asm volatile("s_barrier" ::: "memory");
     const auto first_operands = [&]() {
         static_for<RM>([&](auto i_tag) { read_a(std::integral_constant<int, 0>{}, i_tag); });
@@ -650,10 +656,14 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
 #pragma unroll
         for (int e = 0; e < CN; ++e) keep(wring[t][e]);
     if constexpr (RAW) {
-#pragma unroll
-        for (int t = 0; t < RAW_TILES; ++t) {
+        const auto raw_store = [&](int t) {
             keep(copied[t]);
             raw_tile(t, [&](const uint8_t*, uint8_t* dst) { *reinterpret_cast<v4i*>(dst) = copied[t]; });
+        };
+        raw_store(0);
+        if (raw_many) {
+#pragma unroll
+            for (int t = 1; t < RAW_TILES; ++t) raw_store(t);
         }
     }
     lds_barrier();
