@@ -881,8 +881,9 @@ static BigPlan big_plan(int M, int N, int K, int w_int4) {
     const int cus = compute_units() > 0 ? compute_units() : 256;
     const int nblocks = (N + 255) / 256, strip = M % 256 > 0 && M % 256 <= 128;
     const int tiles = (M / 256 + (M % 256 > 128)) * nblocks;
-    // microseconds per 64 k of a 128 x 256 tile with every compute unit at work: 554 - 580 cycles at the clock that
-    // the power limit leaves, 1.4 GHz with int8 operands, 1.6 with int4 weights (which ride as 16 * code)
+    // microseconds per 64 k of a 128 x 256 tile with every compute unit at work, at the clock that the power limit leaves.
+    // (Times of the loop on 32x32x32 products, a tenth longer throughout than now; what decides is their ratio to the fixed
+    // part, and forced plans are ahead of this choice nowhere: 23 dense shapes of 160 - 1500 rows and six of the FFN, all within 2 %.)
     const double loop = (w_int4 ? 0.35 : 0.39) * (rkh_align_up(K, RKH_K_ALIGN) / 64);
     const double t_big = 2 * loop + 9.0, t_small = loop + 8.0;
     BigPlan best{0, 0, 0, 1e30, (((M + 127) / 128) * (long)nblocks + cus - 1) / cus * t_small};

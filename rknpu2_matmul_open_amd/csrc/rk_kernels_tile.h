@@ -1,5 +1,5 @@
-// The 32 x 32 accumulator tile of v_mfma_i32_32x32x32_i8 as the MFMA kernels hold it, and the
-// epilogues that turn it into output: shared by rk_kernels_gemm.hip and rk_kernels_stream.hip.
+// The 32 x 32 accumulator tile of v_mfma_i32_32x32x32_i8 as gemm_stream_kernel holds it, and the epilogues that turn it into
+// output; the LDS barrier of rk_kernels_gemm.hip, too, whose 16 x 16 tiles have epilogues of their own.
 #ifndef RK_KERNELS_TILE_H
 #define RK_KERNELS_TILE_H
 
@@ -75,17 +75,6 @@ __device__ __forceinline__ void store_tile(T* C, int ldc, int m0, int n0, int m_
     }
 }
 
-// Weight scales of the 16 columns a lane owns in the tile whose first logical
-// column is n0 (zero beyond the matrix).
-__device__ __forceinline__ void load_col_scales(float* ws, const float* w_scale, int n0, int n_limit,
-                                                int lane) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int n = n0 + tile_col(r, lane);
-        ws[r] = n < n_limit ? w_scale[n] : 0.0f;
-    }
-}
-
 // Dequantize and store one accumulator tile whose physical column block is p;
 // as / ws are the lane's row scale and its 16 column scales.
 template <int EPI>
@@ -116,20 +105,6 @@ __device__ __forceinline__ void epilogue_tile_scaled(const rkh_gemm_args& g, con
     }
 }
 
-template <int EPI>
-__device__ __forceinline__ void epilogue_tile(const rkh_gemm_args& g, const v16i& acc, int m0, int p,
-                                              int lane, const float* a_scale, const float* w_scale,
-                                              int m_limit, uint8_t* stage_lds) {
-    if (g.interleave_F ? p >= g.N / 32 : p * 32 >= g.N) return;
-    float as = 0.0f, ws[16];
-    if constexpr (EPI != RKH_EPI_I32) {
-        const int m = m0 + (lane & 31);
-        as = m < m_limit ? a_scale[m] : 0.0f;
-        load_col_scales(ws, w_scale, block_first_col(p, g.interleave_F), g.N, lane);
-    }
-    epilogue_tile_scaled<EPI>(g, acc, m0, p, lane, as, ws, m_limit, stage_lds);
-}
-
 // gate tile (physical block p, even) + up tile (p + 1) -> 32 columns of the
 // middle and one partial row maximum per (row, 32-column block).  wsg / wsu are
 // the lane's gate and up column scales.
@@ -155,21 +130,6 @@ __device__ __forceinline__ void epilogue_swiglu_scaled(const rkh_gemm_args& g, c
         bits = max(bits, (uint32_t)__shfl_xor((int)bits, 32));
         if (lane < 32 && m < m_limit) g.row_max_bits[(size_t)m * (F / 32) + (p >> 1)] = bits;
     }
-}
-
-__device__ __forceinline__ void epilogue_swiglu(const rkh_gemm_args& g, const v16i& gate,
-                                                const v16i& up, int m0, int p, int lane,
-                                                const float* a_scale, const float* w_scale,
-                                                int m_limit, uint8_t* stage_lds) {
-    const int F = g.interleave_F;
-    const int n0 = (p >> 1) * 32;
-    if (n0 >= F) return;
-    const int m = m0 + (lane & 31);
-    const float as = m < m_limit ? a_scale[m] : 0.0f;
-    float wsg[16], wsu[16];
-    load_col_scales(wsg, w_scale, n0, F, lane);
-    load_col_scales(wsu, w_scale + F, n0, F, lane);
-    epilogue_swiglu_scaled(g, gate, up, m0, p, lane, as, wsg, wsu, m_limit, stage_lds);
 }
 
 } // namespace
