@@ -1763,7 +1763,10 @@ int rkh_quant_gemm(void* stream, const rkh_quant_args* qargs, const rkh_gemm_arg
     // Exact products on narrow tiles of the LDS-ring kernel take the caller's rows in whole lines (wk_tile, RAW).
     if (qargs->mode == RKH_Q_COPY_I8 && qargs->in_dtype == RKH_I8 && !qargs->src_is_host && qargs->M > 0) {
         const GemmRoute r = gemm_route(*gargs);
-        if (r.kernel == RKH_GEMM_TILES_NARROW && rkk::wk_takes_rows(*gargs, qargs->src, r.tile)) {
+        // (a result that is written over the rows needs them copied first)
+        const uintptr_t a = reinterpret_cast<uintptr_t>(qargs->src), c = reinterpret_cast<uintptr_t>(gargs->C);
+        const bool apart = a + (size_t)gargs->M * gargs->K <= c || c + (size_t)gargs->M * gargs->ldc * 4 <= a;
+        if (apart && r.kernel == RKH_GEMM_TILES_NARROW && rkk::wk_takes_rows(*gargs, qargs->src, r.tile)) {
             rkh_gemm_args g = *gargs;
             g.A_rows = static_cast<const uint8_t*>(qargs->src);
             return launch_gemm_wk_narrow((hipStream_t)stream, g, r.tile);

@@ -84,3 +84,21 @@ def test_rows_as_given(sess, oracle, M, N, K, rows, offset):
         sess.free_device(base)
         sess.free_device(dC)
         op.close()
+
+
+def test_a_result_over_the_rows(sess, oracle):
+    """The result may be written over the rows it is made of: they are copied first then."""
+    M, N, K = 129, 4100, 512
+    rng = np.random.default_rng(7)
+    A, B = rng.integers(-128, 128, (M, K)).astype(np.int8), rng.integers(-128, 128, (K, N)).astype(np.int8)
+    op = ops.W8A8Linear(sess, capi.I8I8I32, M, B)
+    want = oracle.gemm_i8(A, B)
+    buf = sess.empty_device(M * N * 4 + 4096)
+    try:
+        for offset in (0, 1024):
+            assert sess.lib.rk_npu_hip_upload(sess.ctx, buf + offset, capi.ptr(A), A.nbytes) == 0
+            assert op.run_device(buf + offset, buf) == 0 and sess.sync() == 0
+            assert np.array_equal(sess.from_device(buf, (M, N), np.int32), want)
+    finally:
+        sess.free_device(buf)
+        op.close()
