@@ -87,8 +87,9 @@ def _instructions(lines):
 _ENDS = re.compile(r"^\s*(s_endpgm|s_branch\b|s_setpc_b64|s_trap)")
 
 
-def _blocks(instrs):
-    """Basic blocks of a function: (first, last + 1, successor block starts)."""
+def _blocks(instrs, unknown=None):
+    """Basic blocks of a function: (first, last + 1, successor block starts).  unknown: takes the branches to labels that
+    the text does not hold, whose paths nobody can follow."""
     label_at = {t[:-1]: i for i, (t, _) in enumerate(instrs) if t.endswith(":")}
     starts = {0}
     for i, (t, _) in enumerate(instrs):
@@ -107,6 +108,8 @@ def _blocks(instrs):
             target = b.group(1) or b.group(2)
             if target in label_at:
                 succ.append(label_at[target])
+            elif unknown is not None:
+                unknown.append(last.strip())
         if not _ENDS.match(last) and hi < len(instrs):
             succ.append(hi)
         blocks[lo] = (lo, hi, succ)
@@ -254,7 +257,9 @@ def _check_mfma(name, instrs, violations):
 def audit_function(name, lines):
     """Violations (strings) of one kernel's assembly."""
     instrs = _instructions(lines)
-    violations, seen = [], set()
+    violations, seen, unknown = [], set(), []
+    _blocks(instrs, unknown)
+    violations += ["%s: `%s` leads out of the kernel's text" % (name, branch) for branch in unknown]
     _check_m0(name, instrs, violations)
     _check_mfma(name, instrs, violations)
     loads = [i for i, (t, a) in enumerate(instrs) if a and (_ASM_VLOAD.match(t) or _ASM_DSREAD.match(t))]
@@ -274,16 +279,17 @@ def audit_function(name, lines):
 def audit_text(asm_text, only=("gemm_wk_kernel", "gemm_wk_big_kernel", "gemm_stream_kernel")):
     """Violations in every kernel of an assembly file whose (mangled) name contains one of `only`."""
     violations, checked = [], 0
-    lines = asm_text.splitlines()
+    lines = asm_text.splitlines() + [".Lfunc_end:"]
     start, name = None, None
     for n, line in enumerate(lines):
         m = re.match(r"^(_Z\w+):\s", line + " ")
-        if m and any(k in m.group(1) for k in only):
-            start, name = n + 1, m.group(1)
-        elif start is not None and "s_endpgm" in line:
-            violations += audit_function(name, lines[start:n + 1])
+        # (a kernel ends where its text does and not at an s_endpgm: the compiler may lay a branch's end ahead of the rest)
+        if start is not None and (m or line.startswith(".Lfunc_end")):
+            violations += audit_function(name, lines[start:n])
             checked += 1
             start = None
+        if m and any(k in m.group(1) for k in only):
+            start, name = n + 1, m.group(1)
     return violations, checked
 
 

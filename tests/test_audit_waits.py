@@ -178,3 +178,32 @@ def test_counted_waits_for_lds_reads():
     assert audit_waits.audit_text(_kernel(body % 10))[0] == []
     found, _ = audit_waits.audit_text(_kernel(body % 14))
     assert found and "v[14:17]" in found[0]
+
+
+# A branch that ends the program ahead of the rest: what lies behind its s_endpgm is part of the kernel
+EARLY_END = """
+	;;#ASMSTART
+	global_load_dwordx4 v[10:13], v1, s[2:3] offset:0
+	;;#ASMEND
+	s_cbranch_scc1 .LBB0_2
+	s_endpgm
+.LBB0_2:
+%s	v_mov_b32_e32 v50, v11
+	;;#ASMSTART
+	s_waitcnt vmcnt(0)
+	;;#ASMEND
+"""
+
+
+def test_what_lies_behind_an_early_end_is_checked():
+    wait = "	;;#ASMSTART\n	s_waitcnt vmcnt(0)\n	;;#ASMEND\n"
+    assert audit_waits.audit_text(_kernel(EARLY_END % wait) + ".Lfunc_end0:\n") == ([], 1)
+    found, checked = audit_waits.audit_text(_kernel(EARLY_END % "") + ".Lfunc_end0:\n")
+    assert checked == 1 and len(found) == 1 and "v[10:13]" in found[0] and "v_mov" in found[0]
+    # ... of each of two kernels that follow one another
+    assert audit_waits.audit_text((_kernel(EARLY_END % "") + ".Lfunc_end0:\n") * 2)[1] == 2
+
+
+def test_a_branch_out_of_the_text_is_flagged():
+    found, _ = audit_waits.audit_text(_kernel(RING_OK.replace("s_cbranch_scc1 .LBB0_1", "s_cbranch_scc1 .LBB0_7")))
+    assert any(".LBB0_7" in f for f in found)
