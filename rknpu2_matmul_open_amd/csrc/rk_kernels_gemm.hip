@@ -674,18 +674,21 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
         constexpr int KEEP = RM / 2, XT = KEEP * CN; // operands kept; tiles per exchange slot
         v4i sum[KEEP][CN];
         v4i* xch = reinterpret_cast<v4i*>(lds_raw);
-        const auto hand_over = [&](auto wk_tag) {
+        // (The comment at the end, which differs between the two branches, keeps the compiler from making one of them: it
+        // would select each accumulator with a vector instruction, 128 in a tile of 128 x 256.  From the loop to the
+        // first store 2.1 -> 1.5 us; calls, us: int4 2048 x 512 x 4096 14.2 -> 13.3, 4036 x 640 x 1920 19.1 -> 18.1, int8 786 x 661 x 8720
+        // 18.1 -> 17.3, exact 950 x 1408 x 5120 15.9 -> 15.4, the FFN 188 x 4576 x 11584 57.0 -> 55.3.)
+        const auto meet = [&](auto wk_tag) {
             constexpr int GIVE0 = (decltype(wk_tag)::value ^ 1) * KEEP, KEEP0 = decltype(wk_tag)::value * KEEP;
 #pragma unroll
             for (int t = 0; t < XT; ++t) xch[(wave * XT + t) * 64 + lane] = acc[GIVE0 + t / CN][t % CN];
+            lds_barrier();
 #pragma unroll
-            for (int t = 0; t < XT; ++t) sum[t / CN][t % CN] = acc[KEEP0 + t / CN][t % CN];
+            for (int t = 0; t < XT; ++t) sum[t / CN][t % CN] = acc[KEEP0 + t / CN][t % CN] + xch[((wave ^ 4) * XT + t) * 64 + lane];
+            asm volatile("; rows of k-half %0" ::"n"(KEEP0));
         };
-        if (wk == 0) hand_over(std::integral_constant<int, 0>{});
-        else hand_over(std::integral_constant<int, 1>{});
-        lds_barrier();
-#pragma unroll
-        for (int t = 0; t < XT; ++t) sum[t / CN][t % CN] += xch[((wave ^ 4) * XT + t) * 64 + lane];
+        if (wk == 0) meet(std::integral_constant<int, 0>{});
+        else meet(std::integral_constant<int, 1>{});
         if (ksplit > 1) { // partial tile in accumulator order: [tile][part][wave][kept tile][lane] x 4 ints
             v4i* dst = reinterpret_cast<v4i*>(g.splitk_acc) + (((size_t)tile * ksplit + kpart) * 8 + wave) * (XT * 64);
 #pragma unroll
