@@ -770,32 +770,43 @@ __global__ __launch_bounds__(512) void gemm_wk_big_kernel(const uint8_t* h_A, co
     }
 }
 
-// Second half of a K-split launch.  Workgroup = one wave = what one wave of gemm_wk_kernel kept of an output tile:
-// blockIdx.x = tile * 8 + wave.  Adds the ksplit partial tiles and runs the epilogue.
+// Second half of a K-split launch.  Workgroup = one wave = up to 32 rows of what one wave of gemm_wk_kernel kept of an output
+// tile: blockIdx.x = (tile * 8 + wave) * PARTS + part.  Adds the ksplit partial tiles and runs the epilogue.  Bound by the latency
+// of its loads, which a wave has in flight for one part of K at a time: the loads of a part go out together (left to itself the
+// compiler waited for each of them ahead of the next in the exact product of 128-row tiles), and the 64 rows that a wave of
+// the 128-row tile kept go to two waves.  us, one wave with loads as the compiler had them -> loads together -> two
+// waves: exact 737 x 10240 x 700 29.7 -> 25.1 -> 24.1, 2076 x 10240 x 512 35.8 -> 33.9 -> 33.2, 453 x 8733 x 628 (64-row tiles) 25.4 ->
+// 24.1, int8 737 x 10240 x 700 30.0 -> 29.7 -> 27.6, 1135 x 8960 x 2176 42.8 -> 43.0 -> 42.0.
 template <int TM, bool W4, int EPI>
 __global__ __launch_bounds__(64) void gemm_wk_reduce_kernel(rkh_gemm_args g, int mblocks, int nblocks, int ksplit) {
-    constexpr int TN = 2, CN = 4, BM = 32 * TM, KEEP = TM; // (rows of operands a wave keeps)
+    constexpr int TN = 2, CN = 4, BM = 32 * TM, KEEP = TM; // (operands of 16 rows that a wave kept)
+    constexpr int ROWS = KEEP > 2 ? 2 : KEEP, PARTS = KEEP / ROWS;
     __shared__ __attribute__((aligned(16))) uint8_t stage_lds[WK_STAGE];
     const int lane = lane_id();
-    const int tile = blockIdx.x / 8, wave = blockIdx.x % 8, wn = wave & 3, wk = wave >> 2;
+    const int owner = blockIdx.x / PARTS, part = blockIdx.x % PARTS;
+    const int tile = owner / 8, wave = owner % 8, wn = wave & 3, wk = wave >> 2;
     int mblk, nblk;
     wk_tile_coords(tile, mblocks, nblocks, mblk, nblk);
-    const int m0 = mblk * BM + wk * KEEP * 16, pb0 = nblk * 8 + wn * TN;
-    const v4i* src = reinterpret_cast<const v4i*>(g.splitk_acc) + ((size_t)tile * ksplit * 8 + wave) * (KEEP * CN * 64) + lane;
-    v4i sum[KEEP][CN];
+    const int m0 = mblk * BM + (wk * KEEP + part * ROWS) * 16, pb0 = nblk * 8 + wn * TN;
+    const v4i* src = reinterpret_cast<const v4i*>(g.splitk_acc) + ((size_t)tile * ksplit * 8 + wave) * (KEEP * CN * 64) + part * (ROWS * CN * 64) + lane;
+    v4i sum[ROWS][CN];
 #pragma unroll
-    for (int t = 0; t < KEEP * CN; ++t) sum[t / CN][t % CN] = v4i{0, 0, 0, 0};
+    for (int t = 0; t < ROWS * CN; ++t) sum[t / CN][t % CN] = v4i{0, 0, 0, 0};
     for (int p = 0; p < ksplit; ++p, src += 8 * KEEP * CN * 64) {
         // int4 weights ride as 16 * code: a part's sum is an exact multiple of 16 that fits
         // int32 (a part spans at most 2^17 k), but the sum of the parts times 16 need not --
         // so the factor comes off each part before it is added
+        v4i got[ROWS * CN];
 #pragma unroll
-        for (int t = 0; t < KEEP * CN; ++t) sum[t / CN][t % CN] += src[t * 64] >> (W4 ? 4 : 0);
+        for (int t = 0; t < ROWS * CN; ++t) got[t] = src[t * 64];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < ROWS * CN; ++t) sum[t / CN][t % CN] += got[t] >> (W4 ? 4 : 0);
     }
-    float as[KEEP], ws[CN][4];
+    float as[ROWS], ws[CN][4];
     if constexpr (EPI != RKH_EPI_I32) {
 #pragma unroll
-        for (int i = 0; i < KEEP; ++i) {
+        for (int i = 0; i < ROWS; ++i) {
             const int m = m0 + 16 * i + (lane & 15);
             as[i] = m < g.M ? g.a_scale[m] : 0.0f;
         }
@@ -808,7 +819,7 @@ __global__ __launch_bounds__(64) void gemm_wk_reduce_kernel(rkh_gemm_args g, int
                 ws[j][e] = live ? g.w_scale[n] : 0.0f;
             }
     }
-    wk_store<KEEP, CN, false, EPI>(g, [&](int i, int j) -> const v4i& { return sum[i][j]; }, [&](int i) { return as[i]; },
+    wk_store<ROWS, CN, false, EPI>(g, [&](int i, int j) -> const v4i& { return sum[i][j]; }, [&](int i) { return as[i]; },
                                    [&](int j, int e) { return ws[j][e]; }, m0, pb0, g.M, stage_lds, lane);
 }
 
@@ -857,7 +868,7 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
         if (ksplit > 1) mark(st, "gemm_wk_reduce_kernel");                                          \
         if (ksplit > 1)                                                                             \
             hipLaunchKernelGGL((gemm_wk_reduce_kernel<TM, W4, EPI>),                                \
-                               dim3(mblocks * nblocks * 8), dim3(64), 0, st, g,     \
+                               dim3(mblocks * nblocks * 8 * (TM > 2 ? TM / 2 : 1)), dim3(64), 0, st, g, \
                                mblocks, nblocks, ksplit);                                           \
     } while (0)
     // (a dense SwiGLU GEMM exists for int4 weights only: the w4a8 FFN; the MoE layer's is grouped)

@@ -48,3 +48,15 @@ def test_k_halves_meet_without_a_select_per_accumulator(gemm_kernels):
             assert text.count("v_cndmask") < accumulators / 2, name
             checked += 1
     assert checked >= 20
+
+
+def test_the_reduce_launch_has_a_parts_loads_in_flight_together(gemm_kernels):
+    """A wave adds up to 32 rows x 64 columns of each part of K: eight loads per 32 rows, none of which waits for another."""
+    checked = 0
+    for name, text in gemm_kernels.items():
+        m = re.search(r"gemm_wk_reduce_kernelILi(\d)E", name)
+        if m:
+            up_to_wait = text[text.index("global_load_dwordx4"):].split("vmcnt")[0]
+            assert up_to_wait.count("global_load_dwordx4") == 4 * min(int(m.group(1)), 2), name
+            checked += 1
+    assert checked >= 15

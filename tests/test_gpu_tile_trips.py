@@ -102,3 +102,26 @@ def test_a_result_over_the_rows(sess, oracle):
     finally:
         sess.free_device(buf)
         op.close()
+
+
+# K split over workgroups: the reduce launch takes the 64 rows that a wave of a 128-row tile kept in two halves; rows that end in
+# either half of either wave, at its edges, and with the tile
+@pytest.mark.parametrize("M", [673, 704, 705, 737, 767, 768])
+@pytest.mark.parametrize("kind", [capi.I8I8I32, capi.F16I8F16_DYNAMIC, capi.F32I8F32_DYNAMIC])
+def test_k_split_of_128_row_tiles(sess, oracle, one_piece, M, kind):
+    N, K = 700, 10240
+    assert _route(M, N, K, 0, I32 if kind == capi.I8I8I32 else F16) == (TILES, 128)
+    c = workloads.w8a8_case(M, K, N, seed_w=N, seed_a=M)
+    if kind == capi.I8I8I32:
+        A, scale = np.random.default_rng(M).integers(-128, 128, (M, K)).astype(np.int8), None
+        want = oracle.gemm_i8(A, c["B"])
+    else:
+        A, scale = (c["A"] if kind == capi.F16I8F16_DYNAMIC else workloads.normal_f32(M, (M, K))), c["w_scale"]
+        want = oracle.w8a8(A, c["B"], scale)["C"]
+    op = ops.W8A8Linear(sess, kind, M, c["B"], scale)
+    try:
+        (rc, got), kernels = one_piece(lambda: op.run(A))
+        assert rc == 0 and kernels[-1] == "gemm_wk_reduce_kernel"
+        assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, got.dtype).view(np.uint8))
+    finally:
+        op.close()
