@@ -403,13 +403,6 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
     if constexpr (RS) a_next = asrc + (size_t)(ksteps - 1) * A_STEP;
 
     v4i acc[RM][CN];
-    if constexpr (!RS) {
-#pragma unroll
-        for (int i = 0; i < RM; ++i)
-#pragma unroll
-            for (int j = 0; j < CN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
-    }
-
     v4i a[RM];                  // activation operands
     v4i wring[NSW][CN];         // weights as loaded: of a unit, or, int4, of a step
     [[maybe_unused]] v4i wop[2][CN]; // int4 only: unpacked operands, this unit / next
@@ -565,6 +558,17 @@ __device__ __forceinline__ void wk_tile(const rkh_gemm_args& g, uint8_t* lds_raw
         if (raw_many) {
 #pragma unroll
             for (int t = 1; t < RAW_TILES; ++t) raw_fetch(t);
+        }
+    }
+    // The sums' zeros, while the first loads are on their way.  Named, so that they are written here: the compiler wrote them
+    // behind the wait for the first data, and of a workgroup's small tiles it kept zeros in scratch memory, whose loads
+    // and stores wait among the prologue's.  us: int8 4000 x 1024 x 14336 73.8 -> 72.7, 786 x 661 x 8720 18.9 -> 18.5, 505 x 544 x 8320 12.8 ->
+    // 12.7, int4 2156 x 640 x 2176 13.8 -> 13.6, exact 4007 x 1024 x 9088 58.7 -> 57.5, the FFN 1300 x 512 x 12288 95.2 -> 91.9.
+    if constexpr (!RS) {
+#pragma unroll
+        for (int t = 0; t < RM * CN; ++t) {
+            acc[t / CN][t % CN] = v4i{0, 0, 0, 0};
+            keep(acc[t / CN][t % CN]);
         }
     }
     // weights of unit 0 and the copies of steps 0..G land (RAW: one load or RAW_TILES behind them, the count of one)

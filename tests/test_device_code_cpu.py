@@ -60,3 +60,16 @@ def test_the_reduce_launch_has_a_parts_loads_in_flight_together(gemm_kernels):
             assert up_to_wait.count("global_load_dwordx4") == 4 * min(int(m.group(1)), 2), name
             checked += 1
     assert checked >= 15
+
+
+def test_no_large_tile_kernel_keeps_registers_in_memory(code_objects):
+    """Registers spilled to scratch memory are loads and stores that wait among those of the loop's own."""
+    checked = 0
+    for obj in code_objects:
+        notes = subprocess.run([os.path.join(TOOLS, "llvm-readelf"), "--notes", obj], check=True, capture_output=True, text=True).stdout
+        for entry in notes.split("- .agpr_count:")[1:]:
+            name = re.search(r"\.name:\s+(\w+)", entry).group(1)
+            if "gemm_wk_" in name:
+                assert int(re.search(r"\.private_segment_fixed_size: (\d+)", entry).group(1)) == 0, name
+                checked += 1
+    assert checked >= 39
