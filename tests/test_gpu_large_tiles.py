@@ -7,6 +7,8 @@ of each shape), one and several trips of the unrolled K loop with and without a
 remainder, columns that are no multiple of anything, and every epilogue.  Integer sums and a fixed order of
 the floating-point steps: exact.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -99,3 +101,41 @@ def test_several_tiles_of_a_workgroup(sess, oracle, one_piece, M, N, K, int4):
         op.close()
     assert rc == 0 and kernels[-1] == "gemm_wk_big_kernel"
     assert np.array_equal(got.view(np.uint16), np.asarray(want).view(np.uint16))
+
+
+# Small tiles behind a chain: (workgroups without a large tile in the last round, three small ones each; small ones on the others)
+# 20 of 256 and 22, all of a last strip; 28 and 172, all halves of large tiles
+@pytest.mark.parametrize("M,N,K,big,small,kind", [(1550, 20992, 512, 492, 82, kind) for kind in ("w8 f16", "w8 i32", "w4 f16", "w4 swiglu")] +
+                         [(2968, 12951, 1024, 484, 256, kind) for kind in ("w8 f16", "w8 i32")])
+def test_several_small_tiles_of_a_workgroup(sess, oracle, one_piece, M, N, K, big, small, kind):
+    bits, kind = kind.split()
+    v = [C.c_int() for _ in range(5)]
+    epilogue = {"i32": 0, "f16": 1, "swiglu": 3}[kind]
+    assert capi.load_library().rkh_gemm_route(M, N, K, int(bits == "w4"), epilogue, *[C.byref(x) for x in v]) == 0
+    assert [x.value for x in v[1:]] == [256, 1, big, small]
+    assert small > 3 * (256 - big % 256)  # (more than those without a large one take)
+    if bits == "w4":
+        c = workloads.w4a8_case(M, K, N, seed_w=N, seed_a=M)
+        w, ws = ops.W4A8Weights(sess, c["B"], c["w_scale"]), ops.W4A8Workspace(sess, M, N, K)
+        if kind == "f16":
+            (rc, got), kernels = one_piece(lambda: ws.run_f16(w, c["A"]))
+            want = oracle.w4a8(c["A"], c["B"], c["w_scale"])["C"]
+        else:
+            A32 = oracle.half_to_float(c["A"]).astype(np.float32).reshape(M, K)
+            (rc, got), kernels = one_piece(lambda: ws.run_swiglu_f32(w, A32))
+            want = oracle.w4a8_swiglu(A32, c["B"], c["w_scale"])["middle"]
+        ws.close()
+        w.close()
+    else:
+        c = workloads.w8a8_case(M, K, N, seed_w=M, seed_a=K)
+        if kind == "f16":
+            op, A = ops.W8A8Linear(sess, capi.F16I8F16_DYNAMIC, M, c["B"], c["w_scale"]), c["A"]
+            want = oracle.w8a8(A, c["B"], c["w_scale"])["C"]
+        else:
+            A = np.random.default_rng(M).integers(-128, 128, (M, K)).astype(np.int8)
+            op = ops.W8A8Linear(sess, capi.I8I8I32, M, c["B"])
+            want = oracle.gemm_i8(A, c["B"])
+        (rc, got), kernels = one_piece(lambda: op.run(A))
+        op.close()
+    assert rc == 0 and kernels[-1] == "gemm_wk_big_kernel"
+    assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want, got.dtype).view(np.uint8))
