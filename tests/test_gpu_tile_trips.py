@@ -86,19 +86,55 @@ def test_rows_as_given(sess, oracle, M, N, K, rows, offset):
         op.close()
 
 
+# The tiles that such a call owes its workspace, 9 .. 32 to a workgroup: two, three and four to a wave, up to the most that a
+# wave takes; beyond it the rows are re-tiled by a launch of their own
+@pytest.mark.parametrize("M,N,K,rows,share", [(600, 500, 752, 64, 12), (600, 500, 1040, 64, 20), (600, 500, 1792, 64, 28), (600, 500, 2048, 64, 32),
+                                              (600, 384, 1536, 64, 32), (600, 500, 2064, 64, 36), (300, 4096, 14336, 64, 28),
+                                              (2500, 1000, 752, 128, 12), (2500, 1000, 1264, 128, 20), (2500, 1000, 1792, 128, 28),
+                                              (2500, 1000, 2048, 128, 32), (2500, 1000, 2064, 128, 36)])
+def test_tiles_owed_to_the_workspace(sess, oracle, M, N, K, rows, share):
+    assert _route(M, N, K, 0, I32) == (NARROW, rows)
+    assert -(-(rows // 32 * ((K + 255) // 256 * 8)) // -(-N // 128)) == share
+    rng = np.random.default_rng(K)
+    B = rng.integers(-128, 128, (K, N)).astype(np.int8)
+    op = ops.W8A8Linear(sess, capi.I8I8I32, M, B)
+    dA, dC = sess.empty_device(M * K), sess.empty_device(M * N * 4)
+    try:
+        for _ in range(2):  # (the second call's rows take the place of the first one's)
+            A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+            assert sess.lib.rk_npu_hip_upload(sess.ctx, dA, capi.ptr(A), A.nbytes) == 0
+            kernels = [name for name, _ in ops.profile_kernels(sess, lambda: op.run_device(dA, dC), iters=1, warmup=0)]
+            assert ("quant_rows_kernel" in kernels) == (share > 32), kernels
+            want = oracle.gemm_i8(A, B)
+            assert np.array_equal(sess.from_device(dC, (M, N), np.int32), want)
+            q = np.empty((M, K), np.int8)
+            assert sess.lib.rk_npu_matmul_workspace_read_quantized(op.ws, capi.ptr(q), None) == 0
+            assert np.array_equal(q, A)
+        assert sess.lib.rk_npu_matmul_workspace_rerun_gemm_device(op.ws, op.w, dC) == 0 and sess.sync() == 0
+        assert np.array_equal(sess.from_device(dC, (M, N), np.int32), want)
+    finally:
+        sess.free_device(dA)
+        sess.free_device(dC)
+        op.close()
+
+
 def test_a_result_over_the_rows(sess, oracle):
-    """The result may be written over the rows it is made of: they are copied first then."""
+    """The result may be written over the rows it is made of: they are copied first then, down to 16 common bytes on
+    either side, and are not where one ends as the other begins.  (The values alone would not show it: the few
+    workgroups of this size read all their rows before any of them writes.)"""
     M, N, K = 129, 4100, 512
     rng = np.random.default_rng(7)
     A, B = rng.integers(-128, 128, (M, K)).astype(np.int8), rng.integers(-128, 128, (K, N)).astype(np.int8)
     op = ops.W8A8Linear(sess, capi.I8I8I32, M, B)
     want = oracle.gemm_i8(A, B)
-    buf = sess.empty_device(M * N * 4 + 4096)
+    a, c = A.nbytes, M * N * 4
+    buf = sess.empty_device(a + c)
     try:
-        for offset in (0, 1024):
-            assert sess.lib.rk_npu_hip_upload(sess.ctx, buf + offset, capi.ptr(A), A.nbytes) == 0
-            assert op.run_device(buf + offset, buf) == 0 and sess.sync() == 0
-            assert np.array_equal(sess.from_device(buf, (M, N), np.int32), want)
+        for rows_at, result_at, apart in ((0, 0, False), (1024, 0, False), (0, a - 16, False), (c - 16, 0, False), (0, a, True), (c, 0, True)):
+            assert sess.lib.rk_npu_hip_upload(sess.ctx, buf + rows_at, capi.ptr(A), a) == 0
+            kernels = [name for name, _ in ops.profile_kernels(sess, lambda: op.run_device(buf + rows_at, buf + result_at), iters=1, warmup=0)]
+            assert ("quant_rows_kernel" in kernels) == (not apart), (rows_at, result_at, kernels)
+            assert np.array_equal(sess.from_device(buf + result_at, (M, N), np.int32), want)
     finally:
         sess.free_device(buf)
         op.close()
