@@ -1489,7 +1489,7 @@ static long dense_tiles(int M, int N, int bm) { return (long)((M + bm - 1) / bm)
 // on the device, and, for a split, the second launch and the int32 partial tiles written and read
 // back; the coefficients are a least-squares fit to measured times (int8, fp16 in / out, 4096 x 4096,
 // 4096 x 11008, 11008 x 4096, 4096 x 14336 at 192 to 1024 rows, nine forced plans each: the fit
-// picks the fastest or second-fastest plan for all of them).  Against the earlier rule (shrink
+// picks the fastest or second-fastest plan for all of them; loops of 32x32x32 products, which were a tenth slower).  Against the earlier rule (shrink
 // the tile until 160 tiles exist, then split): K = 11008, N = 4096 at 192 / 256 / 512 / 1024 rows
 // 50.0 -> 33.5, 53.9 -> 44.9, 71.7 -> 55.0, 82.6 -> 78.4 us; 4096 x 11008 at 192 rows 36.6 -> 31.0.
 static DensePlan dense_plan(int M, int N, int K, int w_int4) {
@@ -1548,6 +1548,8 @@ static DensePlan effective_plan(int M, int N, int K, int w_int4) {
 //         M 128, K 4096, N 14336: 20.9 vs 20.9
 //   int4  M 64, 2048 x 2048:  9.9 vs 14.1   M 128, 4096 x 4096: 11.9 vs 19.4   M 128, K 14336, N 4096: 22.2 vs 25.7
 //         M 32, K 4096, N 14336: 11.4 vs 18.4
+// (The large-tile kernel's times here and below are those of its 32x32x32 products and, for exact results on narrow
+// tiles, of a re-tiling launch in front that they no longer have; the lines have not been drawn anew.)
 // From about 160 rows on the large tile wins for wide N (each row block streams
 // the weights again).  The same holds earlier for the gate/up + SwiGLU GEMM of
 // an FFN, whose N is twice as wide: the whole FFN (4096 -> 14336 -> 4096, weights
@@ -1607,7 +1609,8 @@ static bool dense_streams(const rkh_gemm_args& g) {
 // other plans with int4 weights; those instantiations are gone.)  It loses where the tiles outnumber
 // the compute units (int8 4096 x 4096 at 768 rows 30.8 -> 31.9, 4096 x 14336 at 512 rows 41 -> 68; int4
 // 4096 x 11008 at 160 rows, 258 tiles: 20.6 -> 23.2) and for a long K on few tiles (below), which is where the
-// rule stops.  RK_NPU_HIP_NARROW_TILES = 0 switches it off,
+// rule stops.  (All of these are times of 32x32x32 products, and exact results then had a re-tiling launch in front; the
+// lines have not been drawn anew.)  RK_NPU_HIP_NARROW_TILES = 0 switches it off,
 // 1 forces it (2: the 128-row tiles below) for every dense GEMM beyond the streaming kernel's rows that
 // needs no K split (tuning aid).
 static int dense_narrow(const rkh_gemm_args& g) { // rows of the tile, or 0: another plan

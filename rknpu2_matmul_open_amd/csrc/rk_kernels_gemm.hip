@@ -8,11 +8,12 @@ namespace {
 // ---- tiles of (32 * TM) rows x (128 * TN) columns ------------------------------
 // v_mfma_i32_16x16x64_i8.  Large launches run at the clock that the power limit leaves, so energy per product
 // is what counts: a loop of nothing but MFMAs on quantized activations (codes of N(0, 2.5) with outliers) and
-// N(0, 30) weights reaches 3.53 POP/s with 32x32x32 and 4.19 with 16x16x64 (int4 weights as 16 * code: 3.77 and 4.67),
-// presumably because an instruction moves half the accumulator bytes per product.  Calls with quantization, us, from
-// 32x32x32 with each sub-step's loads issued together to this loop, one box: int4 2048 x 4096 x 4096 39.1 -> 34.8, 4096^3
-// 68.5 -> 59.5, int8 4096 x 4096 x 14336 202 -> 190, 1000 x 4096 x 4096 26.2 -> 24.2; int4 512 x 14336 x 4096 40.0 -> 36.3,
-// the FFN 4096 -> 14336 -> 4096 of 128 / 512 rows 42.6 -> 40.8 / 102 -> 94.
+// N(0, 30) weights reaches 3.53 POP/s with 32x32x32 and 4.19 with 16x16x64 (int4 weights as 16 * code: 3.77 and 4.67).
+// Calls with quantization, us, from the kernel of 32x32x32 products whose sub-steps issued their loads together to this one, one
+// box, two sets of operands in turn (partly from the last-level cache): int4 2048 x 4096 x 4096 38.3 -> 33.2, 4096^3 67.1 -> 59.4, 512 x
+// 14336 x 4096 36.9 -> 33.4, int8 4096 x 4096 x 14336 205 -> 188, 1000 x 4096 x 4096 26.3 -> 23.0, the FFN 4096 -> 14336 -> 4096 of
+// 128 / 512 rows 42.7 -> 39.6 / 101 -> 94 (weights from memory: 48.7 -> 47.3 / 105 -> 98).  Of 260 shapes drawn from 65 - 4096
+// rows, 512 - 14336 columns and k one that this kernel serves is slower beyond the noise of three runs: int8 1241 x 13825 x 1152 71.1 -> 71.25.
 //
 // Eight waves = 4 column groups (wn) x 2.  In the tiles of up to 128 rows the two waves of a column group
 // split K (k-half wk): each accumulates all rows x 32 * TN columns over every second 128 k, and the halves are
@@ -234,8 +235,8 @@ template <int OFF> __device__ __forceinline__ void load_regs(v4i& x, unsigned la
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(x) : "v"(lane_off), "s"(base), "n"(OFF));
 }
 __device__ __forceinline__ void load_far(v4i& x, const uint8_t* src) { asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(x) : "v"(src)); }
-// The product as an asm statement, for the chained tiles: sums stay in one place (left to itself the compiler rotates 128
-// sums through the register file, and with the next tile's weights beside them spills some around the tile's first products).
+// The product as an asm statement, for the chained tiles: sums stay in one place (of products that it knows the compiler rotated 128
+// sums through the register file, and with the next tile's weights beside them spilled some around the tile's first products).
 // What the compiler then does not order: a vector instruction that writes an operand has to be two wait states ahead
 // of the product -- the weights are unpacked well ahead --, and one that reads a sum waits for the last products, settle().
 // The build checks both in the compiled code (audit_waits.py).
@@ -328,7 +329,8 @@ struct WkChain { int v, stride, big, mblocks, nblocks; };
 // rows of an operand, which are a multiple of 128 bytes apart, are read from 16 different places.  The tiles that the call owes its
 // caller (g.A) are written by the workgroups of a row block together, up to RAW_TILES per wave: fetched behind the
 // prologue, stored behind the loop.  Without the re-tiling launch in front, us: exact
-// 128 x 4096 x 11008 13.6 -> 11.8, 512 x 4096 x 4096 15.3 -> 12.8, 1000 x 2048 x 4096 15.4 -> 13.1, 300 x 14336 x 4096 38.2 -> 33.6.
+// 128 x 4096 x 11008 13.6 -> 11.8, 512 x 4096 x 4096 15.3 -> 12.8, 1000 x 2048 x 4096 15.4 -> 13.1, 300 x 14336 x 4096 38.2 -> 33.6 (and 11.6, 13.0,
+// 12.4 and 33.5 since the k-halves meet in branches and the zeros are written early, another box).
 constexpr int RAW_TILES = 4;
 
 template <int TM, bool W4, int EPI, int TN, bool RS, bool RAW = false>
@@ -732,9 +734,11 @@ __global__ __launch_bounds__(512) void gemm_wk_kernel(const uint8_t* h_A, const 
 // last strip of at most 128 rows.  Workgroup = 8 waves in 4 column groups x 2 row halves: a wave multiplies
 // 128 x 64 over the whole K, so there is no exchange of k-halves and all eight waves convert and store.
 // What bounds it: the matrix pipes at the clock that the power limit leaves, and the conversion and stores of a tile.
-// A workgroup per compute unit multiplies its tiles one after the other as one stream of steps (wk_tile, RS), so that only its first
-// tile waits for memory: int8 4000 x 1024 x 14336 77.9 -> 73.2 us, 4000 x 512 x 14336 67.3 -> 62.4, 4096 x 4096 x 14336 187 -> 184;
-// a launch of one round measures the same.
+// A workgroup per compute unit multiplies its tiles one after the other as one stream of steps (wk_tile, RS), so that the first
+// operands of every tile but its first are in LDS and registers when the tile before has been stored (its first wait for
+// weights, two units later, stands behind that tile's 16 or 32 stores, which the counter counts too): int8 4000 x 1024 x 14336
+// 77.9 -> 73.2 us, 4000 x 512 x 14336 67.3 -> 62.4, 4096 x 4096 x 14336 187 -> 184; a launch of one round measures the same.  The small tiles behind a chain
+// start with a round trip to memory each.
 // Against 128 x 256 tiles: the second operand of a column group comes once per 256 rows (16 instead of 24 KB from L2 per 512
 // cycles of MFMAs), one prologue and one epilogue per 256 rows.  us, quantization included, when the tiles were
 // introduced: int8 4096 x 4096 x 14336 241 -> 203, 2048 x 4096 x 14336 122 -> 108, 4096^3 74.7 -> 68.1; int4 214 -> 195, 75 -> 69.
@@ -889,19 +893,23 @@ int launch_gemm_wk(hipStream_t st, const rkh_gemm_args& g, int ksplit) {
 }
 
 // How a dense launch is cut into 256 x 256 tiles (the first `big`, in tile order) and 128 x 256 ones, and
-// the microseconds to expect.  A 256 x 256 tile costs 9 us beside its loop, a 128 x 256 one 8 (time stamps:
-// prologue 2.5, epilogue and stores 5 - 6, the next workgroup's start 0.6), so one big tile is cheaper
+// the microseconds to expect.  A 256 x 256 tile costs 9 us beside its loop, a 128 x 256 one 8 (time stamps of tiles that were
+// a workgroup each: prologue 2.5, epilogue and stores 5 - 6, the next workgroup's start 0.6), so one big tile is cheaper
 // than two small ones (K = 4096: 58 against 2 x 33 us, int8 weights) but leaves more compute units idle in
 // the last round: the tiles of that round go as halves where that ends sooner.
+// The model is older than the kernels: every tile of a chain is charged the start that only the first one has, and the loop's
+// times are those of 32x32x32 products.  Against forced plans (128 / 64 / 32-row tiles, one and two parts of K, narrow tiles) on
+// 46 shapes of 64 - 4096 rows, int8, int4 and exact results, the dispatch as a whole is fastest or within 1 % on 43; behind by 3.0 %
+// at int4 400 x 14336 x 2048 (narrow tiles), 5.6 % at int8 3000 x 1024 x 9000 (128 x 128 tiles), 16 % at exact 300 x 4096 x 11008 (128 x 256).
+// (A forced 256:1 is cut by this function too, so the cut itself is compared with nothing.)
 // `rounds`: small tiles that a compute unit without one of the last round's big tiles multiplies; the rest go to the others.
 struct BigPlan { int big, small, rounds; double us, us_128; };
 static BigPlan big_plan(int M, int N, int K, int w_int4) {
     const int cus = compute_units() > 0 ? compute_units() : 256;
     const int nblocks = (N + 255) / 256, strip = M % 256 > 0 && M % 256 <= 128;
     const int tiles = (M / 256 + (M % 256 > 128)) * nblocks;
-    // microseconds per 64 k of a 128 x 256 tile with every compute unit at work, at the clock that the power limit leaves.
-    // (Times of the loop on 32x32x32 products, a tenth longer throughout than now; what decides is their ratio to the fixed
-    // part, and forced plans are ahead of this choice nowhere: 23 dense shapes of 160 - 1500 rows and six of the FFN, all within 2 %.)
+    // microseconds per 64 k of a 128 x 256 tile with every compute unit at work, at the clock that the power limit leaves
+    // (32x32x32 products, a tenth longer than now)
     const double loop = (w_int4 ? 0.35 : 0.39) * (rkh_align_up(K, RKH_K_ALIGN) / 64);
     const double t_big = 2 * loop + 9.0, t_small = loop + 8.0;
     BigPlan best{0, 0, 0, 1e30, (((M + 127) / 128) * (long)nblocks + cus - 1) / cus * t_small};
